@@ -80,7 +80,7 @@ def draw(rng):
             if rng.random() < 0.75:                       # hidden sizes are usually multiples of 64
                 m, n = m // 64 * 64, n // 64 * 64
             return dict(path=path, kernel="gemv", m=m, n=n, bpw=bpw, rows=_log_int(rng, 1, 16), dtype=dtype)
-        m, n = _log_int(rng, 1024, 16384) // 32 * 32, _log_int(rng, 1024, 16384) // 256 * 256
+        m, n = _log_int(rng, 1024, 13824) // 32 * 32, _log_int(rng, 1024, 13824) // 256 * 256
         return dict(path=path, kernel="gemm", m=m, n=n, bpw=bpw, rows=_log_int(rng, 128, 4096), dtype=dtype)
     if path == "decode_layers":
         return dict(path=path, model=small, layers=rng.randint(4, 9), bpw=bpw, rows=_log_int(rng, 1, 16), dtype=dtype)
