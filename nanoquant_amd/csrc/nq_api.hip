@@ -65,55 +65,43 @@ int nq_gemv_forward(const void* x, const void* s_in, const uint32_t* vt_bits, co
     return nq_gemv_forward_bias(x, s_in, vt_bits, s_mid, u_bits, s_out, nullptr, h_scratch, y, batch, n, r, m, dtype, stream);
 }
 
-// Both stages of every linear for `batch` rows.  Groups of independent linears in pieces of 1, 2 and 4 batch rows go
-// through nq::gemv_fused (two launches per nq::gemv_fused_max() linears, or one with `one_launch`); a single linear,
-// and pieces of 8 and 16 rows, take two launches per linear.
+// First and second stage of linear l for batch rows [done, done + piece).  The h of a piece sits in l.h as 16-bit values.
+static void linear_stages(const nq_linear& l, int done, nq::RowsStage* first, nq::RowsStage* second) {
+    const int hs = nq::gemv_rows_h_stride(l.r);
+    float* h = l.h + (size_t)done * l.r;
+    *first = nq::RowsStage{l.vt_bits, (const char*)l.x + (size_t)done * l.n * 2, l.s_in, l.s_mid, nullptr, nullptr, h,
+                           l.r, words_of(l.n), l.n, l.n, hs, 2};
+    *second = nq::RowsStage{l.u_bits, h, nullptr, l.s_out, l.bias, nullptr, (char*)l.y + (size_t)done * l.m * 2,
+                            l.m, words_of(l.r), hs, hs, l.m, 0};
+}
+
+// Both stages of every linear for `batch` rows, in pieces of 16 rows: two launches (all first stages, all second stages)
+// per nq::gemv_rows_group_max() linears, or one with `one_launch`.
 static int forward_linears(const nq_linear* ls, int count, int batch, int dtype, bool one_launch, hipStream_t st) {
-    const int group = nq::gemv_fused_max();
-    int done = 0;
-    while (done < batch) {
-        int piece = 16;
-        while (piece > batch - done) piece >>= 1;
-        if (piece >= 8 || (count == 1 && !one_launch)) {
-            for (int i = 0; i < count; ++i) {
-                const nq_linear& l = ls[i];
-                if (l.m == 0) continue;
-                const char* x = (const char*)l.x + (size_t)done * l.n * 2;
-                float* h = l.h + (size_t)done * l.r;
-                char* y = (char*)l.y + (size_t)done * l.m * 2;
-                hipError_t e = nq::gemv_stage(dtype, true, l.vt_bits, x, l.s_in, l.s_mid, nullptr, h, true, piece, l.r,
-                                              words_of(l.n), l.n, l.n, l.r, st);
-                if (e != hipSuccess) return hip_status(e);
-                e = nq::gemv_stage(dtype, false, l.u_bits, h, nullptr, l.s_out, nullptr, y, false, piece, l.m,
-                                   words_of(l.r), l.r, l.r, l.m, st, l.bias);
-                if (e != hipSuccess) return hip_status(e);
+    constexpr int kMax = 16;
+    const int group = nq::gemv_rows_group_max() < kMax ? nq::gemv_rows_group_max() : kMax;
+    for (int done = 0; done < batch; done += 16) {
+        const int piece = std::min(16, batch - done);
+        for (int i0 = 0; i0 < count;) {
+            nq::RowsStage a[kMax], b[kMax];
+            int k = 0;
+            bool all_ranks = true;
+            for (; i0 < count && k < group; ++i0) {
+                if (ls[i0].m == 0) continue;
+                linear_stages(ls[i0], done, &a[k], &b[k]);
+                if (ls[i0].r == 0) all_ranks = false;
+                ++k;
             }
-        } else {
-            for (int i0 = 0; i0 < count; i0 += group) {
-                const int c = count - i0 < group ? count - i0 : group;
-                const void *x[16], *s_in[16], *s_mid[16], *s_out[16], *bias[16];
-                const uint32_t *vt[16], *u[16];
-                float* h[16];
-                void* y[16];
-                int n[16], r[16], m[16];
-                int k = 0;
-                for (int i = i0; i < i0 + c; ++i) {
-                    const nq_linear& l = ls[i];
-                    if (l.m == 0) continue;
-                    x[k] = (const char*)l.x + (size_t)done * l.n * 2;
-                    h[k] = l.h + (size_t)done * l.r;
-                    y[k] = (char*)l.y + (size_t)done * l.m * 2;
-                    s_in[k] = l.s_in; s_mid[k] = l.s_mid; s_out[k] = l.s_out; bias[k] = l.bias;
-                    vt[k] = l.vt_bits; u[k] = l.u_bits;
-                    n[k] = l.n; r[k] = l.r; m[k] = l.m;
-                    ++k;
-                }
-                if (k == 0) continue;
-                hipError_t e = nq::gemv_fused(dtype, k, piece, x, s_in, vt, s_mid, u, s_out, bias, h, y, n, r, m, one_launch, st);
-                if (e != hipSuccess) return hip_status(e);
+            if (k == 0) continue;
+            hipError_t e;
+            if (one_launch && all_ranks) {
+                e = nq::gemv_rows_fused(dtype, k, a, b, piece, st);
+            } else {
+                e = nq::gemv_rows(dtype, true, k, a, piece, st);
+                if (e == hipSuccess) e = nq::gemv_rows(dtype, false, k, b, piece, st);
             }
+            if (e != hipSuccess) return hip_status(e);
         }
-        done += piece;
     }
     return NQ_OK;
 }
@@ -131,7 +119,7 @@ int nq_gemv_forward_bias(const void* x, const void* s_in, const uint32_t* vt_bit
     return forward_linears(&l, 1, batch, dtype, false, (hipStream_t)stream);
 }
 
-int nq_gemv_group_max(void) { return nq::gemv_fused_max(); }
+int nq_gemv_group_max(void) { return nq::gemv_rows_group_max(); }
 
 int nq_gemv_forward_group(const nq_linear* linears, int count, int batch, int dtype, int one_launch, void* stream) {
     if (dtype != NQ_F16 && dtype != NQ_BF16) return NQ_ERR_DTYPE;
@@ -219,15 +207,38 @@ int nq_gemv_mixture(const void* x, const void* const* s_in, const uint32_t* cons
     }
     if (batch == 0 || m == 0) return NQ_OK;
     hipStream_t st = (hipStream_t)stream;
-    for (int t = 0; t < nterms; ++t) {
-        hipError_t e = nq::gemv_stage(dtype, true, vt_bits[t], x, s_in[t], s_mid[t], nullptr, h_scratch, true,
-                                      batch, r[t], words_of(n), n, n, r[t], st);
-        if (e != hipSuccess) return hip_status(e);
-        const bool last = (t == nterms - 1);
-        // Partial sums over terms stay in fp32; only the last term rounds to the activation type.
-        e = nq::gemv_stage(dtype, false, u_bits[t], h_scratch, nullptr, s_out[t], t ? y_scratch : nullptr,
-                           last ? y : (void*)y_scratch, !last, batch, m, words_of(r[t]), r[t], r[t], m, st);
-        if (e != hipSuccess) return hip_status(e);
+    int max_r = 0;
+    for (int t = 0; t < nterms; ++t) max_r = std::max(max_r, r[t]);
+    for (int done = 0; done < batch; done += 16) {
+        const int piece = std::min(16, batch - done);
+        const char* xp = (const char*)x + (size_t)done * n * 2;
+        char* yp = (char*)y + (size_t)done * m * 2;
+        float* yacc = nterms > 1 ? y_scratch + (size_t)done * m : nullptr;
+        // Two terms at a time where their two 16-bit h fit the [batch, max r] fp32 scratch: both first stages in one
+        // launch, then one launch that adds the two second stages.  Partial sums over further terms stay in fp32; only
+        // the last launch rounds to the activation type.
+        for (int t = 0; t < nterms;) {
+            nq::RowsStage a[2], b[2];
+            size_t used = 0;
+            int k = 0;
+            for (; k < 2 && t + k < nterms; ++k) {
+                const int rt = r[t + k], hs = nq::gemv_rows_h_stride(rt);
+                const size_t bytes = ((size_t)piece * hs * 2 + 15) / 16 * 16;
+                if (k > 0 && used + bytes > (size_t)piece * max_r * 4) break;
+                void* h = (char*)h_scratch + used;
+                used += bytes;
+                a[k] = nq::RowsStage{vt_bits[t + k], xp, s_in[t + k], s_mid[t + k], nullptr, nullptr, h, rt, words_of(n), n, n, hs, 2};
+                b[k] = nq::RowsStage{u_bits[t + k], h, nullptr, s_out[t + k], nullptr, nullptr, nullptr, m, words_of(rt), hs, hs, m, 0};
+            }
+            const bool last = t + k == nterms;
+            b[0].addend = t ? yacc : nullptr;
+            b[0].out = last ? (void*)yp : (void*)yacc;
+            b[0].out_kind = last ? 0 : 1;
+            hipError_t e = nq::gemv_rows(dtype, true, k, a, piece, st);
+            if (e == hipSuccess) e = k == 2 ? nq::gemv_rows_sum2(dtype, b, piece, st) : nq::gemv_rows(dtype, false, 1, b, piece, st);
+            if (e != hipSuccess) return hip_status(e);
+            t += k;
+        }
     }
     return NQ_OK;
 }
@@ -238,8 +249,13 @@ int nq_gemv_stage(const void* in, const void* s_col, const uint32_t* bits, const
     if (batch < 0 || cols < 0 || rows < 0) return NQ_ERR_SHAPE;
     if (batch == 0 || rows == 0) return NQ_OK;
     if (!in || !bits || !out) return NQ_ERR_NULL;
-    return hip_status(nq::gemv_stage(dtype, true, bits, in, s_col, s_row, nullptr, out, false, batch, rows,
-                                     words_of(cols), cols, cols, rows, (hipStream_t)stream));
+    for (int done = 0; done < batch; done += 16) {
+        const nq::RowsStage st{bits, (const char*)in + (size_t)done * cols * 2, s_col, s_row, nullptr, nullptr,
+                               (char*)out + (size_t)done * rows * 2, rows, words_of(cols), cols, cols, rows, 0};
+        hipError_t e = nq::gemv_rows(dtype, s_col != nullptr, 1, &st, std::min(16, batch - done), (hipStream_t)stream);
+        if (e != hipSuccess) return hip_status(e);
+    }
+    return NQ_OK;
 }
 
 // ---- run list ---------------------------------------------------------------------------------

@@ -1,35 +1,13 @@
-// Shared device code of the matmul-free decode stages: staging of the (scaled) input vector in LDS
+// Shared device code of the run-list kernel: staging of the (scaled) input vector in LDS
 // and the arithmetic of one 16-byte unit of packed signs (4 words = 128 columns of one row).
 //
-// LDS layout of the staged input (per batch row b): 16-byte chunk (b, i, cu) at
-// xs[xs_chunk(b, i, upad, cu)] = xs[b*(16*upad+1) + i*upad + cu] holds the 8 consecutive columns 128*(c0+cu) + 8*i .. +7 as 16-bit values;
-// upad is odd.  For a fixed i the lanes of a row read consecutive chunks (conflict-free) and lanes of
-// different rows read the same chunk (broadcast).  xsum[b*upad + cu] is the fp32 sum of the 128
-// staged values of unit cu.
-//
-// Arithmetic, fp16.  The packed "half2" order puts the signs of the element pair j (j = 0..15) of a
-// word at bits 15-j and 31-j, i.e. at the same position of both 16-bit halves.  A 16-bit pattern with
-// only bit p set is itself a valid fp16 number when p is one of the exponent bits 10..14: its value
-// is 2^-14, 2^-13, 2^-11, 2^-7, 2^+1.  So `word & mask_p` IS the operand pair (b_lo*c_p, b_hi*c_p)
-// with b the packed bits, and one v_dot2_f32_f16 adds c_p * (b_lo*x_lo + b_hi*x_hi) to an fp32
-// accumulator of class p.  Three shifted copies of the word (>>1, <<5, <<10) bring every one of the
-// 16 pair positions onto an exponent bit, which makes 3 shifts + 16 ANDs + 16 dot2 per word instead
-// of a shift, a mask and an OR per pair.  All scalings are powers of two and the products of two fp16
-// numbers are exact in fp32, so sum_c acc_c / c_p = sum b*x exactly as accumulated, and the signed
-// sum follows from  sum (1-2b) x = sum x - 2 sum b x  with sum x taken from xsum.
-//
-// bf16 has no such luck (its single exponent bits reach 2^-126, which underflows fp32 products), so
-// the bf16 path keeps the +-1 operand: ((word << j) & 0x80008000) | (1.0, 1.0).
+// A staged unit (128 columns = 64 pairs P = 0..63, pair P = columns 2P, 2P+1) is kept pair-major: its 16-byte chunk
+// j = P & 15 holds pair j of each of the four 32-column words (dword wi = P >> 4), the order in which one sign-bit
+// position of the four words of a unit addresses the columns; chunks are stored unit by unit, batch row by batch row.
 #pragma once
 #include "nq_common.h"
 
 namespace nq {
-
-constexpr int kXsumStride = 576;   // floats of unit sums per batch row: >= largest staged chunk (| 1), multiple of 4
-
-__device__ __forceinline__ uint32_t comp_d(const uint4& v, int i) {
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
 
 // Description of a stage input as the staging code sees it.
 struct StageInput {
@@ -58,60 +36,23 @@ constexpr uint32_t kPastEnd = 0x7FFFFFF0u;
 constexpr int kCacheDefault = 0;
 constexpr int kCacheAgentCoherent = 16;   // sc1: served coherently at device scope, not from this XCD's L2
 
-// Two LDS layouts of a staged unit (128 columns = 64 pairs P = 0..63, pair P = columns 2P, 2P+1):
-//   chunk-major (PM = false): 16-byte chunk i = P >> 2 holds pairs 4i..4i+3 = 8 consecutive columns;
-//   pair-major  (PM = true):  16-byte chunk j = P & 15 holds pair j of each of the four 32-column words
-//                             (dword wi = P >> 4), the order in which one sign-bit position of the
-//                             four words of a unit addresses the columns; chunks are stored unit by unit.
-// Returns the dword index into xs.
-// 16-byte chunk index of (batch row b, chunk i, unit cu).  The batch-row pitch 16*upad + 1 chunks is
+// 16-byte chunks of staged input for `batch` rows of `upad` units (odd).  The batch-row pitch 16*upad + 1 chunks is
 // 4 dwords off a multiple of 64: the 16 lanes of an MFMA operand read that differ only in the batch row
 // fall into 16 different bank groups (a pitch of 16*upad chunks puts all of them into the same one).
-__device__ __forceinline__ int xs_chunk(int b, int i, int upad, int cu) { return b * (16 * upad + 1) + i * upad + cu; }
-// chunks of staged input for `batch` rows
 __host__ __device__ constexpr int xs_chunks(int batch, int upad) { return batch * (16 * upad + 1); }
 
-// Pair-major chunks are stored unit by unit (chunk j of unit cu at b*pitch + 16*cu + j): the 16 reads of
-// one unit differ by compile-time offsets.
+// Chunk j of unit cu of batch row b: the 16 reads of one unit differ by compile-time offsets.
 __device__ __forceinline__ int xs_chunk_pm(int b, int j, int upad, int cu) { return b * (16 * upad + 1) + 16 * cu + j; }
 
-template <bool PM>
-__device__ __forceinline__ int xs_dword(int b, int P, int upad, int cu) {
-    if constexpr (PM) return xs_chunk_pm(b, P & 15, upad, cu) * 4 + (P >> 4);
-    else return xs_chunk(b, P >> 2, upad, cu) * 4 + (P & 3);
-}
-
-// Stores the 8 consecutive 16-bit values r[0..7] of chunk i (columns 8i..8i+7) of unit cu.
-template <bool PM>
-__device__ __forceinline__ void store_chunk(uint4* xs, int b, int i, int upad, int cu, const uint16_t (&r)[8]) {
-    if constexpr (PM) {
-        uint32_t* xd = (uint32_t*)xs;
+// Stores the 8 consecutive 16-bit values (columns 8i..8i+7 of unit cu) as 4 packed pairs.
+__device__ __forceinline__ void store_pairs(uint4* xs, int b, int i, int upad, int cu, const uint32_t (&rp)[4]) {
+    uint32_t* xd = (uint32_t*)xs;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) xd[xs_dword<true>(b, 4 * i + k, upad, cu)] = (uint32_t)r[2 * k] | ((uint32_t)r[2 * k + 1] << 16);
-    } else {
-        uint4 pk;
-        pk.x = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
-        pk.y = (uint32_t)r[2] | ((uint32_t)r[3] << 16);
-        pk.z = (uint32_t)r[4] | ((uint32_t)r[5] << 16);
-        pk.w = (uint32_t)r[6] | ((uint32_t)r[7] << 16);
-        xs[xs_chunk(b, i, upad, cu)] = pk;
+    for (int k = 0; k < 4; ++k) {
+        const int P = 4 * i + k;
+        xd[xs_chunk_pm(b, P & 15, upad, cu) * 4 + (P >> 4)] = rp[k];
     }
 }
-
-// The same with the 8 values as 4 packed pairs.
-template <bool PM>
-__device__ __forceinline__ void store_chunk_packed(uint4* xs, int b, int i, int upad, int cu, const uint32_t (&rp)[4]) {
-    if constexpr (PM) {
-        uint32_t* xd = (uint32_t*)xs;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) xd[xs_dword<true>(b, 4 * i + k, upad, cu)] = rp[k];
-    } else {
-        xs[xs_chunk(b, i, upad, cu)] = make_uint4(rp[0], rp[1], rp[2], rp[3]);
-    }
-}
-
-// Staging variants below: `xsum` (may be null) receives the per-unit sums, `xtot` (may be null) the sum over all staged units per batch row
-// (LDS float atomics; the caller zeroes it and puts a barrier before and after).
 
 // it / n for 0 <= it < 2^23 with rcp = 1.f / n: the float product is off by one at most (the compiler's exact 32-bit
 // division costs some 25 lane instructions, as much as the rest of a staged chunk).
@@ -123,162 +64,10 @@ __device__ __forceinline__ int small_div(int it, int n, float rcp) {
     return q;
 }
 
-// Coherent fp32 input (the intermediate h written by other workgroups of this launch): 16-byte
-// device-coherent loads, kBurst per lane in flight before the first is consumed (a round trip to the
-// memory side costs about a microsecond; 256 lanes x 4 loads cover 4096 values in one round trip).
-// One lane holds 4 consecutive values = 2 pairs; the 128 values of a unit sit in 32 consecutive lanes.
-// Requires K % 4 == 0 and 16-byte aligned rows.
-template <int DT, int BATCH, bool PM>
-__device__ __forceinline__ void stage_units_coherent(uint4* xs, float* xsum, float* xtot, const StageInput& st, int c0,
-                                                     int cu_n, int upad, int nthreads) {
-    using E = Elem<DT>;
-    constexpr int kBurst = 4;
-    const int nquads = cu_n * 32;
-    const int total = BATCH * nquads;
-    const __amdgpu_buffer_rsrc_t rsrc =
-        raw_buffer(st.in, (uint32_t)(((size_t)(BATCH - 1) * st.in_stride + st.K) * sizeof(float)));
-    const float rcp = 1.f / (float)nquads;
-#pragma unroll 1
-    for (int it0 = threadIdx.x; it0 < total; it0 += nthreads * kBurst) {   // wave-uniform trip count: it0 - lane
-        u32x4_t raw[kBurst];
-        int bq[kBurst];
-#pragma unroll
-        for (int j = 0; j < kBurst; ++j) {
-            const int it = it0 + j * nthreads;
-            const int b = small_div(it, nquads, rcp), q = it - b * nquads;
-            bq[j] = b;
-            const int col = c0 * 128 + 4 * q;
-            const uint32_t off = (it < total && col < st.K) ? (uint32_t)(((size_t)b * st.in_stride + col) * sizeof(float)) : kPastEnd;
-            raw[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, kCacheAgentCoherent);
-        }
-#pragma unroll
-        for (int j = 0; j < kBurst; ++j) {
-            const int it = it0 + j * nthreads;
-            const int b = bq[j], q = it - b * nquads;
-            const uint16_t r0 = E::from_float(as_float(raw[j].x));
-            const uint16_t r1 = E::from_float(as_float(raw[j].y));
-            const uint16_t r2 = E::from_float(as_float(raw[j].z));
-            const uint16_t r3 = E::from_float(as_float(raw[j].w));
-            // the sum of what the dot products will actually see; lanes past the end hold zeros
-            const float tot = group_sum((E::to_float(r0) + E::to_float(r1)) + (E::to_float(r2) + E::to_float(r3)), 32);
-            if (it < total) {
-                const int cu = q >> 5, P = 2 * (q & 31);
-                uint32_t* xd = (uint32_t*)xs;
-                xd[xs_dword<PM>(b, P, upad, cu)] = (uint32_t)r0 | ((uint32_t)r1 << 16);
-                xd[xs_dword<PM>(b, P + 1, upad, cu)] = (uint32_t)r2 | ((uint32_t)r3 << 16);
-                if ((q & 31) == 0) {
-                    if (xsum) xsum[b * upad + cu] = tot;
-                    if (xtot) atomicAdd(&xtot[b], tot);
-                }
-            }
-        }
-    }
-}
-
-// 16-bit input (times its per-column scale) or non-coherent fp32 input, 8 columns per lane and load.
-// Requires 16-byte aligned rows and K % 8 == 0 (st.vec_in).
-template <int DT, int BATCH, bool PM>
-__device__ __forceinline__ void stage_units_vector(uint4* xs, float* xsum, float* xtot, const StageInput& st, int c0,
-                                                   int cu_n, int upad, int nthreads) {
-    using E = Elem<DT>;
-    constexpr int kBurst = 6;   // 256 lanes x 6 chunks = 12288 columns in one round trip
-    const int nchunks = cu_n * 16;
-    const int total = BATCH * nchunks;
-    const uint32_t esize = st.in_f32 ? 4u : 2u;
-    const __amdgpu_buffer_rsrc_t rin = raw_buffer(st.in, (uint32_t)(((size_t)(BATCH - 1) * st.in_stride + st.K) * esize));
-    const bool scaled = !st.in_f32 && st.s_col != nullptr;
-    const __amdgpu_buffer_rsrc_t rsc = raw_buffer(scaled ? (const void*)st.s_col : st.in, scaled ? (uint32_t)st.K * 2u : 0u);
-    const float rcp = 1.f / (float)nchunks;
-#pragma unroll 1
-    for (int it0 = threadIdx.x; it0 < total; it0 += nthreads * kBurst) {
-        u32x4_t raw_a[kBurst], raw_b[kBurst];
-        int bq[kBurst];
-#pragma unroll
-        for (int j = 0; j < kBurst; ++j) {
-            const int it = it0 + j * nthreads;
-            const int b = small_div(it, nchunks, rcp), q = it - b * nchunks;
-            bq[j] = b;
-            const int col = c0 * 128 + 8 * q;
-            const bool live = it < total && col < st.K;
-            const uint32_t off = live ? (uint32_t)(((size_t)b * st.in_stride + col) * esize) : kPastEnd;
-            raw_a[j] = __builtin_amdgcn_raw_buffer_load_b128(rin, off, 0, kCacheDefault);
-            if (st.in_f32) raw_b[j] = __builtin_amdgcn_raw_buffer_load_b128(rin, live ? off + 16u : kPastEnd, 0, kCacheDefault);
-            else raw_b[j] = __builtin_amdgcn_raw_buffer_load_b128(rsc, live ? (uint32_t)col * 2u : kPastEnd, 0, kCacheDefault);
-        }
-        // a wavefront whose 64 chunks of a burst slot all lie past the end skips the slot (wave-uniform branch)
-        const int wave_first = __builtin_amdgcn_readfirstlane(it0 - (int)(threadIdx.x & 63));
-#pragma unroll
-        for (int j = 0; j < kBurst; ++j) {
-            if (wave_first + j * nthreads >= total) continue;
-            const int it = it0 + j * nthreads;
-            const int b = bq[j], q = it - b * nchunks;
-            if constexpr (DT == 0) {
-                if (!st.in_f32) {
-                    // fp16 input: packed products, rounded once to fp16 like the fp32 product below (the product of two
-                    // fp16 numbers is exact in fp32), and their sum with the packed dot product: 8 lane operations per
-                    // chunk instead of 50
-                    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-                    uint32_t rp[4];
-                    float tot = 0.f;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        half2_t xv = __builtin_bit_cast(half2_t, (uint32_t)raw_a[j][e]);
-                        if (scaled) xv = xv * __builtin_bit_cast(half2_t, (uint32_t)raw_b[j][e]);
-                        rp[e] = __builtin_bit_cast(uint32_t, xv);
-                        tot = __builtin_amdgcn_fdot2(xv, (half2_t){(_Float16)1.f, (_Float16)1.f}, tot, false);
-                    }
-                    tot = group_sum(tot, 16);
-                    if (it < total) {
-                        const int cu = q >> 4, i = q & 15;
-                        store_chunk_packed<PM>(xs, b, i, upad, cu, rp);
-                        if (i == 0) {
-                            if (xsum) xsum[b * upad + cu] = tot;
-                            if (xtot) atomicAdd(&xtot[b], tot);
-                        }
-                    }
-                    continue;
-                }
-            }
-            float v[8];
-            if (!st.in_f32) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t xw = raw_a[j][e], sw = scaled ? raw_b[j][e] : E::kOnePair;
-                    v[2 * e] = E::to_float(xw & 0xFFFFu) * E::to_float(sw & 0xFFFFu);
-                    v[2 * e + 1] = E::to_float(xw >> 16) * E::to_float(sw >> 16);
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = as_float(raw_a[j][e]);
-                    v[4 + e] = as_float(raw_b[j][e]);
-                }
-            }
-            uint16_t r[8];
-            float tot = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                r[e] = E::from_float(v[e]);
-                tot += E::to_float(r[e]);          // the sum of what the dot products will actually see
-            }
-            // the 16 chunks of a unit are held by 16 consecutive lanes: finish the unit sum with DPP
-            tot = group_sum(tot, 16);
-            if (it < total) {
-                const int cu = q >> 4, i = q & 15;
-                store_chunk<PM>(xs, b, i, upad, cu, r);
-                if (i == 0) {
-                    if (xsum) xsum[b * upad + cu] = tot;
-                    if (xtot) atomicAdd(&xtot[b], tot);
-                }
-            }
-        }
-    }
-}
-
 // Element-wise fallback for inputs that allow no 16-byte loads (odd K, unaligned rows).
-template <int DT, int BATCH, bool PM>
-__device__ __forceinline__ void stage_units_scalar(uint4* xs, float* xsum, float* xtot, const StageInput& st, int c0,
-                                                   int cu_n, int upad, int nthreads) {
+template <int DT, int BATCH>
+__device__ __forceinline__ void stage_units_scalar(uint4* xs, float* unit_tot, const StageInput& st, int c0, int cu_n,
+                                                   int upad, int nthreads) {
     using E = Elem<DT>;
     const int nchunks = cu_n * 16;
 #pragma unroll 1
@@ -310,24 +99,14 @@ __device__ __forceinline__ void stage_units_scalar(uint4* xs, float* xsum, float
             }
             tot = group_sum(tot, 16);
             if (q < nchunks) {
-                store_chunk<PM>(xs, b, i, upad, cu, r);
-                if (i == 0) {
-                    if (xsum) xsum[b * upad + cu] = tot;
-                    if (xtot) atomicAdd(&xtot[b], tot);
-                }
+                uint32_t rp[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rp[e] = (uint32_t)r[2 * e] | ((uint32_t)r[2 * e + 1] << 16);
+                store_pairs(xs, b, i, upad, cu, rp);
+                if (i == 0) unit_tot[b * upad + cu] = tot;
             }
         }
     }
-}
-
-// Stage units [c0, c0+cu_n) for BATCH rows.  All threads of the workgroup call this; nthreads is the
-// workgroup size (a multiple of 64).  Must be followed by a barrier before xs/xsum/xtot are read.
-template <int DT, int BATCH, bool PM = false>
-__device__ __forceinline__ void stage_units(uint4* xs, float* xsum, const StageInput& st, int c0, int cu_n, int upad,
-                                            int nthreads, float* xtot = nullptr) {
-    if (!st.vec_in || (st.K & 7)) stage_units_scalar<DT, BATCH, PM>(xs, xsum, xtot, st, c0, cu_n, upad, nthreads);
-    else if (st.in_f32 && st.in_coherent) stage_units_coherent<DT, BATCH, PM>(xs, xsum, xtot, st, c0, cu_n, upad, nthreads);
-    else stage_units_vector<DT, BATCH, PM>(xs, xsum, xtot, st, c0, cu_n, upad, nthreads);
 }
 
 // Staging for the run-list kernel's 16-bit arithmetic (pair-major layout, unit totals to unit_tot[b * upad + cu]):
@@ -335,12 +114,12 @@ __device__ __forceinline__ void stage_units(uint4* xs, float* xsum, const StageI
 // them, every load of a lane is in flight before the first is used (an input of 4096 columns at batch 16 is one round
 // trip to the memory side for the workgroup instead of two or three), and no index is divided.  A wavefront's 64
 // chunks belong to one half of the batch rows (the chunk count is padded to a multiple of 64).  Requires 16-byte
-// aligned rows and K % 8 == 0; everything else goes through stage_units.
+// aligned rows and K % 8 == 0; everything else goes through stage_units_scalar.
 template <int DT, int BATCH, int THREADS>
 __device__ __forceinline__ void stage_units_rows(uint4* xs, float* unit_tot, const StageInput& st, int c0, int cu_n,
                                                  int upad) {
     if (!st.vec_in || (st.K & 7)) {
-        stage_units<DT, BATCH, true>(xs, unit_tot, st, c0, cu_n, upad, THREADS, nullptr);
+        stage_units_scalar<DT, BATCH>(xs, unit_tot, st, c0, cu_n, upad, THREADS);
         return;
     }
     using E = Elem<DT>;
@@ -360,7 +139,7 @@ __device__ __forceinline__ void stage_units_rows(uint4* xs, float* unit_tot, con
     auto put = [&](int b, int q, const uint32_t (&rp)[4], float tot) {
         tot = group_sum(tot, 16);                            // the 16 chunks of a unit sit in 16 consecutive lanes
         if (q < nchunks) {
-            store_chunk_packed<true>(xs, b, q & 15, upad, q >> 4, rp);
+            store_pairs(xs, b, q & 15, upad, q >> 4, rp);
             if ((q & 15) == 0) unit_tot[b * upad + (q >> 4)] = tot;
         }
     };
@@ -444,99 +223,6 @@ __device__ __forceinline__ void stage_units_rows(uint4* xs, float* unit_tot, con
     }
 }
 
-// Signed sum over one unit for BATCH rows: out[b] = sum_{c in unit} sgn(bit c) * x[b][c].
-template <int DT, int BATCH>
-struct UnitDot;
-
-template <int BATCH>
-struct UnitDot<0, BATCH> {   // fp16: single-exponent-bit operands, 5 accumulator classes
-    static __device__ __forceinline__ void run(const uint4& w, const uint4* xs, const float* xsum, int upad, int cu,
-                                               float (&out)[BATCH]) {
-        using E = Elem<0>;
-        constexpr uint32_t M14 = 0x40004000u, M13 = 0x20002000u, M12 = 0x10001000u, M11 = 0x08000800u, M10 = 0x04000400u;
-        float a14[BATCH], a13[BATCH], a12[BATCH], a11[BATCH], a10[BATCH];
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b) a14[b] = a13[b] = a12[b] = a11[b] = a10[b] = 0.f;
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            const uint32_t w0 = comp_d(w, wi);
-            const uint32_t wa = w0 >> 1, wb = w0 << 5, wc = w0 << 10;
-            // pair j -> (source, class): j=0 (wa,14); j=1..5 (w0,14..10); j=6..10 (wb,14..10); j=11..15 (wc,14..10)
-            const uint32_t m0 = wa & M14;
-            const uint32_t m1 = w0 & M14, m2 = w0 & M13, m3 = w0 & M12, m4 = w0 & M11, m5 = w0 & M10;
-            const uint32_t m6 = wb & M14, m7 = wb & M13, m8 = wb & M12, m9 = wb & M11, m10 = wb & M10;
-            const uint32_t m11 = wc & M14, m12 = wc & M13, m13 = wc & M12, m14 = wc & M11, m15 = wc & M10;
-#pragma unroll
-            for (int b = 0; b < BATCH; ++b) {
-                const uint4 x0 = xs[xs_chunk(b, 4 * wi + 0, upad, cu)];
-                const uint4 x1 = xs[xs_chunk(b, 4 * wi + 1, upad, cu)];
-                const uint4 x2 = xs[xs_chunk(b, 4 * wi + 2, upad, cu)];
-                const uint4 x3 = xs[xs_chunk(b, 4 * wi + 3, upad, cu)];
-                a14[b] = E::dot2(x0.x, m0, a14[b]);
-                a14[b] = E::dot2(x0.y, m1, a14[b]);
-                a13[b] = E::dot2(x0.z, m2, a13[b]);
-                a12[b] = E::dot2(x0.w, m3, a12[b]);
-                a11[b] = E::dot2(x1.x, m4, a11[b]);
-                a10[b] = E::dot2(x1.y, m5, a10[b]);
-                a14[b] = E::dot2(x1.z, m6, a14[b]);
-                a13[b] = E::dot2(x1.w, m7, a13[b]);
-                a12[b] = E::dot2(x2.x, m8, a12[b]);
-                a11[b] = E::dot2(x2.y, m9, a11[b]);
-                a10[b] = E::dot2(x2.z, m10, a10[b]);
-                a14[b] = E::dot2(x2.w, m11, a14[b]);
-                a13[b] = E::dot2(x3.x, m12, a13[b]);
-                a12[b] = E::dot2(x3.y, m13, a12[b]);
-                a11[b] = E::dot2(x3.z, m14, a11[b]);
-                a10[b] = E::dot2(x3.w, m15, a10[b]);
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b) {
-            // undo the class scalings (exact powers of two): 2^1, 2^-7, 2^-11, 2^-13, 2^-14
-            const float bx = a14[b] * 0.5f + a13[b] * 128.f + a12[b] * 2048.f + a11[b] * 8192.f + a10[b] * 16384.f;
-            out[b] = xsum[b * upad + cu] - 2.f * bx;
-        }
-    }
-};
-
-template <int BATCH>
-struct UnitDot<1, BATCH> {   // bf16: +-1 operand pairs
-    static __device__ __forceinline__ void run(const uint4& w, const uint4* xs, const float* xsum, int upad, int cu,
-                                               float (&out)[BATCH]) {
-        using E = Elem<1>;
-        (void)xsum;
-        constexpr int NACC = BATCH >= 4 ? 1 : 4;
-        float acc[BATCH][NACC];
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b)
-#pragma unroll
-            for (int a = 0; a < NACC; ++a) acc[b][a] = 0.f;
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            const uint32_t word = comp_d(w, wi);
-            uint32_t sp[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) sp[j] = ((word << j) & kSignPair) | E::kOnePair;
-#pragma unroll
-            for (int b = 0; b < BATCH; ++b) {
-                uint4 xv[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) xv[q] = xs[xs_chunk(b, 4 * wi + q, upad, cu)];
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    acc[b][j % NACC] = E::dot2(comp_d(xv[j >> 2], j & 3), sp[j], acc[b][j % NACC]);
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b) {
-            float t = acc[b][0];
-#pragma unroll
-            for (int a = 1; a < NACC; ++a) t += acc[b][a];
-            out[b] = t;
-        }
-    }
-};
-
 // ---- MFMA-assisted unit arithmetic (batch >= 4) -----------------------------------------------------
 // One v_mfma_f32_16x16x32 multiplies a 16-row x 32-column block of +-1 (A operand) with 32 columns x
 // 16 batch rows of staged activations (B operand).  Lane l of the wavefront owns matrix row l & 15 and
@@ -561,7 +247,7 @@ struct Mfma16<1> {
     }
 };
 
-// The single-exponent-bit operand of the matmul-free loop as the MFMA weight operand.  A 16-bit pattern with only one
+// The single-exponent-bit operand as the MFMA weight operand.  A 16-bit pattern with only one
 // exponent bit set is itself a number of the type: fp16 bits 14..10 = 2^1, 2^-7, 2^-11, 2^-13, 2^-14 (five classes);
 // bf16 bits 14, 13, 12 = 2^1, 2^-63, 2^-95 (three classes: the lower exponent bits would put the products of small
 // activations below the fp32 normal range).  For a pair position j the four dwords `word_wi & mask` (wi = 0..3) ARE the

@@ -5,21 +5,26 @@
 
 namespace nq {
 
-// nq_gemv.hip: one matmul-free stage.  dtype 0 = fp16, 1 = bf16.  first: input is 16-bit activations
-// scaled by s_col; otherwise input is the fp32 intermediate.  Output is fp32 when out_f32, else the
-// activation type (clamped); `addend` (fp32, same shape as out) is added before the store.
-hipError_t gemv_stage(int dtype, bool first, const uint32_t* bits, const void* in, const void* s_col,
-                      const void* s_row, const float* addend, void* out, bool out_f32, int batch, int rows,
-                      int words, int K, int in_stride, int out_stride, hipStream_t stream,
-                      const void* bias = nullptr);
-
-// Both stages of up to gemv_fused_max() independent linears (batch 1, 2 or 4) in two launches, or in one whose second
-// stages wait inside the kernel; see nq_gemv.hip.
-int gemv_fused_max();
-hipError_t gemv_fused(int dtype, int count, int batch, const void* const* x, const void* const* s_in,
-                      const uint32_t* const* vt_bits, const void* const* s_mid, const uint32_t* const* u_bits,
-                      const void* const* s_out, const void* const* bias, float* const* h, void* const* y,
-                      const int* n, const int* r, const int* m, bool one_launch, hipStream_t stream);
+// nq_rows.hip: one stage of the per-linear decode path on 1 to 16 batch rows.  dtype 0 = fp16, 1 = bf16.
+struct RowsStage {
+    const uint32_t* bits;   // [rows, words], row-major "half2" order
+    const void* in;         // [batch, in_stride] 16-bit: activations, or the h of an earlier stage (K = in_stride then)
+    const void* s_col;      // [K] column scale, or null
+    const void* s_row;      // [rows] row scale, or null
+    const void* bias;       // [rows] added after the row scale, or null
+    const float* addend;    // [batch, out_stride] fp32 added before the store, or null
+    void* out;              // [batch, out_stride]
+    int rows, words, K, in_stride, out_stride;
+    int out_kind;           // 0: 16-bit result (clamped), 1: fp32 result, 2: 16-bit h (with zeros up to out_stride rows)
+};
+int gemv_rows_group_max();
+int gemv_rows_h_stride(int r);
+// `count` (<= gemv_rows_group_max()) independent stages in one launch; scaled: all of them have s_col, or none.
+hipError_t gemv_rows(int dtype, bool scaled, int count, const RowsStage* s, int batch, hipStream_t stream);
+// out = the sum of two stages without column scale on the same rows (out, bias, addend from the first).
+hipError_t gemv_rows_sum2(int dtype, const RowsStage* two, int batch, hipStream_t stream);
+// Both stages of `count` linears in one launch whose second stages wait inside the kernel (first: out_kind 2).
+hipError_t gemv_rows_fused(int dtype, int count, const RowsStage* first, const RowsStage* second, int batch, hipStream_t stream);
 hipError_t gemv_fused_status(unsigned* out, hipStream_t stream);
 void gemv_fused_set_spin_limit(unsigned polls);          // 0: the default
 
@@ -76,9 +81,6 @@ hipError_t gemv_stream(int dtype, int batch, int nstages, const RunSlice* slices
 bool stream_needs_uniform_order(int dtype, int batch, bool alt = false);
 bool stream_has_deterministic(int dtype, int batch);
 bool stream_has_alt(int dtype, int batch);
-
-// One stage on its own through the run-list kernel (no tables, no counters); batch 16 only.
-hipError_t gemv_stream_single(int dtype, int batch, const RunStage& st, hipStream_t stream);
 
 // nq_gemm.hip: C[T,R] = s_out * ((x * s_in) . sgn(W)^T) with W in the 32x256 tile layout.
 // scratch: fp32 [T,R] when gemm_scratch_bytes(T,K,R) > 0.

@@ -128,11 +128,10 @@ __host__ __device__ __forceinline__ int mfma_items_per_wave(int nitems, int wave
 // no row sums in LDS, no LDS atomics, no barrier and no epilogue pass per row block.  The first pair of wavefront w is
 // pair w; every further one comes from a counter in LDS, so a wavefront that is served faster takes more pairs (the
 // four wavefronts of a SIMD are served oldest first; with equal shares the oldest waits 40 % of every pass).
-template <int DT, int BATCH, int ARITH, int THREADS, bool SINGLE, bool TILED, bool DET = false, bool OWN = false>
+template <int DT, int BATCH, int ARITH, int THREADS, bool TILED, bool DET = false, bool OWN = false>
 __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const RunSlice* __restrict__ slices,
                                                                      unsigned long long* counters, unsigned* status,
                                                                      unsigned spin_limit, int chunk_cap,
-                                                                     RunStage single, int single_rows,
                                                                      const void* ext_in, void* ext_out) {
     using E = Elem<DT>;
     constexpr int kStreamThreads = THREADS;
@@ -141,7 +140,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
     extern __shared__ uint4 lds_raw[];
     static_assert(ARITH == 1 || ARITH == 2, "unknown arithmetic");
     constexpr bool kQ8 = ARITH == 2;
-    static_assert(!OWN || (kQ8 && TILED && !SINGLE), "owned row pairs exist for the tile-order fp4 x fp8 kernel only");
+    static_assert(!OWN || (kQ8 && TILED), "owned row pairs exist for the tile-order fp4 x fp8 kernel only");
     constexpr bool kTotals = true;                              // both arithmetics: signed sum = (sum of x) - 2 (sum of b x)
     static_assert(!kQ8 || BATCH * kQ8Pieces <= 16, "pieces of all batch rows must fit the 16 operand columns");
     constexpr int kRaccFloats = kQ8 ? (OWN ? 0 : kRowBlock * BATCH) : kUnitTotalsBytes / (int)sizeof(float);   // 16-bit arithmetic: the unit totals
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
     // its latency is hidden behind phase 0.
     unsigned long long gen_raw = 0;
     unsigned members = 1;
-    if (tid < kWave && !SINGLE) {
+    if (tid < kWave) {
         const unsigned long long* exit_sub = counters + (size_t)nstages * kSubCounters * kCounterStride;
         const unsigned total = gridDim.x;
         const unsigned sub = (unsigned)wg & (kExitSubs - 1);
@@ -232,32 +231,24 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
     };
 
     {
-        // SINGLE: one stage given by value, no tables and no counters; workgroup w takes rows
-        // [w * single_rows, (w + 1) * single_rows)
 #pragma unroll 1
         for (int sg = wg, nth = 0;; ++nth) {
             RunSegment seg;
             RunStage st;
-            if constexpr (SINGLE) {
-                seg = RunSegment{0, wg * single_rows, min(single.rows, (wg + 1) * single_rows), 0};
-                st = single;
-                if (nth || seg.row_end <= seg.row_begin) break;
-            } else {
-                if (nth) {
-                    if (sg_more >= sg_more_end) break;
-                    sg = sg_more++;
-                }
-                const RunSlice& sl = slices[sg];
-                seg = sl.seg;
-                st = sl.st;
-                if (nth == 0) {
-                    sg_more = sl.more_begin;
-                    sg_more_end = sl.more_end;
-                    if (seg.stage < 0) break;           // nothing for this workgroup
-                }
-                if (st.in_ext) st.in = ext_in;          // bound with the launch
-                if (st.out_ext) st.out = ext_out;
+            if (nth) {
+                if (sg_more >= sg_more_end) break;
+                sg = sg_more++;
             }
+            const RunSlice& sl = slices[sg];
+            seg = sl.seg;
+            st = sl.st;
+            if (nth == 0) {
+                sg_more = sl.more_begin;
+                sg_more_end = sl.more_end;
+                if (seg.stage < 0) break;               // nothing for this workgroup
+            }
+            if (st.in_ext) st.in = ext_in;              // bound with the launch
+            if (st.out_ext) st.out = ext_out;
             const BitsView bv = bits_view(st);
             const int chunk_units = min(st.units, chunk_cap);
             const int upad = kQ8 ? q8_pitch(q8_units4(chunk_units)) : (chunk_units | 1);
@@ -305,7 +296,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
             RunSegment seg_n = seg;
             const uint32_t* bits_n = nullptr;
             int rows_n = 0, words_n = 0, units_n = 0;
-            if constexpr (kQ8 && TILED && !SINGLE) {
+            if constexpr (kQ8 && TILED) {
                 if (sg_more < sg_more_end) {
                     const RunSlice& sn = slices[sg_more];
                     seg_n = sn.seg;
@@ -1019,7 +1010,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
         }
     }
 
-    if (tid == 0 && !SINGLE) {
+    if (tid == 0) {
         unsigned long long* exit_sub = counters + (size_t)nstages * kSubCounters * kCounterStride;
         __hip_atomic_fetch_add(exit_sub + (size_t)(wg & (kExitSubs - 1)) * kCounterStride, 1ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
@@ -1079,21 +1070,20 @@ template <int DT, int BATCH, int ARITH = NQ_STREAM_ARITH(DT, BATCH)>
 struct StreamKernel {
     static constexpr int kArith = ARITH;
     static constexpr int kThreads = NQ_STREAM_THREADS(DT, BATCH);
-    static constexpr auto fn = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, false>;
-    static constexpr auto fn_tiled = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, kArith == 2>;
+    static constexpr auto fn = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false>;
+    static constexpr auto fn_tiled = gemv_stream_kernel<DT, BATCH, kArith, kThreads, kArith == 2>;
     // tile order, fp4 x fp8 arithmetic, wavefronts own row pairs: for lists whose longest input is staged in one chunk.
     // It has no row sums in LDS and no LDS atomics, which pays at batch 4 (four batch rows cost four times the flushes)
     // and in long lists at batch 1 and 2; a short slice has fewer row pairs than the workgroup has wavefronts, so the
     // builder asks for it at batch 4 and, for long lists, at batch 1 and 2.
     static constexpr bool kHasOwn = kArith == 2 && BATCH <= 4;
-    static constexpr auto fn_tiled_own = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, kArith == 2, false, kHasOwn>;
-    static constexpr auto fn_tiled_own_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, kArith == 2, kHasOwn, kHasOwn>;
-    static constexpr auto fn_single = gemv_stream_kernel<DT, BATCH, kArith, kThreads, true, false>;
+    static constexpr auto fn_tiled_own = gemv_stream_kernel<DT, BATCH, kArith, kThreads, kArith == 2, false, kHasOwn>;
+    static constexpr auto fn_tiled_own_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, kArith == 2, kHasOwn, kHasOwn>;
     // reproducible sums
     // the 16-bit arithmetic is reproducible as it is: the same instance
     static constexpr bool kHasDet = true;
-    static constexpr auto fn_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, false, kArith == 2>;
-    static constexpr auto fn_tiled_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, kArith == 2, kArith == 2>;
+    static constexpr auto fn_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, false, kArith == 2>;
+    static constexpr auto fn_tiled_det = gemv_stream_kernel<DT, BATCH, kArith, kThreads, kArith == 2, kArith == 2>;
 };
 
 template <int DT, int BATCH, int ARITH>
@@ -1213,54 +1203,8 @@ static hipError_t launch_stream(int nstages, const RunSlice* slices, unsigned lo
     if (cap <= 0) return hipErrorInvalidValue;
     if (nwg > cap) return hipErrorLaunchOutOfResources;
     hipLaunchKernelGGL(fn, dim3(nwg), dim3(SK::kThreads), lds, stream, nstages, slices, counters, status, spin_limit, chunk_cap,
-                       RunStage{}, 0, ext_in, ext_out);
+                       ext_in, ext_out);
     return hipGetLastError();
-}
-
-// One stage on its own: the same kernel without tables, dependencies or counters.
-template <int DT, int BATCH>
-static hipError_t launch_single(const RunStage& st, hipStream_t stream) {
-    using SK = StreamKernel<DT, BATCH>;
-    int chunk_cap;
-    size_t lds;
-    stream_lds_plan(BATCH, SK::kArith, st.units, &chunk_cap, &lds);
-    static PerDeviceFlag attr_done;              // per template instance and device
-    const int dev = current_device();
-    if (lds > 64 * 1024 && !attr_done.test(dev)) {
-        hipError_t e = hipFuncSetAttribute((const void*)SK::fn_single, hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLdsMax);
-        if (e != hipSuccess) return e;
-        attr_done.set(dev);
-    }
-    // resident workgroups of this kernel on this device: the query is host time, so the last answer per calling thread
-    // is kept (keyed by device and LDS size)
-    static thread_local size_t cached_lds = 0;
-    static thread_local int cached_dev = -1, cached_cap = 0;
-    if (cached_cap <= 0 || cached_lds != lds || cached_dev != dev) {
-        int per_cu = 0, cus = 0;
-        if (dev < 0 ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)SK::fn_single, SK::kThreads, lds) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return hipErrorInvalidValue;
-        cached_cap = per_cu * cus;
-        cached_lds = lds;
-        cached_dev = dev;
-    }
-    const int cap = cached_cap;
-    if (cap <= 0) return hipErrorInvalidValue;
-    // whole 16-row groups per workgroup, as few rows as the resident grid allows
-    const int rows_per_wg = ((st.rows + cap - 1) / cap + 15) & ~15;
-    const int nwg = (st.rows + rows_per_wg - 1) / rows_per_wg;
-    hipLaunchKernelGGL((SK::fn_single), dim3(nwg), dim3(SK::kThreads), lds, stream, 0, (const RunSlice*)nullptr,
-                       (unsigned long long*)nullptr, (unsigned*)nullptr, 0u, chunk_cap, st, rows_per_wg, (const void*)nullptr,
-                       (void*)nullptr);
-    return hipGetLastError();
-}
-
-// Only the batch sizes that the per-linear path sends here are instantiated.
-hipError_t gemv_stream_single(int dtype, int batch, const RunStage& st, hipStream_t stream) {
-    if (batch == 8) return dtype == 0 ? launch_single<0, 8>(st, stream) : launch_single<1, 8>(st, stream);
-    if (batch != 16) return hipErrorInvalidValue;
-    return dtype == 0 ? launch_single<0, 16>(st, stream) : launch_single<1, 16>(st, stream);
 }
 
 // CALL(dtype, batch, arithmetic); `alt` selects the 16-bit arithmetic where the batch size has both
