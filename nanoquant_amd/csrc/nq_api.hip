@@ -410,8 +410,23 @@ int nq_runlist_build(const nq_linear* linears, int nlinears, int batch, int dtyp
         for (const auto& st : table) work += (long long)st.rows * st.units;
         own = batch == 4 || work / std::max(1, nq::stream_capacity(dtype, batch, max_units, false)) >= 40000;
     }
+    // Batch 8 and 16 with every word in tile order: one-bit fp4 weights x fp6 pieces of the input, for lists with at least
+    // 60000 rows x units per workgroup.  A shorter list gives a workgroup a few row pairs per slice for its eight wavefronts
+    // and stages as much for them (us per launch, 16-bit operands against fp6, batch 8 / batch 16: two Llama-3-70B layers,
+    // 52000: 85 / 125 against 89 / 130; three, 78000: 121 / 177 against 110 / 155; Llama-2-7B, 6 layers, 37000: 63 / 73
+    // against 57 / 77; 10 layers, 62000: 105 / 116 against 77 / 103; 32 layers: 295 / 320 against 204 / 247).
+    bool f6 = batch >= 8;
+    if (f6) {
+        long long work = 0;
+        for (const auto& st : table) {
+            work += (long long)st.rows * st.units;
+            f6 = f6 && st.tiled != 0;
+        }
+        f6 = f6 && work / std::max(1, nq::stream_capacity(dtype, batch, max_units, alt)) >= 60000;
+    }
     const int granule = nq::stream_row_granule(dtype, batch);
     int nwg = nq::stream_capacity(dtype, batch, max_units, alt);
+    if (f6) nwg = std::min(nwg, nq::stream_f6_capacity(dtype, batch, max_units));
     if (nwg <= 0) return NQ_ERR_HIP;
     if (nwg > kMaxResidentWorkgroups) nwg = kMaxResidentWorkgroups;
     // A family: a stage and the stages that add onto its rows on the same workgroups (addend_local), in list order.
@@ -450,7 +465,7 @@ int nq_runlist_build(const nq_linear* linears, int nlinears, int batch, int dtyp
             // max_s (units_s * rows_s / n_s + fixed_s).
             const double overhead_rows = batch >= 16 ? 64.0 : wide ? 48.0 : 12.0;
             const double pass_cost = wide ? 700.0 : 0.0;
-            const int chunk_cap = std::max(1, nq::stream_chunk_cap(dtype, batch, max_units, alt));
+            const int chunk_cap = std::max(1, nq::stream_chunk_cap(dtype, batch, max_units, alt, f6));
             std::vector<double> fixed(ids.size(), 0.0), width(ids.size(), 0.0);
             for (size_t k = 0; k < ids.size(); ++k)
                 for (int s : family[(size_t)ids[k]]) {
@@ -537,16 +552,18 @@ int nq_runlist_build(const nq_linear* linears, int nlinears, int batch, int dtyp
         {
             // (the variant whose wavefronts own row pairs starts every slice without fetches in flight, so a slice
             // costs it more to start: 16000, and 10000 at batch 1, the best of sweeps on the Llama-2-7B stack)
-            const long long fixed_one = own ? (batch == 1 ? 10000 : 16000) : wide ? 2200 : batch == 1 ? 8800 : batch == 2 ? 6600 : 4400;
+            // (fp6: 9000, of 2200 .. 20000 at Llama-2-7B and Llama-3-70B stacks, within 5 % of each other up to 9000)
+            const long long fixed_one = f6 ? 9000 : own ? (batch == 1 ? 10000 : 16000) : wide ? 2200 : batch == 1 ? 8800 : batch == 2 ? 6600 : 4400;
             auto gran = [&](size_t k) { return table[ids[k]].tiled ? granule : 1; };
             // Batch 8 and 16: an input too long to be staged at once is staged again, chunk by chunk, for every 256 rows
             // of a slice (three barriers and a round trip to memory per chunk): charged as 10 more units per chunk and
             // row, from per-workgroup time accounts of the Llama-2-7B stack (down projection, 86 units in 3 chunks
-            // at batch 16: without the charge its workgroups end 20 % behind the others).
-            const long long chunk_cap_long = std::max(1, nq::stream_chunk_cap(dtype, batch, max_units, alt));
+            // at batch 16: without the charge its workgroups end 20 % behind the others).  The fp6 kernel stages a chunk once
+            // for 1024 rows: 4 (the 32-layer stack at batch 8 / 16 with 10, 4, 0: 206 / 253, 204 / 247, 217 / 268 us).
+            const long long chunk_cap_long = std::max(1, nq::stream_chunk_cap(dtype, batch, max_units, alt, f6));
             auto restage = [&](long long units) -> long long {
                 const long long chunks = (units + chunk_cap_long - 1) / chunk_cap_long;
-                return wide && chunks > 1 ? 10 * chunks : 0;
+                return wide && chunks > 1 ? (f6 ? 4 : 10) * chunks : 0;
             };
             // fills workgroups with budget T; returns how many it needs (emits the slices when `emit`)
             auto fill = [&](long long T, bool emit) -> long long {
@@ -642,6 +659,7 @@ int nq_runlist_build(const nq_linear* linears, int nlinears, int batch, int dtyp
     if (linears[0].tiled) plan_out->bound |= 4;
     if (alt) plan_out->bound |= 16;
     if (own) plan_out->bound |= 32;
+    if (f6) plan_out->bound |= 64;
     return hip_status(hipStreamSynchronize(hs));   // the tables are host memory: finish before they die
 }
 
@@ -666,7 +684,7 @@ int nq_runlist_run_bound(const void* workspace, const nq_runlist_plan* plan, con
                                       (unsigned*)base, plan->workgroups, plan->max_units, (hipStream_t)stream, x, y,
                                       (plan->bound & 4) != 0, (plan->bound & 8) != 0,
                                       plan->spin_limit > 0 ? (unsigned)plan->spin_limit : 0u, (plan->bound & 16) != 0,
-                                      (plan->bound & 32) != 0));
+                                      (plan->bound & 32) != 0, (plan->bound & 64) != 0));
 }
 
 int nq_runlist_capacity(int batch, int dtype, int max_units, int variant) {

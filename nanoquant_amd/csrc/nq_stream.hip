@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "nq_decode.h"
+#include "nq_fp6.h"
 #include "nq_kernels.h"
 
 namespace nq {
@@ -114,6 +115,100 @@ __host__ __device__ constexpr size_t stream_head_bytes(int batch, int arith, boo
 
 // fp4 x fp8 arithmetic: items that each wavefront of a workgroup takes (contiguous runs).
 __host__ __device__ __forceinline__ int mfma_items_per_wave(int nitems, int waves) { return (nitems + waves - 1) / waves; }
+
+// Rows row0 .. row0 + 3 of batch row b: row scale, bias, addend, store.  vec_rows: 8-byte accesses are aligned.
+template <int DT>
+__device__ __forceinline__ void emit_rows(const RunStage& st, int row_end, bool vec_rows, int row0, int b, float4_t v4) {
+    using E = Elem<DT>;
+    float v[4] = {v4[0], v4[1], v4[2], v4[3]};   // scalars: a device-scope atomic store of a vector element stored element 0 four times
+    const size_t o = (size_t)b * st.out_stride + row0;
+    if (vec_rows && row0 + 3 < row_end) {
+        if (st.s_row) {
+            const uint2 sw = *(const uint2*)(st.s_row + row0);
+            v[0] *= E::to_float((uint16_t)(sw.x & 0xFFFFu)); v[1] *= E::to_float((uint16_t)(sw.x >> 16));
+            v[2] *= E::to_float((uint16_t)(sw.y & 0xFFFFu)); v[3] *= E::to_float((uint16_t)(sw.y >> 16));
+        }
+        if (st.bias) {
+            const uint2 bw = *(const uint2*)(st.bias + row0);
+            v[0] += E::to_float((uint16_t)(bw.x & 0xFFFFu)); v[1] += E::to_float((uint16_t)(bw.x >> 16));
+            v[2] += E::to_float((uint16_t)(bw.y & 0xFFFFu)); v[3] += E::to_float((uint16_t)(bw.y >> 16));
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (row0 + k >= row_end) break;
+            if (st.s_row) v[k] *= E::to_float(st.s_row[row0 + k]);
+            if (st.bias) v[k] += E::to_float(st.bias[row0 + k]);
+        }
+    }
+    if (st.addend) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (row0 + k >= row_end) break;
+            if (st.dep2 >= 0)
+                v[k] += __builtin_bit_cast(float, __hip_atomic_load((const uint32_t*)st.addend + o + k, __ATOMIC_RELAXED,
+                                                                    __HIP_MEMORY_SCOPE_AGENT));
+            else
+                v[k] += st.addend[o + k];
+        }
+    }
+    if (!st.out_f32 && vec_rows && row0 + 3 < row_end) {
+        uint2 pk;
+        pk.x = (uint32_t)E::from_float_clamped(v[0]) | ((uint32_t)E::from_float_clamped(v[1]) << 16);
+        pk.y = (uint32_t)E::from_float_clamped(v[2]) | ((uint32_t)E::from_float_clamped(v[3]) << 16);
+        *(uint2*)((uint16_t*)st.out + o) = pk;
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (row0 + k >= row_end) break;
+        if (st.out_f32) {
+            // fp32 results (h, partial sums over terms) may be read by other workgroups of this launch:
+            // device-coherent store, completed before the counter of the slice is bumped
+            if (st.signal) __hip_atomic_store((uint32_t*)st.out + o + k, __builtin_bit_cast(uint32_t, v[k]),
+                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else ((float*)st.out)[o + k] = v[k];
+        } else {
+            ((uint16_t*)st.out)[o + k] = E::from_float_clamped(v[k]);
+        }
+    }
+}
+
+// Called by one wavefront: waits until the stages that `st` depends on are complete in launch `gen`; true if the bound ran
+// out (or another workgroup's did).
+__device__ __forceinline__ bool wait_for_stages(const RunStage& st, unsigned long long gen, const unsigned long long* counters,
+                                                unsigned* status, unsigned spin_limit) {
+    const int lane = threadIdx.x & 63;
+    unsigned spins = 0;
+    bool bad = false;
+#pragma unroll 1
+    for (int which = 0; which < 2 && !bad; ++which) {
+        const int d = which ? st.dep2 : st.dep;
+        if (d < 0 || (which && st.addend_local)) continue;
+        const unsigned long long want = (gen + 1) * (unsigned long long)(which ? st.dep2_segs : st.dep_segs);
+        while (true) {
+            unsigned long long c = 0;
+            if (lane < kSubCounters)
+                c = __hip_atomic_load(counters + ((size_t)d * kSubCounters + lane) * kCounterStride,
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            c += __shfl_xor(c, 1, kWave);
+            c += __shfl_xor(c, 2, kWave);
+            c += __shfl_xor(c, 4, kWave);
+            const unsigned long long sum0 = __shfl(c, 0, kWave);
+            if (sum0 >= want) break;
+            __builtin_amdgcn_s_sleep(8);   // pollers must not crowd out the producers' atomics
+            unsigned flagged = 0;
+            if (lane == 0) flagged = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            flagged = __shfl(flagged, 0, kWave);
+            if (++spins >= spin_limit || flagged) {
+                if (lane == 0) atomicOr(status, 1u);   // bounded wait: flag it, let the grid drain
+                bad = true;
+                break;
+            }
+        }
+    }
+    return bad;
+}
 
 // ARITH: 1 = MFMA with 16-bit operands, 2 = MFMA with one-bit fp4 weights and fp8 pieces of the input (batch <= 4).
 // DET, fp4 x fp8 arithmetic: row sums that do not depend on the order in which the wavefronts of a workgroup add
@@ -340,35 +435,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
 
             if ((st.dep >= 0 || st.dep2 >= 0) && !aborted) {
                 if (tid < kWave) {                               // wavefront 0 polls; lanes 0..7 own one sub-counter each
-                    const unsigned long long gen = gen_raw / members;
-                    unsigned spins = 0;
-                    bool bad = false;
-#pragma unroll 1
-                    for (int which = 0; which < 2 && !bad; ++which) {
-                        const int d = which ? st.dep2 : st.dep;
-                        if (d < 0 || (which && st.addend_local)) continue;
-                        const unsigned long long want = (gen + 1) * (unsigned long long)(which ? st.dep2_segs : st.dep_segs);
-                        while (true) {
-                            unsigned long long c = 0;
-                            if (tid < kSubCounters)
-                                c = __hip_atomic_load(counters + ((size_t)d * kSubCounters + tid) * kCounterStride,
-                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            c += __shfl_xor(c, 1, kWave);
-                            c += __shfl_xor(c, 2, kWave);
-                            c += __shfl_xor(c, 4, kWave);
-                            const unsigned long long sum0 = __shfl(c, 0, kWave);
-                            if (sum0 >= want) break;
-                            __builtin_amdgcn_s_sleep(8);   // pollers must not crowd out the producers' atomics
-                            unsigned flagged = 0;
-                            if (tid == 0) flagged = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            flagged = __shfl(flagged, 0, kWave);
-                            if (++spins >= spin_limit || flagged) {
-                                if (tid == 0) atomicOr(status, 1u);   // bounded wait: flag it, let the grid drain
-                                bad = true;
-                                break;
-                            }
-                        }
-                    }
+                    const bool bad = wait_for_stages(st, gen_raw / members, counters, status, spin_limit);
                     if (bad && tid == 0) s_flag = 1;
                     // 16-bit input written by another stage of this launch: ordinary loads follow, so the
                     // caches of this CU / XCD have to drop what they hold (rare; h and addend never need it).
@@ -387,60 +454,7 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
             // loop).  The four rows of a lane are consecutive: 8-byte accesses where the alignment allows them.
             const bool vec_rows = (seg.row_begin & 3) == 0 && (st.out_stride & 3) == 0 &&
                                   ((((uintptr_t)st.s_row) | ((uintptr_t)st.bias) | ((uintptr_t)st.out)) & 7u) == 0;
-            auto emit4 = [&](int row0, int b, float4_t v4) __attribute__((always_inline)) {
-                float v[4] = {v4[0], v4[1], v4[2], v4[3]};   // scalars: a device-scope atomic store of a vector element stored element 0 four times
-                const size_t o = (size_t)b * st.out_stride + row0;
-                if (vec_rows && row0 + 3 < seg.row_end) {
-                    if (st.s_row) {
-                        const uint2 sw = *(const uint2*)(st.s_row + row0);
-                        v[0] *= E::to_float((uint16_t)(sw.x & 0xFFFFu)); v[1] *= E::to_float((uint16_t)(sw.x >> 16));
-                        v[2] *= E::to_float((uint16_t)(sw.y & 0xFFFFu)); v[3] *= E::to_float((uint16_t)(sw.y >> 16));
-                    }
-                    if (st.bias) {
-                        const uint2 bw = *(const uint2*)(st.bias + row0);
-                        v[0] += E::to_float((uint16_t)(bw.x & 0xFFFFu)); v[1] += E::to_float((uint16_t)(bw.x >> 16));
-                        v[2] += E::to_float((uint16_t)(bw.y & 0xFFFFu)); v[3] += E::to_float((uint16_t)(bw.y >> 16));
-                    }
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        if (row0 + k >= seg.row_end) break;
-                        if (st.s_row) v[k] *= E::to_float(st.s_row[row0 + k]);
-                        if (st.bias) v[k] += E::to_float(st.bias[row0 + k]);
-                    }
-                }
-                if (st.addend) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        if (row0 + k >= seg.row_end) break;
-                        if (st.dep2 >= 0)
-                            v[k] += __builtin_bit_cast(float, __hip_atomic_load((const uint32_t*)st.addend + o + k, __ATOMIC_RELAXED,
-                                                                                __HIP_MEMORY_SCOPE_AGENT));
-                        else
-                            v[k] += st.addend[o + k];
-                    }
-                }
-                if (!st.out_f32 && vec_rows && row0 + 3 < seg.row_end) {
-                    uint2 pk;
-                    pk.x = (uint32_t)E::from_float_clamped(v[0]) | ((uint32_t)E::from_float_clamped(v[1]) << 16);
-                    pk.y = (uint32_t)E::from_float_clamped(v[2]) | ((uint32_t)E::from_float_clamped(v[3]) << 16);
-                    *(uint2*)((uint16_t*)st.out + o) = pk;
-                    return;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (row0 + k >= seg.row_end) break;
-                    if (st.out_f32) {
-                        // fp32 results (h, partial sums over terms) may be read by other workgroups of this launch:
-                        // device-coherent store, completed before the counter of the slice is bumped
-                        if (st.signal) __hip_atomic_store((uint32_t*)st.out + o + k, __builtin_bit_cast(uint32_t, v[k]),
-                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        else ((float*)st.out)[o + k] = v[k];
-                    } else {
-                        ((uint16_t*)st.out)[o + k] = E::from_float_clamped(v[k]);
-                    }
-                }
-            };
+            auto emit4 = [&](int row0, int b, float4_t v4) __attribute__((always_inline)) { emit_rows<DT>(st, seg.row_end, vec_rows, row0, b, v4); };
             if constexpr (!kQ8) {
               if (!aborted) {
                 // ---- 16-bit MFMA arithmetic (batch 8 and 16): wavefronts own whole row groups ----
@@ -1017,11 +1031,285 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
     }
 }
 
+// The run list at batch 8 and 16 with every word in tile order: one-bit fp4 weights x fp6 pieces (nq_fp6.h).  Slices, waits
+// and completion counts as in gemv_stream_kernel; a workgroup is 8 wavefronts with twice the registers each.
+//
+// What bounds it: no single unit; of 370 K cycles of the 32-layer Llama-2-7B stack at batch 8 the matrix cores are busy 27 %,
+// lane instructions 40 %, HBM moves 4.2 TB/s; the rest is the start of a slice (staging, its barrier, the first fetches) and
+// its end, where wavefronts run out of pairs.  Measured, 16-bit operands before -> now: that stack at batch 16 (bf16) 338 ->
+// 240 us, 80 Llama-3-70B layers at batch 8 (fp16) 2798 -> 1838 us (3.2 -> 4.8 TB/s).  The wavefronts own row pairs (32 rows, so one read of the input operand from
+// LDS serves two row groups) and walk all their columns; sums stay in the accumulators and go straight to the output.
+// An input that fits the staging area (4096 columns at batch 16, 8192 at batch 8) is staged once and the pairs are handed
+// out by a counter; for a longer one a wavefront takes kF6Pairs pairs at a time, whose sums it keeps from chunk to chunk.
+// Four item fetches (2 KB each) are in flight per wavefront; each carries the pair and unit group it belongs to, so the
+// stream runs on from pair to pair.
+template <int DT, int BATCH>
+__global__ __launch_bounds__(kF6Threads, 2) void gemv_stream_f6_kernel(int nstages, const RunSlice* __restrict__ slices,
+                                                                     unsigned long long* counters, unsigned* status,
+                                                                     unsigned spin_limit, int chunk_cap, const void* ext_in,
+                                                                     void* ext_out) {
+    using E = Elem<DT>;
+    using L = F6Layout<BATCH>;
+    constexpr int kWaves = kF6Threads / kWave;
+    extern __shared__ uint4 lds_raw[];
+    __shared__ int s_flag, s_pair;
+    const int tid = threadIdx.x, wg = blockIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // batch 8: operand columns 8 .. 15 are the batch rows again, a piece further
+    const int col = BATCH == 8 ? r16 & 7 : r16, upper = BATCH == 8 ? r16 >> 3 : 0;
+    unsigned long long* const exit_sub = counters + (size_t)nstages * kSubCounters * kCounterStride + (size_t)(wg & (kExitSubs - 1)) * kCounterStride;
+    unsigned long long gen_raw = 0;
+    if (tid < kWave) gen_raw = __hip_atomic_load(exit_sub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned members = (gridDim.x + kExitSubs - 1 - ((unsigned)wg & (kExitSubs - 1))) / kExitSubs;
+    if (tid == 0) s_flag = 0;
+    uint32_t ones = 0x22222222u;
+    asm volatile("" : "+v"(ones));
+    bool aborted = false;
+    int more = 0, more_end = 0;
+#pragma unroll 1
+    for (int sg = wg, nth = 0;; ++nth) {
+        if (nth) {
+            if (more >= more_end) break;
+            sg = more++;
+        }
+        const RunSlice& sl = slices[sg];
+        const RunSegment seg = sl.seg;
+        RunStage st = sl.st;
+        if (nth == 0) {
+            more = sl.more_begin;
+            more_end = sl.more_end;
+            if (seg.stage < 0) break;                       // nothing for this workgroup
+        }
+        if (st.in_ext) st.in = ext_in;
+        if (st.out_ext) st.out = ext_out;
+        StageInput sin;
+        sin.in = st.in; sin.s_col = st.s_col; sin.K = st.K; sin.in_stride = st.in_stride;
+        sin.in_f32 = st.in_f32; sin.in_coherent = st.in_coherent; sin.vec_in = st.vec_in;
+
+        const int nrows = seg.row_end - seg.row_begin, npairs = (nrows + 31) >> 5;
+        const int groups_all = (st.words + 15) >> 4;        // tiles per row pair in memory
+        const int tile0 = (seg.row_begin >> 5) * groups_all;
+        const __amdgpu_buffer_rsrc_t rbits = raw_buffer(st.bits, (uint32_t)((size_t)((st.rows + 31) >> 5) * groups_all * 2048));
+        const bool vec_rows = (seg.row_begin & 3) == 0 && (st.out_stride & 3) == 0 &&
+                              ((((uintptr_t)st.s_row) | ((uintptr_t)st.bias) | ((uintptr_t)st.out)) & 7u) == 0;
+        const size_t out_elems = (size_t)(BATCH - 1) * st.out_stride + st.rows;
+        const bool plain_out = vec_rows && (nrows & 31) == 0 && st.s_row && !st.bias && !st.addend && out_elems < (1u << 28);
+        const __amdgpu_buffer_rsrc_t rout = raw_buffer(st.out, (uint32_t)(out_elems * (st.out_f32 ? 4u : 2u)));
+        const int chunk_units = min(st.units, chunk_cap);
+        const bool whole = chunk_units == st.units;
+
+        // A fetch: the 2 KB of a (pair, unit group), asked for and not yet used.
+        struct Item {
+            u32x4_t a, b;
+            int pair, j;
+        };
+        Item it0, it1, it2, it3;
+        // fetch cursor over the pairs of a round and the unit groups of a chunk; pairs past `limit` load nothing
+        int f_pair = 0, f_j = 0, f_limit = 0, f_groups = 1, f_tile = 0;
+        int taken = 0;                                      // whole inputs: lane 0 holds the pair after the current one
+        auto take_pair = [&]() __attribute__((always_inline)) { if (lane == 0) taken = atomicAdd(&s_pair, 1); };
+        auto fetch = [&](Item& it) __attribute__((always_inline)) {
+            if (f_j == f_groups) {
+                f_j = 0;
+                if (whole) {
+                    f_pair = __builtin_amdgcn_readfirstlane(taken);
+                    take_pair();
+                } else {
+                    f_pair += kWaves;
+                }
+            }
+            const bool live = f_pair < f_limit;
+            const uint32_t soff = live ? (uint32_t)__builtin_amdgcn_readfirstlane(f_tile + f_pair * groups_all + f_j) * 2048u : 0u;
+            const uint32_t voff = live ? (uint32_t)lane * 16u : kPastEnd;
+            it.a = __builtin_amdgcn_raw_buffer_load_b128(rbits, voff, soff, 2 /* nt */);
+            it.b = __builtin_amdgcn_raw_buffer_load_b128(rbits, voff + 1024u, soff, 2 /* nt */);
+            it.pair = f_pair;
+            it.j = f_j++;
+        };
+        auto fetch_from = [&](int first, int limit, int c0, int cu_n) __attribute__((always_inline)) {
+            f_pair = first + wave; f_j = 0; f_limit = limit;
+            f_groups = (cu_n + 3) >> 2;
+            f_tile = tile0 + (c0 >> 2);
+            fetch(it0); fetch(it1); fetch(it2); fetch(it3);
+        };
+        // Where the first four fetches stay inside one pair they are sent out ahead of everything else: packed words
+        // depend on nothing.
+        const bool early = whole && !aborted && st.units > 12;
+        if (early) fetch_from(0, npairs, 0, st.units);
+
+        if ((st.dep >= 0 || st.dep2 >= 0) && !aborted) {
+            if (tid < kWave) {
+                const bool bad = wait_for_stages(st, gen_raw / members, counters, status, spin_limit);
+                if (bad && tid == 0) s_flag = 1;
+                if (st.heavy_acquire && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            }
+        }
+        lds_barrier();                                      // s_flag; the previous slice is done with the staged input
+        aborted = aborted || s_flag != 0;
+        // Pairs 0 .. kWaves - 1 are the wavefronts' first ones.  Nobody takes a pair of the previous slice any more, and the
+        // barrier behind the staging comes before the first one of this slice is taken.
+        if (tid == 0) s_pair = kWaves;
+
+        // 16 rows whose results need nothing but their row scale, without a lane load or a varying number of stores (see
+        // store_plain's twin in gemv_stream_kernel): rows grow + 4 g .. + 3 of the slice, batch row r16
+        const uint32_t past32 = st.out_f32 ? 0u : kPastEnd, past16 = st.out_f32 ? kPastEnd : 0u;
+        auto store_plain = [&](int grow, float4_t v) __attribute__((always_inline)) {
+            typedef const uint32_t __attribute__((address_space(4)))* scalar_words_t;
+            const int prow = seg.row_begin + __builtin_amdgcn_readfirstlane(grow);
+            const scalar_words_t sp = (scalar_words_t)(uintptr_t)(st.s_row + prow);
+            uint32_t sw[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                sw[i] = sp[i];
+                asm volatile("" : "+s"(sw[i]));             // kept in scalar registers: one scalar load each
+            }
+            uint32_t s0 = sw[0], s1 = sw[1];                // rows 4g .. 4g + 3
+#pragma unroll
+            for (int q = 1; q < 4; ++q) {
+                s0 = g == q ? sw[2 * q] : s0;
+                s1 = g == q ? sw[2 * q + 1] : s1;
+            }
+            v[0] *= E::to_float((uint16_t)(s0 & 0xFFFFu)); v[1] *= E::to_float((uint16_t)(s0 >> 16));
+            v[2] *= E::to_float((uint16_t)(s1 & 0xFFFFu)); v[3] *= E::to_float((uint16_t)(s1 >> 16));
+            const bool live = r16 < BATCH;
+            const uint32_t elem = (uint32_t)min(r16, BATCH - 1) * (uint32_t)st.out_stride + (uint32_t)(prow + 4 * g);
+            const uint32_t o32 = live ? (elem * 4u) | past32 : kPastEnd;
+            const uint32_t o16 = live ? (elem * 2u) | past16 : kPastEnd;
+            const u32x4_t f = {as_bits(v[0]), as_bits(v[1]), as_bits(v[2]), as_bits(v[3])};
+            __builtin_amdgcn_raw_buffer_store_b128(f, rout, o32, 0, kCacheAgentCoherent);   // fp32: read by other workgroups
+            const u32x2_t h = {(uint32_t)E::from_float_clamped(v[0]) | ((uint32_t)E::from_float_clamped(v[1]) << 16),
+                               (uint32_t)E::from_float_clamped(v[2]) | ((uint32_t)E::from_float_clamped(v[3]) << 16)};
+            __builtin_amdgcn_raw_buffer_store_b64(h, rout, o16, 0, kCacheDefault);
+        };
+        // PLAIN: every pair of the slice leaves by store_plain.  A loop of its own: where loads through generic addresses
+        // and a varying number of stores may lie behind the fetches, the compiler waits for all of them at every item.
+        auto store_pair = [&](auto plain_tag, int pair, const float4_t& acc_a, const float4_t& acc_b) __attribute__((always_inline)) {
+            const float4_t va = f6_columns<BATCH>(acc_a), vb = f6_columns<BATCH>(acc_b);
+            const int grow = 32 * pair;
+            if constexpr (decltype(plain_tag)::value) {
+                store_plain(grow, va);
+                store_plain(grow + 16, vb);
+            } else {
+                const int row0 = seg.row_begin + grow + 4 * g;
+                if (r16 < BATCH) {
+                    if (row0 < seg.row_end) emit_rows<DT>(st, seg.row_end, vec_rows, row0, r16, va);
+                    if (row0 + 16 < seg.row_end) emit_rows<DT>(st, seg.row_end, vec_rows, row0 + 16, r16, vb);
+                }
+                __builtin_amdgcn_s_waitcnt(0);
+            }
+        };
+        auto walk = [&](auto whole_tag, auto plain_tag) __attribute__((always_inline)) {
+            constexpr bool WHOLE = decltype(whole_tag)::value;
+            const int round_pairs = WHOLE ? npairs : kWaves * kF6Pairs;
+            bool staged = false;
+#pragma unroll 1
+            for (int first = 0; first < npairs; first += round_pairs) {
+                const int limit = min(npairs, first + round_pairs);
+                float4_t sums[kF6Pairs][2];
+#pragma unroll
+                for (int k = 0; k < kF6Pairs; ++k) sums[k][0] = sums[k][1] = f6_zero();
+#pragma unroll 1
+                for (int c0 = 0; c0 < st.units; c0 += chunk_units) {
+                    const int cu_n = min(chunk_units, st.units - c0);
+                    const int units4 = (cu_n + 3) & ~3, ngroups = units4 >> 2;
+                    uint4* x16 = lds_raw;
+                    uint2* x8 = (uint2*)((char*)x16 + L::bytes16(units4));
+                    uint32_t* scl = (uint32_t*)((char*)x8 + L::bytes8(units4));
+                    if (staged) lds_barrier();              // every wavefront is done with the staged chunk
+                    stage_units_f6<DT, BATCH>(x16, x8, scl, sin, c0, cu_n);
+                    staged = true;
+                    lds_barrier();
+                    if (WHOLE) take_pair();
+                    __builtin_amdgcn_s_waitcnt(0);          // what the staging loaded has been used: only fetches from here on
+                    if (!early) fetch_from(first, limit, c0, cu_n);
+                    const uint4* p16 = x16 + col * L::pitch16(units4) + g + L::kPiece * upper;
+                    const uint2* p8 = x8 + col * L::pitch8(units4) + g + L::kPiece * upper;
+                    const uint32_t* ps = scl + col * L::pitch_scale(units4) + g;
+                    const bool last = WHOLE || c0 + chunk_units >= st.units;
+                    int slot = 0;
+                    float4_t acc_a = WHOLE ? f6_zero() : sums[0][0], acc_b = WHOLE ? f6_zero() : sums[0][1];
+                    float4_t tail_a = f6_zero(), tail_b = f6_zero();       // batch 8 only
+                    auto work = [&](Item& it) __attribute__((always_inline)) {
+                        f6_item<BATCH>(it.a, it.b, p16 + L::kGroup * it.j, p8 + L::kGroup * it.j,
+                                       (int)(ps[4 * it.j] >> (8 * upper)), ones, acc_a, acc_b, BATCH == 8 ? tail_a : acc_a, BATCH == 8 ? tail_b : acc_b);
+                        if (it.j + 1 == ngroups) {
+                            if constexpr (BATCH == 8) {
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) {
+                                    acc_a[k] += upper ? 0.f : tail_a[k];
+                                    acc_b[k] += upper ? 0.f : tail_b[k];
+                                }
+                                tail_a = f6_zero();
+                                tail_b = f6_zero();
+                            }
+                            if (last) store_pair(plain_tag, it.pair, acc_a, acc_b);
+                            if constexpr (WHOLE) {
+                                acc_a = f6_zero();
+                                acc_b = f6_zero();
+                            } else {
+#pragma unroll
+                                for (int k = 0; k < kF6Pairs; ++k)
+                                    if (slot == k) { sums[k][0] = acc_a; sums[k][1] = acc_b; }
+                                ++slot;
+#pragma unroll
+                                for (int k = 1; k < kF6Pairs; ++k)
+                                    if (slot == k) { acc_a = sums[k][0]; acc_b = sums[k][1]; }
+                            }
+                        }
+                    };
+                    // (one way through the loop, with the same loads on it whether or not an item is left: the compiler
+                    // counts the loads behind a fetch to know how long to wait for it)
+                    auto slot_turn = [&](Item& it) __attribute__((always_inline)) {
+                        if (it.pair < limit) work(it);
+                        fetch(it);
+                    };
+#pragma unroll 1
+                    while (it0.pair < limit) {
+                        slot_turn(it0);
+                        slot_turn(it1);
+                        slot_turn(it2);
+                        slot_turn(it3);
+                    }
+                }
+            }
+        };
+        if (!aborted) {
+            if (whole && plain_out) walk(std::true_type{}, std::true_type{});
+            else if (whole) walk(std::true_type{}, std::false_type{});
+            else if (plain_out) walk(std::false_type{}, std::true_type{});
+            else walk(std::false_type{}, std::false_type{});
+        }
+        if (st.signal) {
+            // stores of every wavefront acknowledged, then the slice is counted (see gemv_stream_kernel)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __syncthreads();
+            if (tid == 0) {
+                unsigned long long* c = counters + ((size_t)seg.stage * kSubCounters + (wg & (kSubCounters - 1))) * kCounterStride;
+                if (st.heavy_release) __hip_atomic_fetch_add(c, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                else __hip_atomic_fetch_add(c, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    if (tid == 0) __hip_atomic_fetch_add(exit_sub, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 size_t stream_counter_bytes(int nstages) {
     return ((size_t)nstages * kSubCounters + kExitSubs) * kCounterStride * sizeof(unsigned long long);
 }
 
 // ---- host side --------------------------------------------------------------------------------
+// f6: one workgroup per compute unit (the grid has no more, and two on one would leave another idle)
+constexpr size_t kF6LdsMin = 81 * 1024;
+template <int BATCH>
+static void f6_lds_plan(int max_units, int* chunk_cap_out, size_t* lds_out) {
+    int chunk_cap = 4;
+    while (F6Layout<BATCH>::bytes(chunk_cap + 4) <= (size_t)kStreamLdsMax) chunk_cap += 4;
+    *chunk_cap_out = chunk_cap;
+    const size_t need = F6Layout<BATCH>::bytes(max_units < chunk_cap ? (max_units + 3) & ~3 : chunk_cap);
+    *lds_out = need > kF6LdsMin ? need : kF6LdsMin;
+}
+
 static void stream_lds_plan(int batch, int arith, int max_units, int* chunk_cap_out, size_t* lds_out, bool det = false,
                             bool own = false) {
     const int racc_bytes = (int)stream_head_bytes(batch, arith, det && arith == 2, own && arith == 2);
@@ -1176,6 +1464,53 @@ static int capacity_of(int max_units, int variant = -1) {
     return best;
 }
 
+template <int DT, int BATCH>
+static const void* f6_kernel(int max_units, int* chunk_cap, size_t* lds) {
+    f6_lds_plan<BATCH>(max_units, chunk_cap, lds);
+    static PerDeviceFlag attr_done;
+    const int dev = current_device();
+    const void* fn = (const void*)gemv_stream_f6_kernel<DT, BATCH>;
+    if (!attr_done.test(dev)) {
+        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLdsMax) != hipSuccess) return nullptr;
+        attr_done.set(dev);
+    }
+    return fn;
+}
+#define NQ_F6_DISPATCH(CALL)                                          \
+    if (batch == 8) return dtype == 0 ? CALL(0, 8) : CALL(1, 8);      \
+    if (batch == 16) return dtype == 0 ? CALL(0, 16) : CALL(1, 16);
+
+// Workgroups of the fp6 kernel that the device keeps resident; 0 where there is none or on error.
+template <int DT, int BATCH>
+static int f6_capacity(int max_units) {
+    int chunk_cap;
+    size_t lds;
+    const void* fn = f6_kernel<DT, BATCH>(max_units, &chunk_cap, &lds);
+    return fn ? resident_workgroups(fn, kF6Threads, lds) : 0;
+}
+int stream_f6_capacity(int dtype, int batch, int max_units) {
+#define NQ_CAP6(D, B) f6_capacity<D, B>(max_units)
+    NQ_F6_DISPATCH(NQ_CAP6)
+#undef NQ_CAP6
+    return 0;
+}
+
+template <int DT, int BATCH>
+static hipError_t launch_f6(int nstages, const RunSlice* slices, unsigned long long* counters, unsigned* status, int nwg,
+                            int max_units, hipStream_t stream, const void* ext_in, void* ext_out, unsigned spin_limit) {
+    int chunk_cap;
+    size_t lds;
+    const void* fn = f6_kernel<DT, BATCH>(max_units, &chunk_cap, &lds);
+    if (!fn) return hipErrorInvalidValue;
+    const int cap = resident_workgroups(fn, kF6Threads, lds);
+    if (cap <= 0) return hipErrorInvalidValue;
+    if (nwg > cap) return hipErrorLaunchOutOfResources;
+    if (spin_limit == 0) spin_limit = 1u << 21;
+    hipLaunchKernelGGL((gemv_stream_f6_kernel<DT, BATCH>), dim3(nwg), dim3(kF6Threads), lds, stream, nstages, slices, counters, status,
+                       spin_limit, chunk_cap, ext_in, ext_out);
+    return hipGetLastError();
+}
+
 template <int DT, int BATCH, int ARITH>
 static hipError_t launch_stream(int nstages, const RunSlice* slices, unsigned long long* counters, unsigned* status, int nwg,
                                 int max_units, hipStream_t stream, const void* ext_in, void* ext_out, bool tiled, bool det,
@@ -1229,9 +1564,14 @@ int stream_capacity(int dtype, int batch, int max_units, bool alt, int variant) 
 }
 
 // Units of an input vector that are staged at once (longer inputs take several passes over the rows of a slice).
-int stream_chunk_cap(int dtype, int batch, int max_units, bool alt) {
+int stream_chunk_cap(int dtype, int batch, int max_units, bool alt, bool f6) {
     int cap = 0;
     size_t lds = 0;
+    if (f6) {
+        if (batch == 8) f6_lds_plan<8>(max_units, &cap, &lds);
+        else f6_lds_plan<16>(max_units, &cap, &lds);
+        return cap;
+    }
 #define NQ_CHUNK(D, B, A) (stream_lds_plan(B, A, max_units, &cap, &lds), cap)
     NQ_STREAM_DISPATCH(NQ_CHUNK)
 #undef NQ_CHUNK
@@ -1266,7 +1606,13 @@ bool stream_has_deterministic(int dtype, int batch) {
 
 hipError_t gemv_stream(int dtype, int batch, int nstages, const RunSlice* slices, unsigned long long* counters,
                        unsigned* status, int nwg, int max_units, hipStream_t stream, const void* ext_in, void* ext_out,
-                       bool tiled, bool det, unsigned spin_limit, bool alt, bool own) {
+                       bool tiled, bool det, unsigned spin_limit, bool alt, bool own, bool f6) {
+    if (f6) {
+#define NQ_RUN6(D, B) launch_f6<D, B>(nstages, slices, counters, status, nwg, max_units, stream, ext_in, ext_out, spin_limit)
+        NQ_F6_DISPATCH(NQ_RUN6)
+#undef NQ_RUN6
+        return hipErrorInvalidValue;
+    }
 #define NQ_RUN(D, B, A) launch_stream<D, B, A>(nstages, slices, counters, status, nwg, max_units, stream, ext_in, ext_out, tiled, det, spin_limit, own)
     NQ_STREAM_DISPATCH(NQ_RUN)
 #undef NQ_RUN
