@@ -51,6 +51,7 @@ _SWEEPS = {
     "n_acc": (1, 2, 4),
     "n_pipe": (1, 2, 4, 8, 16),
 }
+_N_TH, _N_RPW, _N_ACC, _N_PIPE = (_SWEEPS[k] for k in ("n_th", "n_rpw", "n_acc", "n_pipe"))
 
 
 def _dtype_id(t: torch.Tensor) -> int:
@@ -81,7 +82,7 @@ def _sweep(name: str, value: int) -> None:
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()     # the declared argument type makes a pointer of it
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -91,8 +92,8 @@ def _stream(dev: torch.device):
     """The current stream of `dev` as the C ABI takes it.  The raw-handle query costs a tenth of building a
     `torch.cuda.Stream` object, which counts on a decode call that the GPU finishes in microseconds."""
     if _raw_stream is not None and dev.index is not None:
-        return ctypes.c_void_p(_raw_stream(dev.index))
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        return _raw_stream(dev.index)
+    return torch.cuda.current_stream(dev).cuda_stream
 
 
 class _on_device:
@@ -116,18 +117,26 @@ class _on_device:
 # decode op
 # ---------------------------------------------------------------------------------------------
 def _check_gemv_args(x, scale_g, Ubits, scale_l, Vbits, scale_h):
-    if x.dtype not in (torch.float16, torch.bfloat16):
+    dt = x.dtype
+    if dt not in _FLOAT_WHAT:
         raise RuntimeError("Support only Half or BFloat16")
-    what = _FLOAT_WHAT[x.dtype]
-    _check_dev_cont(x, "x", x.dtype, what)
-    _check_dev_cont(scale_g, "scale_g", x.dtype, what)
-    _check_dev_cont(scale_h, "scale_h", x.dtype, what)
-    _check_dev_cont(Ubits, "Ubits", torch.int32, "tensor dtype must be int32")
-    _check_dev_cont(Vbits, "Vbits", torch.int32, "tensor dtype must be int32")
-    if scale_l is not None:
-        _check_dev_cont(scale_l, "(*scale_l)", x.dtype, what)
-        if scale_l.size(0) != Ubits.size(0):
-            raise RuntimeError("scale_l size mismatch")
+    # One expression for a call in order (this is host time of every decode call); the calls below find out what is wrong.
+    if not (x.is_cuda and x.is_contiguous() and
+            scale_g.is_cuda and scale_g.dtype == dt and scale_g.is_contiguous() and
+            scale_h.is_cuda and scale_h.dtype == dt and scale_h.is_contiguous() and
+            Ubits.is_cuda and Ubits.dtype == torch.int32 and Ubits.is_contiguous() and
+            Vbits.is_cuda and Vbits.dtype == torch.int32 and Vbits.is_contiguous() and
+            (scale_l is None or (scale_l.is_cuda and scale_l.dtype == dt and scale_l.is_contiguous()))):
+        what = _FLOAT_WHAT[dt]
+        _check_dev_cont(x, "x", dt, what)
+        _check_dev_cont(scale_g, "scale_g", dt, what)
+        _check_dev_cont(scale_h, "scale_h", dt, what)
+        _check_dev_cont(Ubits, "Ubits", torch.int32, "tensor dtype must be int32")
+        _check_dev_cont(Vbits, "Vbits", torch.int32, "tensor dtype must be int32")
+        if scale_l is not None:
+            _check_dev_cont(scale_l, "(*scale_l)", dt, what)
+    if scale_l is not None and scale_l.size(0) != Ubits.size(0):
+        raise RuntimeError("scale_l size mismatch")
     if x.dim() < 1:
         raise RuntimeError("x must have at least one dimension")
     n = x.size(-1)
@@ -156,18 +165,23 @@ def _check_bias(bias, m, x):
 def _gemv_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias=None, dims=None):
     n, r, m = dims if dims is not None else _check_gemv_args(x, scale_g, Ubits, scale_l, Vbits, scale_h)
     _check_bias(bias, m, x)
-    lead = x.shape[:-1]
-    batch = 1
-    for d in lead:
-        batch *= d
-    y = torch.empty((batch, m), dtype=x.dtype, device=x.device)
+    flat = x.dim() == 2
+    dev, dt = x.device, x.dtype
+    if flat:
+        batch = x.size(0)
+    else:
+        batch = 1
+        for d in x.shape[:-1]:
+            batch *= d
+    y = torch.empty((batch, m), dtype=dt, device=dev)
     if batch > 0 and m > 0:
-        h = torch.empty((batch, max(r, 1)), dtype=torch.float32, device=x.device)
-        with _on_device(x.device):
-            _lib.check(_lib.lib().nq_gemv_forward_bias(_ptr(x), _ptr(scale_g), _ptr(Ubits), _ptr(scale_l), _ptr(Vbits),
-                                                       _ptr(scale_h), _ptr(bias), _ptr(h), _ptr(y), batch, n, r, m,
-                                                       _dtype_id(x), _stream(x.device)))
-    return y.reshape(*lead, m)
+        h = torch.empty((batch, max(r, 1)), dtype=torch.float32, device=dev)
+        with _on_device(dev):
+            _lib.check(_lib.lib().nq_gemv_forward_bias(x.data_ptr(), scale_g.data_ptr(), Ubits.data_ptr(), _ptr(scale_l),
+                                                       Vbits.data_ptr(), scale_h.data_ptr(), _ptr(bias), h.data_ptr(),
+                                                       y.data_ptr(), batch, n, r, m,
+                                                       _lib.NQ_F16 if dt == torch.float16 else _lib.NQ_BF16, _stream(dev)))
+    return y if flat else y.reshape(*x.shape[:-1], m)
 
 
 def nanoquant_dyn_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h,
@@ -178,14 +192,18 @@ def nanoquant_dyn_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h,
     """y = scale_h * (Vbits (scale_l * (Ubits (scale_g * x)))): `Ubits` [r, n/32] is the FIRST stage,
     `Vbits` [m, r/32] the second (the reference's argument names, pybind.cpp:86-90)."""
     dims = _check_gemv_args(x, scale_g, Ubits, scale_l, Vbits, scale_h)
-    _sweep("n_th1", num_thread_stage1)
-    _sweep("n_rpw1", num_row_per_warp_stage1)
-    _sweep("n_acc1", num_acc_stage1)
-    _sweep("n_pipe1", num_pipeline_stage1)
-    _sweep("n_th2", num_thread_stage2)
-    _sweep("n_rpw2", num_row_per_warp_stage2)
-    _sweep("n_acc2", num_acc_stage2)
-    _sweep("n_pipe2", num_pipeline_stage2)
+    if not (num_thread_stage1 in _N_TH and num_thread_stage2 in _N_TH and
+            num_row_per_warp_stage1 in _N_RPW and num_row_per_warp_stage2 in _N_RPW and
+            num_acc_stage1 in _N_ACC and num_acc_stage2 in _N_ACC and
+            num_pipeline_stage1 in _N_PIPE and num_pipeline_stage2 in _N_PIPE):
+        _sweep("n_th1", num_thread_stage1)
+        _sweep("n_rpw1", num_row_per_warp_stage1)
+        _sweep("n_acc1", num_acc_stage1)
+        _sweep("n_pipe1", num_pipeline_stage1)
+        _sweep("n_th2", num_thread_stage2)
+        _sweep("n_rpw2", num_row_per_warp_stage2)
+        _sweep("n_acc2", num_acc_stage2)
+        _sweep("n_pipe2", num_pipeline_stage2)
     return _gemv_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, dims=dims)
 
 
