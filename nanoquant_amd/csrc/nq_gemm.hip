@@ -616,14 +616,31 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 #undef NQ_BG
 }
 
+// More than kKwaveGroupMaxTokens tokens: whether the few-token tiles are still the faster ones.  A block tile walks the whole
+// k by itself, at 1.6 us per weight tile however few workgroups there are, while the four wavefronts of a few-token tile
+// share the k and there are eight times as many workgroups.  us per launch, block tiles against few-token tiles, by block
+// workgroups (64 tokens x 128 rows), 200 to 768 tokens of Llama-2-7B- and Qwen3-8B-shaped groups:
+//   k 4096:         40: 26 / 12    80: 26 / 18    176: 28 / 23    264: 36 / 28    352: 38 / 34    528: 51 / 50
+//   k 11008, 12288: 56: 65 / 26    88: 71 / 39    132: 72 / 52    264: 105 / 80
+//   k 1792 - 2816:  128: 14 / 10   192: 14 / 13   256: 15 / 15    384: 19 / 20    768: 40 / 50
+//   k below 1792:   128: 10 / 9    192: 10 / 12   384: 11 / 16
+bool gemm_group_few_tiles(int count, int T, const int* K, const int* R) {
+    long wgs = 0;
+    int shortest = 0x7FFFFFFF;
+    for (int p = 0; p < count; ++p) {
+        wgs += (long)((R[p] + 127) / 128) * ((T + 63) / 64);
+        shortest = K[p] / kTileK < shortest ? K[p] / kTileK : shortest;
+    }
+    return T <= kKwaveGroupMaxTokens || (shortest >= 16 && wgs <= 360) || (shortest >= 7 && wgs <= 192);
+}
+
 // GEMMs of several problems on the same token count in one launch; every problem: K % 256 == 0, R % 32 == 0, and
-// either all have input scales or none (checked by the caller).  Up to kKwaveGroupMaxTokens tokens the few-token
-// tiles, above them block tiles.
+// either all have input scales or none (checked by the caller).  Few-token tiles or block tiles: gemm_group_few_tiles.
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                              const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                              int T, const int* K, const int* R, hipStream_t stream) {
     if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
-    if (T > kKwaveGroupMaxTokens) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
+    if (T > kKwaveGroupMaxTokens && !gemm_group_few_tiles(count, T, K, R)) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     const int gy = (T + 31) / 32;
     int rt = 4;                                  // widest row blocks that still leave two workgroups per CU
     for (; rt > 1; rt /= 2) {

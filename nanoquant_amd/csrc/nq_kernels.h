@@ -92,7 +92,8 @@ hipError_t gemm_onebit(int dtype, const void* x, const uint32_t* tiles, const vo
                        void* y, float* scratch, int T, int K, int R, hipStream_t stream, const void* bias = nullptr);
 
 // Up to gemm_group_max() GEMMs on the same token count in one launch (s_in: all or none); few-token tiles up to
-// gemm_group_max_tokens() tokens, block tiles above.
+// gemm_group_max_tokens() tokens and where gemm_group_few_tiles says so, block tiles otherwise.
+bool gemm_group_few_tiles(int count, int T, const int* K, const int* R);
 int gemm_group_max();
 int gemm_group_max_tokens();
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,

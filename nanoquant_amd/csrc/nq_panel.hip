@@ -567,11 +567,23 @@ bool panel_applies(int count, int T, const int* K, const int* R) {
         longest = longest > K[p] / kTileK ? longest : K[p] / kTileK;
     }
     const double per_wg = (double)units / G;
+    const double fill = (double)T / (tblocks * kPanelTok);
+    if (T > gemm_group_max_tokens()) {
+        // Above the few-token counts.  A long k (more than 16 tiles): panels from some 90 block workgroups on (us, panels
+        // against few-token tiles: 56 workgroups 42 / 26, 88 40 / 39, 112 42 / 50, 168 49 / 53; block tiles 60 to 80).
+        // Up to 16 tiles panels start where the few-token tiles end; a k of less than 7 tiles, or a short one with less than
+        // 5 units per workgroup, is faster on block tiles (5 tiles, 3.2 units: 26 against 21; 10.5 units: 50 against 47;
+        // 8 tiles, 3.6 units: 27 against 24; 7 to 11 tiles, 7 to 25 units: 35 to 88 against 40 to 103).
+        long wgs = 0;
+        for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
+        if (longest > 16) return wgs > 88 && per_wg >= 3.0;
+        if (gemm_group_few_tiles(count, T, K, R)) return false;
+        return fill >= 0.70 && (longest >= 16 ? per_wg >= 3.0 : longest >= 7 && per_wg >= 5.0);
+    }
     if (per_wg < 3.0) return false;
     // up to two token blocks the few-token tiles are the alternative, and a strong one; beyond, panels win more easily
     const bool few = T <= 2 * kPanelTok;
     if (longest > (few ? 4.0 : 8.0) * per_wg) return false;
-    const double fill = (double)T / (tblocks * kPanelTok);
     return fill >= (few ? 0.78 : 0.70) || longest > 16;
 }
 

@@ -1034,8 +1034,8 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
 // The run list at batch 8 and 16 with every word in tile order: one-bit fp4 weights x fp6 pieces (nq_fp6.h).  Slices, waits
 // and completion counts as in gemv_stream_kernel; a workgroup is 8 wavefronts with twice the registers each.
 //
-// What bounds it: no single unit; of 370 K cycles of the 32-layer Llama-2-7B stack at batch 8 the matrix cores are busy 27 %,
-// lane instructions 40 %, HBM moves 4.2 TB/s; the rest is the start of a slice (staging, its barrier, the first fetches) and
+// What bounds it: no single unit; of 366 K cycles of the 32-layer Llama-2-7B stack at batch 8 the matrix cores are busy 27 %,
+// lane and matrix instructions together issue in 63 %, HBM moves 4.2 TB/s; the rest is the start of a slice (staging, its barrier, the first fetches) and
 // its end, where wavefronts run out of pairs.  Measured, 16-bit operands before -> now: that stack at batch 16 (bf16) 338 ->
 // 240 us, 80 Llama-3-70B layers at batch 8 (fp16) 2798 -> 1838 us (3.2 -> 4.8 TB/s).  The wavefronts own row pairs (32 rows, so one read of the input operand from
 // LDS serves two row groups) and walk all their columns; sums stay in the accumulators and go straight to the output.

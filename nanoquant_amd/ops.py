@@ -516,7 +516,7 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     the stages may run as persistent panel launches (around 128 tokens, see include/nq_gfx950.h).  Returns the list of
     outputs.  The terms share
     launches (a single linear leaves most of the device idle up to some hundred tokens): few-token tiles up to 160
-    tokens, 64-token block tiles without k-split above.  The
+    tokens and where a group is too small for more, 64-token block tiles without k-split above.  The
     reference launches every linear by itself (modules/linear.py:131-133)."""
     lib = _lib.lib()
     count = len(terms)

@@ -1,0 +1,38 @@
+"""Grouped prefill above 160 tokens: both sides of the lines between few-token tiles, block tiles and panels."""
+import numpy as np
+import pytest
+import torch
+
+from nanoquant_amd import ops, packing
+from oracle import nq_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+# (tokens, n, r, m): 64-token x 128-row block workgroups of the two GEMMs in the comments
+@pytest.mark.parametrize("tokens,n,r,m", [
+    (161, 4096, 256, 320),       # 6 and 9: few-token tiles (16 k tiles), block tiles (one)
+    (384, 1792, 4096, 512),      # 192 on 7 k tiles: the last one on few-token tiles; 24 on 16
+    (384, 1792, 4352, 256),      # 204: block tiles
+    (384, 4096, 7680, 288),      # 360 on 16 k tiles: the last one on few-token tiles
+    (330, 4096, 7936, 288),      # 372: panels or block tiles; 18 on 31 k tiles
+    (450, 11008, 1280, 256),     # 80 on 43 k tiles: few-token tiles
+    (450, 11008, 1536, 256),     # 96: panels
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_either_side_of_the_lines(dev, dtype, tokens, n, r, m):
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(dtype)
+    f32 = lambda t: t.float().cpu().numpy()
+    vt, u, s_in, s_mid, s_out = oracle.synth_term(m, n, r, 9500)
+    sc = (to(s_in), to(s_mid), to(s_out))
+    packed = packing.marlin_nanoquant_packer(torch.from_numpy(vt).T.contiguous().to(dev), torch.from_numpy(u).T.contiguous().to(dev), *sc)
+    x = to(oracle.synth_x(tokens, n, 9501))
+    ref = oracle.layer_forward(f32(x), vt, u, *(f32(s) for s in sc))
+    for panel in ("auto", "never"):
+        y = ops.gemm_group_forward([x], [packed], panel=panel)[0]
+        torch.cuda.synchronize()
+        err = oracle.max_rel_err(f32(y), ref)
+        print(f"group {tokens} tokens {n}->{r}->{m} {dtype} panel={panel}: {err:.2e}", flush=True)
+        # h and the result are rounded to the 16-bit type: half an ulp each, 2^-11 (fp16) or 2^-8 (bf16), of values near the largest
+        assert err < 3 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), (panel, err)
+    assert ops.panel_status(dev) == 0
