@@ -1337,7 +1337,8 @@ static void stream_lds_plan(int batch, int arith, int max_units, int* chunk_cap_
 // 16-bit MFMA operands (ARITH 1), but every workgroup quantises the whole input vector of its stage (about 110 lane
 // instructions per 8 columns and batch row): at batch 4 that costs as much as the arithmetic saves when a launch
 // covers only one layer, and a third less time in long run lists.  Its staging does not depend on the element type,
-// so bf16 runs as fast as fp16.  Batch 8 and 16 need more operand columns (batch rows x 3 pieces) than one MFMA has.
+// so bf16 runs as fast as fp16.  Batch 8 and 16 need more operand columns (batch rows x 3 pieces) than one MFMA has; long
+// lists in tile order run on gemv_stream_f6_kernel there.
 // Every workgroup stages the whole input vector of its stage, so larger workgroups mean less staging work per
 // row: 1024 lanes everywhere.
 #ifndef NQ_STREAM_ARITH
