@@ -1,0 +1,61 @@
+"""Registers of the built run-list kernels, from the metadata notes of the code objects inside the library (no GPU): the
+batch 4 instances are at the register limit of 1024 lanes, and what spills there is time in the inner loop."""
+import struct
+
+import pytest
+
+from nanoquant_amd import _lib
+
+msgpack = pytest.importorskip("msgpack")
+
+_AMDGPU, _METADATA_NOTE, _SHT_NOTE = 224, 32, 7
+
+
+def _notes(elf):
+    """(type, descriptor) of every note of a 64-bit little-endian ELF image."""
+    shoff, = struct.unpack_from("<Q", elf, 40)
+    shentsize, shnum = struct.unpack_from("<HH", elf, 58)
+    for i in range(shnum):
+        kind, = struct.unpack_from("<I", elf, shoff + i * shentsize + 4)
+        if kind != _SHT_NOTE:
+            continue
+        at, size = struct.unpack_from("<QQ", elf, shoff + i * shentsize + 24)
+        end = at + size
+        while at < end:
+            namesz, descsz, note = struct.unpack_from("<III", elf, at)
+            desc = at + 12 + (namesz + 3) // 4 * 4
+            yield note, elf[desc:desc + descsz]
+            at = desc + (descsz + 3) // 4 * 4
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    with open(_lib.LIB_PATH, "rb") as f:
+        image = f.read()
+    found, at = {}, image.find(b"\x7fELF", 1)
+    while at > 0:
+        if struct.unpack_from("<H", image, at + 18)[0] == _AMDGPU:
+            for note, desc in _notes(memoryview(image)[at:]):
+                if note == _METADATA_NOTE:
+                    found.update((k[".name"], k) for k in msgpack.unpackb(bytes(desc))["amdhsa.kernels"])
+        at = image.find(b"\x7fELF", at + 1)
+    assert found
+    return found
+
+
+def _stream_kernel(kernels, dtype, batch, arith, tiled, det, own):
+    prefix = f"_ZN2nq18gemv_stream_kernelILi{dtype}ELi{batch}ELi{arith}ELi1024ELb{tiled}ELb{det}ELb{own}EEE"
+    hits = [k for name, k in kernels.items() if name.startswith(prefix)]
+    assert len(hits) == 1, prefix
+    return hits[0]
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_owned_row_pairs_at_batch_4_spill_no_vector_register(kernels, dtype):
+    k = _stream_kernel(kernels, dtype, 4, 2, 1, 0, 1)
+    assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0
+
+
+def test_short_fp16_lists_at_batch_4_spill_no_more_than_five(kernels):
+    # 16-bit operands: 5 of 128 (24 bytes) with the class operands of eight steps in flight; every further one showed in time
+    assert _stream_kernel(kernels, 0, 4, 1, 0, 0, 0)[".vgpr_spill_count"] <= 5
