@@ -618,20 +618,34 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 
 // More than kKwaveGroupMaxTokens tokens: whether the few-token tiles are still the faster ones.  A block tile walks the whole
 // k by itself, at 1.6 us per weight tile however few workgroups there are, while the four wavefronts of a few-token tile
-// share the k and there are eight times as many workgroups.  us per launch, block tiles against few-token tiles, by block
-// workgroups (64 tokens x 128 rows), 200 to 768 tokens of Llama-2-7B- and Qwen3-8B-shaped groups:
-//   k 4096:         40: 26 / 12    80: 26 / 18    176: 28 / 23    264: 36 / 28    352: 38 / 34    528: 51 / 50
-//   k 11008, 12288: 56: 65 / 26    88: 71 / 39    132: 72 / 52    264: 105 / 80
-//   k 1792 - 2816:  128: 14 / 10   192: 14 / 13   256: 15 / 15    384: 19 / 20    768: 40 / 50
-//   k below 1792:   128: 10 / 9    192: 10 / 12   384: 11 / 16
-bool gemm_group_few_tiles(int count, int T, const int* K, const int* R) {
+// share the k and there are eight times as many workgroups, each of which reads its 32 tokens again for every 32 to 128 rows.
+// The limits are block workgroups (64 tokens x 128 rows), from 2494 pairs of timings: k of 5 to 48 tiles, 256 to 8704
+// rows, 161 to 2048 tokens, GEMMs with s_in (the first of a linear) and without (the second, whose block tiles are the faster
+// ones).  At 512 tokens, and at every further multiple, eight token blocks share slabs in one L2 each and block tiles gain;
+// above 1024 tokens the inputs no longer stay in the L2s and the few-token tiles lose.  us per call of a linear whose other
+// GEMM is a few, block tiles / few-token tiles, by block workgroups and tokens:
+//   with s_in, k 4096   64 at 256: 30 / 17    192 at 512: 33 / 29      300 at 900: 41 / 38      96 at 3072: 30 / 39
+//   without             64 at 256: 28 / 18    192 at 512: 28.5 / 31    120 at 900: 34 / 31      64 at 2048: 33 / 37
+//   with s_in, k 1792   64 at 512: 21 / 16    120 at 900: 22 / 20.6    192 at 1024: 24 / 24.4   192 at 1536: 22 / 24
+//   without             96 at 512: 17.2 / 17  160 at 512: 17.5 / 19    128 at 1024: 17.6 / 20   192 at 1536: 19 / 25
+//   without, k 11008    128 at 512: 67 / 46   128 at 1024: 72 / 56     96 at 1536: 78 / 69      256 at 2048: 82 / 91
+bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool scaled) {
+    constexpr int kRanges = 6;
+    constexpr int kTokens[kRanges] = {400, 512, 768, 1280, 1536, 2048};
+    constexpr int kLimits[2][3][kRanges] = {
+        {{150, 96, 144, 80, 0, 0}, {288, 96, 200, 160, 48, 0}, {360, 360, 360, 160, 96, 0}},            // no s_in; k of 7, 16, 24 tiles
+        {{192, 192, 160, 160, 48, 0}, {360, 360, 360, 160, 96, 64}, {360, 360, 360, 320, 192, 128}}};   // s_in
+    if (T <= kKwaveGroupMaxTokens) return true;
     long wgs = 0;
     int shortest = 0x7FFFFFFF;
     for (int p = 0; p < count; ++p) {
         wgs += (long)((R[p] + 127) / 128) * ((T + 63) / 64);
         shortest = K[p] / kTileK < shortest ? K[p] / kTileK : shortest;
     }
-    return T <= kKwaveGroupMaxTokens || (shortest >= 16 && wgs <= 360) || (shortest >= 7 && wgs <= 192);
+    if (shortest < 7) return false;              // block tiles are as short: k below 1792, 128 workgroups 10 / 9, 192 10 / 12, 384 11 / 16
+    for (int i = 0; i < kRanges; ++i)
+        if (T <= kTokens[i]) return wgs <= kLimits[scaled][shortest >= 24 ? 2 : shortest >= 16 ? 1 : 0][i];
+    return false;
 }
 
 // GEMMs of several problems on the same token count in one launch; every problem: K % 256 == 0, R % 32 == 0, and
@@ -640,7 +654,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
                              const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                              int T, const int* K, const int* R, hipStream_t stream) {
     if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
-    if (T > kKwaveGroupMaxTokens && !gemm_group_few_tiles(count, T, K, R)) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
+    if (!gemm_group_few_tiles(count, T, K, R, s_in && s_in[0])) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     const int gy = (T + 31) / 32;
     int rt = 4;                                  // widest row blocks that still leave two workgroups per CU
     for (; rt > 1; rt /= 2) {

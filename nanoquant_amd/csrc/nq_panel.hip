@@ -555,7 +555,7 @@ size_t panel_workspace_bytes() {
 // cut eight ways, is faster on the few-token tiles); token counts that fill their 64-token blocks badly waste MFMAs,
 // which only a stage with a long k makes up for (its block tiles need a k split and a finish launch); and from
 // about 1024 tokens on the block tiles are level.
-bool panel_applies(int count, int T, const int* K, const int* R) {
+bool panel_applies(int count, int T, const int* K, const int* R, bool scaled) {
     const int G = panel_grid();
     if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > 768) return false;
     const int tblocks = (T + kPanelTok - 1) / kPanelTok;
@@ -577,7 +577,7 @@ bool panel_applies(int count, int T, const int* K, const int* R) {
         long wgs = 0;
         for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
         if (longest > 16) return wgs > 88 && per_wg >= 3.0;
-        if (gemm_group_few_tiles(count, T, K, R)) return false;
+        if (gemm_group_few_tiles(count, T, K, R, scaled)) return false;
         return fill >= 0.70 && (longest >= 16 ? per_wg >= 3.0 : longest >= 7 && per_wg >= 5.0);
     }
     if (per_wg < 3.0) return false;

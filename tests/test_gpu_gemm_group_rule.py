@@ -18,6 +18,11 @@ pytestmark = pytest.mark.gpu
     (330, 4096, 7936, 288),      # 372: panels or block tiles; 18 on 31 k tiles
     (450, 11008, 1280, 256),     # 80 on 43 k tiles: few-token tiles
     (450, 11008, 1536, 256),     # 96: panels
+    (500, 256, 4096, 1536),      # second GEMM, 96 on 16 k tiles: the last one on few-token tiles at 401 to 512 tokens
+    (500, 256, 4096, 1664),      # 104: block tiles
+    (1500, 4096, 512, 256),      # 96 on 16 k tiles: the last one on few-token tiles above 1280 tokens
+    (2048, 4096, 256, 256),      # 64: the last one above 1536
+    (2050, 4096, 256, 256),      # 66 above 2048: block tiles
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_either_side_of_the_lines(dev, dtype, tokens, n, r, m):
@@ -36,3 +41,24 @@ def test_either_side_of_the_lines(dev, dtype, tokens, n, r, m):
         # h and the result are rounded to the 16-bit type: half an ulp each, 2^-11 (fp16) or 2^-8 (bf16), of values near the largest
         assert err < 3 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), (panel, err)
     assert ops.panel_status(dev) == 0
+
+
+# (tokens, (n, r, m) of a linear, of a neighbour that puts the launch beyond the few-token tiles)
+@pytest.mark.parametrize("tokens,linear,neighbour", [
+    (3072, (4096, 256, 256), (4096, 2048, 256)),     # few rows at many tokens: 96 block workgroups on 16 k tiles
+    (512, (256, 4096, 3072), (256, 4096, 8192)),     # a second GEMM: 192 on 16 k tiles
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_block_tiles_where_few_token_tiles_are_slower(dev, dtype, tokens, linear, neighbour):
+    # the route shows in the bits: block tiles add the k tiles one behind the other, few-token tiles in four shares
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(11)
+    signs = lambda a, b: torch.randint(0, 2, (a, b), dtype=torch.int8, device=dev, generator=gen) * 2 - 1
+    scale = lambda k: (torch.rand(k, device=dev, generator=gen) + 0.01).to(dtype)
+    terms = [packing.marlin_nanoquant_packer(signs(n, r), signs(r, m), scale(n), scale(r), scale(m)) for n, r, m in (linear, neighbour)]
+    x = torch.randn(tokens, linear[0], device=dev, generator=gen).to(dtype)
+    print(f"group {tokens} tokens {linear} beside {neighbour} {dtype}", flush=True)
+    alone = ops.gemm_group_forward([x], terms[:1], panel="never")[0]
+    beside = ops.gemm_group_forward([x, x], terms, panel="never")[0]
+    torch.cuda.synchronize()
+    assert torch.equal(alone, beside)
