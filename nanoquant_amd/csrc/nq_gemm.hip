@@ -629,6 +629,9 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 //   with s_in, k 1792   64 at 512: 21 / 16    120 at 900: 22 / 20.6    192 at 1024: 24 / 24.4   192 at 1536: 22 / 24
 //   without             96 at 512: 17.2 / 17  160 at 512: 17.5 / 19    128 at 1024: 17.6 / 20   192 at 1536: 19 / 25
 //   without, k 11008    128 at 512: 67 / 46   128 at 1024: 72 / 56     96 at 1536: 78 / 69      256 at 2048: 82 / 91
+// The longest k of a group decides: the launch lasts as long as its block tiles, and the few-token tiles cost a short k little
+// (with s_in, k 11008 and 1024, 1024 rows each: 64 workgroups at 256 tokens 69 / 34, 128 at 512: 72 / 43; k 4096 and 1024, 1024
+// and 512 rows: 96 at 512: 34 / 27; k 2304 and 768, 4096 rows each: 192 at 161: 25 / 22).
 bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool scaled) {
     constexpr int kRanges = 6;
     constexpr int kTokens[kRanges] = {400, 512, 768, 1280, 1536, 2048};
@@ -637,14 +640,14 @@ bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool sca
         {{192, 192, 160, 160, 48, 0}, {360, 360, 360, 160, 96, 64}, {360, 360, 360, 320, 192, 128}}};   // s_in
     if (T <= kKwaveGroupMaxTokens) return true;
     long wgs = 0;
-    int shortest = 0x7FFFFFFF;
+    int longest = 0;
     for (int p = 0; p < count; ++p) {
         wgs += (long)((R[p] + 127) / 128) * ((T + 63) / 64);
-        shortest = K[p] / kTileK < shortest ? K[p] / kTileK : shortest;
+        longest = K[p] / kTileK > longest ? K[p] / kTileK : longest;
     }
-    if (shortest < 7) return false;              // block tiles are as short: k below 1792, 128 workgroups 10 / 9, 192 10 / 12, 384 11 / 16
+    if (longest < 7) return false;               // block tiles are as short: k below 1792, 128 workgroups 10 / 9, 192 10 / 12, 384 11 / 16
     for (int i = 0; i < kRanges; ++i)
-        if (T <= kTokens[i]) return wgs <= kLimits[scaled][shortest >= 24 ? 2 : shortest >= 16 ? 1 : 0][i];
+        if (T <= kTokens[i]) return wgs <= kLimits[scaled][longest >= 24 ? 2 : longest >= 16 ? 1 : 0][i];
     return false;
 }
 

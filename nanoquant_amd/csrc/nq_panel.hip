@@ -576,8 +576,9 @@ bool panel_applies(int count, int T, const int* K, const int* R, bool scaled) {
         // 8 tiles, 3.6 units: 27 against 24; 7 to 11 tiles, 7 to 25 units: 35 to 88 against 40 to 103).
         long wgs = 0;
         for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
-        if (longest > 16) return wgs > 88 && per_wg >= 3.0;
-        if (gemm_group_few_tiles(count, T, K, R, scaled)) return false;
+        const bool few = gemm_group_few_tiles(count, T, K, R, scaled);
+        if (longest > 16) return (wgs > 88 || !few) && per_wg >= 3.0;
+        if (few) return false;
         return fill >= 0.70 && (longest >= 16 ? per_wg >= 3.0 : longest >= 7 && per_wg >= 5.0);
     }
     if (per_wg < 3.0) return false;

@@ -62,3 +62,31 @@ def test_block_tiles_where_few_token_tiles_are_slower(dev, dtype, tokens, linear
     beside = ops.gemm_group_forward([x, x], terms, panel="never")[0]
     torch.cuda.synchronize()
     assert torch.equal(alone, beside)
+
+
+# (tokens, linears [(n, r, m)]): a first GEMM of 43, a second one of 16 k tiles beside ones of 4 and 6
+@pytest.mark.parametrize("tokens,linears", [
+    (256, [(11008, 1024, 256), (1024, 1024, 256)]),
+    (333, [(256, 4096, 512), (256, 1536, 1024), (256, 1536, 1024)]),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_the_longest_k_of_a_group_decides(dev, dtype, tokens, linears):
+    # the one of the long k gets the bits it gets alone: few-token tiles in both calls
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(dtype)
+    f32 = lambda t: t.float().cpu().numpy()
+    packed, xs, refs = [], [], []
+    for i, (n, r, m) in enumerate(linears):
+        vt, u, *scales = oracle.synth_term(m, n, r, 9600 + i)
+        sc = [to(s) for s in scales]
+        packed.append(packing.marlin_nanoquant_packer(torch.from_numpy(vt).T.contiguous().to(dev), torch.from_numpy(u).T.contiguous().to(dev), *sc))
+        xs.append(to(oracle.synth_x(tokens, n, 9610 + i)))
+        refs.append(oracle.layer_forward(f32(xs[-1]), vt, u, *(f32(s) for s in sc)))
+    print(f"mixed group {tokens} tokens {linears} {dtype}", flush=True)
+    alone = ops.gemm_group_forward(xs[:1], packed[:1])[0]
+    together = ops.gemm_group_forward(xs, packed)
+    torch.cuda.synchronize()
+    assert torch.equal(alone, together[0])
+    for y, ref in zip(together, refs):
+        # h and the result are rounded to the 16-bit type, as above
+        assert oracle.max_rel_err(f32(y), ref) < 3 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)
+    assert ops.panel_status(dev) == 0
