@@ -9,12 +9,18 @@
 // The input is staged as kF6Pieces numbers per element, u = x * s / 2^k ~ q0 + q1 / 2^4 + q2 / 2^9, each the fp6 number
 // nearest to what the ones before it left over; k is the power of two that brings the largest |u| of the element's UNIT
 // (128 consecutive columns) into (3.75, 7.5], the top of the fp6 range, and rides along as the block scale of the MFMA
-// (so do the factors 2^-4 and 2^-9).  Rounding to nearest leaves |error| <= 2^-12 for |u| >= 4 and <= 2^-13 below, of a unit
-// whose largest |u| is above 3.75: at most 2^-14.9 of the unit's maximum but for the few largest elements, where the 16-bit
-// staging has 2^-12 (fp16) and 2^-9 (bf16) of every element; since the maximum of 128 numbers is at most 11.3 times
-// their root mean square, the fp16 error of a unit is never the smaller one.  All signs are +-1 and products are exact,
-// so nothing is subtracted again afterwards; all pieces of a batch row add into one fp32 accumulator (batch 16) or two
-// (batch 8).  A unit that holds an infinity or a NaN gets the block scale NaN: its batch row comes out NaN.
+// (so do the factors 2^-4 and 2^-9).  Rounding to nearest leaves |error| <= 2^-12 for |u| >= 4 and <= 2^-13 below: an absolute
+// step of at most 2^-13.9 and 2^-14.9 of the unit's largest value, the same for all of its 128 columns.  16-bit staging errs
+// by a share of every element instead (2^-12 of it in fp16, 2^-9 in bf16) and not at all where x * s has 16 bits: it keeps
+// more of an element below some 2^-3 (fp16) or 2^-6 (bf16) of its unit's maximum, and one below 2^-15 of it is lost here.
+// What a sum keeps is decided by the large elements, and h, an fp32 vector, is not rounded to 16 bits either.  Error of a
+// whole linear against 64 bits (2-norm; 16-bit operands -> here, batch 8 and 16 alike, 1024 x 4096 to 4096 x 11008):
+//   channels of one size      fp16 2.9e-4 -> 1.0e-4, bf16 2.3e-3 -> 1.0e-4
+//   four channels 100 times   fp16 3.0e-4 -> 1.4e-4, bf16 2.4e-3 -> 1.4e-4;   1000 times  3.1e-4 -> 1.6e-4, 2.9e-3 -> 1.6e-4
+//   the same, s a power of 2  fp16 2.1e-4 -> 1.6e-4, bf16 1.6e-3 -> 1.5e-4;   1000 times  2.1e-4 -> 1.5e-4, 1.6e-3 -> 1.6e-4
+// All signs are +-1 and products are exact, so nothing is subtracted again afterwards; all pieces of a batch row add into one
+// fp32 accumulator (batch 16) or two (batch 8).  A unit that holds an infinity or a NaN gets the block scale NaN: its batch
+// row comes out NaN, as it does with 16-bit operands (whose class sums take an infinity from itself).
 //
 // Operand geometry (one-hot operands on gfx950): lane (i = l & 15, g = l >> 4) supplies
 //   A (fp4, 4 dwords): row i, k = 32 g + idx, idx = 8 d + e for nibble e of dword d;

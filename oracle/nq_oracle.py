@@ -26,11 +26,14 @@ checkout):
                           round to nearest even) and the three-piece decomposition, with one power-of-two scale
                           per block of 128 columns, in which the gfx950 run-list kernel stages its input; lets a
                           test state exactly what that kernel must compute
+  fp6_e2m3_round / fp6_pieces / staged_input_fp6   the same for its long lists at batch 8 and 16: OCP e2m3 numbers,
+                          pieces in units of 1, 2^-4 and 2^-9, one power-of-two scale per block of 128 columns
   max_rel_err / elementwise_err   the two error figures of the tests: max|dy| / max|y_ref| (the tolerance
                           metric) and max(|dy| / (|y_ref| + 0.1 rms(y_ref))) (every element judged on its own)
 
 Pinning of the fp8 helpers: against torch.float8_e4m3fn conversion on every finite fp8 value, on midpoints and on
-random inputs, and against the closed-form error bound of the decomposition (tests/test_oracle_layer.py).
+random inputs, and against the closed-form error bound of the decomposition; of the fp6 helpers: against the table of
+the 32 magnitudes of the format, its midpoints, and the closed-form bound (tests/test_oracle_layer.py).
 
 Pinning (tests/test_oracle_*.py): pack/unpack against hand-derived known-answer words and the
 committed fixtures in tests/golden/, a brute-force per-bit Python loop, the popcount and
@@ -313,6 +316,42 @@ def staged_input(v, pieces: int = 3, block: int = 128) -> np.ndarray:
                 continue
             s = np.exp2(7 - np.floor(np.log2(mx)))
             out[b, c:c + block] = fp8_pieces(seg * s, pieces).sum(axis=0) / s
+    return out
+
+
+def fp6_e2m3_round(v) -> np.ndarray:
+    """Round to the nearest OCP e2m3 number (ties to even; spacing 1/8 below 2, 1/4 below 4, 1/2 up to the largest, 7.5)."""
+    v = np.asarray(v, dtype=np.float64)
+    a = np.abs(v)
+    q = np.exp2(np.clip(np.floor(np.log2(np.where(a > 0, a, 1.0))), 0, 2) - 3)
+    return np.sign(v) * np.minimum(np.round(a / q) * q, 7.5)
+
+
+def fp6_pieces(u, shifts=(0, 4, 9)) -> np.ndarray:
+    """[pieces, ...]: piece k is the multiple of 2^-shifts[k] times an fp6 number nearest to what is left of u."""
+    rest = np.array(u, dtype=np.float64)
+    out = []
+    for s in shifts:
+        out.append(fp6_e2m3_round(rest * 2.0 ** s) / 2.0 ** s)
+        rest = rest - out[-1]
+    return np.stack(out)
+
+
+def staged_input_fp6(v, block: int = 128, shifts=(0, 4, 9)) -> np.ndarray:
+    """What the run-list kernel multiplies the signs with in long lists at batch 8 and 16, per row of v [batch, K]: every
+    block of 128 columns scaled by the power of two that brings its max |v| into (3.75, 7.5], cut into fp6 pieces, summed
+    and scaled back."""
+    v = np.asarray(v, dtype=np.float64)
+    out = np.zeros_like(v)
+    for b in range(v.shape[0]):
+        for c in range(0, v.shape[1], block):
+            seg = v[b, c:c + block]
+            mx = np.abs(seg).max()
+            if mx == 0:
+                continue
+            e = np.floor(np.log2(mx))
+            s = np.exp2(2 - e - (mx > 1.875 * np.exp2(e)))
+            out[b, c:c + block] = fp6_pieces(seg * s, shifts).sum(axis=0) / s
     return out
 
 

@@ -170,6 +170,43 @@ def test_three_fp8_pieces_reproduce_the_input():
     assert np.array_equal(oracle.staged_input(np.zeros((1, 64))), np.zeros((1, 64)))
 
 
+def test_fp6_rounding_matches_the_format():
+    # e2m3, bias 1: subnormals k / 8, then (1 + k / 8) 2^(e - 1) for e = 1 .. 3
+    mags = [k / 8 for k in range(8)] + [(1 + k / 8) * 2.0 ** (e - 1) for e in (1, 2, 3) for k in range(8)]
+    assert len(set(mags)) == 32 and max(mags) == 7.5
+    grid = np.array(mags)
+    both = np.concatenate([grid, -grid])
+    assert np.array_equal(oracle.fp6_e2m3_round(both), both)
+    mid = (grid[:-1] + grid[1:]) / 2                       # ties: the neighbour whose last mantissa bit (code) is even
+    even = np.where(np.arange(31) % 2 == 0, grid[:-1], grid[1:])
+    assert np.array_equal(oracle.fp6_e2m3_round(mid), even) and np.array_equal(oracle.fp6_e2m3_round(-mid), -even)
+    x = np.random.default_rng(2).uniform(-7.5, 7.5, 20000)
+    nearest = both[np.abs(x[:, None] - both[None, :]).argmin(axis=1)]
+    assert np.array_equal(oracle.fp6_e2m3_round(x), nearest)
+    assert oracle.fp6_e2m3_round(9.0) == 7.5
+
+
+def test_three_fp6_pieces_reproduce_the_input_up_to_a_step_of_the_units_maximum():
+    rng = np.random.default_rng(3)
+    u = np.concatenate([rng.uniform(-7.5, 7.5, 100000), rng.normal(0, 1e-3, 20000), [0.0, 7.5, -4.0, 3.75]])
+    p = oracle.fp6_pieces(u)
+    assert np.abs(p * np.array([1.0, 2.0 ** 4, 2.0 ** 9])[:, None]).max() <= 7.5
+    err = np.abs(p.sum(axis=0) - u)
+    assert np.all(err <= np.where(np.abs(u) >= 4, 2.0 ** -12, 2.0 ** -13))
+    assert err[np.abs(u) < 4].max() > 0.9 * 2.0 ** -13     # the bound is reached
+    assert np.abs(oracle.fp6_pieces(u, (0, 4)).sum(axis=0) - u).max() > 2.0 ** -9
+    # whole vectors: an absolute step of the block's maximum whatever the element, other blocks untouched by an outlier
+    v = rng.normal(0, 0.02, (2, 512))
+    v[0, 130] = 50.0
+    sv = oracle.staged_input_fp6(v)
+    for c in range(0, 512, 128):
+        mx = np.abs(v[:, c:c + 128]).max(axis=1, keepdims=True)
+        assert np.all(np.abs(sv - v)[:, c:c + 128] <= 2.0 ** -13.9 * mx)
+    assert np.abs(sv - v)[0, 128:256].max() > 100 * np.abs(sv - v)[0, :128].max()
+    assert np.array_equal(oracle.staged_input_fp6(v * 8.0), sv * 8.0)
+    assert np.array_equal(oracle.staged_input_fp6(np.zeros((1, 64))), np.zeros((1, 64)))
+
+
 def test_error_figures_known_answers():
     ref = np.array([3.0, -4.0, 0.0, 5.0])                              # rms = sqrt(50 / 4)
     y = ref + np.array([0.0, 0.5, 0.25, -1.0])
