@@ -557,18 +557,18 @@ def main():
         mods = [[decode_module(lin) for lin in layer] for layer in layers]
         for layer in mods:
             for mod in layer:
-                mod.mfma_from_rows = 3         # opt in to the few-token MFMA tiles from 3 rows on
-                mod.prepare_mfma_route()       # set-up: otherwise the first call of 3 or more rows builds the tiles
+                mod.mfma_from_rows = 17        # opt in to the few-token MFMA tiles where the decode kernels take a second pass
+                mod.prepare_mfma_route()       # set-up: otherwise the first such call builds the tiles
         by_rows = {}
         with torch.no_grad():
-            for rows in (1, 2, 4, 16):
+            for rows in (1, 2, 4, 16, 32):
                 xs_m = {n: torch.randn(rows, n, device=dev).to(torch.float16) for n in (4096, 11008)}
                 fns = [(lambda layer=layer: [mod(xs_m[mod.in_features]) for mod in layer]) for layer in mods]
                 by_rows[str(rows)] = round(timed(fns, 2 * len(layers), len(layers)) * 1e3, 1)
         extra["module_forward_us_per_layer_by_rows"] = dict(
             by_rows, note="NanoQuantLinear.forward of 7 modules prepared with kernel_type='gemv', graph replays over the "
-                          "rotating weight copies: one decode launch per linear up to 2 rows, the few-token MFMA tiles "
-                          "(mfma_from_rows = 3, built once from the decode words) from 3 rows on")
+                          "rotating weight copies: the decode kernels up to 16 rows, the few-token MFMA tiles "
+                          "(mfma_from_rows = 17, built once from the decode words) above")
         del mods
         # ---- prefill GEMM over the three distinct linear shapes of the layer ----
         # Timed as HIP graph replays: through Python the two-GEMM op costs more host time than GPU time.

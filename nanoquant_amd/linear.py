@@ -51,8 +51,9 @@ class NanoQuantLinear(nn.Module):
         # expired wait raises; the first launch of a list is always checked.  0: only `fused_status()` tells.
         self.fused_status_every = 256
         # Opt-in (0: never): a module prepared for decode ("gemv") sends calls of at least this many rows to the
-        # few-token MFMA tiles of the prefill path, whose cost does not grow with the row count while that of the
-        # decode kernels does; 3 is the break-even on a Llama-2-7B layer.  The price is a second copy of the packed
+        # few-token MFMA tiles of the prefill path.  17 is the break-even: the decode kernels run 16 rows at a time (the
+        # seven linears of a Llama-2-7B layer, one call each, us on 1 / 4 / 16 / 17 / 32 / 64 rows: decode 69 / 74 / 94 / 157 /
+        # 179 / 349, tiles 108 / 109 / 112 / 113 / 116 / 121).  The price is a second copy of the packed
         # factors (the prefill tiles, built once from the decode words on the device, on the first such call or by
         # `prepare_mfma_route()`, and kept beside them), and results that differ in the last bits from the decode
         # kernels' (other order of the fp32 additions, h rounded to 16 bits in between).  Needs
