@@ -174,42 +174,6 @@ __device__ __forceinline__ void emit_rows(const RunStage& st, int row_end, bool 
     }
 }
 
-// Called by one wavefront: waits until the stages that `st` depends on are complete in launch `gen`; true if the bound ran
-// out (or another workgroup's did).
-__device__ __forceinline__ bool wait_for_stages(const RunStage& st, unsigned long long gen, const unsigned long long* counters,
-                                                unsigned* status, unsigned spin_limit) {
-    const int lane = threadIdx.x & 63;
-    unsigned spins = 0;
-    bool bad = false;
-#pragma unroll 1
-    for (int which = 0; which < 2 && !bad; ++which) {
-        const int d = which ? st.dep2 : st.dep;
-        if (d < 0 || (which && st.addend_local)) continue;
-        const unsigned long long want = (gen + 1) * (unsigned long long)(which ? st.dep2_segs : st.dep_segs);
-        while (true) {
-            unsigned long long c = 0;
-            if (lane < kSubCounters)
-                c = __hip_atomic_load(counters + ((size_t)d * kSubCounters + lane) * kCounterStride,
-                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            c += __shfl_xor(c, 1, kWave);
-            c += __shfl_xor(c, 2, kWave);
-            c += __shfl_xor(c, 4, kWave);
-            const unsigned long long sum0 = __shfl(c, 0, kWave);
-            if (sum0 >= want) break;
-            __builtin_amdgcn_s_sleep(8);   // pollers must not crowd out the producers' atomics
-            unsigned flagged = 0;
-            if (lane == 0) flagged = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            flagged = __shfl(flagged, 0, kWave);
-            if (++spins >= spin_limit || flagged) {
-                if (lane == 0) atomicOr(status, 1u);   // bounded wait: flag it, let the grid drain
-                bad = true;
-                break;
-            }
-        }
-    }
-    return bad;
-}
-
 // ARITH: 1 = MFMA with 16-bit operands, 2 = MFMA with one-bit fp4 weights and fp8 pieces of the input (batch <= 4).
 // DET, fp4 x fp8 arithmetic: row sums that do not depend on the order in which the wavefronts of a workgroup add
 // their partial sums.  Every partial sum is rounded to a grid fine enough (2^-22 of columns x largest staged value, a
@@ -440,7 +404,37 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
 
             if ((st.dep >= 0 || st.dep2 >= 0) && !aborted) {
                 if (tid < kWave) {                               // wavefront 0 polls; lanes 0..7 own one sub-counter each
-                    const bool bad = wait_for_stages(st, gen_raw / members, counters, status, spin_limit);
+                    // (written out: as a call of wait_for_stages, which is the same, it costs the instances for batch 1, 2 and 4
+                    // scalar registers: one 2048 x 2048 linear 12.75 us against 12.45)
+                    const unsigned long long gen = gen_raw / members;
+                    unsigned spins = 0;
+                    bool bad = false;
+#pragma unroll 1
+                    for (int which = 0; which < 2 && !bad; ++which) {
+                        const int d = which ? st.dep2 : st.dep;
+                        if (d < 0 || (which && st.addend_local)) continue;
+                        const unsigned long long want = (gen + 1) * (unsigned long long)(which ? st.dep2_segs : st.dep_segs);
+                        while (true) {
+                            unsigned long long c = 0;
+                            if (tid < kSubCounters)
+                                c = __hip_atomic_load(counters + ((size_t)d * kSubCounters + tid) * kCounterStride,
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            c += __shfl_xor(c, 1, kWave);
+                            c += __shfl_xor(c, 2, kWave);
+                            c += __shfl_xor(c, 4, kWave);
+                            const unsigned long long sum0 = __shfl(c, 0, kWave);
+                            if (sum0 >= want) break;
+                            __builtin_amdgcn_s_sleep(8);   // pollers must not crowd out the producers' atomics
+                            unsigned flagged = 0;
+                            if (tid == 0) flagged = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            flagged = __shfl(flagged, 0, kWave);
+                            if (++spins >= spin_limit || flagged) {
+                                if (tid == 0) atomicOr(status, 1u);   // bounded wait: flag it, let the grid drain
+                                bad = true;
+                                break;
+                            }
+                        }
+                    }
                     if (bad && tid == 0) s_flag = 1;
                     // 16-bit input written by another stage of this launch: ordinary loads follow, so the
                     // caches of this CU / XCD have to drop what they hold (rare; h and addend never need it).
@@ -1034,6 +1028,42 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
         __hip_atomic_fetch_add(exit_sub + (size_t)(wg & (kExitSubs - 1)) * kCounterStride, 1ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// Called by one wavefront: waits until the stages that `st` depends on are complete in launch `gen`; true if the bound ran
+// out (or another workgroup's did).
+__device__ __forceinline__ bool wait_for_stages(const RunStage& st, unsigned long long gen, const unsigned long long* counters,
+                                                unsigned* status, unsigned spin_limit) {
+    const int lane = threadIdx.x & 63;
+    unsigned spins = 0;
+    bool bad = false;
+#pragma unroll 1
+    for (int which = 0; which < 2 && !bad; ++which) {
+        const int d = which ? st.dep2 : st.dep;
+        if (d < 0 || (which && st.addend_local)) continue;
+        const unsigned long long want = (gen + 1) * (unsigned long long)(which ? st.dep2_segs : st.dep_segs);
+        while (true) {
+            unsigned long long c = 0;
+            if (lane < kSubCounters)
+                c = __hip_atomic_load(counters + ((size_t)d * kSubCounters + lane) * kCounterStride,
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            c += __shfl_xor(c, 1, kWave);
+            c += __shfl_xor(c, 2, kWave);
+            c += __shfl_xor(c, 4, kWave);
+            const unsigned long long sum0 = __shfl(c, 0, kWave);
+            if (sum0 >= want) break;
+            __builtin_amdgcn_s_sleep(8);   // pollers must not crowd out the producers' atomics
+            unsigned flagged = 0;
+            if (lane == 0) flagged = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            flagged = __shfl(flagged, 0, kWave);
+            if (++spins >= spin_limit || flagged) {
+                if (lane == 0) atomicOr(status, 1u);   // bounded wait: flag it, let the grid drain
+                bad = true;
+                break;
+            }
+        }
+    }
+    return bad;
 }
 
 // The run list at batch 8 and 16 with every word in tile order: one-bit fp4 weights x fp6 pieces (nq_fp6.h).  Slices, waits

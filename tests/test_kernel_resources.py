@@ -59,3 +59,8 @@ def test_owned_row_pairs_at_batch_4_spill_no_vector_register(kernels, dtype):
 def test_short_fp16_lists_at_batch_4_spill_no_more_than_five(kernels):
     # 16-bit operands: 5 of 128 (24 bytes) with the class operands of eight steps in flight; every further one showed in time
     assert _stream_kernel(kernels, 0, 4, 1, 0, 0, 0)[".vgpr_spill_count"] <= 5
+
+
+def test_short_lists_at_batch_1_spill_no_more_scalar_registers_than_with_the_wait_written_out(kernels):
+    # 103 of the slice's record and the fetch addresses; a wait in a function of its own made it 107 and one linear 2 % slower
+    assert _stream_kernel(kernels, 0, 1, 2, 1, 0, 0)[".sgpr_spill_count"] <= 103
