@@ -294,10 +294,25 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
         for (int sg = wg, nth = 0;; ++nth) {
             RunSegment seg;
             RunStage st;
-            // In a scope of its own: with the record's name alive to the end of the slice the compiler spills vector registers
-            // in the batch 4 instances (us per launch, without and with the scope: one Llama-2-7B layer, fp16 26.3 and 25.6;
-            // three layers, both types 34.6 and 33.1).
-            {
+            // The same statements twice: where the record has a name of its own scope, the compiler spills fewer vector registers
+            // in most instances, and more in the reproducible ones for row-major words and owned row pairs (us per launch,
+            // below / above: one Llama-2-7B layer at batch 4, fp16 26.3 / 25.6; three layers 34.6 / 33.1; reproducible
+            // row-major list at batch 1, one layer 22.3 / 26.7).
+            if constexpr (DET && (OWN || !TILED)) {
+                if (nth) {
+                    if (sg_more >= sg_more_end) break;
+                    sg = sg_more++;
+                }
+                seg = slices[sg].seg;
+                st = slices[sg].st;
+                if (nth == 0) {
+                    sg_more = slices[sg].more_begin;
+                    sg_more_end = slices[sg].more_end;
+                    if (seg.stage < 0) break;           // nothing for this workgroup
+                }
+                if (st.in_ext) st.in = ext_in;          // bound with the launch
+                if (st.out_ext) st.out = ext_out;
+            } else {
                 if (nth) {
                     if (sg_more >= sg_more_end) break;
                     sg = sg_more++;
@@ -308,9 +323,9 @@ __global__ __launch_bounds__(THREADS) void gemv_stream_kernel(int nstages, const
                 if (nth == 0) {
                     sg_more = sl.more_begin;
                     sg_more_end = sl.more_end;
-                    if (seg.stage < 0) break;               // nothing for this workgroup
+                    if (seg.stage < 0) break;
                 }
-                if (st.in_ext) st.in = ext_in;              // bound with the launch
+                if (st.in_ext) st.in = ext_in;
                 if (st.out_ext) st.out = ext_out;
             }
             const BitsView bv = bits_view(st);

@@ -64,3 +64,8 @@ def test_short_fp16_lists_at_batch_4_spill_no_more_than_five(kernels):
 def test_short_lists_at_batch_1_spill_no_more_scalar_registers_than_with_the_wait_written_out(kernels):
     # 103 of the slice's record and the fetch addresses; a wait in a function of its own made it 107 and one linear 2 % slower
     assert _stream_kernel(kernels, 0, 1, 2, 1, 0, 0)[".sgpr_spill_count"] <= 103
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_reproducible_row_major_lists_at_batch_1_spill_no_vector_register(kernels, dtype):
+    assert _stream_kernel(kernels, dtype, 1, 2, 0, 1, 0)[".vgpr_spill_count"] == 0
