@@ -619,11 +619,12 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 // More than kKwaveGroupMaxTokens tokens: whether the few-token tiles are still the faster ones.  A block tile walks the whole
 // k by itself, at 1.6 us per weight tile however few workgroups there are, while the four wavefronts of a few-token tile
 // share the k and there are eight times as many workgroups, each of which reads its 32 tokens again for every 32 to 128 rows.
-// The limits are block workgroups (64 tokens x 128 rows), from 2494 pairs of timings: k of 5 to 48 tiles, 256 to 8704
+// The limits are block workgroups (64 tokens x 128 rows), from 2494 sets of timings: k of 5 to 48 tiles, 256 to 8704
 // rows, 161 to 2048 tokens, GEMMs with s_in (the first of a linear) and without (the second, whose block tiles are the faster
-// ones).  At 512 tokens, and at every further multiple, eight token blocks share slabs in one L2 each and block tiles gain;
-// above 1024 tokens the inputs no longer stay in the L2s and the few-token tiles lose.  us per call of a linear whose other
-// GEMM is a few, block tiles / few-token tiles, by block workgroups and tokens:
+// ones).  Two things move them.  Block tiles whose workgroups share slabs in one L2 (group_mode 0 and 1: four or eight token
+// blocks, or a multiple of eight) are faster than at the token counts between; and above 1024 tokens the inputs no longer stay
+// in the L2s, so that the few-token tiles lose.  us per call of a linear whose other GEMM is a few, block tiles / few-token
+// tiles, by block workgroups and tokens:
 //   with s_in, k 4096   64 at 256: 30 / 17    192 at 512: 33 / 29      300 at 900: 41 / 38      96 at 3072: 30 / 39
 //   without             64 at 256: 28 / 18    192 at 512: 28.5 / 31    120 at 900: 34 / 31      64 at 2048: 33 / 37
 //   with s_in, k 1792   64 at 512: 21 / 16    120 at 900: 22 / 20.6    192 at 1024: 24 / 24.4   192 at 1536: 22 / 24
@@ -633,21 +634,30 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 // (with s_in, k 11008 and 1024, 1024 rows each: 64 workgroups at 256 tokens 69 / 34, 128 at 512: 72 / 43; k 4096 and 1024, 1024
 // and 512 rows: 96 at 512: 34 / 27; k 2304 and 768, 4096 rows each: 192 at 161: 25 / 22).
 bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool scaled) {
-    constexpr int kRanges = 6;
-    constexpr int kTokens[kRanges] = {400, 512, 768, 1280, 1536, 2048};
-    constexpr int kLimits[2][3][kRanges] = {
-        {{150, 96, 144, 80, 0, 0}, {288, 96, 200, 160, 48, 0}, {360, 360, 360, 160, 96, 0}},            // no s_in; k of 7, 16, 24 tiles
-        {{192, 192, 160, 160, 48, 0}, {360, 360, 360, 160, 96, 64}, {360, 360, 360, 320, 192, 128}}};   // s_in
+    // [s_in][k of 7, 16, 24 tiles and more][token range]
+    constexpr int kBetween[4] = {512, 768, 1024, 1536};
+    constexpr int kBetweenLimits[2][3][4] = {{{160, 160, 150, 80}, {360, 200, 180, 160}, {360, 360, 480, 160}},
+                                             {{192, 192, 180, 160}, {360, 360, 300, 160}, {360, 360, 480, 360}}};
+    constexpr int kShared[5] = {256, 512, 1024, 1536, 2048};
+    constexpr int kSharedLimits[2][3][5] = {{{128, 96, 32, 0, 0}, {288, 96, 128, 48, 0}, {360, 360, 160, 96, 0}},
+                                            {{256, 256, 128, 48, 0}, {288, 360, 192, 96, 64}, {360, 360, 512, 288, 128}}};
     if (T <= kKwaveGroupMaxTokens) return true;
+    const int gy = (T + 63) / 64;
     long wgs = 0;
     int longest = 0;
     for (int p = 0; p < count; ++p) {
-        wgs += (long)((R[p] + 127) / 128) * ((T + 63) / 64);
+        wgs += (long)((R[p] + 127) / 128) * gy;
         longest = K[p] / kTileK > longest ? K[p] / kTileK : longest;
     }
     if (longest < 7) return false;               // block tiles are as short: k below 1792, 128 workgroups 10 / 9, 192 10 / 12, 384 11 / 16
-    for (int i = 0; i < kRanges; ++i)
-        if (T <= kTokens[i]) return wgs <= kLimits[scaled][longest >= 24 ? 2 : longest >= 16 ? 1 : 0][i];
+    const int k = longest >= 24 ? 2 : longest >= 16 ? 1 : 0;
+    if (group_mode(gy) == 2) {
+        for (int i = 0; i < 4; ++i)
+            if (T <= kBetween[i]) return wgs <= kBetweenLimits[scaled][k][i];
+    } else {
+        for (int i = 0; i < 5; ++i)
+            if (T <= kShared[i]) return wgs <= kSharedLimits[scaled][k][i];
+    }
     return false;
 }
 

@@ -572,14 +572,15 @@ bool panel_applies(int count, int T, const int* K, const int* R, bool scaled) {
         // Above the few-token counts.  A long k (more than 16 tiles): panels from some 90 block workgroups on (us, panels
         // against few-token tiles: 56 workgroups 42 / 26, 88 40 / 39, 112 42 / 50, 168 49 / 53; block tiles 60 to 80).
         // Up to 16 tiles panels start where the few-token tiles end; a k of less than 7 tiles, or a short one with less than
-        // 5 units per workgroup, is faster on block tiles (5 tiles, 3.2 units: 26 against 21; 10.5 units: 50 against 47;
-        // 8 tiles, 3.6 units: 27 against 24; 7 to 11 tiles, 7 to 25 units: 35 to 88 against 40 to 103).
+        // 5 units per workgroup (16 tiles: 4.2), is faster on block tiles (5 tiles, 3.2 units: 26 against 21; 10.5 units: 50
+        // against 47; 8 tiles, 3.6 units: 27 against 24; 7 to 11 tiles, 7 to 25 units: 35 to 88 against 40 to 103; 16 tiles without
+        // s_in, 3 and 3.75 units: 37 and 38 against 28 and 34, 4.25 and 4.7: 38 and 39 against 39 and 41).
         long wgs = 0;
         for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
         const bool few = gemm_group_few_tiles(count, T, K, R, scaled);
         if (longest > 16) return (wgs > 88 || !few) && per_wg >= 3.0;
         if (few) return false;
-        return fill >= 0.70 && (longest >= 16 ? per_wg >= 3.0 : longest >= 7 && per_wg >= 5.0);
+        return fill >= 0.70 && (longest >= 16 ? per_wg >= 4.2 : longest >= 7 && per_wg >= 5.0);
     }
     if (per_wg < 3.0) return false;
     // up to two token blocks the few-token tiles are the alternative, and a strong one; beyond, panels win more easily
