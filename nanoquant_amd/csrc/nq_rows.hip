@@ -579,6 +579,7 @@ static hipError_t launch_any(int count, const RowsStage* s, int batch, hipStream
         vec = vec && stage_vec(s[i]);
     }
     if (!vec) {                                          // the same sums in the same order from 2-byte loads
+        if (batch == 1) return launch_group<DT, SCALED, 1, 1, NT, false>(count, s, batch, stream);
         if (batch <= 4) return launch_group<DT, SCALED, 4, 1, NT, false>(count, s, batch, stream);
         return launch_group<DT, SCALED, 16, 1, NT, false>(count, s, batch, stream);
     }
