@@ -51,7 +51,8 @@ int nq_device_query(int attr, int* value);   /* current device */
 /* Decode path, one term:  y = s_out * (U (s_mid * (Vt (s_in * x)))).
  * Replaces nanoquant_dyn_forward (kernel/cuda/gemv_kernel.cu:308-429; schema kernel/pybind.cpp:86-90).
  *   x [batch, n], s_in [n], s_mid [r] or NULL, s_out [m], y [batch, m]: all of `dtype`, contiguous.
- *   h_scratch: fp32 [batch, r] owned by the caller (the reference allocates `interm` itself, :345).
+ *   h_scratch: storage of the size and alignment of an fp32 [batch, r], owned by the caller (the reference allocates
+ *   `interm` itself, :345).  Its contents are the library's own: 16-bit values in padded rows, not fp32.
  * Any batch >= 1 is accepted; every packed word is read once per 16 batch rows. */
 int nq_gemv_forward(const void* x, const void* s_in, const uint32_t* vt_bits, const void* s_mid,
                     const uint32_t* u_bits, const void* s_out, float* h_scratch, void* y,
@@ -66,7 +67,7 @@ int nq_gemv_forward_bias(const void* x, const void* s_in, const uint32_t* vt_bit
 
 /* nq_gemv_forward_bias for callers that cannot allocate device memory or hand over a workspace: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference (whose
- * wrapper allocates `interm` with torch::empty on every call, kernel/cuda/gemv_kernel.cu:345).  The fp32
+ * wrapper allocates `interm` with torch::empty on every call, kernel/cuda/gemv_kernel.cu:345).  The
  * intermediate h lives in a device array inside the library, NQ_NOALLOC_MAX_H_FLOATS floats (1 MiB) per GPU, held
  * until the process ends: batch * r above that returns NQ_ERR_SCRATCH_LIMIT.  The call allocates and frees nothing.
  * All calls on one GPU share that array: calls that overlap in time on one GPU (two streams, two threads) race on
@@ -79,7 +80,7 @@ int nq_gemv_forward_noalloc(const void* x, const void* s_in, const uint32_t* vt_
 
 /* Decode path, sum of `nterms` terms that share x (the mixture-of-rank layer; no counterpart in the
  * reference's code, defined as the sum of single-term layers).  Arrays hold one pointer / rank per
- * term; s_mid[t] may be NULL.  h_scratch: fp32 [batch, max r]; y_scratch: fp32 [batch, m]. */
+ * term; s_mid[t] may be NULL.  h_scratch: storage of an fp32 [batch, max r], contents as above; y_scratch: fp32 [batch, m]. */
 int nq_gemv_mixture(const void* x, const void* const* s_in, const uint32_t* const* vt_bits,
                     const void* const* s_mid, const uint32_t* const* u_bits, const void* const* s_out,
                     const int* r, int nterms, float* h_scratch, float* y_scratch, void* y,
@@ -182,13 +183,13 @@ int nq_runlist_set_deterministic(nq_runlist_plan* plan, int on);
  * launches per nq_gemv_group_max() linears (all first stages, then all second stages) instead of the two launches
  * per linear of nq_gemv_forward and of the reference (kernel/cuda/gemv_kernel.cu:406-425), without a built run list:
  * nothing to prepare, any pointers on every call, no requirement on what else the GPU runs.
- *   linears: x_from = y_from = -1, no addend, out_f32 = 0, tiled = 0; h buffers distinct, fp32 [batch, r] each.
- *   Pieces of 1, 2 and 4 batch rows are grouped; pieces of 8 and 16 rows take two launches per linear.
+ *   linears: x_from = y_from = -1, no addend, out_f32 = 0, tiled = 0; h buffers distinct, storage of an fp32 [batch, r] each.
+ *   Batch rows are taken 16 at a time, at any count.
  * one_launch = 1: ONE ordinary launch per group instead of two.  The workgroups of the second stages sit behind those
- * of the first in the same grid, fetch their first sign words, and wait on flags until their linear's h is complete
+ * of the first in the same grid and wait on flags, before anything else, until their linear's h is complete
  * (workgroups start in the order of their ids, so whatever a workgroup waits for is running or done: no resident
  * grid is needed).  On MI355X the signalling through device-coherent memory costs more than the launch boundary it
- * replaces (a Llama-2-7B layer at batch 1 in four groups: 82 us with one launch per group, 48 us with two); the
+ * replaces (a Llama-2-7B layer at batch 1 in four groups: 76 us with one launch per group, 44 us with two); the
  * switch is kept for measurement and for callers that are charged per launch.  Its flags live in a device
  * array inside the library (4.5 MiB per GPU, 256 slots dealt round robin, every launch puts its slot back to zero);
  * the first call on each device looks up its address and should be made outside graph capture.  The wait is bounded
@@ -202,7 +203,7 @@ int nq_gemv_group_status(int* status_out, void* stream);
  * host; every kernel still runs to its end. */
 int nq_gemv_group_set_spin_limit(unsigned polls);
 
-/* One matmul-free stage: out[b,row] = s_row[row] * sum_c sgn(bits[row,c]) * in[b,c] * s_col[c].
+/* One stage on its own: out[b,row] = s_row[row] * sum_c sgn(bits[row,c]) * in[b,c] * s_col[c].
  * Replaces nanoquant_stage1_dyn_kernel / nanoquant_stage2_dyn_kernel launches
  * (kernel/cuda/gemv_kernel.cu:283-301).  in/out are `dtype`; s_col, s_row may be NULL. */
 int nq_gemv_stage(const void* in, const void* s_col, const uint32_t* bits, const void* s_row, void* out,
@@ -242,9 +243,11 @@ int nq_gemm_nanoquant_bias(const void* x, const uint32_t* vt_tiles, const uint32
 /* Several terms with the same token count in two launches instead of two per term: the first GEMMs of all
  * terms, then the second ones (the projections of a decoder block that read the same tokens: q/k/v, gate/up, or
  * independent linears of a layer).  Up to 128 tokens a single term cannot fill the device and is bound by launch
- * and load latencies; grouped, the same launches carry several times the work.  Above 160 tokens a group
- * large enough to fill the device runs on 64-token block tiles whose workgroups walk the whole k of their term (no k-split, no scratch): together the
- * terms fill the device where one term needs a k-split and a finish launch to do so.  Only when some terms have
+ * and load latencies; grouped, the same launches carry several times the work.  Above 160 tokens a group large enough to
+ * fill the device runs on 64-token block tiles whose workgroups walk the whole k of their term (no k-split, no scratch):
+ * together the terms fill the device where one term needs a k-split and a finish launch to do so; smaller groups stay on
+ * the few-token tiles.  The choice is made per launch from all of its terms, so above 160 tokens the last bits of a term's
+ * result may depend on what shares the call.  Only when some terms have
  * s_in and others do not does the call run the terms one after another (nq_gemm_nanoquant_bias); it then needs
  * their scratch, max over terms of nq_gemm_scratch_bytes for both GEMMs (may be NULL otherwise).
  * count <= nq_gemm_group_max(); h and y of different terms must not coincide.  No counterpart in the reference, which launches each linear by itself

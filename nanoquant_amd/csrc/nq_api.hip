@@ -153,7 +153,8 @@ int nq_gemv_group_status(int* status_out, void* stream) {
 }
 
 // ---- the allocation-free variant of nq_gemv_forward_bias ---------------------------------------------
-// The fp32 intermediate h lives in a file-scope device array instead of a caller's buffer.  In host code the
+// The intermediate h lives in a file-scope device array of the size of an fp32 [batch, r] (it holds 16-bit values, rows padded
+// to a multiple of eight) instead of a caller's buffer.  In host code the
 // array's name is only a handle: its device address is asked for once per device (each device holds its own copy)
 // and only that address is ever handed to a kernel.
 constexpr size_t kScratchFloats = NQ_NOALLOC_MAX_H_FLOATS;
@@ -414,7 +415,9 @@ int nq_runlist_build(const nq_linear* linears, int nlinears, int batch, int dtyp
     // 60000 rows x units per workgroup.  A shorter list gives a workgroup a few row pairs per slice for its eight wavefronts
     // and stages as much for them (us per launch, 16-bit operands against fp6, batch 8 / batch 16: two Llama-3-70B layers,
     // 52000: 85 / 125 against 89 / 130; three, 78000: 121 / 177 against 110 / 155; Llama-2-7B, 6 layers, 37000: 63 / 73
-    // against 57 / 77; 10 layers, 62000: 105 / 116 against 77 / 103; 32 layers: 295 / 320 against 204 / 247).
+    // against 57 / 77; 10 layers, 62000: 105 / 116 against 77 / 103; 32 layers: 295 / 320 against 204 / 247).  The line lies
+    // where every list that was measured above it gains; what separates the ones below is row pairs per slice rather than this
+    // product (six layers of the smaller shape would gain at batch 8 and not at 16, two of the larger one at neither).
     bool f6 = batch >= 8;
     if (f6) {
         long long work = 0;

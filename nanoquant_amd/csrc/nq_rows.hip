@@ -39,7 +39,11 @@ constexpr int kRowsMaxWaves = 8;     // wavefronts of a workgroup
 //   CUs run in rounds; with few rows a second block only makes a wavefront's chain longer)
 //   four wavefronts instead of eight                out 22016 of rank 2992  10.5 / 8.1 / 7.5  against 14.1 / 9.0 / 7.8
 //                                                   rank 2985 of 11008      12.4 / 8.4 / 7.1  against 10.3 / 7.1 / 5.8
-//   (many rows: more workgroups stay resident and each stages less; few rows: eight keep more loads in flight)
+//   (many rows: more workgroups stay resident and each stages less; few rows: eight keep more loads in flight).  The line
+//   between is a compromise over the batch sizes, since the split decides the order of the sums and must not depend on them: whole
+//   linears of 8192 to 14336 rows lose 3 to 5 % on four wavefronts at 1 to 8 rows (9216 x 4096, 1 row fp16: 10.0 against 9.4) and
+//   gain 11 to 15 % at 16 rows (13.8 against 15.4), from 14336 rows on four are level (2 %) or ahead at every batch size; below 8192
+//   rows they lose 1 to 6 % throughout (5120 x 8192: 12.3 against 11.6 at 8 rows).
 constexpr int kTwoBlocksFrom = 257;  // 16-row blocks of a launch, 5 batch rows and more
 constexpr int kFewWavesFrom = 8192;  // rows of a linear
 constexpr int kStagePitch = 1040;    // LDS bytes per staged input row of a chunk: 512 x 2 + 16 (8 lanes of an operand

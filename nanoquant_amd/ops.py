@@ -372,7 +372,7 @@ def gemv_forward_with_bias(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias):
 
 def gemv_group_forward(xs, linears, biases=None, outs=None, one_launch=False):
     """`[nanoquant_dyn_forward(x_i, *linears[i]) (+ biases[i])]` for independent linears in two launches per
-    `nq_gemv_group_max()` linears and piece of 1, 2 or 4 rows (`nq_gemv_forward_group`: all first stages, then all
+    `nq_gemv_group_max()` linears and piece of up to 16 rows (`nq_gemv_forward_group`: all first stages, then all
     second stages): the q/k/v or gate/up projections of a decoder layer at decode time, which the reference launches
     one module and two kernels at a time (modules/linear.py:121-130).  `xs`: one tensor [rows, n] for all linears or
     one per linear (same row count); `linears`: (scale_g, Ubits, scale_l, Vbits, scale_h) per linear, the operands of
@@ -680,7 +680,7 @@ def pack_gemm_tiles_device(words: torch.Tensor, rows_padded: int, k_padded: int,
 
 def gemv_stage_forward(inp: torch.Tensor, s_col: Optional[torch.Tensor], bits: torch.Tensor,
                        s_row: Optional[torch.Tensor]) -> torch.Tensor:
-    """One matmul-free stage on its own: out[b, row] = s_row[row] * sum_c sgn(bits[row, c]) * inp[b, c] * s_col[c]
+    """One stage on its own: out[b, row] = s_row[row] * sum_c sgn(bits[row, c]) * inp[b, c] * s_col[c]
     (what one of the reference's two launches computes, kernel/cuda/gemv_kernel.cu:283-301).  `bits` [rows,
     ceil(cols/32)] in the "half2" order; the result has inp's dtype."""
     if inp.dtype not in (torch.float16, torch.bfloat16):
