@@ -833,7 +833,7 @@ int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens,
     }
     // one stage: the panel launch where a workspace was given and the shapes make it the faster one
     auto stage = [&]() -> hipError_t {
-        if (have_ws && (panel_mode == NQ_PANEL_ALWAYS || nq::panel_applies(count, tokens, K, R, si[0] != nullptr)))
+        if (have_ws && (panel_mode == NQ_PANEL_ALWAYS || nq::panel_applies(count, x, tokens, K, R, si[0] != nullptr)))
             return nq::gemm_panel_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, panel_ws, g_panel_spin_limit.load(),
                                         (hipStream_t)stream);
         return nq::gemm_onebit_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, (hipStream_t)stream);

@@ -620,7 +620,7 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 // k by itself, at 1.6 us per weight tile however few workgroups there are, while the four wavefronts of a few-token tile
 // share the k and there are eight times as many workgroups, each of which reads its 32 tokens again for every 32 to 128 rows.
 // The limits are block workgroups (64 tokens x 128 rows), from 2494 sets of timings: k of 5 to 48 tiles, 256 to 8704
-// rows, 161 to 2048 tokens, GEMMs with s_in (the first of a linear) and without (the second, whose block tiles are the faster
+// rows, 161 to 2048 tokens, and from 1350 sets of two to eight equal terms, GEMMs with s_in (the first of a linear) and without (the second, whose block tiles are the faster
 // ones).  Two things move them.  Block tiles whose workgroups share slabs in one L2 (group_mode 0 and 1: four or eight token
 // blocks, or a multiple of eight) are faster than at the token counts between; and above 1024 tokens the inputs no longer stay
 // in the L2s, so that the few-token tiles lose.  us per call of a linear whose other GEMM is a few, block tiles / few-token
@@ -630,32 +630,41 @@ static hipError_t gemm_block_group(int dtype, int count, const void* const* x, c
 //   with s_in, k 1792   64 at 512: 21 / 16    120 at 900: 22 / 20.6    192 at 1024: 24 / 24.4   192 at 1536: 22 / 24
 //   without             96 at 512: 17.2 / 17  160 at 512: 17.5 / 19    128 at 1024: 17.6 / 20   192 at 1536: 19 / 25
 //   without, k 11008    128 at 512: 67 / 46   128 at 1024: 72 / 56     96 at 1536: 78 / 69      256 at 2048: 82 / 91
+// What is read again counts once per INPUT: terms of inputs of their own (every second GEMM, whose inputs are the h) bring as
+// many token rows as so many times the tokens, and beyond some 1800 of them the few-token tiles lose whatever the rest says
+// (three k of 4096 on 256 rows each, with s_in: 512 tokens 30 / 24, 640 32 / 29, 1024 31 / 39; six at 640: 33 / 47; the six on
+// one input: 400 tokens 30 / 21, 640 31 / 30, 1024 30 / 27).
 // The longest k of a group decides: the launch lasts as long as its block tiles, and the few-token tiles cost a short k little
 // (with s_in, k 11008 and 1024, 1024 rows each: 64 workgroups at 256 tokens 69 / 34, 128 at 512: 72 / 43; k 4096 and 1024, 1024
 // and 512 rows: 96 at 512: 34 / 27; k 2304 and 768, 4096 rows each: 192 at 161: 25 / 22).
-bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool scaled) {
+bool gemm_group_few_tiles(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
     // [s_in][k of 7, 16, 24 tiles and more][token range]
     constexpr int kBetween[4] = {512, 768, 1024, 1536};
     constexpr int kBetweenLimits[2][3][4] = {{{160, 160, 150, 80}, {360, 200, 180, 160}, {360, 360, 480, 160}},
                                              {{192, 192, 180, 160}, {360, 360, 300, 160}, {360, 360, 480, 360}}};
-    constexpr int kShared[5] = {256, 512, 1024, 1536, 2048};
-    constexpr int kSharedLimits[2][3][5] = {{{128, 96, 32, 0, 0}, {288, 96, 128, 48, 0}, {360, 360, 160, 96, 0}},
-                                            {{256, 256, 128, 48, 0}, {288, 360, 192, 96, 64}, {360, 360, 512, 288, 128}}};
+    constexpr int kShared[4] = {256, 512, 1024, 1536};
+    constexpr int kSharedLimits[2][3][4] = {{{128, 96, 32, 0}, {288, 96, 128, 48}, {360, 360, 160, 96}},
+                                            {{256, 256, 128, 48}, {288, 360, 192, 96}, {360, 360, 512, 288}}};
+    constexpr long kMostTokens = 1800;           // of all inputs together, weighed by their k
     if (T <= kKwaveGroupMaxTokens) return true;
     const int gy = (T + 63) / 64;
-    long wgs = 0;
+    long wgs = 0, tiles = 0;
     int longest = 0;
     for (int p = 0; p < count; ++p) {
         wgs += (long)((R[p] + 127) / 128) * gy;
         longest = K[p] / kTileK > longest ? K[p] / kTileK : longest;
+        bool seen = false;
+        for (int q = 0; q < p; ++q) seen = seen || x[q] == x[p];
+        if (!seen) tiles += K[p] / kTileK;
     }
+    if (T * tiles > kMostTokens * longest) return false;
     if (longest < 7) return false;               // block tiles are as short: k below 1792, 128 workgroups 10 / 9, 192 10 / 12, 384 11 / 16
     const int k = longest >= 24 ? 2 : longest >= 16 ? 1 : 0;
     if (group_mode(gy) == 2) {
         for (int i = 0; i < 4; ++i)
             if (T <= kBetween[i]) return wgs <= kBetweenLimits[scaled][k][i];
     } else {
-        for (int i = 0; i < 5; ++i)
+        for (int i = 0; i < 4; ++i)
             if (T <= kShared[i]) return wgs <= kSharedLimits[scaled][k][i];
     }
     return false;
@@ -667,7 +676,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
                              const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                              int T, const int* K, const int* R, hipStream_t stream) {
     if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
-    if (!gemm_group_few_tiles(count, T, K, R, s_in && s_in[0])) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
+    if (!gemm_group_few_tiles(count, x, T, K, R, s_in && s_in[0])) return gemm_block_group(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     const int gy = (T + 31) / 32;
     int rt = 4;                                  // widest row blocks that still leave two workgroups per CU
     for (; rt > 1; rt /= 2) {

@@ -93,7 +93,7 @@ hipError_t gemm_onebit(int dtype, const void* x, const uint32_t* tiles, const vo
 
 // Up to gemm_group_max() GEMMs on the same token count in one launch (s_in: all or none); few-token tiles up to
 // gemm_group_max_tokens() tokens and where gemm_group_few_tiles says so, block tiles otherwise.
-bool gemm_group_few_tiles(int count, int T, const int* K, const int* R, bool scaled);
+bool gemm_group_few_tiles(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 int gemm_group_max();
 int gemm_group_max_tokens();
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
@@ -103,7 +103,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
 // nq_panel.hip: the same GEMMs at about 128 to 768 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
 size_t panel_workspace_bytes();
-bool panel_applies(int count, int T, const int* K, const int* R, bool scaled);
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 hipError_t gemm_panel_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                             const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                             int T, const int* K, const int* R, void* workspace, unsigned spin_limit, hipStream_t stream);

@@ -555,7 +555,7 @@ size_t panel_workspace_bytes() {
 // cut eight ways, is faster on the few-token tiles); token counts that fill their 64-token blocks badly waste MFMAs,
 // which only a stage with a long k makes up for (its block tiles need a k split and a finish launch); and from
 // about 1024 tokens on the block tiles are level.
-bool panel_applies(int count, int T, const int* K, const int* R, bool scaled) {
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
     const int G = panel_grid();
     if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > 768) return false;
     const int tblocks = (T + kPanelTok - 1) / kPanelTok;
@@ -577,7 +577,7 @@ bool panel_applies(int count, int T, const int* K, const int* R, bool scaled) {
         // s_in, 3 and 3.75 units: 37 and 38 against 28 and 34, 4.25 and 4.7: 38 and 39 against 39 and 41).
         long wgs = 0;
         for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
-        const bool few = gemm_group_few_tiles(count, T, K, R, scaled);
+        const bool few = gemm_group_few_tiles(count, x, T, K, R, scaled);
         if (longest > 16) return (wgs > 88 || !few) && per_wg >= 3.0;
         if (few) return false;
         return fill >= 0.70 && (longest >= 16 ? per_wg >= 4.2 : longest >= 7 && per_wg >= 5.0);

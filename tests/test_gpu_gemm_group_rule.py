@@ -21,8 +21,7 @@ pytestmark = pytest.mark.gpu
     (500, 256, 4096, 1536),      # second GEMM, 96 on 16 k tiles: the last one on few-token tiles at 401 to 512 tokens
     (500, 256, 4096, 1664),      # 104: block tiles
     (1500, 4096, 512, 256),      # 96 on 16 k tiles: the last one on few-token tiles above 1280 tokens
-    (2048, 4096, 256, 256),      # 64: the last one above 1536
-    (2050, 4096, 256, 256),      # 66 above 2048: block tiles
+    (1800, 4096, 256, 256),      # 58 above 1536: block tiles
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_either_side_of_the_lines(dev, dtype, tokens, n, r, m):
@@ -90,3 +89,22 @@ def test_the_longest_k_of_a_group_decides(dev, dtype, tokens, linears):
         # h and the result are rounded to the 16-bit type, as above
         assert oracle.max_rel_err(f32(y), ref) < 3 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)
     assert ops.panel_status(dev) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_inputs_of_their_own_count_by_themselves(dev, dtype):
+    # six linears of 256 rows on 640 tokens: few-token tiles on one input (the bits of one of them alone), block tiles on six
+    # inputs (the bits beside a neighbour that fills the device)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(12)
+    signs = lambda a, b: torch.randint(0, 2, (a, b), dtype=torch.int8, device=dev, generator=gen) * 2 - 1
+    scale = lambda k: (torch.rand(k, device=dev, generator=gen) + 0.01).to(dtype)
+    make = lambda r: packing.marlin_nanoquant_packer(signs(4096, r), signs(r, 256), scale(4096), scale(r), scale(256))
+    terms, big = [make(256) for _ in range(6)], make(8192)
+    xs = [torch.randn(640, 4096, device=dev, generator=gen).to(dtype) for _ in range(6)]
+    print(f"six linears on one input and on six {dtype}", flush=True)
+    run = lambda x, t: ops.gemm_group_forward(x, t, panel="never")
+    few, block = run(xs[:1], terms[:1])[0], run([xs[0], xs[0]], [terms[0], big])[0]
+    one, six = run([xs[0]] * 6, terms)[0], run(xs, terms)[0]
+    torch.cuda.synchronize()
+    assert torch.equal(one, few) and torch.equal(six, block) and not torch.equal(few, block)
