@@ -216,9 +216,7 @@ int nq_gemv_stage(const void* in, const void* s_col, const uint32_t* bits, const
  *   layout is private to packer and kernel, as the reference's Marlin layout is).
  *   Requires k % 256 == 0 and rows % 32 == 0 (else NQ_ERR_PROB_SHAPE, the reference's error class
  *   for shapes its tiles do not cover).  scratch: nq_gemm_scratch_bytes(tokens, k, rows) bytes of
- *   device memory (may be NULL when that is 0).  It holds fp32 partial sums and tile counters when k
- *   is split; it MUST BE ZERO ON ENTRY and is zero again when the enqueued work has finished, so a
- *   caller zeroes it once and reuses it (calls sharing a scratch must not overlap in time). */
+ *   device memory; that is 0 for every shape (no kernel splits k between workgroups), so NULL will do. */
 size_t nq_gemm_scratch_bytes(int tokens, int k, int rows);
 int nq_gemm_onebit(const void* x, const uint32_t* tiles, const void* s_in, const void* s_out, void* y,
                    void* scratch, size_t scratch_bytes, int tokens, int k, int rows, int dtype, void* stream);
@@ -243,13 +241,10 @@ int nq_gemm_nanoquant_bias(const void* x, const uint32_t* vt_tiles, const uint32
 /* Several terms with the same token count in two launches instead of two per term: the first GEMMs of all
  * terms, then the second ones (the projections of a decoder block that read the same tokens: q/k/v, gate/up, or
  * independent linears of a layer).  Up to 128 tokens a single term cannot fill the device and is bound by launch
- * and load latencies; grouped, the same launches carry several times the work.  Above 160 tokens a group large enough to
- * fill the device runs on 64-token block tiles whose workgroups walk the whole k of their term (no k-split, no scratch):
- * together the terms fill the device where one term needs a k-split and a finish launch to do so; smaller groups stay on
- * the few-token tiles.  The choice is made per launch from all of its terms, so above 160 tokens the last bits of a term's
- * result may depend on what shares the call.  Only when some terms have
- * s_in and others do not does the call run the terms one after another (nq_gemm_nanoquant_bias); it then needs
- * their scratch, max over terms of nq_gemm_scratch_bytes for both GEMMs (may be NULL otherwise).
+ * and load latencies; grouped, the same launches carry several times the work.  The tiles are chosen per launch from all of
+ * its terms, so above 160 tokens the last bits of a term's result may depend on what shares the call; up to 160 tokens they are
+ * those of nq_gemm_nanoquant.  Only when some terms have s_in and others do not does the call run the terms one after another
+ * (nq_gemm_nanoquant_bias).  scratch is not needed (NULL).
  * count <= nq_gemm_group_max(); h and y of different terms must not coincide.  No counterpart in the reference, which launches each linear by itself
  * (modules/linear.py:131-133). */
 typedef struct nq_gemm_term {
@@ -268,8 +263,8 @@ int nq_gemm_group_max(void);
 int nq_gemm_nanoquant_group(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                             size_t scratch_bytes, void* stream);
 
-/* The same with a workspace for the panel launches.  From about 100 to 768 tokens a group that gives every
- * workgroup a few k steps of work runs a stage as ONE persistent launch (two workgroups per compute unit) over panels
+/* The same with a workspace for the panel launches.  Up to 2048 tokens a group whose tiles would leave the device unevenly
+ * loaded runs a stage as ONE persistent launch (two workgroups per compute unit) over panels
  * of 64 tokens x 256 rows whose k ranges are shared out evenly over the workgroups (what the reference's stream-k
  * stripes do, kernel/cuda/gemm_kernel.cu:335-400, :594-640): panels cut by a share boundary are finished together by
  * the workgroups that end inside them, which exchange partial fp32 tiles through `panel_ws`.
@@ -277,8 +272,8 @@ int nq_gemm_nanoquant_group(const nq_gemm_term* terms, int count, int tokens, in
  *   left to these launches from then on (it holds partial tiles, hand-over flags and a count of finished
  *   workgroups from which every launch derives its own flag value, so nothing is cleared between launches or graph
  *   replays).  It must not be `scratch` and launches that share it must not overlap in time.
- *   panel_mode: NQ_PANEL_AUTO picks per stage (other token counts and small groups take the launches of
- *   nq_gemm_nanoquant_group), NQ_PANEL_ALWAYS forces the panel launch for any token count, NQ_PANEL_NEVER (or
+ *   panel_mode: NQ_PANEL_AUTO picks per stage whatever is fastest (panels, or the tiles of nq_gemm_nanoquant_group, of which
+ *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count, NQ_PANEL_NEVER (or
  *   panel_ws NULL) never takes it.
  * A panel launch keeps two workgroups per compute unit resident and its workgroups wait for each other's partial
  * tiles: it may share the GPU with other kernels (its waits then last until those free their compute units), but a

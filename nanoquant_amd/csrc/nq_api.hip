@@ -719,7 +719,8 @@ int nq_runlist_status(const void* workspace, int* status_out, void* stream) {
     return hip_status(e);
 }
 
-size_t nq_gemm_scratch_bytes(int tokens, int k, int rows) { return nq::gemm_scratch_bytes(tokens, k, rows); }
+// No kernel splits k between workgroups, so none needs scratch.
+size_t nq_gemm_scratch_bytes(int, int, int) { return 0; }
 
 int nq_gemm_onebit(const void* x, const uint32_t* tiles, const void* s_in, const void* s_out, void* y,
                    void* scratch, size_t scratch_bytes, int tokens, int k, int rows, int dtype, void* stream) {
@@ -736,10 +737,9 @@ int nq_gemm_onebit_bias(const void* x, const uint32_t* tiles, const void* s_in, 
     if (!x || !tiles || !y) return NQ_ERR_NULL;
     if (((uintptr_t)x | (uintptr_t)tiles | (uintptr_t)y | (uintptr_t)s_in | (uintptr_t)scratch | (uintptr_t)bias) & 15u)
         return NQ_ERR_ALIGN;
-    const size_t need = nq::gemm_scratch_bytes(tokens, k, rows);
-    if (need > 0 && (!scratch || scratch_bytes < need)) return NQ_ERR_WORKSPACE;
-    return hip_status(nq::gemm_onebit(dtype, x, tiles, s_in, s_out, y, (float*)scratch, tokens, k, rows,
-                                      (hipStream_t)stream, bias));
+    (void)scratch_bytes;
+    return hip_status(nq::gemm_onebit_group(dtype, 1, &x, &tiles, &s_in, &s_out, &bias, &y, tokens, &k, &rows, nq::kGemmAlone,
+                                            (hipStream_t)stream));
 }
 
 int nq_gemm_nanoquant(const void* x, const uint32_t* vt_tiles, const uint32_t* u_tiles, const void* s_in,
@@ -836,7 +836,8 @@ int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens,
         if (have_ws && (panel_mode == NQ_PANEL_ALWAYS || nq::panel_applies(count, x, tokens, K, R, si[0] != nullptr)))
             return nq::gemm_panel_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, panel_ws, g_panel_spin_limit.load(),
                                         (hipStream_t)stream);
-        return nq::gemm_onebit_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, (hipStream_t)stream);
+        return nq::gemm_onebit_group(dtype, count, x, w, si, so, bs, out, tokens, K, R,
+                                     panel_mode == NQ_PANEL_AUTO && have_ws ? nq::kGemmAnyTile : nq::kGemmGroup, (hipStream_t)stream);
     };
     for (int i = 0; i < count; ++i) {
         const nq_gemm_term& t = terms[i];

@@ -85,20 +85,19 @@ bool stream_needs_uniform_order(int dtype, int batch, bool alt = false);
 bool stream_has_deterministic(int dtype, int batch);
 bool stream_has_alt(int dtype, int batch);
 
-// nq_gemm.hip: C[T,R] = s_out * ((x * s_in) . sgn(W)^T) with W in the 32x256 tile layout.
-// scratch: fp32 [T,R] when gemm_scratch_bytes(T,K,R) > 0.
-size_t gemm_scratch_bytes(int T, int K, int R);
-hipError_t gemm_onebit(int dtype, const void* x, const uint32_t* tiles, const void* s_in, const void* s_out,
-                       void* y, float* scratch, int T, int K, int R, hipStream_t stream, const void* bias = nullptr);
-
-// Up to gemm_group_max() GEMMs on the same token count in one launch (s_in: all or none); few-token tiles up to
-// gemm_group_max_tokens() tokens and where gemm_group_few_tiles says so, block tiles otherwise.
-bool gemm_group_few_tiles(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
+// nq_gemm.hip: C[T,R] = s_out * ((x * s_in) . sgn(W)^T) with W in the 32x256 tile layout, up to gemm_group_max() GEMMs on the
+// same token count in one launch (s_in: all or none).  use: which tiles may be taken (see choose_tile).
+enum GemmUse {
+    kGemmAlone,      // one linear by itself
+    kGemmGroup,      // up to 160 tokens the bits that it gets by itself
+    kGemmAnyTile,    // whatever is fastest
+};
 int gemm_group_max();
-int gemm_group_max_tokens();
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                              const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
-                             int T, const int* K, const int* R, hipStream_t stream);
+                             int T, const int* K, const int* R, int use, hipStream_t stream);
+// Estimated time of that launch with kGemmAnyTile, in us.
+double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 
 // nq_panel.hip: the same GEMMs at about 128 to 768 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.

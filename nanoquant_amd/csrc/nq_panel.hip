@@ -1,4 +1,4 @@
-// Prefill at about 128 to 768 tokens: one persistent launch per GEMM stage of a group of linears.
+// Prefill up to 2048 tokens, where tiles leave the device unevenly loaded: one persistent launch per GEMM stage of a group.
 //
 //   C[t, j] = s_out[j] * sum_k (x[t, k] * s_in[k]) * sgn(W[j, k])       (same function as nq_gemm.hip)
 //
@@ -548,16 +548,16 @@ size_t panel_workspace_bytes() {
     return kPanelHeadBytes + flags + (size_t)2 * G * kPanelSlotFloats * sizeof(float);
 }
 
-// Whether one stage of a group is better off as a panel launch than on the tiles of nq_gemm.hip (measured on
-// Llama-2-7B layers, per stage, 64 .. 4096 tokens).  Every workgroup must get a few k steps (otherwise panels are cut
-// into many pieces and the hand-over of partial tiles costs more than the shared slabs save); the longest k range
-// must not be shared by too many workgroups (the first stage of a 128-token layer, whose 43-tile down projection is
-// cut eight ways, is faster on the few-token tiles); token counts that fill their 64-token blocks badly waste MFMAs,
-// which only a stage with a long k makes up for (its block tiles need a k split and a finish launch); and from
-// about 1024 tokens on the block tiles are level.
+// Whether one stage of a group is better off as a panel launch than on the tiles of nq_gemm.hip: where tiles leave the last of
+// their rounds nearly empty, which equal shares of k steps do not (11008 -> 6144 rows on 700 tokens: 123 / 95; on 512 tokens
+// 78 / 77; 4096 -> 22016 on 333: 76 / 66).  A panel launch takes, in us, 12.4 + 3.1 per k step of a workgroup (3.3 with s_in)
+// + 1 for every workgroup that a panel is shared by: the middle 90 % of 445 launches are within -8 .. +8 % of that (128 to 2048
+// tokens, 1 to 43 k tiles, 512 to 22016 rows); with fewer than three k steps the hand-over takes most of the time (128
+// tokens, 3072 -> 4096 rows: tiles 7, panels 35).
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
+    constexpr int kMostTokens = 2048;            // of the launches that were timed
     const int G = panel_grid();
-    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > 768) return false;
+    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > kMostTokens) return false;
     const int tblocks = (T + kPanelTok - 1) / kPanelTok;
     long long units = 0;
     int longest = 0;
@@ -567,26 +567,10 @@ bool panel_applies(int count, const void* const* x, int T, const int* K, const i
         longest = longest > K[p] / kTileK ? longest : K[p] / kTileK;
     }
     const double per_wg = (double)units / G;
-    const double fill = (double)T / (tblocks * kPanelTok);
-    if (T > gemm_group_max_tokens()) {
-        // Above the few-token counts.  A long k (more than 16 tiles): panels from some 90 block workgroups on (us, panels
-        // against few-token tiles: 56 workgroups 42 / 26, 88 40 / 39, 112 42 / 50, 168 49 / 53; block tiles 60 to 80).
-        // Up to 16 tiles panels start where the few-token tiles end; a k of less than 7 tiles, or a short one with less than
-        // 5 units per workgroup (16 tiles: 4.2), is faster on block tiles (5 tiles, 3.2 units: 26 against 21; 10.5 units: 50
-        // against 47; 8 tiles, 3.6 units: 27 against 24; 7 to 11 tiles, 7 to 25 units: 35 to 88 against 40 to 103; 16 tiles without
-        // s_in, 3 and 3.75 units: 37 and 38 against 28 and 34, 4.25 and 4.7: 38 and 39 against 39 and 41).
-        long wgs = 0;
-        for (int p = 0; p < count; ++p) wgs += (long)((R[p] + 127) / 128) * tblocks;
-        const bool few = gemm_group_few_tiles(count, x, T, K, R, scaled);
-        if (longest > 16) return (wgs > 88 || !few) && per_wg >= 3.0;
-        if (few) return false;
-        return fill >= 0.70 && (longest >= 16 ? per_wg >= 4.2 : longest >= 7 && per_wg >= 5.0);
-    }
     if (per_wg < 3.0) return false;
-    // up to two token blocks the few-token tiles are the alternative, and a strong one; beyond, panels win more easily
-    const bool few = T <= 2 * kPanelTok;
-    if (longest > (few ? 4.0 : 8.0) * per_wg) return false;
-    return fill >= (few ? 0.78 : 0.70) || longest > 16;
+    const double steps = (double)((units + G - 1) / G);
+    const double time = 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
+    return time < 0.95 * gemm_tiles_time(count, x, T, K, R, scaled);
 }
 
 template <int DT, bool SCALED>

@@ -251,23 +251,6 @@ def _check_gemm_tensor(t, name, dtype=None):
         raise RuntimeError(f"{name} must have dtype {dtype}")
 
 
-# Split-k scratch (fp32 partial sums + tile counters).  The kernels require it to be zero on entry and
-# leave it zero on exit, so one buffer per (device, stream) is allocated zeroed once, grown on demand and
-# reused; no per-call memset.
-_scratch_cache = {}
-
-
-def _scratch(nbytes, device):
-    if nbytes == 0:
-        return None
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    buf = _scratch_cache.get(key)
-    if buf is None or buf.numel() * 4 < nbytes:
-        buf = torch.zeros((nbytes + 3) // 4, dtype=torch.float32, device=device)
-        _scratch_cache[key] = buf
-    return buf
-
-
 # Workspace of the panel launches (partial tiles, hand-over flags, the count of finished workgroups): zero when
 # first used, then owned by the launches; one per (device, stream) so that launches sharing it are stream-ordered.
 _panel_ws_cache = {}
@@ -312,11 +295,9 @@ def marlin_onebit_forward(x, weight, scale_g, scale_h, workspace):
     C = torch.empty((m, n), dtype=x.dtype, device=x.device)
     if m == 0 or n == 0:
         return C
-    nbytes = int(_lib.lib().nq_gemm_scratch_bytes(m, k, n))
-    scratch = _scratch(nbytes, x.device)
     with torch.cuda.device(x.device):
         _lib.check(_lib.lib().nq_gemm_onebit(_ptr(x), _ptr(weight), _ptr(scale_g), _ptr(scale_h), _ptr(C),
-                                             _ptr(scratch), nbytes, m, k, n, dt, _stream(x.device)))
+                                             None, 0, m, k, n, dt, _stream(x.device)))
     return C
 
 
@@ -339,11 +320,9 @@ def _gemm_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, wo
     out = torch.empty((t, m), dtype=x.dtype, device=x.device)
     if t == 0 or m == 0:
         return out
-    nbytes = max(int(_lib.lib().nq_gemm_scratch_bytes(t, n, r)), int(_lib.lib().nq_gemm_scratch_bytes(t, r, m)))
-    scratch = _scratch(nbytes, x.device)
     with torch.cuda.device(x.device):
         _lib.check(_lib.lib().nq_gemm_nanoquant_bias(_ptr(x), _ptr(weight_u), _ptr(weight_v), _ptr(scale_g), _ptr(scale_l),
-                                                     _ptr(scale_h), _ptr(bias), _ptr(imm), _ptr(out), _ptr(scratch), nbytes,
+                                                     _ptr(scale_h), _ptr(bias), _ptr(imm), _ptr(out), None, 0,
                                                      t, n, r, m, dt, _stream(x.device)))
     return out
 
@@ -513,11 +492,10 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     op takes them after x; `xs` is one tensor [tokens, n] read by every term or a list of one tensor per term;
     `biases` an optional list of [m] tensors / None; `outs` an optional list of contiguous [tokens, m] tensors of
     the activation type to write into (allocated here when absent); `panel` ("auto", "always", "never") says whether
-    the stages may run as persistent panel launches (around 128 tokens, see include/nq_gfx950.h).  Returns the list of
-    outputs.  The terms share
-    launches (a single linear leaves most of the device idle up to some hundred tokens): few-token tiles up to 160
-    tokens and where a group is too small for more, 64-token block tiles without k-split above.  The
-    reference launches every linear by itself (modules/linear.py:131-133)."""
+    the stages may run as persistent panel launches and, up to 160 tokens, on tiles other than the ones a linear gets by
+    itself (see include/nq_gfx950.h).  Returns the list of outputs.  The terms share launches: a single linear leaves most
+    of the device idle up to some hundred tokens.  The reference launches every linear by itself
+    (modules/linear.py:131-133)."""
     lib = _lib.lib()
     count = len(terms)
     if count == 0:
@@ -527,7 +505,7 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     if len(xs) != count or (biases is not None and len(biases) != count) or (outs is not None and len(outs) != count):
         raise RuntimeError("one x (and one bias / output entry) per term")
     dt = _gemm_dtype(xs[0])
-    given, outs, keep, arr_items, nbytes = outs, [], [], [], 0
+    given, outs, keep, arr_items = outs, [], [], []
     for i, (x, term) in enumerate(zip(xs, terms)):
         weight_u, weight_v, scale_g, scale_l, scale_h, workspace = term
         bias = None if biases is None else biases[i]
@@ -551,7 +529,6 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
                 raise RuntimeError(f"outs[{i}] must be a contiguous, 16-byte aligned [{t}, {m}] tensor of {x.dtype} on {x.device}")
         outs.append(out)
         keep.append(imm)
-        nbytes = max(nbytes, int(lib.nq_gemm_scratch_bytes(t, n, r)), int(lib.nq_gemm_scratch_bytes(t, r, m)))
         pv = lambda ten: None if ten is None else ten.data_ptr()
         arr_items.append(NqGemmTerm(pv(x), pv(weight_u), pv(weight_v), pv(scale_g), pv(scale_l), pv(scale_h), pv(bias),
                                     pv(imm), pv(out), n, r, m))
@@ -560,14 +537,13 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
         return outs
     device = xs[0].device
     group_max = int(lib.nq_gemm_group_max())
-    scratch = _scratch(nbytes, device)
     mode = PANEL_MODES[panel]
     ws = None if mode == 2 else _panel_workspace(device)
     with torch.cuda.device(device):
         for lo in range(0, count, group_max):
             part = arr_items[lo:lo + group_max]
             arr = (NqGemmTerm * len(part))(*part)
-            _lib.check(lib.nq_gemm_nanoquant_group_ws(arr, len(part), tokens, dt, _ptr(scratch), nbytes, _ptr(ws),
+            _lib.check(lib.nq_gemm_nanoquant_group_ws(arr, len(part), tokens, dt, None, 0, _ptr(ws),
                                                       0 if ws is None else ws.numel(), mode, _stream(device)))
     return outs
 

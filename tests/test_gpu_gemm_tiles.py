@@ -1,0 +1,67 @@
+"""Prefill tiles at their edges: every tile size of csrc/nq_gemm.hip with ragged tokens and rows, k of one tile up to more than
+the ring and the k groups hold, against the dense definition in 64 bits (src/nanoquant/modules/linear.py:248-257 of the
+reference)."""
+import numpy as np
+import pytest
+import torch
+
+from nanoquant_amd import ops, packing
+from oracle import nq_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+# half an ulp of the 16-bit result, and as much again for the h that feeds the second GEMM
+ROUND = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _onebit(dev, tokens, k, rows, dtype, scaled, seed):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    signs = torch.randint(0, 2, (rows, k), dtype=torch.int8, device=dev, generator=gen) * 2 - 1
+    scale = lambda n: (torch.rand(n, device=dev, generator=gen) + 0.01).to(dtype)
+    s_in, s_out = scale(k) if scaled else None, scale(rows)
+    bits, si, so, words = packing.marlin_onebit_packer(signs, s_in, s_out)
+    x = torch.randn(tokens, k, device=dev, generator=gen).to(dtype)
+    xs = x.double() * (s_in.double() if scaled else 1.0)
+    return x, bits, si, so, torch.zeros(max(words, 1), dtype=torch.int32, device=dev), (xs @ signs.double().T) * s_out.double()
+
+
+# (tokens, k, rows): 32 x 32 tiles up to 32 x 96 where k is split four ways (k tiles left over for none, one, three of the four
+# wavefronts), 64 x 128 to 128 x 256 where it is not
+@pytest.mark.parametrize("tokens,k,rows", [
+    (1, 256, 32), (31, 512, 64), (33, 1280, 96), (65, 2304, 160),              # 32 x 32: 1, 2, 5, 9 k tiles
+    (128, 4096, 3104), (200, 1792, 2080), (161, 2816, 3072),                   # 32 x 64, rows left over
+    (333, 4096, 3104), (250, 2048, 3136),                                      # 32 x 96, one and two row tiles left over
+    (333, 1024, 3168), (700, 256, 2080), (193, 2560, 8224),                    # 64 x 128
+    (400, 768, 16416), (1000, 1280, 4128),                                     # 64 x 256
+    (2049, 512, 12320), (4097, 256, 8224),                                     # 128 x 256
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("scaled", [True, False])
+def test_tiles_at_their_edges(dev, tokens, k, rows, dtype, scaled):
+    x, bits, si, so, workspace, ref = _onebit(dev, tokens, k, rows, dtype, scaled, tokens + k)
+    print(f"tile {tokens} tokens {k} -> {rows} {dtype} scaled={scaled}", flush=True)
+    y = torch.ops.binary_kernels.marlin_onebit_forward(x, bits, si, so, workspace)
+    torch.cuda.synchronize()
+    err = ((y.double() - ref).abs().max() / ref.abs().max()).item()
+    assert err < 1.2 * ROUND[dtype], err                     # products are exact, sums are fp32: the rounding of the result
+
+
+@pytest.mark.parametrize("tokens", [100, 128, 160])
+def test_other_tiles_for_many_rows_below_160_tokens(dev, tokens):
+    # 2 x 8192 rows over a short rank: block tiles where the group may take any, the bits of the linear alone where it may not
+    dtype, n = torch.float16, 512
+    f = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev).to(dtype)
+    packed, refs = [], []
+    x = f(oracle.synth_x(tokens, n, 5))
+    for i in range(2):
+        vt, u, *scales = oracle.synth_term(8192, n, 512, 70 + i)
+        sc = [f(s) for s in scales]
+        packed.append(packing.marlin_nanoquant_packer(torch.from_numpy(vt).T.contiguous().to(dev), torch.from_numpy(u).T.contiguous().to(dev), *sc))
+        refs.append(oracle.layer_forward(x.float().cpu().numpy(), vt, u, *(s.float().cpu().numpy() for s in sc)))
+    print(f"many rows {tokens} tokens", flush=True)
+    alone = [torch.ops.binary_kernels.marlin_nanoquant_forward(x, *p) for p in packed]
+    same, free = ops.gemm_group_forward(x, packed, panel="never"), ops.gemm_group_forward(x, packed)
+    torch.cuda.synchronize()
+    for a, s, y, ref in zip(alone, same, free, refs):
+        assert torch.equal(a, s)
+        assert oracle.max_rel_err(y.float().cpu().numpy(), ref) < 3 * ROUND[dtype]
