@@ -67,13 +67,16 @@ struct RowsProblem {
     int rows, out_stride, waves;
     int out_kind;           // RowsOut
 };
-// Up to kGroupMax linears per launch: their workgroups one behind the other.
+// Up to N linears per launch: their workgroups one behind the other.  A launch takes the smallest table that holds its
+// linears (one, {gate, up} and {q, k, v}, more): kernel arguments are read from memory at the start of every workgroup, with all
+// else waiting, and eight entries are 800 bytes of them.  Llama-2-7B layer as four groups of two launches in a graph, 1 / 4 / 11
+// rows of fp16: always eight entries and an entry looked up by its index 43.0 / 47.6 / 58.4 us, this 38.3 / 42.9 / 54.6.
 constexpr int kGroupMax = 8;
-template <int NT>
+template <int NT, int N>
 struct RowsGroup {
-    RowsProblem<NT> p[kGroupMax];
-    int first[kGroupMax + 1];        // first workgroup of every problem; [kGroupMax] = the grid
     int batch;
+    int first[N + 1];                // first workgroup of every problem; [N] = the grid
+    RowsProblem<NT> p[N];
 };
 
 template <bool COHERENT>
@@ -404,19 +407,25 @@ __device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, i
     }
 }
 
-template <int NT>
-__device__ __forceinline__ int problem_of(const int (&first)[kGroupMax + 1], int b) {
+template <int N>
+__device__ __forceinline__ int problem_of(const int (&first)[N + 1], int b) {
     int i = 0;
 #pragma unroll
-    for (int k = 1; k < kGroupMax; ++k) i += b >= first[k] ? 1 : 0;
+    for (int k = 1; k < N; ++k) i += b >= first[k] ? 1 : 0;
     return i;
 }
 
-template <int DT, bool SCALED, int NB, int F, int NT, bool VEC>
-__global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_rows_kernel(RowsGroup<NT> gr) {
+template <int DT, bool SCALED, int NB, int F, int NT, bool VEC, int N>
+__global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_rows_kernel(RowsGroup<NT, N> gr) {
     const int b = (int)blockIdx.x;
-    const int i = problem_of<NT>(gr.first, b);
-    rows_body<DT, SCALED, NB, F, NT, VEC, false>(gr.p[i], b - gr.first[i], gr.batch, StageWait{});
+    int i = 0, first = 0;
+#pragma unroll
+    for (int k = 1; k < N; ++k)
+        if (b >= gr.first[k]) {
+            i = k;
+            first = gr.first[k];
+        }
+    rows_body<DT, SCALED, NB, F, NT, VEC, false>(gr.p[i], b - first, gr.batch, StageWait{});
 }
 
 // Both stages of up to kGroupMax linears in ONE ordinary launch (no resident-grid requirement): the workgroups of all
@@ -435,7 +444,7 @@ constexpr int kFusedFlagLine0 = 16;                                  // flag j o
 constexpr int kFusedSlotLines = kFusedFlagLine0 + kGroupMax * kFusedFlagLines;
 constexpr int kFusedSlotWords = kFusedSlotLines * kFusedLineWords;   // 18 KiB
 struct FusedArgs {
-    RowsGroup<1> a, b;               // first and second stages; b.first counts from the end of the first stages
+    RowsGroup<1, kGroupMax> a, b;    // first and second stages; b.first counts from the end of the first stages
     unsigned* slot;                  // kFusedSlotWords words, zero between launches
     unsigned* status;
     unsigned spin_limit;
@@ -446,7 +455,7 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_fused_kernel(FusedArg
     const int b = (int)blockIdx.x;
     const int n1 = f.a.first[kGroupMax];
     if (b < n1) {
-        const int i = problem_of<1>(f.a.first, b);
+        const int i = problem_of<kGroupMax>(f.a.first, b);
         rows_body<DT, true, NB, 1, 1, VEC, true>(f.a.p[i], b - f.a.first[i], f.a.batch, StageWait{});
         // every wavefront waits until its own stores of h have been acknowledged, the barrier collects all of them,
         // then the arrival is counted
@@ -463,7 +472,7 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_fused_kernel(FusedArg
         }
     } else {
         const int lb = b - n1;
-        const int i = problem_of<1>(f.b.first, lb);
+        const int i = problem_of<kGroupMax>(f.b.first, lb);
         StageWait w;
         w.counter = f.slot + (kFusedFlagLine0 + i * kFusedFlagLines + (lb & (kFusedFlagLines - 1))) * kFusedLineWords;
         w.target = 1u;
@@ -529,11 +538,11 @@ static RowsProblem<NT> make_problem(const RowsStage* s) {
 }
 
 // Fills a group; returns the grid, or 0 when there is nothing to do.
-template <int NT>
-static int make_group(RowsGroup<NT>& g, int count, const RowsStage* s, int batch, int F, int* waves) {
+template <int NT, int N>
+static int make_group(RowsGroup<NT, N>& g, int count, const RowsStage* s, int batch, int F, int* waves) {
     int at = 0;
     *waves = F;                          // wavefront f finishes tile f
-    for (int i = 0; i < kGroupMax; ++i) {
+    for (int i = 0; i < N; ++i) {
         g.p[i] = make_problem<NT>(s + NT * (i < count ? i : count - 1));
         g.first[i] = at;
         if (i < count) {
@@ -541,7 +550,8 @@ static int make_group(RowsGroup<NT>& g, int count, const RowsStage* s, int batch
             *waves = std::max(*waves, g.p[i].waves);
         }
     }
-    g.first[kGroupMax] = at;
+    g.first[N] = at;                     // so that no workgroup belongs to an unused entry
+    for (int i = count; i < N; ++i) g.first[i] = at;
     g.batch = batch;
     return at;
 }
@@ -559,14 +569,23 @@ static hipError_t launch_rows(K kern, const A& args, int grid, int waves, int wa
     return hipGetLastError();
 }
 
-template <int DT, bool SCALED, int NB, int F, int NT, bool VEC>
-static hipError_t launch_group(int count, const RowsStage* s, int batch, hipStream_t stream) {
-    RowsGroup<NT> g;
+template <int DT, bool SCALED, int NB, int F, int NT, bool VEC, int N>
+static hipError_t launch_table(int count, const RowsStage* s, int batch, hipStream_t stream) {
+    RowsGroup<NT, N> g;
     int waves = 1;
-    const int grid = make_group<NT>(g, count, s, batch, F, &waves);
+    const int grid = make_group(g, count, s, batch, F, &waves);
     if (grid == 0) return hipSuccess;
     static PerDeviceFlag raised;
-    return launch_rows(gemv_rows_kernel<DT, SCALED, NB, F, NT, VEC>, g, grid, waves, rows_wave_lds<DT, SCALED, NB, F>(), raised, stream);
+    return launch_rows(gemv_rows_kernel<DT, SCALED, NB, F, NT, VEC, N>, g, grid, waves, rows_wave_lds<DT, SCALED, NB, F>(), raised, stream);
+}
+template <int DT, bool SCALED, int NB, int F, int NT, bool VEC>
+static hipError_t launch_group(int count, const RowsStage* s, int batch, hipStream_t stream) {
+    if constexpr (VEC) {
+        if (count == 1) return launch_table<DT, SCALED, NB, F, NT, VEC, 1>(count, s, batch, stream);
+        if constexpr (NT == 1)
+            if (count <= 3) return launch_table<DT, SCALED, NB, F, NT, VEC, 3>(count, s, batch, stream);
+    }
+    return launch_table<DT, SCALED, NB, F, NT, VEC, kGroupMax>(count, s, batch, stream);
 }
 
 // Whether 16-byte loads can read this stage: aligned input rows, and at least 16 bytes of words in the last row block.
@@ -674,8 +693,8 @@ hipError_t gemv_rows_fused(int dtype, int count, const RowsStage* first, const R
     if (count < 1 || count > kGroupMax || batch < 1 || batch > 16) return hipErrorInvalidValue;
     FusedArgs f;
     int wa = 1, wb = 1;
-    const int na = make_group<1>(f.a, count, first, batch, 1, &wa);
-    const int nb = make_group<1>(f.b, count, second, batch, 1, &wb);
+    const int na = make_group(f.a, count, first, batch, 1, &wa);
+    const int nb = make_group(f.b, count, second, batch, 1, &wb);
     if (nb == 0) return hipSuccess;
     for (int i = 0; i < count; ++i)
         if (first[i].rows == 0) return hipErrorInvalidValue;         // nobody would raise its flag: callers use two launches
