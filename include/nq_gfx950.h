@@ -273,8 +273,8 @@ int nq_gemm_nanoquant_group(const nq_gemm_term* terms, int count, int tokens, in
  *   workgroups from which every launch derives its own flag value, so nothing is cleared between launches or graph
  *   replays).  It must not be `scratch` and launches that share it must not overlap in time.
  *   panel_mode: NQ_PANEL_AUTO picks per stage whatever is fastest (panels, or the tiles of nq_gemm_nanoquant_group, of which
- *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count, NQ_PANEL_NEVER (or
- *   panel_ws NULL) never takes it.
+ *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count, NQ_PANEL_NEVER never
+ *   takes it; with panel_ws NULL there is none in any mode.
  * A panel launch keeps two workgroups per compute unit resident and its workgroups wait for each other's partial
  * tiles: it may share the GPU with other kernels (its waits then last until those free their compute units), but a
  * wait that outlasts its bound (2^20 polls, about a second) invalidates the launch's outputs.
@@ -285,6 +285,9 @@ enum { NQ_PANEL_AUTO = 0, NQ_PANEL_ALWAYS = 1, NQ_PANEL_NEVER = 2 };
 size_t nq_gemm_panel_workspace_bytes(void);
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                                size_t scratch_bytes, void* panel_ws, size_t panel_ws_bytes, int panel_mode, void* stream);
+/* 1 when a stage of that call would be a panel launch (0 otherwise, and for NQ_PANEL_NEVER), so that a caller can do without the
+ * workspace until one is. */
+int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode);
 int nq_gemm_panel_status(const void* panel_ws, int* status_out, void* stream);
 /* Polls after which a wait of a panel launch gives up (0 = the default of 2^20).  Process-wide; for exercising a
  * caller's handling of status 1 from the host, as nq_gemv_group_set_spin_limit. */

@@ -7,6 +7,7 @@ import os
 import re
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
 LIB_PATH = os.path.join(_HERE, "libnq_gfx950.so")
 HEADER_PATH = os.path.join(os.path.dirname(_HERE), "include", "nq_gfx950.h")
 
@@ -48,6 +49,7 @@ _SIGNATURES = {
     "nq_gemm_nanoquant_group": (_i, [_vp, _i, _i, _i, _vp, _sz, _vp]),
     "nq_gemm_panel_workspace_bytes": (_sz, []),
     "nq_gemm_nanoquant_group_ws": (_i, [_vp, _i, _i, _i, _vp, _sz, _vp, _sz, _i, _vp]),
+    "nq_gemm_group_wants_panel": (_i, [_vp, _i, _i, _i]),
     "nq_gemm_panel_status": (_i, [_vp, ctypes.POINTER(_i), _vp]),
     "nq_gemm_panel_set_spin_limit": (_i, [ctypes.c_uint]),
     "nq_pack_gemm_tiles": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp]),
@@ -81,6 +83,17 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def host():
+    """The C++ host path (csrc/nq_torch.cpp), linked against the library above."""
+    lib()
+    if not os.path.exists(HOST_PATH):
+        raise ImportError(
+            f"{HOST_PATH} not found: the host path of the operators is not built. "
+            "Run `python -c 'import __graft_entry__ as g; g.build()'` (or nanoquant_amd/build.py).")
+    from . import _host
+    return _host
 
 
 def status_message(status: int) -> str:

@@ -1,4 +1,4 @@
-"""hipcc build of libnq_gfx950.so (the only native artefact of the package)."""
+"""Builds libnq_gfx950.so (hipcc: the kernels behind the C ABI) and _host.so (g++: the operators' host path on top of it)."""
 from __future__ import annotations
 
 import os
@@ -10,6 +10,8 @@ from concurrent.futures import ThreadPoolExecutor
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(_HERE, "libnq_gfx950.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
+HOST_SOURCE = os.path.join(CSRC, "nq_torch.cpp")
 SOURCES = ("nq_rows.hip", "nq_stream.hip", "nq_gemm.hip", "nq_panel.hip", "nq_util.hip", "nq_api.hip")
 # -packed-fp32-ops off: hipcc may otherwise fuse scalar float code into packed-fp32 instructions.
 FLAGS = ("--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
@@ -43,5 +45,26 @@ def build(verbose: bool = False, extra_flags=(), out_path: str = LIB_PATH) -> st
     return out_path
 
 
+def build_host(out_path: str = HOST_PATH) -> str:
+    """Compile the host path against torch's headers and link it to LIB_PATH (found beside it at run time)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    tmp = out_path + ".tmp"
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + os.path.join(root, "include"), "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-I/opt/rocm/include", "-I" + sysconfig.get_paths()["include"], HOST_SOURCE, "-o", tmp,
+           "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
+           "-L" + _HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+    os.replace(tmp, out_path)
+    return out_path
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_host())

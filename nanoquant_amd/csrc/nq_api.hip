@@ -42,7 +42,7 @@ const char* nq_status_string(int status) {
 
 int nq_last_hip_error(void) { return g_last_hip_error; }
 
-int nq_abi_version(void) { return 9; }
+int nq_abi_version(void) { return 10; }
 
 int nq_device_query(int attr, int* value) {
     if (!value) return NQ_ERR_NULL;
@@ -790,6 +790,18 @@ int nq_gemm_panel_status(const void* panel_ws, int* status_out, void* stream) {
     return hip_status(e);
 }
 
+int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode) {
+    if (!terms || count < 1 || count > nq::gemm_group_max() || tokens < 1 || panel_mode == NQ_PANEL_NEVER) return 0;
+    if (panel_mode == NQ_PANEL_ALWAYS) return 1;
+    const void* x[16]; const void* h[16];
+    int n[16], r[16], m[16];
+    static_assert(sizeof(x) / sizeof(x[0]) >= 16, "nq::gemm_group_max()");
+    for (int i = 0; i < count; ++i) {
+        x[i] = terms[i].x; h[i] = terms[i].h; n[i] = terms[i].n; r[i] = terms[i].r; m[i] = terms[i].m;
+    }
+    return nq::panel_applies(count, x, tokens, n, r, terms[0].s_in != nullptr) || nq::panel_applies(count, h, tokens, r, m, false);
+}
+
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                                size_t scratch_bytes, void* panel_ws, size_t panel_ws_bytes, int panel_mode, void* stream) {
     if (dtype != NQ_F16 && dtype != NQ_BF16) return NQ_ERR_DTYPE;
@@ -837,7 +849,7 @@ int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens,
             return nq::gemm_panel_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, panel_ws, g_panel_spin_limit.load(),
                                         (hipStream_t)stream);
         return nq::gemm_onebit_group(dtype, count, x, w, si, so, bs, out, tokens, K, R,
-                                     panel_mode == NQ_PANEL_AUTO && have_ws ? nq::kGemmAnyTile : nq::kGemmGroup, (hipStream_t)stream);
+                                     panel_mode == NQ_PANEL_AUTO ? nq::kGemmAnyTile : nq::kGemmGroup, (hipStream_t)stream);
     };
     for (int i = 0; i < count; ++i) {
         const nq_gemm_term& t = terms[i];

@@ -410,8 +410,8 @@ def prefill_group(modules: Sequence, x) -> list:
         if t.ndim not in (2, 3):
             raise ValueError(f"Expected 2D or 3D input tensor, got {t.ndim}D")
         if id(t) not in cache:                 # a shared input is converted once
-            v = t if t.dtype == mods[0].dtype else t.to(mods[0].dtype)
-            cache[id(t)] = v.contiguous().view(-1, v.size(-1))
+            v = (t if t.dtype == mods[0].dtype else t.to(mods[0].dtype)).contiguous()
+            cache[id(t)] = v if v.ndim == 2 else v.view(-1, v.size(-1))
         flat.append(cache[id(t)])
     biases = []
     for mod in mods:

@@ -6,10 +6,8 @@ shape-only implementations under Meta, as the reference does (pybind.cpp:108-124
 under torch.compile(fullgraph=True).  There is no CPU registration and no fallback: without the
 built library, or on CPU tensors, the ops raise.
 
-Argument checks and their messages follow the reference's host wrappers:
-  nanoquant_dyn_forward     src/nanoquant/kernel/cuda/gemv_kernel.cu:308-346, cuda/meta_utils.h:14-38
-  marlin_onebit_forward     src/nanoquant/kernel/cuda/gemm.cpp:36-98
-  marlin_nanoquant_forward  src/nanoquant/kernel/cuda/gemm.cpp:112-122
+The device implementations, with the argument checks and messages of the reference's host wrappers, are in C++
+(csrc/nq_torch.cpp, built as the extension module `_host`).
 """
 from __future__ import annotations
 
@@ -42,18 +40,6 @@ _SCHEMAS = (
 
 MARLIN_MIN_MAX_PAR = 32
 
-# Legal values of the CUDA tuning hints (gemv_kernel.cu:351-354).  They select template instances in
-# the reference; here they are validated and otherwise ignored -- the gfx950 launch shape is derived
-# from the problem.  4 is added to the accumulator set because it is the schema's own default.
-_SWEEPS = {
-    "n_th": (64, 128, 256),
-    "n_rpw": (1, 2, 4, 8),
-    "n_acc": (1, 2, 4),
-    "n_pipe": (1, 2, 4, 8, 16),
-}
-_N_TH, _N_RPW, _N_ACC, _N_PIPE = (_SWEEPS[k] for k in ("n_th", "n_rpw", "n_acc", "n_pipe"))
-
-
 def _dtype_id(t: torch.Tensor) -> int:
     if t.dtype == torch.float16:
         return _lib.NQ_F16
@@ -75,10 +61,8 @@ _FLOAT_WHAT = {torch.float16: "must be float16 tensor", torch.bfloat16: "must be
 
 
 def _sweep(name: str, value: int) -> None:
-    legal = _SWEEPS[name.rstrip("12")]
-    if value not in legal:
-        choices = ", ".join(str(v) for v in legal)
-        raise ValueError(f"{name} should be one of [{choices}], but {value} was given")
+    """Raises ValueError unless `value` is legal for the tuning hint `name` (gemv_kernel.cu:351-354)."""
+    _host.check_hint(name, value)
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -162,49 +146,16 @@ def _check_bias(bias, m, x):
         raise RuntimeError(f"bias must be [{m}], got {list(bias.shape)}")
 
 
-def _gemv_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias=None, dims=None):
-    n, r, m = dims if dims is not None else _check_gemv_args(x, scale_g, Ubits, scale_l, Vbits, scale_h)
-    _check_bias(bias, m, x)
-    flat = x.dim() == 2
-    dev, dt = x.device, x.dtype
-    if flat:
-        batch = x.size(0)
-    else:
-        batch = 1
-        for d in x.shape[:-1]:
-            batch *= d
-    y = torch.empty((batch, m), dtype=dt, device=dev)
-    if batch > 0 and m > 0:
-        h = torch.empty((batch, max(r, 1)), dtype=torch.float32, device=dev)
-        with _on_device(dev):
-            _lib.check(_lib.lib().nq_gemv_forward_bias(x.data_ptr(), scale_g.data_ptr(), Ubits.data_ptr(), _ptr(scale_l),
-                                                       Vbits.data_ptr(), scale_h.data_ptr(), _ptr(bias), h.data_ptr(),
-                                                       y.data_ptr(), batch, n, r, m,
-                                                       _lib.NQ_F16 if dt == torch.float16 else _lib.NQ_BF16, _stream(dev)))
-    return y if flat else y.reshape(*x.shape[:-1], m)
-
-
 def nanoquant_dyn_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h,
                           num_thread_stage1=128, num_thread_stage2=128,
                           num_row_per_warp_stage1=2, num_row_per_warp_stage2=2,
                           num_acc_stage1=4, num_acc_stage2=4,
                           num_pipeline_stage1=2, num_pipeline_stage2=2):
     """y = scale_h * (Vbits (scale_l * (Ubits (scale_g * x)))): `Ubits` [r, n/32] is the FIRST stage,
-    `Vbits` [m, r/32] the second (the reference's argument names, pybind.cpp:86-90)."""
-    dims = _check_gemv_args(x, scale_g, Ubits, scale_l, Vbits, scale_h)
-    if not (num_thread_stage1 in _N_TH and num_thread_stage2 in _N_TH and
-            num_row_per_warp_stage1 in _N_RPW and num_row_per_warp_stage2 in _N_RPW and
-            num_acc_stage1 in _N_ACC and num_acc_stage2 in _N_ACC and
-            num_pipeline_stage1 in _N_PIPE and num_pipeline_stage2 in _N_PIPE):
-        _sweep("n_th1", num_thread_stage1)
-        _sweep("n_rpw1", num_row_per_warp_stage1)
-        _sweep("n_acc1", num_acc_stage1)
-        _sweep("n_pipe1", num_pipeline_stage1)
-        _sweep("n_th2", num_thread_stage2)
-        _sweep("n_rpw2", num_row_per_warp_stage2)
-        _sweep("n_acc2", num_acc_stage2)
-        _sweep("n_pipe2", num_pipeline_stage2)
-    return _gemv_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, dims=dims)
+    `Vbits` [m, r/32] the second (the reference's argument names, pybind.cpp:86-90).  The operator without its dispatcher."""
+    return _host.nanoquant_dyn_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, num_thread_stage1, num_thread_stage2,
+                                       num_row_per_warp_stage1, num_row_per_warp_stage2, num_acc_stage1, num_acc_stage2,
+                                       num_pipeline_stage1, num_pipeline_stage2)
 
 
 def _nanoquant_dyn_forward_meta(x, scale_g, Ubits, scale_l, Vbits, scale_h, *hints, **kw):
@@ -232,25 +183,6 @@ def _onebit_check(A, B, s_in, s_out, workspace):
     return prob_m, prob_n, prob_k
 
 
-def _gemm_dtype(A):
-    if A.dtype == torch.float16:
-        return _lib.NQ_F16
-    if A.dtype == torch.bfloat16:
-        return _lib.NQ_BF16
-    raise RuntimeError("Unsupported dtype: Marlin only supports Half and BFloat16")
-
-
-def _check_gemm_tensor(t, name, dtype=None):
-    if t is None:
-        return
-    if not t.is_cuda:
-        raise RuntimeError(f"{name} must be a CUDA tensor")
-    if not t.is_contiguous():
-        raise RuntimeError(f"{name} must be contiguous")
-    if dtype is not None and t.dtype != dtype:
-        raise RuntimeError(f"{name} must have dtype {dtype}")
-
-
 # Workspace of the panel launches (partial tiles, hand-over flags, the count of finished workgroups): zero when
 # first used, then owned by the launches; one per (device, stream) so that launches sharing it are stream-ordered.
 _panel_ws_cache = {}
@@ -270,6 +202,10 @@ def _panel_workspace(device):
     return buf
 
 
+def _panel_workspace_of(xs):
+    return lambda: _panel_workspace(xs[0].device)
+
+
 def panel_status(device=None) -> int:
     """Status word of the current stream's panel workspace (synchronises; reads and clears): 0 ok, 1 = a bounded
     wait of a panel launch expired since the last call and that launch's outputs are invalid."""
@@ -284,53 +220,9 @@ def panel_status(device=None) -> int:
     return int(out.value)
 
 
-def marlin_onebit_forward(x, weight, scale_g, scale_h, workspace):
-    """C[m, n] = s_out[n] * sum_k (x[m, k] * s_in[k]) * sgn(weight)[n, k]; weight from marlin_onebit_packer."""
-    dt = _gemm_dtype(x)
-    m, n, k = _onebit_check(x, weight, scale_g, scale_h, workspace)
-    _check_gemm_tensor(x, "x")
-    _check_gemm_tensor(weight, "weight", torch.int32)
-    _check_gemm_tensor(scale_g, "scale_g", x.dtype)
-    _check_gemm_tensor(scale_h, "scale_h", x.dtype)
-    C = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    if m == 0 or n == 0:
-        return C
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().nq_gemm_onebit(_ptr(x), _ptr(weight), _ptr(scale_g), _ptr(scale_h), _ptr(C),
-                                             None, 0, m, k, n, dt, _stream(x.device)))
-    return C
-
-
 def _marlin_onebit_meta(x, weight, scale_g, scale_h, workspace):
     m, n, _ = _onebit_check(x, weight, scale_g, scale_h, workspace)
     return x.new_empty((m, n))
-
-
-def _gemm_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace, bias=None):
-    dt = _gemm_dtype(x)
-    t, r, n = _onebit_check(x, weight_u, scale_g, scale_l, workspace)
-    _check_gemm_tensor(x, "x")
-    _check_gemm_tensor(weight_u, "weight_u", torch.int32)
-    _check_gemm_tensor(weight_v, "weight_v", torch.int32)
-    for name, s in (("scale_g", scale_g), ("scale_l", scale_l), ("scale_h", scale_h)):
-        _check_gemm_tensor(s, name, x.dtype)
-    imm = torch.empty((t, r), dtype=x.dtype, device=x.device)
-    _, m, _ = _onebit_check(imm, weight_v, None, scale_h, workspace)
-    _check_bias(bias, m, x)
-    out = torch.empty((t, m), dtype=x.dtype, device=x.device)
-    if t == 0 or m == 0:
-        return out
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().nq_gemm_nanoquant_bias(_ptr(x), _ptr(weight_u), _ptr(weight_v), _ptr(scale_g), _ptr(scale_l),
-                                                     _ptr(scale_h), _ptr(bias), _ptr(imm), _ptr(out), None, 0,
-                                                     t, n, r, m, dt, _stream(x.device)))
-    return out
-
-
-def marlin_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace):
-    """Two chained one-bit GEMMs (gemm.cpp:112-122): `weight_u` is the FIRST stage [n -> r],
-    `weight_v` the second [r -> m] (the order marlin_nanoquant_packer returns them)."""
-    return _gemm_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace)
 
 
 def _marlin_nanoquant_meta(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace):
@@ -346,7 +238,7 @@ def _marlin_nanoquant_meta(x, weight_u, weight_v, scale_g, scale_l, scale_h, wor
 def gemv_forward_with_bias(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias):
     """nanoquant_dyn_forward + bias [m], added in the epilogue of the second stage.  The reference's kernel paths
     return before the module's bias is added (modules/linear.py:121-141); this keeps it."""
-    return _gemv_forward(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias)
+    return _host.gemv_bias(x, scale_g, Ubits, scale_l, Vbits, scale_h, bias)
 
 
 def gemv_group_forward(xs, linears, biases=None, outs=None, one_launch=False):
@@ -475,7 +367,7 @@ def gemv_group_status(device=None) -> int:
 
 def gemm_forward_with_bias(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace, bias):
     """marlin_nanoquant_forward + bias [m], added in the epilogue of the second GEMM."""
-    return _gemm_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace, bias)
+    return _host.gemm_bias(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace, bias)
 
 
 class NqGemmTerm(ctypes.Structure):
@@ -496,56 +388,9 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     itself (see include/nq_gfx950.h).  Returns the list of outputs.  The terms share launches: a single linear leaves most
     of the device idle up to some hundred tokens.  The reference launches every linear by itself
     (modules/linear.py:131-133)."""
-    lib = _lib.lib()
-    count = len(terms)
-    if count == 0:
-        return []
     if isinstance(xs, torch.Tensor):
-        xs = [xs] * count
-    if len(xs) != count or (biases is not None and len(biases) != count) or (outs is not None and len(outs) != count):
-        raise RuntimeError("one x (and one bias / output entry) per term")
-    dt = _gemm_dtype(xs[0])
-    given, outs, keep, arr_items = outs, [], [], []
-    for i, (x, term) in enumerate(zip(xs, terms)):
-        weight_u, weight_v, scale_g, scale_l, scale_h, workspace = term
-        bias = None if biases is None else biases[i]
-        if x.dtype != xs[0].dtype or x.dim() != 2 or x.size(0) != xs[0].size(0) or x.device != xs[0].device:
-            raise RuntimeError("all inputs of a group must be 2-D with the same token count, dtype and device")
-        t, r, n = _onebit_check(x, weight_u, scale_g, scale_l, workspace)
-        _check_gemm_tensor(x, "x")
-        _check_gemm_tensor(weight_u, "weight_u", torch.int32)
-        _check_gemm_tensor(weight_v, "weight_v", torch.int32)
-        for name, s in (("scale_g", scale_g), ("scale_l", scale_l), ("scale_h", scale_h)):
-            _check_gemm_tensor(s, name, x.dtype)
-        imm = torch.empty((t, r), dtype=x.dtype, device=x.device)
-        _, m, _ = _onebit_check(imm, weight_v, None, scale_h, workspace)
-        _check_bias(bias, m, x)
-        if given is None:
-            out = torch.empty((t, m), dtype=x.dtype, device=x.device)
-        else:
-            out = given[i]
-            if (tuple(out.shape) != (t, m) or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous()
-                    or out.data_ptr() % 16 != 0):
-                raise RuntimeError(f"outs[{i}] must be a contiguous, 16-byte aligned [{t}, {m}] tensor of {x.dtype} on {x.device}")
-        outs.append(out)
-        keep.append(imm)
-        pv = lambda ten: None if ten is None else ten.data_ptr()
-        arr_items.append(NqGemmTerm(pv(x), pv(weight_u), pv(weight_v), pv(scale_g), pv(scale_l), pv(scale_h), pv(bias),
-                                    pv(imm), pv(out), n, r, m))
-    tokens = xs[0].size(0)
-    if tokens == 0:
-        return outs
-    device = xs[0].device
-    group_max = int(lib.nq_gemm_group_max())
-    mode = PANEL_MODES[panel]
-    ws = None if mode == 2 else _panel_workspace(device)
-    with torch.cuda.device(device):
-        for lo in range(0, count, group_max):
-            part = arr_items[lo:lo + group_max]
-            arr = (NqGemmTerm * len(part))(*part)
-            _lib.check(lib.nq_gemm_nanoquant_group_ws(arr, len(part), tokens, dt, None, 0, _ptr(ws),
-                                                      0 if ws is None else ws.numel(), mode, _stream(device)))
-    return outs
+        xs = [xs] * len(terms)
+    return _host.gemm_group(xs, terms, biases, outs, PANEL_MODES[panel], _panel_workspace_of(xs))
 
 
 def gemm_group_sum_forward(xs, term_groups, bias_groups=None, panel="auto"):
@@ -556,42 +401,9 @@ def gemm_group_sum_forward(xs, term_groups, bias_groups=None, panel="auto"):
     per weight.  `xs`: one tensor or one per weight; `bias_groups`: optional list (per weight) of lists (per term) of
     bias tensors / None; `panel` as in `gemm_group_forward`.  Returns one [tokens, m] tensor per weight (views of one
     buffer)."""
-    nw = len(term_groups)
-    if nw == 0:
-        return []
     if isinstance(xs, torch.Tensor):
-        xs = [xs] * nw
-    if len(xs) != nw or any(len(g) == 0 for g in term_groups):
-        raise RuntimeError("one x and at least one term per weight")
-    tokens, dtype, device = xs[0].size(0), xs[0].dtype, xs[0].device
-    ms = [g[0][1].size(1) * 2 for g in term_groups]                  # weight_v [r / 16, m / 2]
-    order = sorted(range(nw), key=lambda i: -len(term_groups[i]))      # stable: more terms first
-    depth = len(term_groups[order[0]])
-    sizes = [sum(tokens * ms[i] for i in order if len(term_groups[i]) > t) for t in range(depth)]
-    bufs = [torch.empty(n, dtype=dtype, device=device) for n in sizes]
-    flat_x, flat_terms, flat_bias, flat_out = [], [], [], []
-    results = [None] * nw
-    for t in range(depth):
-        off = 0
-        for i in order:
-            if len(term_groups[i]) <= t:
-                break
-            m = ms[i]
-            if (off * bufs[t].element_size()) % 16 != 0:
-                raise RuntimeError("tokens * out_features must keep the outputs 16-byte aligned")
-            view = bufs[t][off:off + tokens * m].view(tokens, m)
-            off += tokens * m
-            if t == 0:
-                results[i] = view
-            flat_x.append(xs[i])
-            flat_terms.append(term_groups[i][t])
-            flat_bias.append(None if bias_groups is None or bias_groups[i] is None else bias_groups[i][t])
-            flat_out.append(view)
-    gemm_group_forward(flat_x, flat_terms, flat_bias if any(b is not None for b in flat_bias) else None, outs=flat_out,
-                       panel=panel)
-    for t in range(1, depth):
-        bufs[0][:sizes[t]].add_(bufs[t])
-    return results
+        xs = [xs] * len(term_groups)
+    return _host.gemm_group_sum(xs, term_groups, bias_groups, PANEL_MODES[panel], _panel_workspace_of(xs))
 
 
 def gemv_mixture_forward(x, terms):
@@ -728,12 +540,21 @@ def get_kernel_function(namespace: str, dtype: torch.dtype, kernel_type: str):
 # ---------------------------------------------------------------------------------------------
 # registration
 # ---------------------------------------------------------------------------------------------
+class _Unbuilt:
+    def __init__(self, cause):
+        self._cause = cause
+
+    def __getattr__(self, name):
+        raise ImportError(f"nanoquant_amd._host is not usable: {self._cause}") from self._cause
+
+
 _library = torch.library.Library(_NS, "DEF")
 for _schema in _SCHEMAS:
     _library.define(_schema)
-_library.impl("nanoquant_dyn_forward", nanoquant_dyn_forward, "CUDA")
-_library.impl("marlin_onebit_forward", marlin_onebit_forward, "CUDA")
-_library.impl("marlin_nanoquant_forward", marlin_nanoquant_forward, "CUDA")
+try:
+    _host = _lib.host()                  # registers the CUDA implementations
+except (ImportError, AttributeError) as _exc:      # not built, or built from other sources: importing the package must still
+    _host = _Unbuilt(_exc)                         # work for the build itself; every call raises
 _library.impl("nanoquant_dyn_forward", _nanoquant_dyn_forward_meta, "Meta")
 _library.impl("marlin_onebit_forward", _marlin_onebit_meta, "Meta")
 _library.impl("marlin_nanoquant_forward", _marlin_nanoquant_meta, "Meta")

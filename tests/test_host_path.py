@@ -1,0 +1,78 @@
+"""The operators' C++ host path without a GPU: argument checks and their messages, in the order of the reference's host wrappers
+(src/nanoquant/kernel/cuda/gemm.cpp:36-98, gemv_kernel.cu:308-346), and what happens where it is not built."""
+import pytest
+import torch
+
+from nanoquant_amd import _lib, ops
+
+F16 = lambda *s: torch.zeros(*s, dtype=torch.float16)
+I32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
+
+
+def _term(**other):
+    args = dict(weight_u=I32(32, 128), weight_v=I32(16, 64), scale_g=F16(512), scale_l=F16(256), scale_h=F16(128), workspace=I32(64))
+    args.update(other)
+    return tuple(args.values())
+
+
+# what is wrong, the message; on CPU tensors a call in order ends at the device check
+@pytest.mark.parametrize("x,term,message", [
+    (torch.zeros(5, 512), _term(), "Unsupported dtype: Marlin only supports Half and BFloat16"),
+    (F16(5, 500), _term(), "k dimension mismatch"),
+    (F16(5, 512), _term(scale_g=F16(511)), "s_in size mismatch"),
+    (F16(5, 512), _term(scale_l=F16(255)), "s_out size mismatch"),
+    (F16(5, 512), _term(workspace=I32(63)), "workspace too small"),
+    (F16(5, 512), _term(), "x must be a CUDA tensor"),
+])
+def test_prefill_checks(x, term, message):
+    for call in (lambda: ops.gemm_forward_with_bias(x, *term, None), lambda: ops.gemm_group_forward(x, [term]),
+                 lambda: ops.gemm_group_sum_forward(x, [[term]])):
+        with pytest.raises(RuntimeError, match=message):
+            call()
+
+
+@pytest.mark.parametrize("call", [
+    lambda x, t: ops.gemm_group_forward([x], [t, t]),
+    lambda x, t: ops.gemm_group_forward(x, [t], biases=[None, None]),
+    lambda x, t: ops.gemm_group_forward(x, [t], outs=[]),
+    lambda x, t: ops.gemm_group_sum_forward([x], [[t], [t]]),
+    lambda x, t: ops.gemm_group_sum_forward([x], [[]]),
+])
+def test_lists_of_different_lengths(call):
+    with pytest.raises(RuntimeError, match=r"one x (and at least one term per weight|\(and one bias / output entry\) per term)"):
+        call(F16(5, 512), _term())
+
+
+def test_empty_groups():
+    assert ops.gemm_group_forward(F16(5, 512), []) == [] and ops.gemm_group_sum_forward(F16(5, 512), []) == []
+
+
+def test_terms_that_are_no_terms():
+    with pytest.raises(ValueError, match="a term is"):
+        ops.gemm_group_forward(F16(5, 512), [_term()[:5]])
+    with pytest.raises(TypeError, match="weight_v must be a tensor"):
+        ops.gemm_group_forward(F16(5, 512), [(I32(32, 128), 3, None, None, None, I32(64))])
+
+
+def test_decode_checks_in_order():
+    args = (F16(1, 64), F16(64), I32(32, 2), None, I32(96, 1), F16(96))
+    with pytest.raises(RuntimeError, match="Support only Half or BFloat16"):
+        ops.gemv_forward_with_bias(torch.zeros(1, 64), *args[1:], None)
+    with pytest.raises(RuntimeError, match="x must be a CUDA tensor"):
+        ops.gemv_forward_with_bias(*args, None)
+
+
+def test_a_missing_build_is_an_import_error():
+    broken = ops._Unbuilt(ImportError("not there"))
+    with pytest.raises(ImportError, match="not there"):
+        broken.gemm_group([], [])
+    assert _lib.host().__name__ == "nanoquant_amd._host"
+
+
+def test_no_panel_without_need():
+    # argument checks only: no device is asked
+    lib = _lib.lib()
+    assert lib.nq_gemm_group_wants_panel(None, 1, 128, 0) == 0
+    arr = (ops.NqGemmTerm * 1)(ops.NqGemmTerm(*[None] * 9, 512, 256, 128))
+    assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 2) == 0 and lib.nq_gemm_group_wants_panel(arr, 1, 0, 1) == 0
+    assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 1) == 1
