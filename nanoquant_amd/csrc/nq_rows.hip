@@ -46,6 +46,11 @@ constexpr int kRowsMaxWaves = 8;     // wavefronts of a workgroup
 //   rows they lose 1 to 6 % throughout (5120 x 8192: 12.3 against 11.6 at 8 rows).
 constexpr int kTwoBlocksFrom = 257;  // 16-row blocks of a launch, 5 batch rows and more
 constexpr int kFewWavesFrom = 8192;  // rows of a linear
+// Up to this many staged rows the input operands are read two steps ahead of their products (left to itself the compiler waits
+// for every pair of reads; with more rows the workgroups that share a compute unit hide that, and the registers count): layer of
+// four groups, stages repeated, 1 / 4 / 11 rows fp16: 35.6 / 39.0 / 49.1 us without, 34.3 / 38.6 / 50.6 with; four or eight steps
+// ahead 34.7 / 39.3 / 50.9 and 35.6 / 42.0 / 52.2.
+constexpr int kReadAheadRows = 4;
 constexpr int kStagePitch = 1040;    // LDS bytes per staged input row of a chunk: 512 x 2 + 16 (8 lanes of an operand
                                      // read that differ in the batch row only hit 8 different bank groups)
 
@@ -74,7 +79,7 @@ struct RowsProblem {
 constexpr int kGroupMax = 8;
 template <int NT, int N>
 struct RowsGroup {
-    int batch;
+    int batch, waves;                // wavefronts of a workgroup
     int first[N + 1];                // first workgroup of every problem; [N] = the grid
     RowsProblem<NT> p[N];
 };
@@ -235,7 +240,7 @@ struct StageWait {
 // workgroup of the same launch reads it), the second stage waits until every first-stage workgroup of its linear has
 // arrived and reads h with device-coherent loads.
 template <int DT, bool SCALED, int NB, int F, int NT, bool VEC, bool FUSED>
-__device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, int nb, const StageWait& wait) {
+__device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, int nb, int launch_waves, const StageWait& wait) {
     using E = Elem<DT>;
     constexpr bool kInOperand = rows_scale_in_operand<DT, SCALED, NB>();
     constexpr int kWaveLds = rows_wave_lds<DT, SCALED, NB, F>();
@@ -267,7 +272,7 @@ __device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, i
 
     // What the epilogue needs is asked for up front (by the wavefronts that will run it), not one round trip at a time at
     // the end; rows past the last one read zeros.
-    const int rows = early(p.rows), out_stride = early(p.out_stride), out_kind = early(p.out_kind);
+    const int rows = early(p.rows), out_stride = early(p.out_stride), out_kind = early(p.out_kind), waves = early(launch_waves);
     char* const out_base = early((char*)p.out);
     const uint16_t* const s_row = early(p.t[0].s_row);
     const uint16_t* const bias = early(p.bias);
@@ -332,11 +337,13 @@ __device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, i
             wave_lds_fence();
             load_words<SCALED, VEC, F>(nw, v, ragged, chunk + p.waves, lane);
             load_inputs<SCALED, NB, VEC, FUSED && !SCALED>(nx, ns, v, chunk + p.waves, lane);
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {               // step q: 8 of the 128 columns of every lane group's unit
-                const u32x4_t b = *(const u32x4_t*)(mine + read_off + 16 * q);
-                u32x4_t one = (u32x4_t){one_pair, one_pair, one_pair, one_pair};
+            // step q: 8 of the 128 columns of every lane group's unit
+            auto read = [&](int q, u32x4_t& b, u32x4_t& one) __attribute__((always_inline)) {
+                b = *(const u32x4_t*)(mine + read_off + 16 * q);
+                one = (u32x4_t){one_pair, one_pair, one_pair, one_pair};
                 if constexpr (kInOperand) one = *(const u32x4_t*)(mine + NB * kStagePitch + 256 * g + 16 * q);
+            };
+            auto step = [&](int q, const u32x4_t& b, const u32x4_t& one) __attribute__((always_inline)) {
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
                     const uint32_t word = w[f][q >> 2];
@@ -344,6 +351,31 @@ __device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, i
 #pragma unroll
                     for (int k = 0; k < 4; ++k) a[k] = ((word << (4 * (q & 3) + k)) & mask) ^ one[k];
                     acc[f] = RowsArith<DT>::mfma(a, b, acc[f]);
+                }
+            };
+            if constexpr (NB <= kReadAheadRows) {
+                // the operands of the next two steps are read while two multiply
+                u32x4_t b[2][2], one[2][2];
+                read(0, b[0][0], one[0][0]);
+                read(1, b[0][1], one[0][1]);
+#pragma unroll
+                for (int q = 0; q < 16; q += 2) {
+                    const int now = (q >> 1) & 1;
+                    if (q + 2 < 16) {
+                        read(q + 2, b[now ^ 1][0], one[now ^ 1][0]);
+                        read(q + 3, b[now ^ 1][1], one[now ^ 1][1]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    step(q, b[now][0], one[now][0]);
+                    step(q + 1, b[now][1], one[now][1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    u32x4_t b, one;
+                    read(q, b, one);
+                    step(q, b, one);
                 }
             }
         }
@@ -364,7 +396,6 @@ __device__ __forceinline__ void rows_body(const RowsProblem<NT>& p, int block, i
     for (int f = 0; f < F; ++f) *(float4_t*)(mine + f * 1024 + 16 * lane) = NT > 1 ? tot[f] : acc[f];
     __syncthreads();
     if (wave >= F) return;
-    const int waves = (int)(blockDim.x >> 6);
     float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int wv = 0; wv < kRowsMaxWaves; ++wv) {
@@ -425,7 +456,7 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_rows_kernel(RowsGroup
             i = k;
             first = gr.first[k];
         }
-    rows_body<DT, SCALED, NB, F, NT, VEC, false>(gr.p[i], b - first, gr.batch, StageWait{});
+    rows_body<DT, SCALED, NB, F, NT, VEC, false>(gr.p[i], b - first, gr.batch, gr.waves, StageWait{});
 }
 
 // Both stages of up to kGroupMax linears in ONE ordinary launch (no resident-grid requirement): the workgroups of all
@@ -448,6 +479,7 @@ struct FusedArgs {
     unsigned* slot;                  // kFusedSlotWords words, zero between launches
     unsigned* status;
     unsigned spin_limit;
+    int waves;                       // wavefronts of a workgroup, both stages
 };
 
 template <int DT, int NB, bool VEC>
@@ -456,7 +488,7 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_fused_kernel(FusedArg
     const int n1 = f.a.first[kGroupMax];
     if (b < n1) {
         const int i = problem_of<kGroupMax>(f.a.first, b);
-        rows_body<DT, true, NB, 1, 1, VEC, true>(f.a.p[i], b - f.a.first[i], f.a.batch, StageWait{});
+        rows_body<DT, true, NB, 1, 1, VEC, true>(f.a.p[i], b - f.a.first[i], f.a.batch, f.waves, StageWait{});
         // every wavefront waits until its own stores of h have been acknowledged, the barrier collects all of them,
         // then the arrival is counted
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -478,7 +510,7 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void gemv_fused_kernel(FusedArg
         w.target = 1u;
         w.spin_limit = f.spin_limit;
         w.status = f.status;
-        rows_body<DT, false, NB, 1, 1, VEC, true>(f.b.p[i], lb - f.b.first[i], f.b.batch, w);
+        rows_body<DT, false, NB, 1, 1, VEC, true>(f.b.p[i], lb - f.b.first[i], f.b.batch, f.waves, w);
         __syncthreads();
         if (threadIdx.x < kWave) {
             unsigned before = 0;
@@ -553,6 +585,7 @@ static int make_group(RowsGroup<NT, N>& g, int count, const RowsStage* s, int ba
     g.first[N] = at;                     // so that no workgroup belongs to an unused entry
     for (int i = count; i < N; ++i) g.first[i] = at;
     g.batch = batch;
+    g.waves = *waves;
     return at;
 }
 
@@ -708,6 +741,7 @@ hipError_t gemv_rows_fused(int dtype, int count, const RowsStage* first, const R
     const unsigned spin = g_fused_spin_limit.load();
     f.spin_limit = spin ? spin : (1u << 20);
     const int waves = std::max(wa, wb);
+    f.waves = waves;
     return dtype == 0 ? launch_fused_batch<0>(f, vec, na + nb, waves, batch, stream) : launch_fused_batch<1>(f, vec, na + nb, waves, batch, stream);
 }
 
