@@ -288,6 +288,14 @@ int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens,
 /* 1 when a stage of that call would be a panel launch (0 otherwise, and for NQ_PANEL_NEVER), so that a caller can do without the
  * workspace until one is. */
 int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode);
+/* Weights that are sums of terms, without a pass that adds: next[i] is the term behind term i of the same weight (-1: none;
+ * next[i] > i, the same m), and the y of a weight's first term receives the sum, every term scaled and its bias added in 32 bits
+ * and the sum rounded once; the y of the others is not used (may be NULL).  The first GEMMs are those of the call above with the
+ * same workspace and mode; all terms have s_in or none has (NQ_ERR_SHAPE otherwise). */
+int nq_gemm_nanoquant_sum(const nq_gemm_term* terms, const int* next, int count, int tokens, int dtype, void* panel_ws,
+                          size_t panel_ws_bytes, int panel_mode, void* stream);
+/* 1 when that call is estimated to take less than nq_gemm_nanoquant_group_ws and the additions (0 otherwise, for terms that it refuses and where nothing is summed). */
+int nq_gemm_sum_pays(const nq_gemm_term* terms, const int* next, int count, int tokens);
 int nq_gemm_panel_status(const void* panel_ws, int* status_out, void* stream);
 /* Polls after which a wait of a panel launch gives up (0 = the default of 2^20).  Process-wide; for exercising a
  * caller's handling of status 1 from the host, as nq_gemv_group_set_spin_limit. */

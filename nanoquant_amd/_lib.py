@@ -50,6 +50,8 @@ _SIGNATURES = {
     "nq_gemm_panel_workspace_bytes": (_sz, []),
     "nq_gemm_nanoquant_group_ws": (_i, [_vp, _i, _i, _i, _vp, _sz, _vp, _sz, _i, _vp]),
     "nq_gemm_group_wants_panel": (_i, [_vp, _i, _i, _i]),
+    "nq_gemm_nanoquant_sum": (_i, [_vp, ctypes.POINTER(_i), _i, _i, _i, _vp, _sz, _i, _vp]),
+    "nq_gemm_sum_pays": (_i, [_vp, ctypes.POINTER(_i), _i, _i]),
     "nq_gemm_panel_status": (_i, [_vp, ctypes.POINTER(_i), _vp]),
     "nq_gemm_panel_set_spin_limit": (_i, [ctypes.c_uint]),
     "nq_pack_gemm_tiles": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp]),

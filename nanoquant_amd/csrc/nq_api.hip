@@ -790,78 +790,150 @@ int nq_gemm_panel_status(const void* panel_ws, int* status_out, void* stream) {
     return hip_status(e);
 }
 
-int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode) {
-    if (!terms || count < 1 || count > nq::gemm_group_max() || tokens < 1 || panel_mode == NQ_PANEL_NEVER) return 0;
-    if (panel_mode == NQ_PANEL_ALWAYS) return 1;
-    const void* x[16]; const void* h[16];
-    int n[16], r[16], m[16];
-    static_assert(sizeof(x) / sizeof(x[0]) >= 16, "nq::gemm_group_max()");
+namespace {
+constexpr int kMaxTerms = 16;                    // >= nq::gemm_group_max(), checked at run time
+// One stage of a group, as the launches take it.
+struct GroupStage {
+    const void* x[kMaxTerms]; const uint32_t* w[kMaxTerms]; const void* si[kMaxTerms]; const void* so[kMaxTerms];
+    const void* bs[kMaxTerms]; void* out[kMaxTerms];
+    int K[kMaxTerms], R[kMaxTerms];
+};
+GroupStage first_stage(const nq_gemm_term* terms, int count) {
+    GroupStage s;
     for (int i = 0; i < count; ++i) {
-        x[i] = terms[i].x; h[i] = terms[i].h; n[i] = terms[i].n; r[i] = terms[i].r; m[i] = terms[i].m;
+        const nq_gemm_term& t = terms[i];
+        s.x[i] = t.x; s.w[i] = t.vt_tiles; s.si[i] = t.s_in; s.so[i] = t.s_mid; s.bs[i] = nullptr; s.out[i] = t.h; s.K[i] = t.n; s.R[i] = t.r;
     }
-    return nq::panel_applies(count, x, tokens, n, r, terms[0].s_in != nullptr) || nq::panel_applies(count, h, tokens, r, m, false);
+    return s;
+}
+GroupStage second_stage(const nq_gemm_term* terms, int count) {
+    GroupStage s;
+    for (int i = 0; i < count; ++i) {
+        const nq_gemm_term& t = terms[i];
+        s.x[i] = t.h; s.w[i] = t.u_tiles; s.si[i] = nullptr; s.so[i] = t.s_out; s.bs[i] = t.bias; s.out[i] = t.y; s.K[i] = t.r; s.R[i] = t.m;
+    }
+    return s;
+}
+bool panel_for(const GroupStage& s, int count, int tokens) {
+    return nq::panel_applies(count, s.x, tokens, s.K, s.R, s.si[0] != nullptr);
+}
+struct PanelUse {
+    void* ws;                                    // null: no panel launches
+    int mode;
+};
+// The panel launch where a workspace was given and the shapes make it the faster one.
+hipError_t run_stage(const GroupStage& s, int count, int tokens, int dtype, const PanelUse& panel, hipStream_t stream) {
+    if (panel.ws && (panel.mode == NQ_PANEL_ALWAYS || panel_for(s, count, tokens)))
+        return nq::gemm_panel_group(dtype, count, s.x, s.w, s.si, s.so, s.bs, s.out, tokens, s.K, s.R, panel.ws,
+                                    g_panel_spin_limit.load(), stream);
+    return nq::gemm_onebit_group(dtype, count, s.x, s.w, s.si, s.so, s.bs, s.out, tokens, s.K, s.R,
+                                 panel.mode == NQ_PANEL_AUTO ? nq::kGemmAnyTile : nq::kGemmGroup, stream);
+}
+// next: null, or the chains of a call that sums terms (only their first terms have a y).  *alike: all have s_in or none has.
+int check_terms(const nq_gemm_term* terms, const int* next, int count, bool* alike) {
+    *alike = true;
+    bool chained[kMaxTerms] = {};
+    for (int i = 0; i < count; ++i) {
+        const nq_gemm_term& t = terms[i];
+        if (t.n <= 0 || t.r <= 0 || t.m <= 0) return NQ_ERR_SHAPE;
+        if (t.n % 256 != 0 || t.r % 256 != 0 || t.m % 32 != 0) return NQ_ERR_PROB_SHAPE;
+        if (!t.x || !t.vt_tiles || !t.u_tiles || !t.h || !(t.y || chained[i])) return NQ_ERR_NULL;
+        if (((uintptr_t)t.x | (uintptr_t)t.vt_tiles | (uintptr_t)t.u_tiles | (uintptr_t)t.h | (uintptr_t)t.y |
+             (uintptr_t)t.s_in | (uintptr_t)t.s_mid | (uintptr_t)t.s_out | (uintptr_t)t.bias) & 15u)
+            return NQ_ERR_ALIGN;
+        if ((t.s_in == nullptr) != (terms[0].s_in == nullptr)) *alike = false;
+        for (int j = 0; j < i; ++j)                                                // results would overwrite each other
+            if (terms[j].h == t.h || (terms[j].y == t.y && !chained[i] && !chained[j])) return NQ_ERR_SHAPE;
+        if (next && next[i] >= 0) {                                                // a later term of as many rows, in one chain only
+            if (next[i] <= i || next[i] >= count || terms[next[i]].m != t.m || chained[next[i]]) return NQ_ERR_SHAPE;
+            chained[next[i]] = true;
+        }
+    }
+    return NQ_OK;
+}
+int check_panel(void* panel_ws, size_t panel_ws_bytes, int panel_mode, PanelUse* use) {
+    *use = PanelUse{panel_mode != NQ_PANEL_NEVER ? panel_ws : nullptr, panel_mode};
+    if (!use->ws) return NQ_OK;
+    if (((uintptr_t)panel_ws) & 255u) return NQ_ERR_ALIGN;
+    const size_t need = nq::panel_workspace_bytes();
+    return need == 0 || panel_ws_bytes < need ? NQ_ERR_WORKSPACE : NQ_OK;
+}
+bool known_panel_mode(int mode) { return mode == NQ_PANEL_AUTO || mode == NQ_PANEL_ALWAYS || mode == NQ_PANEL_NEVER; }
+}  // namespace
+
+int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode) {
+    if (!terms || count < 1 || count > nq::gemm_group_max() || count > kMaxTerms || tokens < 1 || panel_mode == NQ_PANEL_NEVER) return 0;
+    if (panel_mode == NQ_PANEL_ALWAYS) return 1;
+    return panel_for(first_stage(terms, count), count, tokens) || panel_for(second_stage(terms, count), count, tokens);
 }
 
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                                size_t scratch_bytes, void* panel_ws, size_t panel_ws_bytes, int panel_mode, void* stream) {
     if (dtype != NQ_F16 && dtype != NQ_BF16) return NQ_ERR_DTYPE;
-    if (count < 0 || tokens < 0) return NQ_ERR_SHAPE;
-    if (panel_mode != NQ_PANEL_AUTO && panel_mode != NQ_PANEL_ALWAYS && panel_mode != NQ_PANEL_NEVER) return NQ_ERR_SHAPE;
+    if (count < 0 || tokens < 0 || !known_panel_mode(panel_mode)) return NQ_ERR_SHAPE;
     if (count == 0 || tokens == 0) return NQ_OK;
     if (!terms) return NQ_ERR_NULL;
-    if (count > nq::gemm_group_max()) return NQ_ERR_SHAPE;
-    bool grouped = true;
-    for (int i = 0; i < count; ++i) {
-        const nq_gemm_term& t = terms[i];
-        if (t.n <= 0 || t.r <= 0 || t.m <= 0) return NQ_ERR_SHAPE;
-        if (t.n % 256 != 0 || t.r % 256 != 0 || t.m % 32 != 0) return NQ_ERR_PROB_SHAPE;
-        if (!t.x || !t.vt_tiles || !t.u_tiles || !t.h || !t.y) return NQ_ERR_NULL;
-        if (((uintptr_t)t.x | (uintptr_t)t.vt_tiles | (uintptr_t)t.u_tiles | (uintptr_t)t.h | (uintptr_t)t.y |
-             (uintptr_t)t.s_in | (uintptr_t)t.s_mid | (uintptr_t)t.s_out | (uintptr_t)t.bias) & 15u)
-            return NQ_ERR_ALIGN;
-        if ((t.s_in == nullptr) != (terms[0].s_in == nullptr)) grouped = false;   // one kernel variant per launch
-        for (int j = 0; j < i; ++j)
-            if (terms[j].h == t.h || terms[j].y == t.y) return NQ_ERR_SHAPE;      // results would overwrite each other
-    }
-    if (!grouped) {                              // mixed kernel variants: one linear after the other
+    if (count > nq::gemm_group_max() || count > kMaxTerms) return NQ_ERR_SHAPE;
+    bool alike = true;                           // one kernel variant per launch
+    int st = check_terms(terms, nullptr, count, &alike);
+    if (st != NQ_OK) return st;
+    if (!alike) {                                // mixed kernel variants: one linear after the other
         for (int i = 0; i < count; ++i) {
             const nq_gemm_term& t = terms[i];
-            int st = nq_gemm_nanoquant_bias(t.x, t.vt_tiles, t.u_tiles, t.s_in, t.s_mid, t.s_out, t.bias, t.h, t.y, scratch,
-                                            scratch_bytes, tokens, t.n, t.r, t.m, dtype, stream);
+            st = nq_gemm_nanoquant_bias(t.x, t.vt_tiles, t.u_tiles, t.s_in, t.s_mid, t.s_out, t.bias, t.h, t.y, scratch,
+                                        scratch_bytes, tokens, t.n, t.r, t.m, dtype, stream);
             if (st != NQ_OK) return st;
         }
         return NQ_OK;
     }
-    constexpr int kMax = 16;                     // >= nq::gemm_group_max(), checked above
-    static_assert(kMax >= 16, "group arrays");
-    const void* x[kMax]; const uint32_t* w[kMax]; const void* si[kMax]; const void* so[kMax]; const void* bs[kMax]; void* out[kMax];
-    int K[kMax], R[kMax];
-    if (count > kMax) return NQ_ERR_SHAPE;
-    const bool have_ws = panel_ws && panel_mode != NQ_PANEL_NEVER;
-    if (have_ws) {
-        if (((uintptr_t)panel_ws) & 255u) return NQ_ERR_ALIGN;
-        const size_t need = nq::panel_workspace_bytes();
-        if (need == 0 || panel_ws_bytes < need) return NQ_ERR_WORKSPACE;
-    }
-    // one stage: the panel launch where a workspace was given and the shapes make it the faster one
-    auto stage = [&]() -> hipError_t {
-        if (have_ws && (panel_mode == NQ_PANEL_ALWAYS || nq::panel_applies(count, x, tokens, K, R, si[0] != nullptr)))
-            return nq::gemm_panel_group(dtype, count, x, w, si, so, bs, out, tokens, K, R, panel_ws, g_panel_spin_limit.load(),
-                                        (hipStream_t)stream);
-        return nq::gemm_onebit_group(dtype, count, x, w, si, so, bs, out, tokens, K, R,
-                                     panel_mode == NQ_PANEL_AUTO ? nq::kGemmAnyTile : nq::kGemmGroup, (hipStream_t)stream);
-    };
-    for (int i = 0; i < count; ++i) {
-        const nq_gemm_term& t = terms[i];
-        x[i] = t.x; w[i] = t.vt_tiles; si[i] = t.s_in; so[i] = t.s_mid; bs[i] = nullptr; out[i] = t.h; K[i] = t.n; R[i] = t.r;
-    }
-    hipError_t e = stage();
+    PanelUse panel;
+    st = check_panel(panel_ws, panel_ws_bytes, panel_mode, &panel);
+    if (st != NQ_OK) return st;
+    hipError_t e = run_stage(first_stage(terms, count), count, tokens, dtype, panel, (hipStream_t)stream);
     if (e != hipSuccess) return hip_status(e);
+    return hip_status(run_stage(second_stage(terms, count), count, tokens, dtype, panel, (hipStream_t)stream));
+}
+
+int nq_gemm_nanoquant_sum(const nq_gemm_term* terms, const int* next, int count, int tokens, int dtype, void* panel_ws,
+                          size_t panel_ws_bytes, int panel_mode, void* stream) {
+    if (dtype != NQ_F16 && dtype != NQ_BF16) return NQ_ERR_DTYPE;
+    if (count < 0 || tokens < 0 || !known_panel_mode(panel_mode)) return NQ_ERR_SHAPE;
+    if (count == 0 || tokens == 0) return NQ_OK;
+    if (!terms || !next) return NQ_ERR_NULL;
+    if (count > nq::gemm_group_max() || count > kMaxTerms) return NQ_ERR_SHAPE;
+    bool alike = true;
+    int st = check_terms(terms, next, count, &alike);
+    if (st != NQ_OK) return st;
+    if (!alike) return NQ_ERR_SHAPE;
+    PanelUse panel;
+    st = check_panel(panel_ws, panel_ws_bytes, panel_mode, &panel);
+    if (st != NQ_OK) return st;
+    hipError_t e = run_stage(first_stage(terms, count), count, tokens, dtype, panel, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_status(e);
+    const GroupStage s = second_stage(terms, count);
+    return hip_status(nq::gemm_onebit_sums(dtype, count, next, s.x, s.w, s.so, s.bs, s.out, tokens, s.K, s.R, (hipStream_t)stream));
+}
+
+// The sums by launches of their own: per pass over a term index 3 us, and two reads and one write of the 16-bit results at the
+// 4.8 TB/s that a large copy reaches.  In us, apart and added / as a sum (two stages): a pair of 4096 x 4096 terms on 64 tokens
+// 14.3 / 13.3, on 512 29 / 25, on 8192 211 / 185; five terms of 2048 x 2048 on 1000 tokens 40 / 25.  Level, and left apart, where
+// one weight of few rows is a sum and a large one is not (256 rows beside 12288 on 512 tokens: 41.6 / 42.2).
+int nq_gemm_sum_pays(const nq_gemm_term* terms, const int* next, int count, int tokens) {
+    if (!terms || !next || count < 1 || count > nq::gemm_group_max() || count > kMaxTerms || tokens < 1) return 0;
+    bool alike = true;
+    if (check_terms(terms, next, count, &alike) != NQ_OK || !alike) return 0;
+    int depth[kMaxTerms] = {}, passes = 0;
+    double adds = 0;
     for (int i = 0; i < count; ++i) {
-        const nq_gemm_term& t = terms[i];
-        x[i] = t.h; w[i] = t.u_tiles; si[i] = nullptr; so[i] = t.s_out; bs[i] = t.bias; out[i] = t.y; K[i] = t.r; R[i] = t.m;
+        if (next[i] < 0) continue;
+        const int d = depth[next[i]] = depth[i] + 1;
+        passes = passes > d ? passes : d;
+        adds += 6.0 * tokens * terms[i].m / 4.8e6;
     }
-    return hip_status(stage());
+    if (passes == 0) return 0;
+    const GroupStage s = second_stage(terms, count);
+    const double tiles = nq::gemm_tiles_time(count, s.x, tokens, s.K, s.R, false), panels = nq::panel_time(count, tokens, s.K, s.R, false);
+    return nq::gemm_sums_time(count, next, tokens, s.K, s.R) < (panels < 0.95 * tiles ? panels : tiles) + 3.0 * passes + adds;
 }
 
 size_t nq_tiled_words(int rows, int words) {

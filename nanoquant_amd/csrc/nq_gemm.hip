@@ -15,7 +15,7 @@ namespace nq {
 // Workgroups of all problems one behind the other: workgroup b belongs to the problem p with first[p] <= b < first[p + 1].
 // A linear by itself has kernels of its own (N = 1): finding the problem is a round trip to the kernel arguments ahead of the
 // first load (2048 x 2048 on 128 tokens, both GEMMs in a graph: 9.95 us with the kernels of 16, 9.3 with these).
-constexpr int kGroupMax = 16;   // 16 problems of 72 bytes: well inside the 4 KB of kernel arguments
+constexpr int kGroupMax = 16;   // 16 problems of 64 bytes: well inside the 4 KB of kernel arguments
 template <int N>
 struct GemmGroup {
     GemmArgs a[N];
@@ -34,19 +34,11 @@ static int group_blocks(int gx, int gy) {
     return (gx * gy + 7) / 8 * 8;
 }
 
-template <int DT, bool SCALED, int TT, int RT, int WR, int WK, int NB, int N>
-__global__ __launch_bounds__(64 * WR * WK, 2) void gemm_tile_kernel(GemmGroup<N> g) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t tile_lds[];
-    const int b = blockIdx.x;
-    // first[i] of the unused entries is the grid size, so no count is needed; all of first[] comes with one load
-    int p = 0;
-#pragma unroll
-    for (int i = 1; i < N; ++i) p += b >= g.first[i] ? 1 : 0;
-    const GemmArgs a = g.a[p];
-    const int local = N > 1 ? b - g.first[p] : b;
+// Row block and token block of workgroup `local` of a problem; false: none.
+template <int TT>
+__device__ __forceinline__ bool tile_of(const GemmArgs& a, int local, int& bx, int& by) {
     const int gx = a.gx, gy = (a.T + 32 * TT - 1) / (32 * TT);
     const int mode = group_mode(gy);
-    int bx, by;
     if (mode == 0) {
         const int slot = local >> 3;
         by = (slot / gx) * 8 + (local & 7);
@@ -59,8 +51,38 @@ __global__ __launch_bounds__(64 * WR * WK, 2) void gemm_tile_kernel(GemmGroup<N>
         bx = local % gx;
         by = local / gx;
     }
-    if (bx >= gx || by >= gy) return;
+    return bx < gx && by < gy;
+}
+
+template <int DT, bool SCALED, int TT, int RT, int WR, int WK, int NB, int N>
+__global__ __launch_bounds__(64 * WR * WK, 2) void gemm_tile_kernel(GemmGroup<N> g) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t tile_lds[];
+    const int b = blockIdx.x;
+    // first[i] of the unused entries is the grid size, so no count is needed; all of first[] comes with one load
+    int p = 0;
+#pragma unroll
+    for (int i = 1; i < N; ++i) p += b >= g.first[i] ? 1 : 0;
+    const GemmArgs a = g.a[p];
+    int bx, by;
+    if (!tile_of<TT>(a, N > 1 ? b - g.first[p] : b, bx, by)) return;
     Tile<DT, SCALED, TT, RT, WR, WK, NB>::run(a, bx, by, tile_lds);
+}
+
+// Sums of terms: the first `heads` entries are one per output, next[p] is the entry of the term behind p (or -1).
+struct GemmSums {
+    GemmGroup<kGroupMax> g;
+    int next[kGroupMax];
+};
+template <int DT, int TT, int RT, int WR, int WK, int NB>
+__global__ __launch_bounds__(64 * WR * WK, 2) void gemm_tile_sum_kernel(GemmSums s) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t tile_lds[];
+    const int b = blockIdx.x;
+    int p = 0;
+#pragma unroll
+    for (int i = 1; i < kGroupMax; ++i) p += b >= s.g.first[i] ? 1 : 0;
+    int bx, by;
+    if (!tile_of<TT>(s.g.a[p], b - s.g.first[p], bx, by)) return;
+    Tile<DT, false, TT, RT, WR, WK, NB>::run_sum(s.g.a, s.next, p, bx, by, tile_lds);
 }
 
 // ---- host side --------------------------------------------------------------------------------
@@ -238,6 +260,117 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
     const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0]}, use, &time);
     if (count == 1) return launch_group<1>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     return launch_group<kGroupMax>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
+}
+
+// ---- sums of terms ------------------------------------------------------------------------------
+// The tiles whose accumulators fit the registers twice.
+constexpr int kSumVariantCount = 5;
+
+template <int DT, int V>
+static hipError_t launch_sums(const GemmSums& s, int blocks, hipStream_t stream) {
+    constexpr TileVariant v = kVariants[V];
+    using S = TileShape<v.tt, v.rt, v.wr, v.wk, v.nb>;
+    auto kern = gemm_tile_sum_kernel<DT, v.tt, v.rt, v.wr, v.wk, v.nb>;
+    static PerDeviceFlag raised;
+    const int dev = current_device();
+    if (S::kLds > 64 * 1024 && !raised.test(dev)) {
+        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLds);
+        if (e != hipSuccess) return e;
+        raised.set(dev);
+    }
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(S::kThreads), S::kLds, stream, s);
+    return hipGetLastError();
+}
+template <int DT>
+static hipError_t launch_sums(int v, const GemmSums& s, int blocks, hipStream_t stream) {
+    static_assert(kSumVariantCount == 5, "one case per entry");
+    switch (v) {
+        case 0: return launch_sums<DT, 0>(s, blocks, stream);
+        case 1: return launch_sums<DT, 1>(s, blocks, stream);
+        case 2: return launch_sums<DT, 2>(s, blocks, stream);
+        case 3: return launch_sums<DT, 3>(s, blocks, stream);
+        default: return launch_sums<DT, 4>(s, blocks, stream);
+    }
+}
+
+// The outputs of a launch of sums: one per term that no other term's next[] names, longest k first.
+struct SumHeads {
+    int count, longest;                                // outputs; most terms of one
+    int at[kGroupMax], K[kGroupMax], R[kGroupMax];     // first term, k summed over the terms, rows
+    int split_k[kGroupMax];                            // the same sum of whole rounds of four wavefronts that split k
+    bool head[kGroupMax];
+};
+static SumHeads sum_heads(int count, const int* next, const int* K, const int* R) {
+    SumHeads h;
+    h.count = h.longest = 0;
+    for (int i = 0; i < count; ++i) h.head[i] = true;
+    for (int i = 0; i < count; ++i)
+        if (next[i] >= 0) h.head[next[i]] = false;
+    for (int i = 0; i < count; ++i) {
+        if (!h.head[i]) continue;
+        int k = 0, split = 0, terms = 0;
+        for (int t = i; t >= 0; t = next[t], ++terms) {
+            k += K[t];
+            split += (K[t] + 4 * kTileK - 1) / (4 * kTileK) * (4 * kTileK);
+        }
+        h.longest = h.longest > terms ? h.longest : terms;
+        int j = h.count++;
+        for (; j > 0 && h.K[j - 1] < k; --j) {
+            h.at[j] = h.at[j - 1]; h.K[j] = h.K[j - 1]; h.R[j] = h.R[j - 1]; h.split_k[j] = h.split_k[j - 1];
+        }
+        h.at[j] = i; h.K[j] = k; h.R[j] = R[i]; h.split_k[j] = split;
+    }
+    return h;
+}
+// A sum costs about what one problem of its terms' k costs, and some 1.5 us for every further term, whose ring is filled anew.
+// Where k is split between wavefronts a term of one k tile takes as long as one of four: counted by its own k, two terms of
+// 256 -> 64 rows on 8192 tokens took such a tile, 20.3 us with the first stage; 17.4 apart and added, 16.6 on the tile taken now.
+static int choose_sum_tile(const SumHeads& h, int T, double* time) {
+    double few_time = 0, block_time = 0;
+    const int few = best_tile(GemmShapes{h.count, T, h.split_k, h.R, false}, 0, kFewTiles, &few_time);
+    const int block = best_tile(GemmShapes{h.count, T, h.K, h.R, false}, kFewTiles, kSumVariantCount, &block_time);
+    const bool take_few = few_time < 0.95 * block_time;
+    *time = (take_few ? few_time : block_time) + 1.5 * (h.longest - 1);
+    return take_few ? few : block;
+}
+double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R) {
+    double time = 0;
+    choose_sum_tile(sum_heads(count, next, K, R), T, &time);
+    return time;
+}
+
+// y of every term that no other term's next[] names = the sum of the GEMMs along next[] (-1: the last); no input scales, the
+// same R along a chain, K % 256 == 0, R % 32 == 0, next[i] > i (checked by the caller).
+hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* const* x, const uint32_t* const* tiles,
+                            const void* const* s_out, const void* const* bias, void* const* y, int T, const int* K, const int* R,
+                            hipStream_t stream) {
+    if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
+    for (int i = 0; i < count; ++i)
+        if (K[i] > kGemmMaxK) return hipErrorInvalidValue;
+    const SumHeads h = sum_heads(count, next, K, R);
+    double time = 0;
+    const int pick = choose_sum_tile(h, T, &time);
+    int slot[kGroupMax];
+    for (int j = 0; j < h.count; ++j) slot[h.at[j]] = j;
+    for (int i = 0, free = h.count; i < count; ++i)
+        if (!h.head[i]) slot[i] = free++;
+    GemmSums s;
+    for (int i = 0; i < kGroupMax; ++i) {
+        const int q = i < count ? i : 0, to = i < count ? slot[i] : i;
+        GemmArgs& a = s.g.a[to];
+        a.x = x[q]; a.tiles = (const uint4*)tiles[q];
+        a.s_in = nullptr; a.s_out = (const uint16_t*)s_out[q]; a.bias = (const uint16_t*)bias[q];
+        a.y = y[q];
+        a.T = T; a.K = K[q]; a.R = R[q];
+        a.gx = tile_gx(kVariants[pick], R[q]);
+        s.next[to] = i < count && next[i] >= 0 ? slot[next[i]] : -1;
+    }
+    int blocks = 0;
+    for (int j = 0; j <= kGroupMax; ++j) {
+        s.g.first[j] = blocks;
+        if (j < h.count) blocks += group_blocks(s.g.a[j].gx, tile_gy(kVariants[pick], T));
+    }
+    return dtype == 0 ? launch_sums<0>(pick, s, blocks, stream) : launch_sums<1>(pick, s, blocks, stream);
 }
 
 int gemm_group_max() { return kGroupMax; }

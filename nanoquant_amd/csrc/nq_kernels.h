@@ -96,12 +96,18 @@ int gemm_group_max();
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                              const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                              int T, const int* K, const int* R, int use, hipStream_t stream);
-// Estimated time of that launch with kGemmAnyTile, in us.
+// Sums of GEMMs without input scales in one launch (see nq_gemm.hip).
+hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* const* x, const uint32_t* const* tiles,
+                            const void* const* s_out, const void* const* bias, void* const* y, int T, const int* K, const int* R,
+                            hipStream_t stream);
+double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R);       // estimate of that launch, us
+// Estimated time of gemm_onebit_group with kGemmAnyTile, in us.
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 
 // nq_panel.hip: the same GEMMs at about 128 to 768 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
 size_t panel_workspace_bytes();
+double panel_time(int count, int T, const int* K, const int* R, bool scaled);      // estimate in us; 1e30: not as panels
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 hipError_t gemm_panel_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                             const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,

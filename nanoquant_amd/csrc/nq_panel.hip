@@ -554,23 +554,27 @@ size_t panel_workspace_bytes() {
 // + 1 for every workgroup that a panel is shared by: the middle 90 % of 445 launches are within -8 .. +8 % of that (128 to 2048
 // tokens, 1 to 43 k tiles, 512 to 22016 rows); with fewer than three k steps the hand-over takes most of the time (128
 // tokens, 3072 -> 4096 rows: tiles 7, panels 35).
-bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
+double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
+    constexpr double kNever = 1e30;
     constexpr int kMostTokens = 2048;            // of the launches that were timed
     const int G = panel_grid();
-    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > kMostTokens) return false;
+    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > kMostTokens) return kNever;
     const int tblocks = (T + kPanelTok - 1) / kPanelTok;
     long long units = 0;
     int longest = 0;
     for (int p = 0; p < count; ++p) {
-        if (K[p] % kTileK != 0 || R[p] % 32 != 0) return false;
+        if (K[p] % kTileK != 0 || R[p] % 32 != 0) return kNever;
         units += (long long)((R[p] + kPanelRows - 1) / kPanelRows) * tblocks * (K[p] / kTileK);
         longest = longest > K[p] / kTileK ? longest : K[p] / kTileK;
     }
     const double per_wg = (double)units / G;
-    if (per_wg < 3.0) return false;
+    if (per_wg < 3.0) return kNever;
     const double steps = (double)((units + G - 1) / G);
-    const double time = 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
-    return time < 0.95 * gemm_tiles_time(count, x, T, K, R, scaled);
+    return 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
+}
+
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
+    return panel_time(count, T, K, R, scaled) < 0.95 * gemm_tiles_time(count, x, T, K, R, scaled);
 }
 
 template <int DT, bool SCALED>

@@ -208,19 +208,33 @@ struct Tile {
         return make_uint2(one(s[0], so.x, bs.x) | (one(s[1], so.x >> 16, bs.x >> 16) << 16), one(s[2], so.y, bs.y) | (one(s[3], so.y >> 16, bs.y >> 16) << 16));
     }
 
-    static __device__ __forceinline__ void run(const GemmArgs& a, int bx, int by, uint16_t* lds) {
-        const int lane = threadIdx.x & 63;
-        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        const int wr = wave % WR, wk = wave / WR;
-        const int tok0 = by * S::kTok, row0 = (bx * WR + wr) * RT * 32;
-        const int hi = lane >> 5;
+    // Where a wavefront stands.
+    struct Place {
+        int lane, hi, wave, wr, wk, tok0, row0;
+    };
+    static __device__ __forceinline__ Place place(int bx, int by) {
+        Place c;
+        c.lane = threadIdx.x & 63;
+        c.hi = c.lane >> 5;
+        c.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        c.wr = c.wave % WR;
+        c.wk = c.wave / WR;
+        c.tok0 = by * S::kTok;
+        c.row0 = (bx * WR + c.wr) * RT * 32;
+        return c;
+    }
+
+    // q.acc = this wavefront's sums over its k tiles.  On return nothing is outstanding; other wavefronts may still be reading
+    // their last slab.
+    static __device__ __forceinline__ void walk(const GemmArgs& a, const Place& c, uint16_t* lds, State& q) {
+        const int lane = c.lane, wr = c.wr, wk = c.wk;
         const char* group = (const char*)lds + wk * S::kGroupBytes;
         Fetch f;
         // both buffers begin with what is this tile's, so that the offsets stay small whatever the matrices' sizes; tokens and
         // rows past the end read zeros
         const int ktiles = a.K / kTileK;
-        f.x = raw_rsrc((const uint16_t*)a.x + (size_t)tok0 * a.K, (uint32_t)min(a.T - tok0, S::kTok) * (uint32_t)a.K * 2u);
-        f.w = raw_rsrc(a.tiles + (size_t)(row0 / 32) * ktiles * 64, (uint32_t)max(0, min(a.R - row0, 32 * RT)) * (uint32_t)a.K / 8u);
+        f.x = raw_rsrc((const uint16_t*)a.x + (size_t)c.tok0 * a.K, (uint32_t)min(a.T - c.tok0, S::kTok) * (uint32_t)a.K * 2u);
+        f.w = raw_rsrc(a.tiles + (size_t)(c.row0 / 32) * ktiles * 64, (uint32_t)max(0, min(a.R - c.row0, 32 * RT)) * (uint32_t)a.K / 8u);
         f.s = raw_rsrc(SCALED ? (const void*)a.s_in : a.x, (uint32_t)a.K * 2u);
         f.wr = wr;
         f.soff = (uint32_t)lane * 16u;
@@ -238,32 +252,12 @@ struct Tile {
         // waves that meet at barriers walk equally many tiles (those past the end are zeros)
         const int count = WR > 1 ? (ktiles + WK - 1) / WK : mine;
         auto slab_k = [&](int j) { return (uint32_t)(wk + (j >> 2) * WK) * 512u + (uint32_t)(j & 3) * 128u; };
-
-        auto row_values = [&](const uint16_t* p, int row, uint32_t pad) { return p && row < a.R ? *(const uint2*)(p + row) : make_uint2(pad, pad); };
-        // piece p of a 32 x 32 tile: rows 8 p + 4 hi .. + 3 of token lane & 31.  With several k groups it is finished by group
-        // p % WK, and the row operands are asked for up front, not one round trip behind the last product
-        constexpr int kPieces = 4 / WK;
-        uint2 so[RT][kPieces], bs[RT][kPieces];
-        auto load_rows = [&] {
-#pragma unroll
-            for (int r = 0; r < RT; ++r)
-#pragma unroll
-                for (int pp = 0; pp < kPieces; ++pp) {
-                    const int row = row0 + 32 * r + 8 * (WK > 1 ? wk + WK * pp : pp) + 4 * hi;
-                    so[r][pp] = row_values(a.s_out, row, E::kOnePair);
-                    bs[r][pp] = row_values(a.bias, row, 0u);
-                }
-        };
-        if constexpr (WK > 1) load_rows();
-
-        State q;
-        auto& acc = q.acc;
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[r][tt][v] = 0.f;
+                for (int v = 0; v < 16; ++v) q.acc[r][tt][v] = 0.f;
         uint32_t one = E::kOnePair;
         asm volatile("" : "+v"(one));
         if (count > 0) {
@@ -277,8 +271,8 @@ struct Tile {
             uint4 sp0 = make_uint4(0, 0, 0, 0);
             q.sp = sp0;
             if constexpr (SCALED) {
-                sp0 = *(const uint4*)(group + S::kScaleAt + 16 * hi);
-                q.sp = *(const uint4*)(group + S::kScaleAt + 16 * hi + 32);
+                sp0 = *(const uint4*)(group + S::kScaleAt + 16 * c.hi);
+                q.sp = *(const uint4*)(group + S::kScaleAt + 16 * c.hi + 32);
             }
 #pragma unroll
             for (int r = 0; r < RT; ++r) q.a[r] = operand(q.w[r][0], 0, sp0, one);
@@ -296,7 +290,31 @@ struct Tile {
             }
         }
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __syncthreads();
+    }
+
+    // Four values of s_out or bias for rows row .. + 3; pad: two of the value where there are none.
+    static __device__ __forceinline__ uint2 row_values(const GemmArgs& a, const uint16_t* p, int row, uint32_t pad) {
+        return p && row < a.R ? *(const uint2*)(p + row) : make_uint2(pad, pad);
+    }
+    // Piece p of a 32 x 32 tile: rows 8 p + 4 hi .. + 3 of token lane & 31.  With several k groups it is finished by group p % WK.
+    static constexpr int kPieces = 4 / WK;
+    struct RowScales {
+        uint2 so[RT][kPieces], bs[RT][kPieces];
+    };
+    static __device__ __forceinline__ void load_rows(const GemmArgs& a, const Place& c, RowScales& s) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int pp = 0; pp < kPieces; ++pp) {
+                const int row = c.row0 + 32 * r + 8 * (WK > 1 ? c.wk + WK * pp : pp) + 4 * c.hi;
+                s.so[r][pp] = row_values(a, a.s_out, row, E::kOnePair);
+                s.bs[r][pp] = row_values(a, a.bias, row, 0u);
+            }
+    }
+
+    // Scales, rounds and stores the sums (all wavefronts are past their last slab).
+    static __device__ __forceinline__ void store(const GemmArgs& a, const Place& c, uint16_t* lds, const float16_t (&acc)[RT][TT], const RowScales& rs) {
+        const int lane = c.lane, hi = c.hi, wave = c.wave, wr = c.wr, wk = c.wk, tok0 = c.tok0, row0 = c.row0;
         if constexpr (WK > 1) {
             // [wave][r][tt][4 pieces][64 lanes] 16 bytes
             float* part = (float*)lds;
@@ -321,14 +339,13 @@ struct Tile {
                         float4_t s = g[0] + g[1];
                         if constexpr (WK == 4) s += g[2] + g[3];
                         const int tok = tok0 + 32 * tt + (lane & 31);
-                        if (row < a.R && tok < a.T) *(uint2*)((uint16_t*)a.y + (size_t)tok * a.R + row) = finish4(s, so[r][pp], bs[r][pp]);
+                        if (row < a.R && tok < a.T) *(uint2*)((uint16_t*)a.y + (size_t)tok * a.R + row) = finish4(s, rs.so[r][pp], rs.bs[r][pp]);
                     }
                 }
         } else {
             constexpr int kPitch = 32 * RT + 8;
             uint16_t* stage = lds + wave * 32 * kPitch;
             if (row0 >= a.R) return;
-            load_rows();
             auto fence = [] {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
                 __builtin_amdgcn_wave_barrier();
@@ -341,7 +358,7 @@ struct Tile {
 #pragma unroll
                     for (int p = 0; p < 4; ++p)
                         *(uint2*)(stage + (lane & 31) * kPitch + 32 * r + 8 * p + 4 * hi) =
-                            finish4((float4_t){acc[r][tt][4 * p], acc[r][tt][4 * p + 1], acc[r][tt][4 * p + 2], acc[r][tt][4 * p + 3]}, so[r][p], bs[r][p]);
+                            finish4((float4_t){acc[r][tt][4 * p], acc[r][tt][4 * p + 1], acc[r][tt][4 * p + 2], acc[r][tt][4 * p + 3]}, rs.so[r][p], rs.bs[r][p]);
                 fence();
                 constexpr int kPer = 4 * RT, kTokPer = 64 / kPer;              // 16-byte chunks of a token, tokens of a store
 #pragma unroll
@@ -354,6 +371,64 @@ struct Tile {
                 fence();
             }
         }
+    }
+
+    static __device__ __forceinline__ void run(const GemmArgs& a, int bx, int by, uint16_t* lds) {
+        const Place c = place(bx, by);
+        RowScales rs;
+        if constexpr (WK > 1) load_rows(a, c, rs);       // asked for up front, not one round trip behind the last product
+        State q;
+        walk(a, c, lds, q);
+        __syncthreads();
+        if constexpr (WK == 1) load_rows(a, c, rs);
+        store(a, c, lds, q.acc, rs);
+    }
+
+    // The sum of terms on the same rows and tokens: table[first], table[next[first]], ...; each is scaled by its own s_out in
+    // 32 bits, and the sum is rounded once.  The terms' 16-bit results and the launches that add them are gone: of 169 us of the
+    // seven two-term linears of a Qwen3-8B layer on 512 tokens 26 went there (now 147).  The registers hold the tile twice, which
+    // the 128 x 256 tile has no room for.
+    static __device__ __forceinline__ void run_sum(const GemmArgs* table, const int* next, int first, int bx, int by, uint16_t* lds) {
+        const Place c = place(bx, by);
+        float16_t tot[RT][TT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) tot[r][tt][v] = 0.f;
+#pragma unroll 1
+        for (int p = first; p >= 0; p = next[p]) {
+            const GemmArgs a = table[p];
+            State q;
+            walk(a, c, lds, q);
+            if constexpr (WR > 1) __syncthreads();       // before the next term's slabs
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int piece = 0; piece < 4; ++piece) {
+                    const int row = c.row0 + 32 * r + 8 * piece + 4 * c.hi;
+                    const uint2 so = row_values(a, a.s_out, row, E::kOnePair);
+                    const uint2 bs = row_values(a, c.wk == 0 ? a.bias : nullptr, row, 0u);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t sw = e < 2 ? so.x : so.y, bw = e < 2 ? bs.x : bs.y;
+                        const float scale = E::to_float((uint16_t)(sw >> (16 * (e & 1)))), bias = E::to_float((uint16_t)(bw >> (16 * (e & 1))));
+#pragma unroll
+                        for (int tt = 0; tt < TT; ++tt) tot[r][tt][4 * piece + e] += q.acc[r][tt][4 * piece + e] * scale + bias;
+                    }
+                }
+        }
+        __syncthreads();
+        RowScales rs;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int pp = 0; pp < kPieces; ++pp) {
+                rs.so[r][pp] = make_uint2(E::kOnePair, E::kOnePair);
+                rs.bs[r][pp] = make_uint2(0u, 0u);
+            }
+        store(table[first], c, lds, tot, rs);
     }
 };
 

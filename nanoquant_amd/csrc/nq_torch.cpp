@@ -277,11 +277,7 @@ GroupTerm group_term(const Tensor& x, const Tensor& x0, PyObject* term, PyObject
     return t;
 }
 
-// The launches of checked terms; y: one output address per term.  panel_ws(): the workspace of the panel launches, asked for
-// only where a stage takes one.
-void launch_group_terms(const std::vector<GroupTerm>& terms, const std::vector<void*>& y, int dt, int panel_mode, const py::object& panel_ws) {
-    const int64_t tokens = terms[0].d.tokens;
-    const int most = nq_gemm_group_max();
+std::vector<nq_gemm_term> terms_of(const std::vector<GroupTerm>& terms, const std::vector<void*>& y) {
     std::vector<nq_gemm_term> arr;
     arr.reserve(terms.size());
     for (size_t i = 0; i < terms.size(); ++i) {
@@ -289,11 +285,23 @@ void launch_group_terms(const std::vector<GroupTerm>& terms, const std::vector<v
         arr.push_back({data(t.x), (const uint32_t*)data(t.weight_u), (const uint32_t*)data(t.weight_v), data(t.scale_g), data(t.scale_l),
                        data(t.scale_h), data(t.bias), t.h.mutable_data_ptr(), y[i], (int)t.d.n, (int)t.d.r, (int)t.d.m});
     }
+    return arr;
+}
+
+// The workspace of the panel launches, panel_ws(), asked for only where a stage takes one.
+MaybeTensor panel_workspace(const nq_gemm_term* terms, int count, int64_t tokens, int panel_mode, const py::object& panel_ws) {
+    if (panel_mode == NQ_PANEL_NEVER || !nq_gemm_group_wants_panel(terms, count, (int)tokens, panel_mode)) return std::nullopt;
+    return tensor_of(panel_ws().ptr(), "the panel workspace");
+}
+
+// The launches of checked terms; y: one output address per term.
+void launch_group_terms(const std::vector<GroupTerm>& terms, const std::vector<void*>& y, int dt, int panel_mode, const py::object& panel_ws) {
+    const int64_t tokens = terms[0].d.tokens;
+    const int most = nq_gemm_group_max();
+    const std::vector<nq_gemm_term> arr = terms_of(terms, y);
     for (size_t lo = 0; lo < arr.size(); lo += most) {
         const int count = (int)std::min<size_t>(most, arr.size() - lo);
-        MaybeTensor ws;
-        if (panel_mode != NQ_PANEL_NEVER && nq_gemm_group_wants_panel(arr.data() + lo, count, (int)tokens, panel_mode))
-            ws = tensor_of(panel_ws().ptr(), "the panel workspace");
+        const MaybeTensor ws = panel_workspace(arr.data() + lo, count, tokens, panel_mode, panel_ws);
         check_status(nq_gemm_nanoquant_group_ws(arr.data() + lo, count, (int)tokens, dt, nullptr, 0, ws ? ws->mutable_data_ptr() : nullptr,
                                                 ws ? (size_t)ws->nbytes() : 0, panel_mode, stream_of(terms[0].x)));
     }
@@ -341,8 +349,9 @@ py::list gemm_group(const py::sequence& xs, const py::sequence& terms, const py:
     return result;
 }
 
-// Weights that are sums of terms: the t-th terms of all weights write into one flat buffer per t, weights with more terms first,
-// so that the sums over the terms are one in-place add per extra term index.
+// Weights that are sums of terms.  Where one call can take all terms the second GEMM adds them up; otherwise the t-th terms of all
+// weights write into one flat buffer per t, weights with more terms first, so that the sums over the terms are one in-place add
+// per extra term index.
 py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups, const py::object& bias_groups, int panel_mode,
                         const py::object& panel_ws) {
     const size_t weights = term_groups.size();
@@ -364,11 +373,10 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return groups[a].size() > groups[b].size(); });
     const size_t depth = groups[order[0]].size();
     std::vector<GroupTerm> checked;
-    std::vector<void*> y;
-    std::vector<Tensor> bufs, firsts(weights);
-    std::vector<int64_t> sizes, rows(weights);
+    std::vector<Tensor> firsts(weights);
+    std::vector<int64_t> rows(weights), offsets, sizes;           // per weight; per checked term; per term index
+    std::vector<int> next, last(weights, -1);
     for (size_t t = 0; t < depth; ++t) {
-        std::vector<std::pair<size_t, int64_t>> at;               // weight, offset in the buffer
         int64_t size = 0;
         for (size_t i : order) {
             if (groups[i].size() <= t) break;
@@ -384,18 +392,37 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
             TORCH_CHECK(rows[i] == d.m, "all terms of a weight must have the same output size");
             checked.back().h = empty({d.tokens, d.r}, x[0]);
             TORCH_CHECK(size * x[0].element_size() % 16 == 0, "tokens * out_features must keep the outputs 16-byte aligned");
-            at.emplace_back(i, size);
+            if (last[i] >= 0) next[last[i]] = (int)next.size();
+            last[i] = (int)next.size();
+            next.push_back(-1);
+            offsets.push_back(size);
             size += tokens * d.m;
         }
-        bufs.push_back(empty({size}, x[0]));
         sizes.push_back(size);
-        for (const auto& [i, offset] : at) {
-            y.push_back((char*)bufs[t].mutable_data_ptr() + offset * x[0].element_size());
-            if (t == 0) firsts[i] = bufs[0].as_strided({tokens, rows[i]}, {rows[i], 1}, offset);
-        }
     }
-    if (tokens > 0) launch_group_terms(checked, y, dt, panel_mode, panel_ws);
-    for (size_t t = 1; t < depth; ++t) (sizes[t] == sizes[0] ? bufs[0] : bufs[0].narrow(0, 0, sizes[t])).add_(bufs[t]);
+    Tensor sum = empty({sizes[0]}, x[0]);
+    std::vector<void*> y(checked.size(), nullptr);
+    for (size_t k = 0; k < weights; ++k) {                        // the first terms, in this order
+        y[k] = (char*)sum.mutable_data_ptr() + offsets[k] * x[0].element_size();
+        firsts[order[k]] = sum.as_strided({tokens, rows[order[k]]}, {rows[order[k]], 1}, offsets[k]);
+    }
+    const int count = (int)checked.size();
+    std::vector<nq_gemm_term> arr;
+    if (tokens > 0 && panel_mode == NQ_PANEL_AUTO && count <= nq_gemm_group_max()) arr = terms_of(checked, y);
+    if (!arr.empty() && nq_gemm_sum_pays(arr.data(), next.data(), count, (int)tokens)) {
+        const MaybeTensor ws = panel_workspace(arr.data(), count, tokens, panel_mode, panel_ws);
+        check_status(nq_gemm_nanoquant_sum(arr.data(), next.data(), count, (int)tokens, dt, ws ? ws->mutable_data_ptr() : nullptr,
+                                           ws ? (size_t)ws->nbytes() : 0, panel_mode, stream_of(x[0])));
+    } else if (tokens > 0) {
+        std::vector<Tensor> more;
+        for (size_t t = 1, k = weights; t < depth; ++t) {
+            more.push_back(empty({sizes[t]}, x[0]));
+            for (size_t i = 0; i < weights && groups[order[i]].size() > t; ++i, ++k)
+                y[k] = (char*)more.back().mutable_data_ptr() + offsets[k] * x[0].element_size();
+        }
+        launch_group_terms(checked, y, dt, panel_mode, panel_ws);
+        for (size_t t = 1; t < depth; ++t) (sizes[t] == sizes[0] ? sum : sum.narrow(0, 0, sizes[t])).add_(more[t - 1]);
+    }
     for (const Tensor& first : firsts) result.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(first)));
     return result;
 }

@@ -396,9 +396,9 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
 def gemm_group_sum_forward(xs, term_groups, bias_groups=None, panel="auto"):
     """`[sum_t marlin_nanoquant_forward(x_i, *term_groups[i][t]) for i]`: weights that are sums of several binary
     low-rank terms (mixture of ranks) on the grouped prefill launches.  All terms of all weights share the two
-    launches of `gemm_group_forward`; the t-th terms of all weights write into one flat buffer per t, weights with
-    more terms first, so that the sums over the terms are one in-place add per extra term index instead of one
-    per weight.  `xs`: one tensor or one per weight; `bias_groups`: optional list (per weight) of lists (per term) of
+    launches of `gemm_group_forward`.  Up to 16 terms, with "auto", the second one adds the terms up in 32 bits; otherwise the
+    t-th terms of all weights write into one flat buffer per t and one in-place add per extra term index adds them.
+    `xs`: one tensor or one per weight; `bias_groups`: optional list (per weight) of lists (per term) of
     bias tensors / None; `panel` as in `gemm_group_forward`.  Returns one [tokens, m] tensor per weight (views of one
     buffer)."""
     if isinstance(xs, torch.Tensor):

@@ -65,3 +65,41 @@ def test_other_tiles_for_many_rows_below_160_tokens(dev, tokens):
     for a, s, y, ref in zip(alone, same, free, refs):
         assert torch.equal(a, s)
         assert oracle.max_rel_err(y.float().cpu().numpy(), ref) < 3 * ROUND[dtype]
+
+
+# Sums of terms: chains of 1 to 3 terms of uneven rank, ranks of one tile up to many, a bias on some terms; the sizes reach every
+# tile that sums (32 x 32, 32 x 64 and 32 x 96 with k split, 64 x 128, 64 x 256) with tokens and rows left over.
+@pytest.mark.parametrize("tokens,spec", [
+    (1, [(32, (200, 100)), (96, (512,))]),
+    (33, [(160, (256, 1280, 300)), (64, (100,)), (3104, (700, 256))]),
+    (200, [(3104, (512, 2304)), (2080, (256,))]),
+    (333, [(3104, (256, 256, 768)), (1056, (2048, 100))]),
+    (700, [(4128, (300, 100)), (2080, (256,))]),
+    (1000, [(8224, (256, 256))]),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_sums_of_terms(dev, tokens, spec, dtype):
+    f = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    host = lambda a: a.float().cpu().numpy()
+    n = 512
+    x = f(oracle.synth_x(tokens, n, tokens)).to(dtype)
+    groups, biases, refs = [], [], []
+    for w, (m, ranks) in enumerate(spec):
+        packed, own, ref = [], [], 0.0
+        for t, rank in enumerate(ranks):
+            vt, u, *scales = oracle.synth_term(m, n, rank, 31 * tokens + 5 * w + t)
+            sc = [f(s).to(dtype) for s in scales]
+            bias = torch.linspace(-1, 1, m, device=dev).to(dtype) if (w + t) % 2 else None
+            packed.append(packing.marlin_nanoquant_packer(f(vt).T.contiguous(), f(u).T.contiguous(), *sc))
+            own.append(bias)
+            ref = ref + oracle.layer_forward(host(x), vt, u, *(host(s) for s in sc)) + (0.0 if bias is None else host(bias))
+        groups.append(packed)
+        biases.append(own)
+        refs.append(ref)
+    print(f"sums {tokens} tokens {spec} {dtype}", flush=True)
+    added, apart = ops.gemm_group_sum_forward(x, groups, biases), ops.gemm_group_sum_forward(x, groups, biases, panel="never")
+    torch.cuda.synchronize()
+    for y, z, ref in zip(added, apart, refs):
+        err, err_apart = oracle.max_rel_err(host(y), ref), oracle.max_rel_err(host(z), ref)
+        assert err < 3 * ROUND[dtype], err                   # h and the result are rounded, the sum is not
+        assert err_apart < 5 * ROUND[dtype], err_apart       # and here every term's result and two additions

@@ -76,3 +76,19 @@ def test_no_panel_without_need():
     arr = (ops.NqGemmTerm * 1)(ops.NqGemmTerm(*[None] * 9, 512, 256, 128))
     assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 2) == 0 and lib.nq_gemm_group_wants_panel(arr, 1, 0, 1) == 0
     assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 1) == 1
+
+
+def test_chains_of_terms_that_are_none():
+    import ctypes
+    term = lambda h, y, m=64, s_in=None: ops.NqGemmTerm(4096, 4096, 4096, s_in, None, None, None, h, y, 256, 256, m)
+    call = lambda terms, nxt: _lib.lib().nq_gemm_nanoquant_sum((ops.NqGemmTerm * len(terms))(*terms), (ctypes.c_int * len(nxt))(*nxt), len(terms), 5, 0,
+                                                               None, 0, 0, None)
+    null, shape = -2, -3                                                                   # NQ_ERR_NULL, NQ_ERR_SHAPE
+    for terms, nxt in [([term(16, 32), term(48, None)], [0, -1]),                          # a term behind itself
+                       ([term(16, 32), term(48, None)], [2, -1]),                          # past the end
+                       ([term(16, 32), term(48, None, m=96)], [1, -1]),                    # other rows
+                       ([term(16, 32), term(48, 64), term(80, None)], [2, 2, -1]),         # one term in two chains
+                       ([term(16, 32), term(48, 32)], [-1, -1]),                           # one output twice
+                       ([term(16, 32), term(48, None, s_in=4096)], [1, -1])]:              # two kernels
+        assert call(terms, nxt) == shape, nxt
+    assert call([term(16, 32), term(48, None)], [-1, -1]) == null               # a first term without y
