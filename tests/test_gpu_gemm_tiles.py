@@ -34,6 +34,7 @@ def _onebit(dev, tokens, k, rows, dtype, scaled, seed):
     (333, 1024, 3168), (700, 256, 2080), (193, 2560, 8224),                    # 64 x 128
     (400, 768, 16416), (1000, 1280, 4128),                                     # 64 x 256
     (2049, 512, 12320), (4097, 256, 8224),                                     # 128 x 256
+    (352, 1024, 3168), (353, 1024, 3168), (2112, 512, 12320), (2113, 512, 12320),   # half a tile of tokens left, one more
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("scaled", [True, False])
@@ -76,6 +77,7 @@ def test_other_tiles_for_many_rows_below_160_tokens(dev, tokens):
     (333, [(3104, (256, 256, 768)), (1056, (2048, 100))]),
     (700, [(4128, (300, 100)), (2080, (256,))]),
     (1000, [(8224, (256, 256))]),
+    (992, [(8224, (256, 256))]), (993, [(8224, (256, 256))]),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_sums_of_terms(dev, tokens, spec, dtype):
