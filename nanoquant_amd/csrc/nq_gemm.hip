@@ -148,12 +148,21 @@ static double tile_time(const TileVariant& v, const GemmShapes& s) {
     }
     int fit = 0;
     while (fit < 4 && c.tile[fit] > 0.f) ++fit;
-    const long per_cu = (long)std::ceil(blocks / 256.0), full = per_cu / fit, rest = per_cu % fit;
     const double mean = work / blocks;
-    const double rounds = (double)full + (rest ? 1 : 0);
-    const double walk = mean * ((double)full * c.tile[fit - 1] + (rest ? c.tile[rest - 1] : 0.f));
-    const double alone = (double)longest * c.tile[0];        // the longest problem's workgroups start first
-    return c.start + c.round * rounds + (walk > alone ? walk : alone);
+    auto walk = [&](double workgroups, double* rounds) {
+        const long per_cu = (long)std::ceil(workgroups / 256.0), full = per_cu / fit, rest = per_cu % fit;
+        *rounds = (double)full + (rest ? 1 : 0);
+        const double all = mean * ((double)full * c.tile[fit - 1] + (rest ? c.tile[rest - 1] : 0.f));
+        // The longest problem's workgroups start first and share their compute units with those of mean length (4096 and 11008 ->
+        // 3072 rows on 768 tokens: 164, not 116, on 128 x 256; panels 128).
+        const long beside = per_cu < fit ? per_cu : fit;
+        const double one = mean * c.tile[beside - 1] + ((double)longest - mean) * c.tile[0];
+        return all > one ? all : one;
+    };
+    double rounds, real_rounds;
+    const double time = walk(blocks, &rounds), real = walk(blocks / whole, &real_rounds);
+    // half the way to what as many whole workgroups would take: the cut ones still share compute units
+    return c.start + c.round * 0.5 * (rounds + real_rounds) + 0.5 * (time + real);
 }
 
 static int best_tile(const GemmShapes& s, int begin, int end, double* time) {
