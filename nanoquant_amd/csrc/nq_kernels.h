@@ -104,7 +104,7 @@ double gemm_sums_time(int count, const int* next, int T, const int* K, const int
 // Estimated time of gemm_onebit_group with kGemmAnyTile, in us.
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 
-// nq_panel.hip: the same GEMMs at about 128 to 768 tokens as one persistent launch over 64-token x 256-row panels
+// nq_panel.hip: the same GEMMs up to 2048 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
 size_t panel_workspace_bytes();
 double panel_time(int count, int T, const int* K, const int* R, bool scaled);      // estimate in us; 1e30: not as panels

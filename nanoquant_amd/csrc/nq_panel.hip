@@ -9,7 +9,7 @@
 //
 //  * A workgroup (4 wavefronts, two workgroups per compute unit) works on a PANEL of 64 tokens x 256 rows.  The
 //    activation slab [64 tokens][256 k] is staged once in LDS for all four wavefronts (32 KiB of L2 traffic per
-//    8.4 MFLOP; the few-token tiles of nq_gemm.hip stage 16 KiB per 2.1 MFLOP).  Two slabs in LDS: one barrier per
+//    8.4 MFLOP; the few-token tiles of nq_gemm.hip stage 16 KiB per 0.5 to 1.6 MFLOP).  Two slabs in LDS: one barrier per
 //    k step.  Two workgroups share a compute unit so that one has MFMAs to issue while the other hands over a
 //    partial tile or stores a panel, and so that token counts are covered in blocks of 64.
 //  * A wavefront holds 64 tokens x 64 rows (four 32x32 accumulators): every sign fragment decoded in registers
@@ -573,8 +573,12 @@ double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
     return 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
 }
 
+// Problems of different k are the estimate's weak side (the seven first GEMMs of a Llama-2-7B layer, k 4096 and 11008, on 1024 tokens:
+// panels 165, tiles 175 by estimate, the layer 409 with panels and 371 without; on 768, estimates 128 / 139, 279 and 297).
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
-    return panel_time(count, T, K, R, scaled) < 0.95 * gemm_tiles_time(count, x, T, K, R, scaled);
+    bool mixed = false;
+    for (int p = 1; p < count; ++p) mixed = mixed || K[p] != K[0];
+    return panel_time(count, T, K, R, scaled) < (mixed ? 0.93 : 0.95) * gemm_tiles_time(count, x, T, K, R, scaled);
 }
 
 template <int DT, bool SCALED>
