@@ -30,10 +30,9 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch of the headline kernel, measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE scaled by a
 # copy kernel of known size (profiles/gemv_stream_llama2_7b_stack_b1.md); valid for the default workload only.
 MEASURED_TRAFFIC_BYTES = 843630592
-# The same for the two launches of the 128-token grouped layer (profiles/gemm_group_llama2_7b_layer_prefill.md):
-# (18756 + 26222) KiB x 2.000 fetched + (4352 + 48686) KiB written; 38.9 MB each way of the second launch are partial
-# tiles that its workgroups hand over through device-coherent memory.
-MEASURED_PREFILL_TRAFFIC_BYTES = (18756 + 26222) * 2 * 1024 + (4352 + 48686) * 1024
+# The same for the two launches of the 128-token grouped layer (profiles/gemm_tile_llama2_7b_layer_prefill.md):
+# (17437 + 20889) KiB x 2.000 fetched + (4352 + 10624) KiB written.
+MEASURED_PREFILL_TRAFFIC_BYTES = (17437 + 20889) * 2 * 1024 + (4352 + 10624) * 1024
 MFMA_F16_PEAK_TFLOPS = 2500.0
 
 LLAMA2_7B_LAYER = (("q", 4096, 4096), ("k", 4096, 4096), ("v", 4096, 4096), ("o", 4096, 4096),
@@ -630,8 +629,8 @@ def main():
                 # the second headline metric (128-token GEMM TFLOP/s) as a roofline object of its own
                 result["roofline_prefill"] = {
                     "bound": "mfma", "tokens": 128,
-                    "kernel": "first GEMMs of the 7 linears: gemm_kwave_group_kernel<fp16> (few-token tiles); second GEMMs: "
-                              "gemm_panel_kernel<fp16> (persistent 64-token x 256-row panels, two workgroups per CU); one launch each",
+                    "kernel": "gemm_tile_kernel<fp16>, one launch each: first GEMMs of the 7 linears on 32-token x 96-row tiles "
+                              "(k split between four wavefronts), second GEMMs on 128 x 256 tiles",
                     "achieved": round(tf, 2), "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": round(tf / MFMA_F16_PEAK_TFLOPS, 4), "flops_per_layer": int(group_flops),
                     "us_per_layer": round(us, 2), "traffic": MEASURED_PREFILL_TRAFFIC_BYTES}

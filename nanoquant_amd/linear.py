@@ -46,7 +46,7 @@ class NanoQuantLinear(nn.Module):
         # True: a decode call of 1, 2, 4, 8 or 16 rows is ONE launch of the run-list kernel (both stages, the
         # scales and the bias) on a list built once per row count, instead of the two launches of the
         # reference's op (linear.py:121-130).  The two launches are the faster form (seven linears of a Llama-2-7B layer at
-        # 1 / 4 / 16 rows: 69 / 74 / 94 us against 108 / 150 / 221); the switch serves callers that are charged per launch.
+        # 1 / 4 / 16 rows: 55 / 62 / 83 us against 108 / 150 / 221); the switch serves callers that are charged per launch.
         # It bypasses the torch op, so leave it off under torch.compile.
         self.fused_launch = False
         # With fused_launch: every so many launches of a list the status word is read back (one synchronisation) and an
@@ -54,8 +54,8 @@ class NanoQuantLinear(nn.Module):
         self.fused_status_every = 256
         # Opt-in (0: never): a module prepared for decode ("gemv") sends calls of at least this many rows to the
         # few-token MFMA tiles of the prefill path.  17 is the break-even: the decode kernels run 16 rows at a time (the
-        # seven linears of a Llama-2-7B layer, one call each, us on 1 / 4 / 16 / 17 / 32 / 64 rows: decode 69 / 74 / 94 / 157 /
-        # 179 / 349, tiles 108 / 109 / 112 / 113 / 116 / 121).  The price is a second copy of the packed
+        # seven linears of a Llama-2-7B layer, one call each, us on 1 / 4 / 16 rows: 55 / 62 / 83, and more than 130 on 17 and more,
+        # where the tiles take 89 on 32).  The price is a second copy of the packed
         # factors (the prefill tiles, built once from the decode words on the device, on the first such call or by
         # `prepare_mfma_route()`, and kept beside them), and results that differ in the last bits from the decode
         # kernels' (other order of the fp32 additions, h rounded to 16 bits in between).  Needs
