@@ -3,7 +3,8 @@
 // A decode call of a small linear takes 7 us on the GPU and a prefill group of a decoder layer 100; checked, allocated
 // and launched from Python they took 20 us and 28 us per group of the host.  This file registers the device implementations
 // of torch.ops.binary_kernels.* (schemas and shape-only implementations are in ops.py) and is the extension module
-// nanoquant_amd._host for the calls beyond the operators.  It holds no state.
+// nanoquant_amd._host for the calls beyond the operators.  It holds no state, and allocates and launches without the interpreter
+// lock: a launch waits while the stream's queue is full, maybe for a host function that needs the lock.
 //
 // Checks and messages are those of the reference's host wrappers:
 //   nanoquant_dyn_forward     src/nanoquant/kernel/cuda/gemv_kernel.cu:308-346, cuda/meta_utils.h:14-38
@@ -288,13 +289,14 @@ std::vector<nq_gemm_term> terms_of(const std::vector<GroupTerm>& terms, const st
     return arr;
 }
 
-// The workspace of the panel launches, panel_ws(), asked for only where a stage takes one.
+// The workspace of the panel launches, panel_ws(), asked for only where a stage takes one.  Without the interpreter lock.
 MaybeTensor panel_workspace(const nq_gemm_term* terms, int count, int64_t tokens, int panel_mode, const py::object& panel_ws) {
     if (panel_mode == NQ_PANEL_NEVER || !nq_gemm_group_wants_panel(terms, count, (int)tokens, panel_mode)) return std::nullopt;
+    const py::gil_scoped_acquire lock;
     return tensor_of(panel_ws().ptr(), "the panel workspace");
 }
 
-// The launches of checked terms; y: one output address per term.
+// The launches of checked terms; y: one output address per term.  Without the interpreter lock.
 void launch_group_terms(const std::vector<GroupTerm>& terms, const std::vector<void*>& y, int dt, int panel_mode, const py::object& panel_ws) {
     const int64_t tokens = terms[0].d.tokens;
     const int most = nq_gemm_group_max();
@@ -325,27 +327,32 @@ py::list gemm_group(const py::sequence& xs, const py::sequence& terms, const py:
     const int dt = gemm_dtype(x[0]);
     const c10::DeviceGuard guard(x[0].device());
     std::vector<GroupTerm> checked;
-    std::vector<void*> y;
+    std::vector<Tensor> out(count);
     checked.reserve(count);
     for (size_t i = 0; i < count; ++i) {
         const py::object term = terms[i], bias = biases.is_none() ? py::object(py::none()) : py::object(py::sequence(biases)[i]);
         checked.push_back(group_term(x[i], x[0], term.ptr(), bias.ptr()));
         const GemmDims& d = checked.back().d;
-        Tensor out;
-        if (outs.is_none()) {
-            out = empty({d.tokens, d.m}, x[0]);
-        } else {
-            out = tensor_of(py::object(py::sequence(outs)[i]).ptr(), "out");
-            TORCH_CHECK(out.dim() == 2 && out.size(0) == d.tokens && out.size(1) == d.m && out.scalar_type() == x[0].scalar_type() &&
-                            out.device() == x[0].device() && out.is_contiguous() && (uintptr_t)out.const_data_ptr() % 16 == 0,
+        if (!outs.is_none()) {
+            out[i] = tensor_of(py::object(py::sequence(outs)[i]).ptr(), "out");
+            TORCH_CHECK(out[i].dim() == 2 && out[i].size(0) == d.tokens && out[i].size(1) == d.m && out[i].scalar_type() == x[0].scalar_type() &&
+                            out[i].device() == x[0].device() && out[i].is_contiguous() && (uintptr_t)out[i].const_data_ptr() % 16 == 0,
                         "outs[", i, "] must be a contiguous, 16-byte aligned [", d.tokens, ", ", d.m, "] tensor of ",
                         dt == NQ_F16 ? "torch.float16" : "torch.bfloat16", " on ", x[0].device().str());
         }
-        checked.back().h = empty({d.tokens, d.r}, x[0]);
-        y.push_back(out.mutable_data_ptr());
-        result.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(out)));
     }
-    if (checked[0].d.tokens > 0) launch_group_terms(checked, y, dt, panel_mode, panel_ws);
+    {
+        const py::gil_scoped_release unlocked;
+        std::vector<void*> y;
+        for (size_t i = 0; i < count; ++i) {
+            const GemmDims& d = checked[i].d;
+            if (outs.is_none()) out[i] = empty({d.tokens, d.m}, x[0]);
+            checked[i].h = empty({d.tokens, d.r}, x[0]);
+            y.push_back(out[i].mutable_data_ptr());
+        }
+        if (checked[0].d.tokens > 0) launch_group_terms(checked, y, dt, panel_mode, panel_ws);
+    }
+    for (const Tensor& t : out) result.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(t)));
     return result;
 }
 
@@ -359,9 +366,11 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
     if (weights == 0) return result;
     bool filled = xs.size() == weights;
     std::vector<py::sequence> groups;
+    std::vector<size_t> terms_of_weight;
     for (size_t i = 0; i < weights; ++i) {
         groups.push_back(py::sequence(term_groups[i]));
-        filled = filled && groups.back().size() > 0;
+        terms_of_weight.push_back(groups.back().size());
+        filled = filled && terms_of_weight.back() > 0;
     }
     TORCH_CHECK(filled, "one x and at least one term per weight");
     const std::vector<Tensor> x = tensors_of(xs, "x");
@@ -370,8 +379,8 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
     const int64_t tokens = x[0].size(0);
     std::vector<size_t> order(weights);
     std::iota(order.begin(), order.end(), (size_t)0);
-    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return groups[a].size() > groups[b].size(); });
-    const size_t depth = groups[order[0]].size();
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return terms_of_weight[a] > terms_of_weight[b]; });
+    const size_t depth = terms_of_weight[order[0]];
     std::vector<GroupTerm> checked;
     std::vector<Tensor> firsts(weights);
     std::vector<int64_t> rows(weights), offsets, sizes;           // per weight; per checked term; per term index
@@ -379,7 +388,7 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
     for (size_t t = 0; t < depth; ++t) {
         int64_t size = 0;
         for (size_t i : order) {
-            if (groups[i].size() <= t) break;
+            if (terms_of_weight[i] <= t) break;
             const py::object term = groups[i][t];
             py::object bias = py::none();
             if (!bias_groups.is_none()) {
@@ -390,7 +399,6 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
             const GemmDims& d = checked.back().d;
             if (t == 0) rows[i] = d.m;
             TORCH_CHECK(rows[i] == d.m, "all terms of a weight must have the same output size");
-            checked.back().h = empty({d.tokens, d.r}, x[0]);
             TORCH_CHECK(size * x[0].element_size() % 16 == 0, "tokens * out_features must keep the outputs 16-byte aligned");
             if (last[i] >= 0) next[last[i]] = (int)next.size();
             last[i] = (int)next.size();
@@ -400,28 +408,32 @@ py::list gemm_group_sum(const py::sequence& xs, const py::sequence& term_groups,
         }
         sizes.push_back(size);
     }
-    Tensor sum = empty({sizes[0]}, x[0]);
-    std::vector<void*> y(checked.size(), nullptr);
-    for (size_t k = 0; k < weights; ++k) {                        // the first terms, in this order
-        y[k] = (char*)sum.mutable_data_ptr() + offsets[k] * x[0].element_size();
-        firsts[order[k]] = sum.as_strided({tokens, rows[order[k]]}, {rows[order[k]], 1}, offsets[k]);
-    }
-    const int count = (int)checked.size();
-    std::vector<nq_gemm_term> arr;
-    if (tokens > 0 && panel_mode == NQ_PANEL_AUTO && count <= nq_gemm_group_max()) arr = terms_of(checked, y);
-    if (!arr.empty() && nq_gemm_sum_pays(arr.data(), next.data(), count, (int)tokens)) {
-        const MaybeTensor ws = panel_workspace(arr.data(), count, tokens, panel_mode, panel_ws);
-        check_status(nq_gemm_nanoquant_sum(arr.data(), next.data(), count, (int)tokens, dt, ws ? ws->mutable_data_ptr() : nullptr,
-                                           ws ? (size_t)ws->nbytes() : 0, panel_mode, stream_of(x[0])));
-    } else if (tokens > 0) {
-        std::vector<Tensor> more;
-        for (size_t t = 1, k = weights; t < depth; ++t) {
-            more.push_back(empty({sizes[t]}, x[0]));
-            for (size_t i = 0; i < weights && groups[order[i]].size() > t; ++i, ++k)
-                y[k] = (char*)more.back().mutable_data_ptr() + offsets[k] * x[0].element_size();
+    {
+        const py::gil_scoped_release unlocked;
+        for (GroupTerm& t : checked) t.h = empty({t.d.tokens, t.d.r}, x[0]);
+        Tensor sum = empty({sizes[0]}, x[0]);
+        std::vector<void*> y(checked.size(), nullptr);
+        for (size_t k = 0; k < weights; ++k) {                        // the first terms, in this order
+            y[k] = (char*)sum.mutable_data_ptr() + offsets[k] * x[0].element_size();
+            firsts[order[k]] = sum.as_strided({tokens, rows[order[k]]}, {rows[order[k]], 1}, offsets[k]);
         }
-        launch_group_terms(checked, y, dt, panel_mode, panel_ws);
-        for (size_t t = 1; t < depth; ++t) (sizes[t] == sizes[0] ? sum : sum.narrow(0, 0, sizes[t])).add_(more[t - 1]);
+        const int count = (int)checked.size();
+        std::vector<nq_gemm_term> arr;
+        if (tokens > 0 && panel_mode == NQ_PANEL_AUTO && count <= nq_gemm_group_max()) arr = terms_of(checked, y);
+        if (!arr.empty() && nq_gemm_sum_pays(arr.data(), next.data(), count, (int)tokens)) {
+            const MaybeTensor ws = panel_workspace(arr.data(), count, tokens, panel_mode, panel_ws);
+            check_status(nq_gemm_nanoquant_sum(arr.data(), next.data(), count, (int)tokens, dt, ws ? ws->mutable_data_ptr() : nullptr,
+                                               ws ? (size_t)ws->nbytes() : 0, panel_mode, stream_of(x[0])));
+        } else if (tokens > 0) {
+            std::vector<Tensor> more;
+            for (size_t t = 1, k = weights; t < depth; ++t) {
+                more.push_back(empty({sizes[t]}, x[0]));
+                for (size_t i = 0; i < weights && terms_of_weight[order[i]] > t; ++i, ++k)
+                    y[k] = (char*)more.back().mutable_data_ptr() + offsets[k] * x[0].element_size();
+            }
+            launch_group_terms(checked, y, dt, panel_mode, panel_ws);
+            for (size_t t = 1; t < depth; ++t) (sizes[t] == sizes[0] ? sum : sum.narrow(0, 0, sizes[t])).add_(more[t - 1]);
+        }
     }
     for (const Tensor& first : firsts) result.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(first)));
     return result;
@@ -436,9 +448,10 @@ TORCH_LIBRARY_IMPL(binary_kernels, CUDA, m) {
 }
 
 PYBIND11_MODULE(_host, m) {
-    m.def("nanoquant_dyn_forward", &nanoquant_dyn_forward);
-    m.def("gemv_bias", &gemv_bias);
-    m.def("gemm_bias", &gemm_bias);
+    using Unlocked = py::call_guard<py::gil_scoped_release>;
+    m.def("nanoquant_dyn_forward", &nanoquant_dyn_forward, Unlocked());
+    m.def("gemv_bias", &gemv_bias, Unlocked());
+    m.def("gemm_bias", &gemm_bias, Unlocked());
     m.def("gemm_group", &gemm_group);
     m.def("gemm_group_sum", &gemm_group_sum);
     m.def("check_hint", &check_hint_by_name);
