@@ -289,11 +289,12 @@ std::vector<nq_gemm_term> terms_of(const std::vector<GroupTerm>& terms, const st
     return arr;
 }
 
-// The workspace of the panel launches, panel_ws(), asked for only where a stage takes one.  Without the interpreter lock.
+// The workspace of the panel launches, panel_ws() (None: there is none now), asked for only where a stage takes one.  Without the
+// interpreter lock.
 MaybeTensor panel_workspace(const nq_gemm_term* terms, int count, int64_t tokens, int panel_mode, const py::object& panel_ws) {
     if (panel_mode == NQ_PANEL_NEVER || !nq_gemm_group_wants_panel(terms, count, (int)tokens, panel_mode)) return std::nullopt;
     const py::gil_scoped_acquire lock;
-    return tensor_of(panel_ws().ptr(), "the panel workspace");
+    return maybe_tensor_of(panel_ws().ptr(), "the panel workspace");
 }
 
 // The launches of checked terms; y: one output address per term.  Without the interpreter lock.

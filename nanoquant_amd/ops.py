@@ -185,6 +185,8 @@ def _onebit_check(A, B, s_in, s_out, workspace):
 
 # Workspace of the panel launches (partial tiles, hand-over flags, the count of finished workgroups): zero when
 # first used, then owned by the launches; one per (device, stream) so that launches sharing it are stream-ordered.
+# None is made while a graph is captured: it would be zero only once the graph has run, and calls outside the graph would find
+# it before.  The call then runs on tiles.
 _panel_ws_cache = {}
 PANEL_MODES = {"auto": 0, "always": 1, "never": 2}
 
@@ -193,6 +195,8 @@ def _panel_workspace(device):
     key = (device.index, torch.cuda.current_stream(device).cuda_stream)
     buf = _panel_ws_cache.get(key)
     if buf is None:
+        if torch.cuda.is_current_stream_capturing():
+            return None
         with torch.cuda.device(device):
             nbytes = int(_lib.lib().nq_gemm_panel_workspace_bytes())
         if nbytes == 0:
@@ -385,7 +389,7 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     `biases` an optional list of [m] tensors / None; `outs` an optional list of contiguous [tokens, m] tensors of
     the activation type to write into (allocated here when absent); `panel` ("auto", "always", "never") says whether
     the stages may run as persistent panel launches and, up to 160 tokens, on tiles other than the ones a linear gets by
-    itself (see include/nq_gfx950.h).  Returns the list of outputs.  The terms share launches: a single linear leaves most
+    itself (see include/nq_gfx950.h); in a graph capture they do only if a call on that stream did before.  Returns the list of outputs.  The terms share launches: a single linear leaves most
     of the device idle up to some hundred tokens.  The reference launches every linear by itself
     (modules/linear.py:131-133)."""
     if isinstance(xs, torch.Tensor):

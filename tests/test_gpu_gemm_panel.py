@@ -119,6 +119,41 @@ def test_panel_launches_repeat_and_replay(dev):
     assert ops.panel_status(dev) == 0
 
 
+def test_a_capture_without_a_workspace_leaves_none_behind(dev):
+    # tiles only before the capture, a shape of panels in it, then the same shape outside before the first replay
+    dtype, n, r, m = torch.float16, 11008, 6144, 256
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(3)
+    signs = lambda a, b: torch.randint(0, 2, (a, b), dtype=torch.int8, device=dev, generator=gen) * 2 - 1
+    scale = lambda k: (torch.rand(k, device=dev, generator=gen) + 0.01).to(dtype)
+    packed = packing.marlin_nanoquant_packer(signs(n, r), signs(r, m), scale(n), scale(r), scale(m))
+    x = (torch.randn(700, n, device=dev, generator=gen) * 0.01).to(dtype)
+    arr = (ops.NqGemmTerm * 1)(ops.NqGemmTerm(*[None] * 9, n, r, m))
+    assert _lib.lib().nq_gemm_group_wants_panel(arr, 1, 700, 0) == 1 and _lib.lib().nq_gemm_group_wants_panel(arr, 1, 32, 0) == 0
+    want = ops.gemm_group_forward(x, [packed], panel="never")[0]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    print("capture without a workspace", flush=True)
+    with torch.cuda.stream(side):
+        ops.gemm_group_forward(x[:32], [packed])
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured = ops.gemm_group_forward(x, [packed])[0]
+        assert (dev.index, side.cuda_stream) not in ops._panel_ws_cache
+        eager = ops.gemm_group_forward(x, [packed])[0]
+        side.synchronize()
+        assert ops.panel_status(dev) == 0
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            again = ops.gemm_group_forward(x, [packed])[0]
+            side.synchronize()
+            assert torch.equal(captured, want) and torch.equal(again, eager)
+        assert ops.panel_status(dev) == 0
+    assert torch.allclose(eager.float(), want.float(), rtol=2e-2, atol=2e-3 * float(want.float().abs().max()))
+
+
 def test_an_expired_wait_of_a_panel_launch_is_reported(dev):
     """The workgroups that finish a shared panel wait a bounded number of polls for the others' partial tiles.  With
     the bound lowered to one poll from the host, a launch whose panels are shared by many workgroups reports an expiry,

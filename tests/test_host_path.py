@@ -92,3 +92,23 @@ def test_chains_of_terms_that_are_none():
                        ([term(16, 32), term(48, None, s_in=4096)], [1, -1])]:              # two kernels
         assert call(terms, nxt) == shape, nxt
     assert call([term(16, 32), term(48, None)], [-1, -1]) == null               # a first term without y
+
+
+def test_no_workspace_is_made_while_a_graph_is_captured(monkeypatch):
+    # it would hold whatever was there until the graph runs, and calls outside the graph would use it
+    import contextlib
+    import types
+    made, capturing = [], [True]
+    monkeypatch.setattr(ops, "_panel_ws_cache", {})
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(_lib, "lib", lambda: types.SimpleNamespace(nq_gemm_panel_workspace_bytes=lambda: 256))
+    monkeypatch.setattr(torch, "zeros", lambda n, **kw: made.append(n) or torch.empty(n))
+    device = torch.device("cuda", 0)
+    assert ops._panel_workspace(device) is None and not made and not ops._panel_ws_cache
+    capturing[0] = False
+    buf = ops._panel_workspace(device)
+    assert made == [256]
+    capturing[0] = True
+    assert ops._panel_workspace(device) is buf and made == [256]
