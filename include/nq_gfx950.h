@@ -273,8 +273,9 @@ int nq_gemm_nanoquant_group(const nq_gemm_term* terms, int count, int tokens, in
  *   workgroups from which every launch derives its own flag value, so nothing is cleared between launches or graph
  *   replays).  It must not be `scratch` and launches that share it must not overlap in time.
  *   panel_mode: NQ_PANEL_AUTO picks per stage whatever is fastest (panels, or the tiles of nq_gemm_nanoquant_group, of which
- *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count, NQ_PANEL_NEVER never
- *   takes it; with panel_ws NULL there is none in any mode.
+ *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count (not where
+ *   x, y or the signs of a term are 4 GiB or more, which its 32-bit offsets do not reach), NQ_PANEL_NEVER never takes it; with
+ *   panel_ws NULL there is none in any mode.
  * A panel launch keeps two workgroups per compute unit resident and its workgroups wait for each other's partial
  * tiles: it may share the GPU with other kernels (its waits then last until those free their compute units), but a
  * wait that outlasts its bound (2^20 polls, about a second) invalidates the launch's outputs.

@@ -814,8 +814,9 @@ GroupStage second_stage(const nq_gemm_term* terms, int count) {
     }
     return s;
 }
-bool panel_for(const GroupStage& s, int count, int tokens) {
-    return nq::panel_applies(count, s.x, tokens, s.K, s.R, s.si[0] != nullptr);
+bool panel_for(const GroupStage& s, int count, int tokens, int mode) {
+    if (mode == NQ_PANEL_ALWAYS) return nq::panel_addresses(count, tokens, s.K, s.R);
+    return mode == NQ_PANEL_AUTO && nq::panel_applies(count, s.x, tokens, s.K, s.R, s.si[0] != nullptr);
 }
 struct PanelUse {
     void* ws;                                    // null: no panel launches
@@ -823,7 +824,7 @@ struct PanelUse {
 };
 // The panel launch where a workspace was given and the shapes make it the faster one.
 hipError_t run_stage(const GroupStage& s, int count, int tokens, int dtype, const PanelUse& panel, hipStream_t stream) {
-    if (panel.ws && (panel.mode == NQ_PANEL_ALWAYS || panel_for(s, count, tokens)))
+    if (panel.ws && panel_for(s, count, tokens, panel.mode))
         return nq::gemm_panel_group(dtype, count, s.x, s.w, s.si, s.so, s.bs, s.out, tokens, s.K, s.R, panel.ws,
                                     g_panel_spin_limit.load(), stream);
     return nq::gemm_onebit_group(dtype, count, s.x, s.w, s.si, s.so, s.bs, s.out, tokens, s.K, s.R,
@@ -863,8 +864,7 @@ bool known_panel_mode(int mode) { return mode == NQ_PANEL_AUTO || mode == NQ_PAN
 
 int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode) {
     if (!terms || count < 1 || count > nq::gemm_group_max() || count > kMaxTerms || tokens < 1 || panel_mode == NQ_PANEL_NEVER) return 0;
-    if (panel_mode == NQ_PANEL_ALWAYS) return 1;
-    return panel_for(first_stage(terms, count), count, tokens) || panel_for(second_stage(terms, count), count, tokens);
+    return panel_for(first_stage(terms, count), count, tokens, panel_mode) || panel_for(second_stage(terms, count), count, tokens, panel_mode);
 }
 
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,

@@ -108,6 +108,7 @@ double gemm_tiles_time(int count, const void* const* x, int T, const int* K, con
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
 size_t panel_workspace_bytes();
 double panel_time(int count, int T, const int* K, const int* R, bool scaled);      // estimate in us; 1e30: not as panels
+bool panel_addresses(int count, int T, const int* K, const int* R);                // small enough for the kernel
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 hipError_t gemm_panel_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                             const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,

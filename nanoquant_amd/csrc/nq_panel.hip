@@ -548,6 +548,16 @@ size_t panel_workspace_bytes() {
     return kPanelHeadBytes + flags + (size_t)2 * G * kPanelSlotFloats * sizeof(float);
 }
 
+// The kernel addresses whole matrices by 32-bit byte offsets; token blocks and panels that reach beyond a matrix count in full.
+bool panel_addresses(int count, int T, const int* K, const int* R) {
+    const unsigned long long most = 1ull << 32, tokens = ((unsigned long long)T + kPanelTok - 1) / kPanelTok * kPanelTok;
+    for (int p = 0; p < count; ++p) {
+        const unsigned long long rows = ((unsigned long long)R[p] + kPanelRows - 1) / kPanelRows * kPanelRows;
+        if (tokens * K[p] * 2 >= most || tokens * R[p] * 2 >= most || rows * K[p] / 8 >= most) return false;
+    }
+    return true;
+}
+
 // Whether one stage of a group is better off as a panel launch than on the tiles of nq_gemm.hip: where tiles leave the last of
 // their rounds nearly empty, which equal shares of k steps do not (11008 -> 6144 rows on 700 tokens: 123 / 95; on 512 tokens
 // 78 / 77; 4096 -> 22016 on 333: 76 / 66).  A panel launch takes, in us, 12.4 + 3.1 per k step of a workgroup (3.3 with s_in)
@@ -558,7 +568,7 @@ double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
     constexpr double kNever = 1e30;
     constexpr int kMostTokens = 2048;            // of the launches that were timed
     const int G = panel_grid();
-    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > kMostTokens) return kNever;
+    if (G <= 0 || count < 1 || count > kPanelMax || T < 1 || T > kMostTokens || !panel_addresses(count, T, K, R)) return kNever;
     const int tblocks = (T + kPanelTok - 1) / kPanelTok;
     long long units = 0;
     int longest = 0;
@@ -606,7 +616,7 @@ hipError_t gemm_panel_group(int dtype, int count, const void* const* x, const ui
                             int T, const int* K, const int* R, void* workspace, unsigned spin_limit, hipStream_t stream) {
     const int G = panel_grid();
     if (G <= 0) return hipErrorInvalidDevice;
-    if (count < 1 || count > kPanelMax || T < 1 || !workspace) return hipErrorInvalidValue;
+    if (count < 1 || count > kPanelMax || T < 1 || !workspace || !panel_addresses(count, T, K, R)) return hipErrorInvalidValue;
     PanelArgs a;
     a.T = T;
     a.tblocks = (T + kPanelTok - 1) / kPanelTok;

@@ -209,3 +209,20 @@ def test_panel_entry_point_argument_checks(dev):
     st = ctypes.c_int(-1)
     assert lib.nq_gemm_panel_status(ws.data_ptr(), ctypes.byref(st), stream) == 0 and st.value == 0
     assert lib.nq_gemm_panel_status(None, ctypes.byref(st), stream) != 0
+
+
+def test_matrices_beyond_32_bit_offsets_run_on_tiles(dev):
+    # 4 GiB of x and of h: a panel's offsets would begin again at the first tokens
+    lib, dtype, tokens, m = _lib.lib(), torch.float16, 2 ** 23 + 40, 32
+    query = lambda t, n, r, mode: lib.nq_gemm_group_wants_panel((ops.NqGemmTerm * 1)(ops.NqGemmTerm(*[None] * 9, n, r, 256)), 1, t, mode)
+    assert query(2048, 2 ** 20, 256, 0) == 0 and query(2048, 2 ** 20 - 256, 256, 0) == 1      # "auto"
+    assert query(tokens, 256, 256, 1) == 0
+    packed, ref = _term(dev, m, 256, 256, 77, dtype)
+    x = torch.empty(tokens, 256, dtype=dtype, device=dev)
+    for part in x.split(2 ** 20):
+        part.normal_()
+    print("4 GiB of activations", flush=True)
+    y = ops.gemm_group_forward(x, [packed], panel="always")[0]
+    torch.cuda.synchronize()
+    for rows in (slice(0, 70), slice(2 ** 22 - 5, 2 ** 22 + 60), slice(tokens - 70, tokens)):
+        assert oracle.max_rel_err(y[rows].float().cpu().numpy(), ref(x[rows].float().cpu().numpy())) < TOL[dtype]

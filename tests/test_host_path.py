@@ -78,6 +78,19 @@ def test_no_panel_without_need():
     assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 1) == 1
 
 
+# tokens, n, r, m; whether a stage can be a panel launch (32-bit offsets into x, h, y and the signs)
+@pytest.mark.parametrize("tokens,n,r,m,fits", [
+    (100000, 28672, 28672, 28672, 0),                        # 5.7 GB of x, h and y
+    (64, 2 ** 25, 256, 32, 1), (64, 2 ** 25, 2 ** 25, 32, 0),     # 4 GiB of x; of h as well
+    (64, 2 ** 25 - 256, 256, 32, 1),
+    (33, 2 ** 25, 2 ** 25, 32, 0),                           # in whole token blocks
+    (1, 2 ** 22, 2 ** 18, 2 ** 18, 0),                       # signs of 128 and 8 GiB
+])
+def test_panels_only_where_their_offsets_reach(tokens, n, r, m, fits):
+    arr = (ops.NqGemmTerm * 1)(ops.NqGemmTerm(*[None] * 9, n, r, m))
+    assert _lib.lib().nq_gemm_group_wants_panel(arr, 1, tokens, 1) == fits
+
+
 def test_chains_of_terms_that_are_none():
     import ctypes
     term = lambda h, y, m=64, s_in=None: ops.NqGemmTerm(4096, 4096, 4096, s_in, None, None, None, h, y, 256, 256, m)
