@@ -286,7 +286,7 @@ enum { NQ_PANEL_AUTO = 0, NQ_PANEL_ALWAYS = 1, NQ_PANEL_NEVER = 2 };
 size_t nq_gemm_panel_workspace_bytes(void);
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                                size_t scratch_bytes, void* panel_ws, size_t panel_ws_bytes, int panel_mode, void* stream);
-/* 1 when a stage of that call would be a panel launch (0 otherwise, and for NQ_PANEL_NEVER), so that a caller can do without the
+/* 1 when a stage of that call would be a panel launch (0 otherwise, for NQ_PANEL_NEVER and for sizes that it refuses), so that a caller can do without the
  * workspace until one is. */
 int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode);
 /* Weights that are sums of terms, without a pass that adds: next[i] is the term behind term i of the same weight (-1: none;

@@ -830,14 +830,19 @@ hipError_t run_stage(const GroupStage& s, int count, int tokens, int dtype, cons
     return nq::gemm_onebit_group(dtype, count, s.x, s.w, s.si, s.so, s.bs, s.out, tokens, s.K, s.R,
                                  panel.mode == NQ_PANEL_AUTO ? nq::kGemmAnyTile : nq::kGemmGroup, stream);
 }
+// What the kernels cover: whole tiles of k and rows.
+int check_sizes(const nq_gemm_term& t) {
+    if (t.n <= 0 || t.r <= 0 || t.m <= 0) return NQ_ERR_SHAPE;
+    return t.n % 256 != 0 || t.r % 256 != 0 || t.m % 32 != 0 ? NQ_ERR_PROB_SHAPE : NQ_OK;
+}
 // next: null, or the chains of a call that sums terms (only their first terms have a y).  *alike: all have s_in or none has.
 int check_terms(const nq_gemm_term* terms, const int* next, int count, bool* alike) {
     *alike = true;
     bool chained[kMaxTerms] = {};
     for (int i = 0; i < count; ++i) {
         const nq_gemm_term& t = terms[i];
-        if (t.n <= 0 || t.r <= 0 || t.m <= 0) return NQ_ERR_SHAPE;
-        if (t.n % 256 != 0 || t.r % 256 != 0 || t.m % 32 != 0) return NQ_ERR_PROB_SHAPE;
+        const int st = check_sizes(t);
+        if (st != NQ_OK) return st;
         if (!t.x || !t.vt_tiles || !t.u_tiles || !t.h || !(t.y || chained[i])) return NQ_ERR_NULL;
         if (((uintptr_t)t.x | (uintptr_t)t.vt_tiles | (uintptr_t)t.u_tiles | (uintptr_t)t.h | (uintptr_t)t.y |
              (uintptr_t)t.s_in | (uintptr_t)t.s_mid | (uintptr_t)t.s_out | (uintptr_t)t.bias) & 15u)
@@ -864,6 +869,8 @@ bool known_panel_mode(int mode) { return mode == NQ_PANEL_AUTO || mode == NQ_PAN
 
 int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode) {
     if (!terms || count < 1 || count > nq::gemm_group_max() || count > kMaxTerms || tokens < 1 || panel_mode == NQ_PANEL_NEVER) return 0;
+    for (int i = 0; i < count; ++i)
+        if (check_sizes(terms[i]) != NQ_OK) return 0;      // the call refuses them; the estimates take sizes that fit
     return panel_for(first_stage(terms, count), count, tokens, panel_mode) || panel_for(second_stage(terms, count), count, tokens, panel_mode);
 }
 

@@ -78,6 +78,13 @@ def test_no_panel_without_need():
     assert lib.nq_gemm_group_wants_panel(arr, 1, 128, 1) == 1
 
 
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,r,m", [(512, 256, 0), (512, 0, 128), (-256, 256, 128), (512, 256, 100), (500, 256, 128), (512, 300, 128)])
+def test_no_panel_for_sizes_that_are_refused(n, r, m, mode):
+    good, bad = (ops.NqGemmTerm(*[None] * 9, *sizes) for sizes in ((512, 256, 128), (n, r, m)))
+    assert _lib.lib().nq_gemm_group_wants_panel((ops.NqGemmTerm * 2)(good, bad), 2, 128, mode) == 0
+
+
 # tokens, n, r, m; whether a stage can be a panel launch (32-bit offsets into x, h, y and the signs)
 @pytest.mark.parametrize("tokens,n,r,m,fits", [
     (100000, 28672, 28672, 28672, 0),                        # 5.7 GB of x, h and y
