@@ -215,7 +215,7 @@ int nq_gemv_stage(const void* in, const void* s_col, const uint32_t* bits, const
  *   tiles: k*rows/32 words in the 32-row x 256-k tile layout of the package's prefill packer (the
  *   layout is private to packer and kernel, as the reference's Marlin layout is).
  *   Requires k % 256 == 0 and rows % 32 == 0 (else NQ_ERR_PROB_SHAPE, the reference's error class
- *   for shapes its tiles do not cover).  scratch: nq_gemm_scratch_bytes(tokens, k, rows) bytes of
+ *   for shapes its tiles do not cover), and k < 2^30; more than 2^22 columns run token by token.  scratch: nq_gemm_scratch_bytes(tokens, k, rows) bytes of
  *   device memory; that is 0 for every shape (no kernel splits k between workgroups), so NULL will do. */
 size_t nq_gemm_scratch_bytes(int tokens, int k, int rows);
 int nq_gemm_onebit(const void* x, const uint32_t* tiles, const void* s_in, const void* s_out, void* y,

@@ -270,6 +270,41 @@ static hipError_t launch_group(int pick, int dtype, int count, const void* const
     return scaled ? launch_tiles<1, true, N>(pick, g, blocks, stream) : launch_tiles<1, false, N>(pick, g, blocks, stream);
 }
 
+// A launch with problems of more than kGemmMaxK columns: one problem after the other, those token by token, every token a problem
+// of its own on the smallest tile (offsets of its further, missing tokens may wrap round: what they read is not stored).
+static hipError_t launch_apart(int dtype, int count, const void* const* x, const uint32_t* const* tiles, const void* const* s_in,
+                               const void* const* s_out, const void* const* bias, void* const* y, int T, const int* K, const int* R,
+                               int use, hipStream_t stream) {
+    for (int p = 0; p < count; ++p)
+        if (K[p] >= kGemmEndK) return hipErrorInvalidValue;
+    for (int p = 0; p < count; ++p) {
+        const void* si = s_in ? s_in[p] : nullptr;
+        const void* so = s_out ? s_out[p] : nullptr;
+        const void* bs = bias ? bias[p] : nullptr;
+        if (K[p] <= kGemmMaxK) {
+            const hipError_t e = gemm_onebit_group(dtype, 1, x + p, tiles + p, &si, &so, &bs, y + p, T, K + p, R + p, use, stream);
+            if (e != hipSuccess) return e;
+            continue;
+        }
+        for (int t = 0; t < T; t += kGroupMax) {
+            const int tokens = T - t < kGroupMax ? T - t : kGroupMax;
+            const void *xs[kGroupMax], *sis[kGroupMax], *sos[kGroupMax], *bss[kGroupMax];
+            const uint32_t* ws[kGroupMax];
+            void* ys[kGroupMax];
+            int Ks[kGroupMax], Rs[kGroupMax];
+            for (int j = 0; j < tokens; ++j) {
+                xs[j] = (const uint16_t*)x[p] + (size_t)(t + j) * K[p];
+                ys[j] = (uint16_t*)y[p] + (size_t)(t + j) * R[p];
+                ws[j] = tiles[p]; sis[j] = si; sos[j] = so; bss[j] = bs;
+                Ks[j] = K[p]; Rs[j] = R[p];
+            }
+            const hipError_t e = launch_group<kGroupMax>(0, dtype, tokens, xs, ws, sis, sos, bss, ys, 1, Ks, Rs, stream);
+            if (e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
 // GEMMs of several problems on the same token count in one launch; every problem: K % 256 == 0, R % 32 == 0, and
 // either all have input scales or none (checked by the caller).
 hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
@@ -277,7 +312,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
                              int T, const int* K, const int* R, int use, hipStream_t stream) {
     if (count < 1 || count > kGroupMax) return hipErrorInvalidValue;
     for (int p = 0; p < count; ++p)
-        if (K[p] > kGemmMaxK) return hipErrorInvalidValue;
+        if (K[p] > kGemmMaxK) return launch_apart(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, use, stream);
     double time = 0;
     const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0]}, use, &time);
     if (count == 1) return launch_group<1>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
@@ -357,6 +392,8 @@ static int choose_sum_tile(const SumHeads& h, int T, double* time) {
 }
 double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R) {
     double time = 0;
+    for (int i = 0; i < count; ++i)
+        if (K[i] > kGemmMaxK) return 1e30;
     choose_sum_tile(sum_heads(count, next, K, R), T, &time);
     return time;
 }

@@ -100,7 +100,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
 hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* const* x, const uint32_t* const* tiles,
                             const void* const* s_out, const void* const* bias, void* const* y, int T, const int* K, const int* R,
                             hipStream_t stream);
-double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R);       // estimate of that launch, us
+double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R);       // estimate of that launch, us; 1e30: not as sums
 // Estimated time of gemm_onebit_group with kGemmAnyTile, in us.
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 

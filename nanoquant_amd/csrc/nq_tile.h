@@ -39,7 +39,8 @@ struct GemmArgs {
 
 constexpr int kSlabK = 64;                   // k of one slab
 constexpr uint32_t kPastOperand = 0x80000000u;   // added to an offset: past the end of any operand (host: K <= kGemmMaxK)
-constexpr int kGemmMaxK = 1 << 22;
+constexpr int kGemmMaxK = 1 << 22;           // 128 tokens and 64 row tiles within 2^31 bytes
+constexpr int kGemmEndK = 1 << 30;           // the signs of 32 rows within 2^32 bytes: fewer, of one token at a time
 
 template <int TT, int RT, int WR, int WK, int NB>
 struct TileShape {

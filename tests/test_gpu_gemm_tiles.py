@@ -47,6 +47,26 @@ def test_tiles_at_their_edges(dev, tokens, k, rows, dtype, scaled):
     assert err < 1.2 * ROUND[dtype], err                     # products are exact, sums are fp32: the rounding of the result
 
 
+@pytest.mark.parametrize("scaled", [True, False])
+def test_more_columns_than_a_tile_of_tokens_can_address(dev, scaled):
+    # token by token, 16 to a launch
+    tokens, k, rows, dtype = 18, 2 ** 22 + 256, 256, torch.float16
+    x, bits, si, so, workspace, ref = _onebit(dev, tokens, k, rows, dtype, scaled, 9)
+    print(f"{k} columns scaled={scaled}", flush=True)
+    y = torch.ops.binary_kernels.marlin_onebit_forward(x, bits, si, so, workspace)
+    torch.cuda.synchronize()
+    err = ((y.double() - ref).abs().max() / ref.abs().max()).item()
+    assert err < 1.2 * ROUND[dtype], err
+    # in a group beside an ordinary linear: the bits that both get by themselves
+    x2, bits2, si2, so2, _, _ = _onebit(dev, tokens, 512, rows, dtype, scaled, 10)
+    out = _onebit(dev, 1, rows, 64, dtype, False, 11)[1]
+    terms = [(bits, out, si, so, None, workspace), (bits2, out, si2, so2, None, workspace)]
+    alone = [torch.ops.binary_kernels.marlin_nanoquant_forward(a, *t) for a, t in zip((x, x2), terms)]
+    group = ops.gemm_group_forward([x, x2], terms, panel="never")
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(alone, group))
+
+
 @pytest.mark.parametrize("tokens", [100, 128, 160])
 def test_other_tiles_for_many_rows_below_160_tokens(dev, tokens):
     # 2 x 8192 rows over a short rank: block tiles where the group may take any, the bits of the linear alone where it may not
