@@ -451,6 +451,8 @@ TORCH_LIBRARY_IMPL(binary_kernels, CUDA, m) {
 PYBIND11_MODULE(_host, m) {
     using Unlocked = py::call_guard<py::gil_scoped_release>;
     m.def("nanoquant_dyn_forward", &nanoquant_dyn_forward, Unlocked());
+    m.def("marlin_onebit_forward", &marlin_onebit_forward, Unlocked());
+    m.def("marlin_nanoquant_forward", &marlin_nanoquant_forward, Unlocked());
     m.def("gemv_bias", &gemv_bias, Unlocked());
     m.def("gemm_bias", &gemm_bias, Unlocked());
     m.def("gemm_group", &gemm_group);

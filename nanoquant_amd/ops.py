@@ -40,6 +40,7 @@ _SCHEMAS = (
 
 MARLIN_MIN_MAX_PAR = 32
 
+
 def _dtype_id(t: torch.Tensor) -> int:
     if t.dtype == torch.float16:
         return _lib.NQ_F16
@@ -224,9 +225,21 @@ def panel_status(device=None) -> int:
     return int(out.value)
 
 
+def marlin_onebit_forward(x, weight, scale_g, scale_h, workspace):
+    """C[m, n] = s_out[n] * sum_k (x[m, k] * s_in[k]) * sgn(weight)[n, k]; weight from marlin_onebit_packer.  The operator
+    without its dispatcher."""
+    return _host.marlin_onebit_forward(x, weight, scale_g, scale_h, workspace)
+
+
 def _marlin_onebit_meta(x, weight, scale_g, scale_h, workspace):
     m, n, _ = _onebit_check(x, weight, scale_g, scale_h, workspace)
     return x.new_empty((m, n))
+
+
+def marlin_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace):
+    """Two chained one-bit GEMMs (gemm.cpp:112-122): `weight_u` is the FIRST stage [n -> r],
+    `weight_v` the second [r -> m] (the order marlin_nanoquant_packer returns them).  The operator without its dispatcher."""
+    return _host.marlin_nanoquant_forward(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace)
 
 
 def _marlin_nanoquant_meta(x, weight_u, weight_v, scale_g, scale_l, scale_h, workspace):

@@ -25,10 +25,20 @@ def _term(**other):
     (F16(5, 512), _term(), "x must be a CUDA tensor"),
 ])
 def test_prefill_checks(x, term, message):
-    for call in (lambda: ops.gemm_forward_with_bias(x, *term, None), lambda: ops.gemm_group_forward(x, [term]),
+    for call in (lambda: ops.marlin_nanoquant_forward(x, *term), lambda: ops.gemm_forward_with_bias(x, *term, None), lambda: ops.gemm_group_forward(x, [term]),
                  lambda: ops.gemm_group_sum_forward(x, [[term]])):
         with pytest.raises(RuntimeError, match=message):
             call()
+
+
+@pytest.mark.parametrize("x,other,message", [
+    (torch.zeros(5, 512), {}, "Unsupported dtype"), (F16(5, 500), {}, "k dimension mismatch"), (F16(5, 512), {"scale_h": F16(255)}, "s_out size mismatch"),
+    (F16(5, 512), {}, "x must be a CUDA tensor"),
+])
+def test_single_matrix_checks(x, other, message):
+    args = dict(weight=I32(32, 128), scale_g=F16(512), scale_h=F16(256), workspace=I32(64))
+    with pytest.raises(RuntimeError, match=message):
+        ops.marlin_onebit_forward(x, **{**args, **other})
 
 
 @pytest.mark.parametrize("call", [
