@@ -293,9 +293,13 @@ struct Tile {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     }
 
-    // Four values of s_out or bias for rows row .. + 3; pad: two of the value where there are none.
+    // Four values of s_out or bias for rows row .. + 3; pad: two of the value where there are none.  s_out may begin at any element,
+    // which the device reads in one load all the same.
+    struct __attribute__((packed, aligned(2))) Four {
+        uint2 v;
+    };
     static __device__ __forceinline__ uint2 row_values(const GemmArgs& a, const uint16_t* p, int row, uint32_t pad) {
-        return p && row < a.R ? *(const uint2*)(p + row) : make_uint2(pad, pad);
+        return p && row < a.R ? ((const Four*)(p + row))->v : make_uint2(pad, pad);
     }
     // Piece p of a 32 x 32 tile: rows 8 p + 4 hi .. + 3 of token lane & 31.  With several k groups it is finished by group p % WK.
     static constexpr int kPieces = 4 / WK;

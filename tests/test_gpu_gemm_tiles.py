@@ -47,6 +47,20 @@ def test_tiles_at_their_edges(dev, tokens, k, rows, dtype, scaled):
     assert err < 1.2 * ROUND[dtype], err                     # products are exact, sums are fp32: the rounding of the result
 
 
+@pytest.mark.parametrize("tokens", [5, 200])
+def test_output_scales_that_begin_anywhere(dev, tokens):
+    # of one linear by itself, on few-token and on block tiles: slices at every element offset give the bits of an aligned scale
+    x, bits, si, so, workspace, _ = _onebit(dev, tokens, 512, 2080, torch.float16, True, 8)
+    want = torch.ops.binary_kernels.marlin_onebit_forward(x, bits, si, so, workspace)
+    for offset in range(1, 8):
+        own = torch.full((offset + so.numel() + 8,), float("nan"), dtype=so.dtype, device=dev)[offset:offset + so.numel()]
+        own.copy_(so)
+        print(f"scale at element {offset}, {tokens} tokens", flush=True)
+        y = torch.ops.binary_kernels.marlin_onebit_forward(x, bits, si, own, workspace)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), offset
+
+
 @pytest.mark.parametrize("scaled", [True, False])
 def test_more_columns_than_a_tile_of_tokens_can_address(dev, scaled):
     # token by token, 16 to a launch
