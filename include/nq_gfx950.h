@@ -297,6 +297,11 @@ int nq_gemm_nanoquant_sum(const nq_gemm_term* terms, const int* next, int count,
                           size_t panel_ws_bytes, int panel_mode, void* stream);
 /* 1 when that call is estimated to take less than nq_gemm_nanoquant_group_ws and the additions (0 otherwise, for terms that it refuses and where nothing is summed). */
 int nq_gemm_sum_pays(const nq_gemm_term* terms, const int* next, int count, int tokens);
+/* Tokens * 65536 + rows of the tiles that a launch of GEMMs on k[i] columns and rows[i] rows is cut into (0: refused sizes), for
+ * tests and for tuning: of one linear by itself, of a group in which it keeps the bits that it has there up to 160 tokens
+ * (NQ_PANEL_NEVER), of any other group, of sums (next as above, else NULL).  scaled: with input scales; all read one input. */
+enum { NQ_TILE_ALONE = 0, NQ_TILE_GROUP = 1, NQ_TILE_ANY = 2, NQ_TILE_SUM = 3 };
+int nq_gemm_tile_size(int use, int count, int tokens, const int* k, const int* rows, int scaled, const int* next);
 int nq_gemm_panel_status(const void* panel_ws, int* status_out, void* stream);
 /* Polls after which a wait of a panel launch gives up (0 = the default of 2^20).  Process-wide; for exercising a
  * caller's handling of status 1 from the host, as nq_gemv_group_set_spin_limit. */

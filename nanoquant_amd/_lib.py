@@ -52,6 +52,7 @@ _SIGNATURES = {
     "nq_gemm_group_wants_panel": (_i, [_vp, _i, _i, _i]),
     "nq_gemm_nanoquant_sum": (_i, [_vp, ctypes.POINTER(_i), _i, _i, _i, _vp, _sz, _i, _vp]),
     "nq_gemm_sum_pays": (_i, [_vp, ctypes.POINTER(_i), _i, _i]),
+    "nq_gemm_tile_size": (_i, [_i, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i), _i, ctypes.POINTER(_i)]),
     "nq_gemm_panel_status": (_i, [_vp, ctypes.POINTER(_i), _vp]),
     "nq_gemm_panel_set_spin_limit": (_i, [ctypes.c_uint]),
     "nq_pack_gemm_tiles": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp]),

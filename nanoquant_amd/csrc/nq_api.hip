@@ -42,7 +42,7 @@ const char* nq_status_string(int status) {
 
 int nq_last_hip_error(void) { return g_last_hip_error; }
 
-int nq_abi_version(void) { return 10; }
+int nq_abi_version(void) { return 11; }
 
 int nq_device_query(int attr, int* value) {
     if (!value) return NQ_ERR_NULL;
@@ -919,6 +919,18 @@ int nq_gemm_nanoquant_sum(const nq_gemm_term* terms, const int* next, int count,
     if (e != hipSuccess) return hip_status(e);
     const GroupStage s = second_stage(terms, count);
     return hip_status(nq::gemm_onebit_sums(dtype, count, next, s.x, s.w, s.so, s.bs, s.out, tokens, s.K, s.R, (hipStream_t)stream));
+}
+
+int nq_gemm_tile_size(int use, int count, int tokens, const int* k, const int* rows, int scaled, const int* next) {
+    if (!k || !rows || count < 1 || count > nq::gemm_group_max() || count > kMaxTerms || tokens < 1) return 0;
+    if (use < NQ_TILE_ALONE || use > NQ_TILE_SUM || (use == NQ_TILE_SUM) != (next != nullptr)) return 0;
+    for (int i = 0; i < count; ++i) {
+        if (k[i] <= 0 || rows[i] <= 0 || k[i] % 256 != 0 || rows[i] % 32 != 0) return 0;
+        if (next && next[i] >= 0 && (next[i] <= i || next[i] >= count || rows[next[i]] != rows[i])) return 0;
+    }
+    if (next) return nq::gemm_sums_tile_size(count, next, tokens, k, rows);
+    const void* const x[kMaxTerms] = {};
+    return nq::gemm_tile_size(use, count, x, tokens, k, rows, scaled != 0);
 }
 
 // The sums by launches of their own: per pass over a term index 3 us, and two reads and one write of the 16-bit results at the

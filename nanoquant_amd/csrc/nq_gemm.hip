@@ -111,22 +111,24 @@ struct TileCost {
 };
 struct TileVariant {
     int tt, rt, wr, wk, nb;
+    int sum_fit;                     // gemm_tile_sum_kernel: workgroups that fit a compute unit (0: none of this size), and what
+    float sum_start;                 // it takes beyond the costs below where a single round of them does it all
     TileCost cost[2];                // without and with s_in
 };
 constexpr int kFewTiles = 3, kVariantCount = 6;      // the first kFewTiles entries are few-token tiles
 constexpr TileVariant kVariants[kVariantCount] = {
-    {1, 1, 1, 4, 4, {{2.27f, 0.89f, {0.75f, 1.77f}}, {2.01f, 1.62f, {0.72f, 1.63f}}}},
-    {1, 2, 1, 4, 4, {{2.30f, 1.22f, {1.10f, 2.44f}}, {1.94f, 2.00f, {1.01f, 2.33f}}}},
-    {1, 3, 1, 4, 3, {{2.46f, 1.30f, {1.60f, 3.38f}}, {1.57f, 2.59f, {1.46f, 3.21f}}}},
-    {2, 1, 4, 1, 4, {{1.35f, 2.84f, {0.69f, 1.63f, 2.83f, 3.60f}}, {2.19f, 1.50f, {0.90f, 1.74f, 2.81f, 3.90f}}}},
-    {2, 2, 4, 1, 4, {{0.84f, 4.08f, {1.14f, 3.04f, 4.89f}}, {0.f, 4.27f, {1.33f, 3.05f, 4.96f}}}},
-    {4, 2, 4, 1, 4, {{0.f, 6.09f, {2.18f, 5.76f}}, {0.f, 5.73f, {2.33f, 5.57f}}}},
+    {1, 1, 1, 4, 4, 2, 0.f, {{2.27f, 0.89f, {0.75f, 1.77f}}, {2.01f, 1.62f, {0.72f, 1.63f}}}},
+    {1, 2, 1, 4, 4, 2, 0.f, {{2.30f, 1.22f, {1.10f, 2.44f}}, {1.94f, 2.00f, {1.01f, 2.33f}}}},
+    {1, 3, 1, 4, 3, 2, 0.f, {{2.46f, 1.30f, {1.60f, 3.38f}}, {1.57f, 2.59f, {1.46f, 3.21f}}}},
+    {2, 1, 4, 1, 4, 4, 0.f, {{1.35f, 2.84f, {0.69f, 1.63f, 2.83f, 3.60f}}, {2.19f, 1.50f, {0.90f, 1.74f, 2.81f, 3.90f}}}},
+    {2, 2, 4, 1, 4, 2, 2.f, {{0.84f, 4.08f, {1.14f, 3.04f, 4.89f}}, {0.f, 4.27f, {1.33f, 3.05f, 4.96f}}}},
+    {4, 2, 4, 1, 4, 0, 0.f, {{0.f, 6.09f, {2.18f, 5.76f}}, {0.f, 5.73f, {2.33f, 5.57f}}}},
 };
 
 struct GemmShapes {
     int count, T;
     const int *K, *R;
-    bool scaled;
+    bool scaled, sums;               // sums: for gemm_tile_sum_kernel
 };
 
 static int tile_gx(const TileVariant& v, int R) { return (R + 32 * v.rt * v.wr - 1) / (32 * v.rt * v.wr); }
@@ -147,7 +149,7 @@ static double tile_time(const TileVariant& v, const GemmShapes& s) {
         longest = tiles > longest ? tiles : longest;
     }
     int fit = 0;
-    while (fit < 4 && c.tile[fit] > 0.f) ++fit;
+    while (fit < (s.sums ? v.sum_fit : 4) && c.tile[fit] > 0.f) ++fit;
     const double mean = work / blocks;
     auto walk = [&](double workgroups, double* rounds) {
         const long per_cu = (long)std::ceil(workgroups / 256.0), full = per_cu / fit, rest = per_cu % fit;
@@ -162,7 +164,7 @@ static double tile_time(const TileVariant& v, const GemmShapes& s) {
     double rounds, real_rounds;
     const double time = walk(blocks, &rounds), real = walk(blocks / whole, &real_rounds);
     // half the way to what as many whole workgroups would take: the cut ones still share compute units
-    return c.start + c.round * 0.5 * (rounds + real_rounds) + 0.5 * (time + real);
+    return c.start + (s.sums && real_rounds <= 1.0 ? v.sum_start : 0.f) + c.round * 0.5 * (rounds + real_rounds) + 0.5 * (time + real);
 }
 
 static int best_tile(const GemmShapes& s, int begin, int end, double* time) {
@@ -209,7 +211,7 @@ static int choose_tile(const void* const* x, const GemmShapes& s, int use, doubl
 
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
     double time = 0;
-    choose_tile(x, GemmShapes{count, T, K, R, scaled}, kGemmAnyTile, &time);
+    choose_tile(x, GemmShapes{count, T, K, R, scaled, false}, kGemmAnyTile, &time);
     return time;
 }
 
@@ -314,7 +316,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
     for (int p = 0; p < count; ++p)
         if (K[p] > kGemmMaxK) return launch_apart(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, use, stream);
     double time = 0;
-    const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0]}, use, &time);
+    const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0], false}, use, &time);
     if (count == 1) return launch_group<1>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     return launch_group<kGroupMax>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
 }
@@ -379,13 +381,17 @@ static SumHeads sum_heads(int count, const int* next, const int* K, const int* R
     }
     return h;
 }
-// A sum costs about what one problem of its terms' k costs, and some 1.5 us for every further term, whose ring is filled anew.
+// A sum costs about what one problem of its terms' k costs, and some 1.5 us for every further term, whose ring is filled anew;
+// but of 64 x 256 tiles, whose accumulators it holds twice (196 registers), only two workgroups fit a compute unit, and in a
+// single round of them nobody multiplies while a ring is filled.  The pick is 0.3 % slower than the best tile on average and 9 %
+// at worst, over 160 pairs of stages (100 to 4096 tokens, seven linears of two models); priced as the plain kernel 0.7 and 12 %
+// ({q, k, v} of Qwen3-8B at 0.9 bits on 333 tokens: both stages 37.5 us on 64 x 256, 33.6 on 64 x 128).
 // Where k is split between wavefronts a term of one k tile takes as long as one of four: counted by its own k, two terms of
 // 256 -> 64 rows on 8192 tokens took such a tile, 20.3 us with the first stage; 17.4 apart and added, 16.6 on the tile taken now.
 static int choose_sum_tile(const SumHeads& h, int T, double* time) {
     double few_time = 0, block_time = 0;
-    const int few = best_tile(GemmShapes{h.count, T, h.split_k, h.R, false}, 0, kFewTiles, &few_time);
-    const int block = best_tile(GemmShapes{h.count, T, h.K, h.R, false}, kFewTiles, kSumVariantCount, &block_time);
+    const int few = best_tile(GemmShapes{h.count, T, h.split_k, h.R, false, true}, 0, kFewTiles, &few_time);
+    const int block = best_tile(GemmShapes{h.count, T, h.K, h.R, false, true}, kFewTiles, kSumVariantCount, &block_time);
     const bool take_few = few_time < 0.95 * block_time;
     *time = (take_few ? few_time : block_time) + 1.5 * (h.longest - 1);
     return take_few ? few : block;
@@ -430,6 +436,17 @@ hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* c
         if (j < h.count) blocks += group_blocks(s.g.a[j].gx, tile_gy(kVariants[pick], T));
     }
     return dtype == 0 ? launch_sums<0>(pick, s, blocks, stream) : launch_sums<1>(pick, s, blocks, stream);
+}
+
+int gemm_tile_size(int use, int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
+    double time = 0;
+    const TileVariant& v = kVariants[choose_tile(x, GemmShapes{count, T, K, R, scaled, false}, use, &time)];
+    return (32 * v.tt) << 16 | 32 * v.rt * v.wr;
+}
+int gemm_sums_tile_size(int count, const int* next, int T, const int* K, const int* R) {
+    double time = 0;
+    const TileVariant& v = kVariants[choose_sum_tile(sum_heads(count, next, K, R), T, &time)];
+    return (32 * v.tt) << 16 | 32 * v.rt * v.wr;
 }
 
 int gemm_group_max() { return kGroupMax; }

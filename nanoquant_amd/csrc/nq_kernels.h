@@ -101,6 +101,9 @@ hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* c
                             const void* const* s_out, const void* const* bias, void* const* y, int T, const int* K, const int* R,
                             hipStream_t stream);
 double gemm_sums_time(int count, const int* next, int T, const int* K, const int* R);       // estimate of that launch, us; 1e30: not as sums
+// The tiles that those launches are cut into: tokens << 16 | rows.
+int gemm_tile_size(int use, int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
+int gemm_sums_tile_size(int count, const int* next, int T, const int* K, const int* R);
 // Estimated time of gemm_onebit_group with kGemmAnyTile, in us.
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
 

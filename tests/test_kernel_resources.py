@@ -1,5 +1,6 @@
-"""Registers of the built run-list kernels, from the metadata notes of the code objects inside the library (no GPU): the
-batch 4 instances are at the register limit of 1024 lanes, and what spills there is time in the inner loop."""
+"""Registers of the built kernels, from the metadata notes of the code objects inside the library (no GPU).  Run lists: the
+batch 4 instances are at the register limit of 1024 lanes, and what spills there is time in the inner loop.  Prefill tiles: the
+choice of sizes counts on so many workgroups per compute unit."""
 import struct
 
 import pytest
@@ -69,3 +70,25 @@ def test_short_lists_at_batch_1_spill_no_more_scalar_registers_than_with_the_wai
 @pytest.mark.parametrize("dtype", [0, 1])
 def test_reproducible_row_major_lists_at_batch_1_spill_no_vector_register(kernels, dtype):
     assert _stream_kernel(kernels, dtype, 1, 2, 0, 1, 0)[".vgpr_spill_count"] == 0
+
+
+# tile of a wavefront (32-token blocks, 32-row blocks), wavefronts over rows and k, slabs; workgroups per compute unit that its
+# costs are for, of the plain kernels and of the summing ones (0: none)
+_TILES = [((1, 1, 1, 4, 4), 2, 2), ((1, 2, 1, 4, 4), 2, 2), ((1, 3, 1, 4, 3), 2, 2), ((2, 1, 4, 1, 4), 4, 4), ((2, 2, 4, 1, 4), 3, 2), ((4, 2, 4, 1, 4), 2, 0)]
+
+
+def _fit(kernel):
+    # a workgroup is four wavefronts, one to each SIMD, whose 512 registers go out in eights
+    assert kernel[".max_flat_workgroup_size"] == 256 and kernel[".vgpr_spill_count"] == 0
+    return 512 // ((kernel[".vgpr_count"] + kernel[".agpr_count"] + 7) // 8 * 8)
+
+
+@pytest.mark.parametrize("tile,plain,sums", _TILES)
+def test_registers_of_the_prefill_tiles(kernels, tile, plain, sums):
+    shape = "E".join(f"Li{v}" for v in tile)
+    found = {kind: [k for name, k in kernels.items() if f"{kind}ILi" in name and shape in name] for kind in ("gemm_tile_kernel", "gemm_tile_sum_kernel")}
+    assert len(found["gemm_tile_kernel"]) == 8 and len(found["gemm_tile_sum_kernel"]) == (2 if sums else 0)
+    assert all(_fit(k) >= plain for k in found["gemm_tile_kernel"])
+    assert all(_fit(k) >= sums for k in found["gemm_tile_sum_kernel"])
+    if sums and sums < plain:
+        assert all(_fit(k) < plain for k in found["gemm_tile_sum_kernel"])      # else its costs are too high
