@@ -816,7 +816,7 @@ GroupStage second_stage(const nq_gemm_term* terms, int count) {
 }
 bool panel_for(const GroupStage& s, int count, int tokens, int mode) {
     if (mode == NQ_PANEL_ALWAYS) return nq::panel_addresses(count, tokens, s.K, s.R);
-    return mode == NQ_PANEL_AUTO && nq::panel_applies(count, s.x, tokens, s.K, s.R, s.si[0] != nullptr);
+    return mode == NQ_PANEL_AUTO && nq::panel_applies(count, s.x, tokens, s.K, s.R, s.si[0] != nullptr, nullptr);
 }
 struct PanelUse {
     void* ws;                                    // null: no panel launches
@@ -951,8 +951,9 @@ int nq_gemm_sum_pays(const nq_gemm_term* terms, const int* next, int count, int 
     }
     if (passes == 0) return 0;
     const GroupStage s = second_stage(terms, count);
-    const double tiles = nq::gemm_tiles_time(count, s.x, tokens, s.K, s.R, false), panels = nq::panel_time(count, tokens, s.K, s.R, false);
-    return nq::gemm_sums_time(count, next, tokens, s.K, s.R) < (panels < 0.95 * tiles ? panels : tiles) + 3.0 * passes + adds;
+    double apart = 0;
+    nq::panel_applies(count, s.x, tokens, s.K, s.R, false, &apart);
+    return nq::gemm_sums_time(count, next, tokens, s.K, s.R) < apart + 3.0 * passes + adds;
 }
 
 size_t nq_tiled_words(int rows, int words) {

@@ -110,9 +110,9 @@ double gemm_tiles_time(int count, const void* const* x, int T, const int* K, con
 // nq_panel.hip: the same GEMMs up to 2048 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
 size_t panel_workspace_bytes();
-double panel_time(int count, int T, const int* K, const int* R, bool scaled);      // estimate in us; 1e30: not as panels
 bool panel_addresses(int count, int T, const int* K, const int* R);                // small enough for the kernel
-bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled);
+// Whether panels are the faster form (automatic choice); *time (or null): estimate of the faster one, in us.
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time);
 hipError_t gemm_panel_group(int dtype, int count, const void* const* x, const uint32_t* const* tiles,
                             const void* const* s_in, const void* const* s_out, const void* const* bias, void* const* y,
                             int T, const int* K, const int* R, void* workspace, unsigned spin_limit, hipStream_t stream);

@@ -564,7 +564,7 @@ bool panel_addresses(int count, int T, const int* K, const int* R) {
 // + 1 for every workgroup that a panel is shared by: the middle 90 % of 445 launches are within -8 .. +8 % of that (128 to 2048
 // tokens, 1 to 43 k tiles, 512 to 22016 rows); with fewer than three k steps the hand-over takes most of the time (128
 // tokens, 3072 -> 4096 rows: tiles 7, panels 35).
-double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
+static double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
     constexpr double kNever = 1e30;
     constexpr int kMostTokens = 2048;            // of the launches that were timed
     const int G = panel_grid();
@@ -585,10 +585,13 @@ double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
 
 // Problems of different k are the estimate's weak side: the seven linears of a Llama-2-7B layer in one group took, in us, 214 on 512
 // tokens and 399 on 1024 with panels at 0.93, 194 and 372 at 0.85; of Qwen3-8B on 1536 497 / 447, on 768 241 / 247.
-bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
+    const double panels = panel_time(count, T, K, R, scaled), tiles = gemm_tiles_time(count, x, T, K, R, scaled);
     bool mixed = false;
     for (int p = 1; p < count; ++p) mixed = mixed || K[p] != K[0];
-    return panel_time(count, T, K, R, scaled) < (mixed ? 0.85 : 0.95) * gemm_tiles_time(count, x, T, K, R, scaled);
+    const bool take = panels < (mixed ? 0.85 : 0.95) * tiles;
+    if (time) *time = take ? panels : tiles;
+    return take;
 }
 
 template <int DT, bool SCALED>

@@ -108,3 +108,21 @@ def test_inputs_of_their_own_count_by_themselves(dev, dtype):
     one, six = run([xs[0]] * 6, terms)[0], run(xs, terms)[0]
     torch.cuda.synchronize()
     assert torch.equal(one, few) and torch.equal(six, block) and not torch.equal(few, block)
+
+
+# (tokens, weights as lists of (n, r, m)): the second GEMMs differ in k, and panels are estimated a little ahead of tiles, too little to
+# be taken.  us apart on tiles / apart on panels / as sums
+@pytest.mark.parametrize("tokens,weights", [
+    (655, [[(8960, 3328, 12288), (8960, 3072, 12288)], [(8960, 3840, 5408)]]),      # 241 / 237 / 223
+    (868, [[(6656, 3584, 12768), (6656, 3840, 12768)]]),                           # 234 / 237 / 228
+    (1037, [[(1792, 3584, 4384), (1792, 2560, 4384)], [(1792, 3840, 7072)]]),       # 151 / 153 / 148
+])
+def test_sums_are_compared_with_the_launch_that_would_be_made(dev, tokens, weights):
+    import ctypes
+
+    from nanoquant_amd import _lib
+    flat = [(w, t) for w, terms in enumerate(weights) for t in range(len(terms))]
+    follows = [flat.index((w, t + 1)) if (w, t + 1) in flat else -1 for w, t in flat]
+    arr = (ops.NqGemmTerm * len(flat))(*[ops.NqGemmTerm(4096, 4096, 4096, 4096, None, None, None, 4096 * (i + 1), 16 * (i + 1), *weights[w][t])
+                                         for i, (w, t) in enumerate(flat)])
+    assert _lib.lib().nq_gemm_sum_pays(arr, (ctypes.c_int * len(flat))(*follows), len(flat), tokens) == 1      # a question, no launch
