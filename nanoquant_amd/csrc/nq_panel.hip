@@ -583,13 +583,25 @@ static double panel_time(int count, int T, const int* K, const int* R, bool scal
     return 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
 }
 
-// Problems of different k are the estimate's weak side: the seven linears of a Llama-2-7B layer in one group took, in us, 214 on 512
-// tokens and 399 on 1024 with panels at 0.93, 194 and 372 at 0.85; of Qwen3-8B on 1536 497 / 447, on 768 241 / 247.
+// How far below the tiles' estimate a panel launch must be.  Problems of different k are the weak side of both estimates.  Over 258
+// stages of such groups (100 to 2048 tokens, of one layer's linears at 0.7 and 1 bit) the slower form was taken for 0.9 % of both
+// stages' time where some k is long (more than 16 tiles; 1.7 % at 0.85), for 0.1 % elsewhere (1.2 % at 1): {o, down} of Qwen3-8B on 1280
+// tokens, first stage 4096 and 12288, 195 us on tiles, 167 on panels; second stages of k 1024 to 3072 on 1536 tokens 501 / 527.
+// For one k 0.95 loses 0.2 %, 0.85 0.5, 1 0.3 (290 stages).
+static double panel_margin(int count, const int* K) {
+    constexpr int kLongK = 16 * kTileK;
+    bool mixed = false;
+    int longest = 0;
+    for (int p = 0; p < count; ++p) {
+        mixed = mixed || K[p] != K[0];
+        longest = longest > K[p] ? longest : K[p];
+    }
+    return !mixed ? 0.95 : longest > kLongK ? 1.0 : 0.85;
+}
+
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
     const double panels = panel_time(count, T, K, R, scaled), tiles = gemm_tiles_time(count, x, T, K, R, scaled);
-    bool mixed = false;
-    for (int p = 1; p < count; ++p) mixed = mixed || K[p] != K[0];
-    const bool take = panels < (mixed ? 0.85 : 0.95) * tiles;
+    const bool take = panels < panel_margin(count, K) * tiles;
     if (time) *time = take ? panels : tiles;
     return take;
 }

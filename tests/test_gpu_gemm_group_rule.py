@@ -126,3 +126,18 @@ def test_sums_are_compared_with_the_launch_that_would_be_made(dev, tokens, weigh
     arr = (ops.NqGemmTerm * len(flat))(*[ops.NqGemmTerm(4096, 4096, 4096, 4096, None, None, None, 4096 * (i + 1), 16 * (i + 1), *weights[w][t])
                                          for i, (w, t) in enumerate(flat)])
     assert _lib.lib().nq_gemm_sum_pays(arr, (ctypes.c_int * len(flat))(*follows), len(flat), tokens) == 1      # a question, no launch
+
+
+# (tokens, linears (n, r, m), whether a stage is a panel launch); us on tiles / with the first stage on panels / the second
+@pytest.mark.parametrize("tokens,linears,panel", [
+    (1280, [(4096, 2048, 4096), (12288, 3072, 4096)], 1),      # k of 16 and 48 tiles: 196 / 167 / 202
+    (640, [(4096, 2048, 4096), (12288, 3072, 4096)], 1),       # 115 / 103 / 117
+    (640, [(4096, 1536, 4096), (11008, 2304, 4096)], 1),       # 90 / 85 / 94
+    (1536, [(1024, 2048, 4096), (1024, 3072, 12288), (1024, 3072, 12288)], 0),      # k of 8 and 12 tiles: tiles ahead by 5 %
+])
+def test_panels_beside_tiles_where_k_differs(dev, tokens, linears, panel):
+    from nanoquant_amd import _lib
+    # inputs by width, h by linear, as a group call has them
+    arr = (ops.NqGemmTerm * len(linears))(*[ops.NqGemmTerm(n, 4096, 4096, 4096, None, None, None, 4096 * (i + 1), 16 * (i + 1), n, r, m)
+                                           for i, (n, r, m) in enumerate(linears)])
+    assert _lib.lib().nq_gemm_group_wants_panel(arr, len(linears), tokens, 0) == panel      # a question, no launch
