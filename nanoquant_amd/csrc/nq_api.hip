@@ -737,7 +737,7 @@ int nq_gemm_onebit_bias(const void* x, const uint32_t* tiles, const void* s_in, 
     if (!x || !tiles || !y) return NQ_ERR_NULL;
     if (((uintptr_t)x | (uintptr_t)tiles | (uintptr_t)y | (uintptr_t)s_in | (uintptr_t)scratch | (uintptr_t)bias) & 15u)
         return NQ_ERR_ALIGN;
-    (void)scratch_bytes;
+    (void)scratch_bytes;                         // scratch is not read; one out of line stays refused
     return hip_status(nq::gemm_onebit_group(dtype, 1, &x, &tiles, &s_in, &s_out, &bias, &y, tokens, &k, &rows, nq::kGemmAlone,
                                             (hipStream_t)stream));
 }

@@ -129,7 +129,13 @@ struct GemmShapes {
     int count, T;
     const int *K, *R;
     bool scaled, sums;               // sums: for gemm_tile_sum_kernel
+    double cus;                      // compute units
 };
+// The costs are of a device of 256, which also stands in where there is none to ask.
+static double device_units() {
+    const int n = compute_units();
+    return n > 0 ? n : 256;
+}
 
 static int tile_gx(const TileVariant& v, int R) { return (R + 32 * v.rt * v.wr - 1) / (32 * v.rt * v.wr); }
 static int tile_gy(const TileVariant& v, int T) { return (T + 32 * v.tt - 1) / (32 * v.tt); }
@@ -152,7 +158,7 @@ static double tile_time(const TileVariant& v, const GemmShapes& s) {
     while (fit < (s.sums ? v.sum_fit : 4) && c.tile[fit] > 0.f) ++fit;
     const double mean = work / blocks;
     auto walk = [&](double workgroups, double* rounds) {
-        const long per_cu = (long)std::ceil(workgroups / 256.0), full = per_cu / fit, rest = per_cu % fit;
+        const long per_cu = (long)std::ceil(workgroups / s.cus), full = per_cu / fit, rest = per_cu % fit;
         *rounds = (double)full + (rest ? 1 : 0);
         const double all = mean * ((double)full * c.tile[fit - 1] + (rest ? c.tile[rest - 1] : 0.f));
         // The longest problem's workgroups start first and share their compute units with those of mean length (4096 and 11008 ->
@@ -211,7 +217,7 @@ static int choose_tile(const void* const* x, const GemmShapes& s, int use, doubl
 
 double gemm_tiles_time(int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
     double time = 0;
-    choose_tile(x, GemmShapes{count, T, K, R, scaled, false}, kGemmAnyTile, &time);
+    choose_tile(x, GemmShapes{count, T, K, R, scaled, false, device_units()}, kGemmAnyTile, &time);
     return time;
 }
 
@@ -316,7 +322,7 @@ hipError_t gemm_onebit_group(int dtype, int count, const void* const* x, const u
     for (int p = 0; p < count; ++p)
         if (K[p] > kGemmMaxK) return launch_apart(dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, use, stream);
     double time = 0;
-    const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0], false}, use, &time);
+    const int pick = choose_tile(x, GemmShapes{count, T, K, R, s_in && s_in[0], false, device_units()}, use, &time);
     if (count == 1) return launch_group<1>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
     return launch_group<kGroupMax>(pick, dtype, count, x, tiles, s_in, s_out, bias, y, T, K, R, stream);
 }
@@ -390,8 +396,9 @@ static SumHeads sum_heads(int count, const int* next, const int* K, const int* R
 // 256 -> 64 rows on 8192 tokens took such a tile, 20.3 us with the first stage; 17.4 apart and added, 16.6 on the tile taken now.
 static int choose_sum_tile(const SumHeads& h, int T, double* time) {
     double few_time = 0, block_time = 0;
-    const int few = best_tile(GemmShapes{h.count, T, h.split_k, h.R, false, true}, 0, kFewTiles, &few_time);
-    const int block = best_tile(GemmShapes{h.count, T, h.K, h.R, false, true}, kFewTiles, kSumVariantCount, &block_time);
+    const double cus = device_units();
+    const int few = best_tile(GemmShapes{h.count, T, h.split_k, h.R, false, true, cus}, 0, kFewTiles, &few_time);
+    const int block = best_tile(GemmShapes{h.count, T, h.K, h.R, false, true, cus}, kFewTiles, kSumVariantCount, &block_time);
     const bool take_few = few_time < 0.95 * block_time;
     *time = (take_few ? few_time : block_time) + 1.5 * (h.longest - 1);
     return take_few ? few : block;
@@ -440,7 +447,7 @@ hipError_t gemm_onebit_sums(int dtype, int count, const int* next, const void* c
 
 int gemm_tile_size(int use, int count, const void* const* x, int T, const int* K, const int* R, bool scaled) {
     double time = 0;
-    const TileVariant& v = kVariants[choose_tile(x, GemmShapes{count, T, K, R, scaled, false}, use, &time)];
+    const TileVariant& v = kVariants[choose_tile(x, GemmShapes{count, T, K, R, scaled, false, device_units()}, use, &time)];
     return (32 * v.tt) << 16 | 32 * v.rt * v.wr;
 }
 int gemm_sums_tile_size(int count, const int* next, int T, const int* K, const int* R) {

@@ -109,6 +109,7 @@ double gemm_tiles_time(int count, const void* const* x, int T, const int* K, con
 
 // nq_panel.hip: the same GEMMs up to 2048 tokens as one persistent launch over 64-token x 256-row panels
 // (see the file header).  workspace: panel_workspace_bytes() bytes, zero when first used.
+int compute_units();                 // of the current device; 0: none
 size_t panel_workspace_bytes();
 bool panel_addresses(int count, int T, const int* K, const int* R);                // small enough for the kernel
 // Whether panels are the faster form (automatic choice); *time (or null): estimate of the faster one, in us.

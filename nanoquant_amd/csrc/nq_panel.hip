@@ -527,19 +527,19 @@ __global__ __launch_bounds__(kPanelThreads, kPanelPerCu * kPanelWaves / 4) void 
 }
 
 // ---- host side --------------------------------------------------------------------------------
-// Workgroups of a launch: kPanelPerCu per compute unit, all resident at once (checked against the occupancy of the
-// kernel before the first launch on a device).
-static int panel_grid() {
+int compute_units() {
     static PerDeviceFlag known;
     static int cus[64];
     const int dev = current_device();
     if (dev >= 0 && dev < 64 && known.test(dev)) return cus[dev];
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev < 0 ? 0 : dev) != hipSuccess || n <= 0) return 0;
-    n *= kPanelPerCu;
     if (dev >= 0 && dev < 64) { cus[dev] = n; known.set(dev); }
     return n;
 }
+// Workgroups of a launch: kPanelPerCu per compute unit, all resident at once (checked against the occupancy of the
+// kernel before the first launch on a device).
+static int panel_grid() { return kPanelPerCu * compute_units(); }
 
 size_t panel_workspace_bytes() {
     const int G = panel_grid();

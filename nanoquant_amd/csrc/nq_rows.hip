@@ -582,8 +582,7 @@ static int make_group(RowsGroup<NT, N>& g, int count, const RowsStage* s, int ba
             *waves = std::max(*waves, g.p[i].waves);
         }
     }
-    g.first[N] = at;                     // so that no workgroup belongs to an unused entry
-    for (int i = count; i < N; ++i) g.first[i] = at;
+    g.first[N] = at;                     // as of every unused entry, so that no workgroup belongs to one
     g.batch = batch;
     g.waves = *waves;
     return at;
