@@ -2,7 +2,7 @@
 (src/nanoquant/modules/linear.py:121-141 returns before :248-257 adds it); the default here mirrors that, and
 `kernel_path_bias = True` adds the bias in the epilogue of the last kernel.  Checked against the dense definition
 plus bias on every kernel that has such an epilogue: per-linear decode (lane-group kernel and 16-row pieces),
-run list (fp8-piece and 16-bit arithmetic), prefill (few-token kernel, unsplit blocks, k-split + finish kernel)."""
+run list (fp8-piece and 16-bit arithmetic), prefill (tiles whose wavefronts split k, and tiles that walk all of it)."""
 import numpy as np
 import pytest
 import torch
@@ -67,9 +67,9 @@ def test_run_list_bias(dev, batch):
     assert oracle.max_rel_err(y.float().cpu().numpy(), ref_bias) < 2e-3
 
 
-@pytest.mark.parametrize("tokens,m,n,r", [(64, 512, 512, 256), (160, 2048, 1024, 512), (512, 512, 4096, 2048)])
+@pytest.mark.parametrize("tokens,m,n,r", [(64, 512, 512, 256), (160, 2048, 1024, 512), (512, 512, 4096, 2048), (700, 4128, 512, 256)])
 def test_prefill_module_bias(dev, tokens, m, n, r):
-    # 64 tokens: few-token kernel; 160 x 2048: unsplit blocks; 512 tokens with few row tiles: k-split + finish kernel
+    # the second GEMM on 32 x 32, 32 x 64, 32 x 32 and 64 x 128 tiles
     mod, term, bias = _module(dev, m, n, r, 70, torch.float16)
     mod._prepare_kernel("gemm", torch.float16)
     x = oracle.synth_x(tokens, n, 71)

@@ -49,9 +49,9 @@ def test_config0_shape(dev, dtype, tokens):
     (256, 256, 32, 1),          # a single token, rank padded 32 -> 256
     (320, 512, 100, 77),        # ragged tokens, rows not a multiple of 128
     (128, 768, 256, 200),
-    (256, 4352, 256, 300),      # k of 17 tiles: few-token tiles beyond 256 tokens (wavefronts split k, no scratch)
-    (256, 4352, 256, 1100),     # the same above 1024 tokens: block tiles with a k-split
-    (384, 512, 1024, 640),      # 32-token blocks without k-split (few 64-token workgroups, short k)
+    (256, 4352, 256, 300),      # k of 17 tiles, few rows
+    (256, 4352, 256, 1100),     # the same on more tokens
+    (384, 512, 1024, 640),      # a short k, few rows
 ])
 def test_shapes_fp16(dev, m, n, r, tokens):
     err = _run_fused(dev, m, n, r, tokens, torch.float16, seed=m + r + tokens)
@@ -101,16 +101,14 @@ def test_tile_bit_exactness_single_minus_one(dev):
         assert np.array_equal(y, expect), (row, col)
 
 
-def test_k_split_matches_single_pass(dev):
-    # small row count forces a k-split (atomic fp32 partial sums); large row count does not
+def test_few_rows_of_a_long_k_and_many_of_a_short_one(dev):
     for (m, n, r) in [(128, 4096, 256), (4096, 512, 256)]:
         err = _run_fused(dev, m, n, r, 128, torch.float16, seed=m)
         assert err < TOL[torch.float16], (m, n, r, err)
 
 
-def test_graph_replay_of_the_split_k_path(dev):
-    # k-split partial sums live in a scratch that the finish kernel re-zeroes: replays of a captured call
-    # must equal the eager result every time (no memset nodes involved, the scratch is never cleared by the host)
+def test_graph_replay_of_a_prefill_call(dev):
+    # replays of a captured call must equal the eager result every time, with eager calls between them
     m, n, r, tokens = 512, 4096, 512, 300
     vt, u, s_in, s_mid, s_out = oracle.synth_term(m, n, r, 77)
     x = torch.from_numpy(oracle.synth_x(tokens, n, 78)).to(dev)
@@ -123,7 +121,7 @@ def test_graph_replay_of_the_split_k_path(dev):
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
-        op(x, *packed)                       # the side stream's scratch exists before the capture
+        op(x, *packed)                       # a warm-up on the side stream
     side.synchronize()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=side):

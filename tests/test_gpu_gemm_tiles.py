@@ -7,6 +7,7 @@ import torch
 
 from nanoquant_amd import ops, packing
 from oracle import nq_oracle as oracle
+from test_tile_choice import ALONE, sum_route, tile
 
 pytestmark = pytest.mark.gpu
 # half an ulp of the 16-bit result, and as much again for the h that feeds the second GEMM
@@ -25,20 +26,22 @@ def _onebit(dev, tokens, k, rows, dtype, scaled, seed):
     return x, bits, si, so, torch.zeros(max(words, 1), dtype=torch.int32, device=dev), (xs @ signs.double().T) * s_out.double()
 
 
-# (tokens, k, rows): 32 x 32 tiles up to 32 x 96 where k is split four ways (k tiles left over for none, one, three of the four
-# wavefronts), 64 x 128 to 128 x 256 where it is not
-@pytest.mark.parametrize("tokens,k,rows", [
-    (1, 256, 32), (31, 512, 64), (33, 1280, 96), (65, 2304, 160),              # 32 x 32: 1, 2, 5, 9 k tiles
-    (128, 4096, 3104), (200, 1792, 2080), (161, 2816, 3072),                   # 32 x 64, rows left over
-    (333, 4096, 3104), (250, 2048, 3136),                                      # 32 x 96, one and two row tiles left over
-    (333, 1024, 3168), (700, 256, 2080), (193, 2560, 8224),                    # 64 x 128
-    (400, 768, 16416), (1000, 1280, 4128),                                     # 64 x 256
-    (2049, 512, 12320), (4097, 256, 8224),                                     # 128 x 256
-    (352, 1024, 3168), (353, 1024, 3168), (2112, 512, 12320), (2113, 512, 12320),   # half a tile of tokens left, one more
+# (tokens, k, rows), the tile with and without input scales: 32 x 32 up to 32 x 96 split k four ways (k tiles left over for none, one,
+# three of the four wavefronts), 64 x 128 up to 128 x 256 do not
+@pytest.mark.parametrize("tokens,k,rows,tiles", [
+    (1, 256, 32, "32x32"), (31, 512, 64, "32x32"), (33, 1280, 96, "32x32"), (65, 2304, 160, "32x32"),      # 1, 2, 5, 9 k tiles
+    (128, 4096, 3104, "32x64"), (200, 1792, 2080, "32x64"), (250, 2048, 3136, "32x64"),      # a row tile left over, the same, none
+    (161, 2816, 3072, "32x96"), (200, 2816, 3104, "32x96"), (250, 2048, 2080, "32x96"),      # none, one and two row tiles left over
+    (333, 4096, 3104, "32x96 64x128"),
+    (333, 1024, 3168, "64x128"), (700, 256, 2080, "64x128"), (193, 2560, 8224, "64x128"), (4097, 256, 8224, "64x128"),
+    (400, 768, 16416, "64x256"), (250, 512, 8224, "64x256"), (2049, 2048, 4128, "64x256"),
+    (1000, 1280, 4128, "128x256"), (2049, 512, 12320, "128x256"),
+    (352, 1024, 3168, "64x128"), (353, 1024, 3168, "64x128"), (2112, 512, 12320, "128x256"), (2113, 512, 12320, "128x256"),   # half a tile of tokens left, one more
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("scaled", [True, False])
-def test_tiles_at_their_edges(dev, tokens, k, rows, dtype, scaled):
+def test_tiles_at_their_edges(dev, tokens, k, rows, tiles, dtype, scaled):
+    assert "%dx%d" % tile(ALONE, tokens, [k], [rows], scaled) == tiles.split()[0 if scaled else -1]
     x, bits, si, so, workspace, ref = _onebit(dev, tokens, k, rows, dtype, scaled, tokens + k)
     print(f"tile {tokens} tokens {k} -> {rows} {dtype} scaled={scaled}", flush=True)
     y = torch.ops.binary_kernels.marlin_onebit_forward(x, bits, si, so, workspace)
@@ -102,19 +105,22 @@ def test_other_tiles_for_many_rows_below_160_tokens(dev, tokens):
         assert oracle.max_rel_err(y.float().cpu().numpy(), ref) < 3 * ROUND[dtype]
 
 
-# Sums of terms: chains of 1 to 3 terms of uneven rank, ranks of one tile up to many, a bias on some terms; the sizes reach every
-# tile that sums (32 x 32, 32 x 64 and 32 x 96 with k split, 64 x 128, 64 x 256) with tokens and rows left over.
-@pytest.mark.parametrize("tokens,spec", [
-    (1, [(32, (200, 100)), (96, (512,))]),
-    (33, [(160, (256, 1280, 300)), (64, (100,)), (3104, (700, 256))]),
-    (200, [(3104, (512, 2304)), (2080, (256,))]),
-    (333, [(3104, (256, 256, 768)), (1056, (2048, 100))]),
-    (700, [(4128, (300, 100)), (2080, (256,))]),
-    (1000, [(8224, (256, 256))]),
-    (992, [(8224, (256, 256))]), (993, [(8224, (256, 256))]),
+# Sums of terms: chains of 1 to 3 terms of uneven rank, ranks of one tile up to many, a bias on some terms; every tile that sums
+# (32 x 32, 32 x 64 and 32 x 96 with k split, 64 x 128, 64 x 256) with tokens and rows left over.
+@pytest.mark.parametrize("tokens,spec,tiles", [
+    (1, [(32, (200, 100)), (96, (512,))], "32x32"),
+    (33, [(160, (256, 1280, 300)), (64, (100,)), (3104, (700, 256))], "32x32"),
+    (70, [(3104, (1280, 300))], "32x64"), (157, [(2080, (512, 300))], "32x64"),
+    (190, [(3104, (2304, 512))], "32x96"), (157, [(4128, (1280, 300))], "32x96"), (520, [(1056, (1280, 300))], "32x96"),
+    (200, [(3104, (512, 2304)), (2080, (256,))], "64x128"),
+    (333, [(3104, (256, 256, 768)), (1056, (2048, 100))], "64x128"),
+    (700, [(4128, (300, 100)), (2080, (256,))], "64x128"),
+    (1000, [(8224, (256, 256))], "64x128"),
+    (992, [(8224, (256, 256))], "64x128"), (993, [(8224, (256, 256))], "64x128"),
+    (157, [(8224, (1280, 512)), (8224, (1280, 512))], "64x256"), (1000, [(2080, (2304, 512))], "64x256"),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_sums_of_terms(dev, tokens, spec, dtype):
+def test_sums_of_terms(dev, tokens, spec, tiles, dtype):
     f = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
     host = lambda a: a.float().cpu().numpy()
     n = 512
@@ -132,6 +138,8 @@ def test_sums_of_terms(dev, tokens, spec, dtype):
         groups.append(packed)
         biases.append(own)
         refs.append(ref)
+    size, pays = sum_route(tokens, [[(n, v.size(0) * 16, v.size(1) * 2) for _, v, *_ in terms] for terms in groups])
+    assert "%dx%d" % size == tiles and pays
     print(f"sums {tokens} tokens {spec} {dtype}", flush=True)
     added, apart = ops.gemm_group_sum_forward(x, groups, biases), ops.gemm_group_sum_forward(x, groups, biases, panel="never")
     torch.cuda.synchronize()

@@ -3,7 +3,7 @@ import ctypes
 
 import pytest
 
-from nanoquant_amd import _lib
+from nanoquant_amd import _lib, ops
 
 ALONE, GROUP, ANY, SUM = range(4)
 
@@ -13,6 +13,18 @@ def tile(use, tokens, k, rows, scaled=False, nxt=None):
     ints = lambda a: None if a is None else (ctypes.c_int * len(a))(*a)
     size = _lib.lib().nq_gemm_tile_size(use, len(k), tokens, ints(k), ints(rows), int(scaled), ints(nxt))
     return (size >> 16, size & 0xFFFF) if size else None
+
+
+def sum_route(tokens, weights):
+    """Tile of the launch that sums the terms (n, r, m) of every weight, and whether gemm_group_sum_forward makes it."""
+    order = sorted(range(len(weights)), key=lambda w: -len(weights[w]))
+    flat = [(w, t) for t in range(len(weights[order[0]])) for w in order if t < len(weights[w])]      # as the call lists them
+    nxt = [flat.index((w, t + 1)) if (w, t + 1) in flat else -1 for w, t in flat]
+    sizes = [weights[w][t] for w, t in flat]
+    arr = (ops.NqGemmTerm * len(flat))(*[ops.NqGemmTerm(4096, 4096, 4096, 4096, None, None, None, 4096 * (i + 1), 16 * (i + 1), *s)
+                                         for i, s in enumerate(sizes)])      # addresses that nobody reads
+    pays = _lib.lib().nq_gemm_sum_pays(arr, (ctypes.c_int * len(flat))(*nxt), len(flat), tokens)
+    return tile(SUM, tokens, [r for _, r, _ in sizes], [m for _, _, m in sizes], nxt=nxt), pays == 1
 
 
 def test_sizes_that_are_refused():
