@@ -215,8 +215,9 @@ int nq_gemv_stage(const void* in, const void* s_col, const uint32_t* bits, const
  *   tiles: k*rows/32 words in the 32-row x 256-k tile layout of the package's prefill packer (the
  *   layout is private to packer and kernel, as the reference's Marlin layout is).
  *   Requires k % 256 == 0 and rows % 32 == 0 (else NQ_ERR_PROB_SHAPE, the reference's error class
- *   for shapes its tiles do not cover), and k < 2^30; more than 2^22 columns run token by token.  scratch: nq_gemm_scratch_bytes(tokens, k, rows) bytes of
- *   device memory; that is 0 for every shape (no kernel splits k between workgroups), so NULL will do. */
+ *   for shapes its tiles do not cover), and k < 2^30; more than 2^22 columns run token by token.
+ *   scratch: nq_gemm_scratch_bytes(tokens, k, rows) bytes of device memory; that is 0 for every shape (no kernel
+ *   splits k between workgroups), so NULL will do. */
 size_t nq_gemm_scratch_bytes(int tokens, int k, int rows);
 int nq_gemm_onebit(const void* x, const uint32_t* tiles, const void* s_in, const void* s_out, void* y,
                    void* scratch, size_t scratch_bytes, int tokens, int k, int rows, int dtype, void* stream);
@@ -245,8 +246,8 @@ int nq_gemm_nanoquant_bias(const void* x, const uint32_t* vt_tiles, const uint32
  * its terms, so above 160 tokens the last bits of a term's result may depend on what shares the call; up to 160 tokens they are
  * those of nq_gemm_nanoquant.  Only when some terms have s_in and others do not does the call run the terms one after another
  * (nq_gemm_nanoquant_bias).  scratch is not needed (NULL).
- * count <= nq_gemm_group_max(); h and y of different terms must not coincide.  No counterpart in the reference, which launches each linear by itself
- * (modules/linear.py:131-133). */
+ * count <= nq_gemm_group_max(); h and y of different terms must not coincide.  No counterpart in the reference, which
+ * launches each linear by itself (modules/linear.py:131-133). */
 typedef struct nq_gemm_term {
     const void* x;               /* [tokens, n] */
     const uint32_t* vt_tiles;    /* first stage, [r rows x n] in the prefill tile layout */
@@ -273,9 +274,9 @@ int nq_gemm_nanoquant_group(const nq_gemm_term* terms, int count, int tokens, in
  *   workgroups from which every launch derives its own flag value, so nothing is cleared between launches or graph
  *   replays).  It must not be `scratch` and launches that share it must not overlap in time.
  *   panel_mode: NQ_PANEL_AUTO picks per stage whatever is fastest (panels, or the tiles of nq_gemm_nanoquant_group, of which
- *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any token count (not where
- *   x, y or the signs of a term are 4 GiB or more, which its 32-bit offsets do not reach), NQ_PANEL_NEVER never takes it; with
- *   panel_ws NULL there is none in any mode.
+ *   launches of many rows may then take others up to 160 tokens too), NQ_PANEL_ALWAYS forces the panel launch for any
+ *   token count (not where x, y or the signs of a term are 4 GiB or more, which its 32-bit offsets do not reach),
+ *   NQ_PANEL_NEVER never takes it; with panel_ws NULL there is none in any mode.
  * A panel launch keeps two workgroups per compute unit resident and its workgroups wait for each other's partial
  * tiles: it may share the GPU with other kernels (its waits then last until those free their compute units), but a
  * wait that outlasts its bound (2^20 polls, about a second) invalidates the launch's outputs.
@@ -286,8 +287,8 @@ enum { NQ_PANEL_AUTO = 0, NQ_PANEL_ALWAYS = 1, NQ_PANEL_NEVER = 2 };
 size_t nq_gemm_panel_workspace_bytes(void);
 int nq_gemm_nanoquant_group_ws(const nq_gemm_term* terms, int count, int tokens, int dtype, void* scratch,
                                size_t scratch_bytes, void* panel_ws, size_t panel_ws_bytes, int panel_mode, void* stream);
-/* 1 when a stage of that call would be a panel launch (0 otherwise, for NQ_PANEL_NEVER and for sizes that it refuses), so that a caller can do without the
- * workspace until one is. */
+/* 1 when a stage of that call would be a panel launch (0 otherwise, for NQ_PANEL_NEVER and for sizes that it refuses),
+ * so that a caller can do without the workspace until one is. */
 int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, int panel_mode);
 /* Weights that are sums of terms, without a pass that adds: next[i] is the term behind term i of the same weight (-1: none;
  * next[i] > i, the same m), and the y of a weight's first term receives the sum, every term scaled and its bias added in 32 bits
@@ -295,7 +296,8 @@ int nq_gemm_group_wants_panel(const nq_gemm_term* terms, int count, int tokens, 
  * same workspace and mode; all terms have s_in or none has (NQ_ERR_SHAPE otherwise). */
 int nq_gemm_nanoquant_sum(const nq_gemm_term* terms, const int* next, int count, int tokens, int dtype, void* panel_ws,
                           size_t panel_ws_bytes, int panel_mode, void* stream);
-/* 1 when that call is estimated to take less than nq_gemm_nanoquant_group_ws and the additions (0 otherwise, for terms that it refuses and where nothing is summed). */
+/* 1 when that call is estimated to take less than nq_gemm_nanoquant_group_ws and the additions (0 otherwise, for terms
+ * that it refuses and where nothing is summed). */
 int nq_gemm_sum_pays(const nq_gemm_term* terms, const int* next, int count, int tokens);
 /* Tokens * 65536 + rows of the tiles that a launch of GEMMs on k[i] columns and rows[i] rows is cut into (0: refused sizes), for
  * tests and for tuning: of one linear by itself, of a group in which it keeps the bits that it has there up to 160 tokens

@@ -49,7 +49,8 @@ constexpr int kFewWavesFrom = 8192;  // rows of a linear
 // Up to this many staged rows the input operands are read two steps ahead of their products (left to itself the compiler waits
 // for every pair of reads; with more rows the workgroups that share a compute unit hide that, and the registers count): layer of
 // four groups, stages repeated, 1 / 4 / 11 rows fp16: 35.6 / 39.0 / 49.1 us without, 34.3 / 38.6 / 50.6 with; four or eight steps
-// ahead 34.7 / 39.3 / 50.9 and 35.6 / 42.0 / 52.2.
+// ahead 34.7 / 39.3 / 50.9 and 35.6 / 42.0 / 52.2.  At 5 and 8 rows the two are within 1 % (four groups of two launches: fp16 42.4 and
+// 42.9 us without, 42.3 and 42.9 with, bf16 43.3 and 43.8, 43.1 and 43.8; linears by themselves in bf16 64.4 and 65.3, 63.9 and 64.9).
 constexpr int kReadAheadRows = 4;
 constexpr int kStagePitch = 1040;    // LDS bytes per staged input row of a chunk: 512 x 2 + 16 (8 lanes of an operand
                                      // read that differ in the batch row only hit 8 different bank groups)

@@ -402,8 +402,9 @@ def gemm_group_forward(xs, terms, biases=None, outs=None, panel="auto"):
     `biases` an optional list of [m] tensors / None; `outs` an optional list of contiguous [tokens, m] tensors of
     the activation type to write into (allocated here when absent); `panel` ("auto", "always", "never") says whether
     the stages may run as persistent panel launches and, up to 160 tokens, on tiles other than the ones a linear gets by
-    itself (see include/nq_gfx950.h); in a graph capture they do only if a call on that stream did before.  Returns the list of outputs.  The terms share launches: a single linear leaves most
-    of the device idle up to some hundred tokens.  The reference launches every linear by itself
+    itself (see include/nq_gfx950.h); in a graph capture they do only if a call on that stream did before.  Returns the
+    list of outputs.  The terms share launches: a single linear leaves most of the device idle up to some hundred
+    tokens.  The reference launches every linear by itself
     (modules/linear.py:131-133)."""
     if isinstance(xs, torch.Tensor):
         xs = [xs] * len(terms)
