@@ -583,12 +583,14 @@ static double panel_time(int count, int T, const int* K, const int* R, bool scal
     return 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
 }
 
-// How far below the tiles' estimate a panel launch must be.  Problems of different k are the weak side of both estimates.  Over 258
-// stages of such groups (100 to 2048 tokens, of one layer's linears at 0.7 and 1 bit) the slower form was taken for 0.9 % of both
-// stages' time where some k is long (more than 16 tiles; 1.7 % at 0.85), for 0.1 % elsewhere (1.2 % at 1): {o, down} of Qwen3-8B on 1280
-// tokens, first stage 4096 and 12288, 195 us on tiles, 167 on panels; second stages of k 1024 to 3072 on 1536 tokens 501 / 527.
-// For one k 0.95 loses 0.2 %, 0.85 0.5, 1 0.3 (290 stages).
-static double panel_margin(int count, const int* K) {
+// Whether panels are taken, and the estimate of what is.  Problems of different k are the weak side of both estimates: with a long k
+// among them (more than 16 tiles) panels are compared with 1.05 of the tiles' estimate, and half of what a panel launch takes beyond
+// 120 us comes on top; otherwise panels must be below 0.85 of it, for one k 0.95.  us of both stages, first stage on tiles / on panels:
+// {o, down} of Qwen3-8B (4096 and 12288) on 1280 tokens 193 / 170, {q, k, v, down} on 1024 180 / 158; all seven linears of Llama-2-7B on
+// 256 tokens 119 / 111, on 1024 347 / 357, on 2048 645 / 684.  What the slower form costs, of both stages' time, over 530 stages with a
+// long k (groups of 2 to 7 linears of two models, 0.55 to 1 bit, 128 to 2048 tokens): this 0.6 %, 1.0 of the tiles' estimate
+// 1.1, 0.95 1.1, 0.85 2.2, tiles alone 3.0.  Over 477 others of mixed k 0.85 0.2 %, 0.95 1.1; over 389 of one k 0.95 0.4, 1 0.6.
+bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
     constexpr int kLongK = 16 * kTileK;
     bool mixed = false;
     int longest = 0;
@@ -596,12 +598,13 @@ static double panel_margin(int count, const int* K) {
         mixed = mixed || K[p] != K[0];
         longest = longest > K[p] ? longest : K[p];
     }
-    return !mixed ? 0.95 : longest > kLongK ? 1.0 : 0.85;
-}
-
-bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
-    const double panels = panel_time(count, T, K, R, scaled), tiles = gemm_tiles_time(count, x, T, K, R, scaled);
-    const bool take = panels < panel_margin(count, K) * tiles;
+    double panels = panel_time(count, T, K, R, scaled), margin = mixed ? 0.85 : 0.95;
+    if (mixed && longest > kLongK) {
+        margin = 1.05;
+        if (panels > 120.0) panels += 0.5 * (panels - 120.0);
+    }
+    const double tiles = gemm_tiles_time(count, x, T, K, R, scaled);
+    const bool take = panels < margin * tiles;
     if (time) *time = take ? panels : tiles;
     return take;
 }

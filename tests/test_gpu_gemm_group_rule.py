@@ -134,6 +134,8 @@ def test_sums_are_compared_with_the_launch_that_would_be_made(dev, tokens, weigh
     (640, [(4096, 2048, 4096), (12288, 3072, 4096)], 1),       # 115 / 103 / 117
     (640, [(4096, 1536, 4096), (11008, 2304, 4096)], 1),       # 90 / 85 / 94
     (1536, [(1024, 2048, 4096), (1024, 3072, 12288), (1024, 3072, 12288)], 0),      # k of 8 and 12 tiles: tiles ahead by 5 %
+    (256, [(4096, 2048, 4096)] * 4 + [(4096, 3072, 11008)] * 2 + [(11008, 3072, 4096)], 1),      # 119 / 111
+    (1024, [(4096, 2048, 4096)] * 4 + [(4096, 3072, 11008)] * 2 + [(11008, 3072, 4096)], 0),     # 347 / 357
 ])
 def test_panels_beside_tiles_where_k_differs(dev, tokens, linears, panel):
     from nanoquant_amd import _lib
