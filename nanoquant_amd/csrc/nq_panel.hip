@@ -564,7 +564,8 @@ bool panel_addresses(int count, int T, const int* K, const int* R) {
 // + 1 for every workgroup that a panel is shared by: the middle 90 % of 445 launches are within -8 .. +8 % of that (128 to 2048
 // tokens, 1 to 43 k tiles, 512 to 22016 rows); with fewer than three k steps the hand-over takes most of the time (128
 // tokens, 3072 -> 4096 rows: tiles 7, panels 35).
-static double panel_time(int count, int T, const int* K, const int* R, bool scaled) {
+// *shared: workgroups to the longest of the panels.
+static double panel_time(int count, int T, const int* K, const int* R, bool scaled, double* shared) {
     constexpr double kNever = 1e30;
     constexpr int kMostTokens = 2048;            // of the launches that were timed
     const int G = panel_grid();
@@ -578,18 +579,21 @@ static double panel_time(int count, int T, const int* K, const int* R, bool scal
         longest = longest > K[p] / kTileK ? longest : K[p] / kTileK;
     }
     const double per_wg = (double)units / G;
+    *shared = longest / per_wg;
     if (per_wg < 3.0) return kNever;
     const double steps = (double)((units + G - 1) / G);
-    return 12.4 + 3.08 * steps + 1.0 * longest / per_wg + (scaled ? 1.35 + 0.25 * steps : 0.0);
+    return 12.4 + 3.08 * steps + 1.0 * *shared + (scaled ? 1.35 + 0.25 * steps : 0.0);
 }
 
 // Whether panels are taken, and the estimate of what is.  Problems of different k are the weak side of both estimates: with a long k
 // among them (more than 16 tiles) panels are compared with 1.05 of the tiles' estimate, and half of what a panel launch takes beyond
-// 120 us comes on top; otherwise panels must be below 0.85 of it, for one k 0.95.  us of both stages, first stage on tiles / on panels:
-// {o, down} of Qwen3-8B (4096 and 12288) on 1280 tokens 193 / 170, {q, k, v, down} on 1024 180 / 158; all seven linears of Llama-2-7B on
-// 256 tokens 119 / 111, on 1024 347 / 357, on 2048 645 / 684.  What the slower form costs, of both stages' time, over 530 stages with a
-// long k (groups of 2 to 7 linears of two models, 0.55 to 1 bit, 128 to 2048 tokens): this 0.6 %, 1.0 of the tiles' estimate
-// 1.1, 0.95 1.1, 0.85 2.2, tiles alone 3.0.  Over 477 others of mixed k 0.85 0.2 %, 0.95 1.1; over 389 of one k 0.95 0.4, 1 0.6.
+// 120 us comes on top; otherwise, and where more than 12 workgroups share a panel, panels must be below 0.85 of it, for one k 0.95.
+// us of both stages, first stage on tiles / on panels: {o, down} of Qwen3-8B (4096 and 12288) on 1280 tokens 193 / 170, {q, k, v, down} on
+// 1024 180 / 158; all seven linears of Llama-2-7B on 256 tokens 119 / 111, on 1024 347 / 357, on 2048 645 / 684; 16 workgroups to a panel:
+// {q, k, v, down} of Llama-3-70B on 40 tokens 51 / 67.  What the slower form costs, of both stages' time, over 782 stages with a long k
+// (groups of 2 to 7 linears of three models, 0.55 to 1 bit, 33 to 2048 tokens): this 0.5 %, 1.0 of the tiles' estimate 1.0, 0.95
+// 1.1, 0.85 1.9, tiles alone 3.1.  Over 608 others of mixed k 0.85 0.2 %, 0.95 1.0, tiles alone 0.3; over 652 of one k 0.95 0.4, 1 0.6,
+// tiles alone 0.9.
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
     constexpr int kLongK = 16 * kTileK;
     bool mixed = false;
@@ -598,8 +602,8 @@ bool panel_applies(int count, const void* const* x, int T, const int* K, const i
         mixed = mixed || K[p] != K[0];
         longest = longest > K[p] ? longest : K[p];
     }
-    double panels = panel_time(count, T, K, R, scaled), margin = mixed ? 0.85 : 0.95;
-    if (mixed && longest > kLongK) {
+    double shared = 0, panels = panel_time(count, T, K, R, scaled, &shared), margin = mixed ? 0.85 : 0.95;
+    if (mixed && longest > kLongK && shared <= 12.0) {
         margin = 1.05;
         if (panels > 120.0) panels += 0.5 * (panels - 120.0);
     }
