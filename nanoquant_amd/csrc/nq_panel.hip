@@ -587,13 +587,14 @@ static double panel_time(int count, int T, const int* K, const int* R, bool scal
 
 // Whether panels are taken, and the estimate of what is.  Problems of different k are the weak side of both estimates: with a long k
 // among them (more than 16 tiles) panels are compared with 1.05 of the tiles' estimate, and half of what a panel launch takes beyond
-// 120 us comes on top; otherwise, and where more than 12 workgroups share a panel, panels must be below 0.85 of it, for one k 0.95.
+// 120 us comes on top; otherwise panels must be below 0.85 of it, for one k 0.95.  0.85 also holds where more than 12 workgroups share
+// a panel, and where fewer than two do and most products have another k (tiles then fill in behind the long ones).
 // us of both stages, first stage on tiles / on panels: {o, down} of Qwen3-8B (4096 and 12288) on 1280 tokens 193 / 170, {q, k, v, down} on
-// 1024 180 / 158; all seven linears of Llama-2-7B on 256 tokens 119 / 111, on 1024 347 / 357, on 2048 645 / 684; 16 workgroups to a panel:
-// {q, k, v, down} of Llama-3-70B on 40 tokens 51 / 67.  What the slower form costs, of both stages' time, over 782 stages with a long k
-// (groups of 2 to 7 linears of three models, 0.55 to 1 bit, 33 to 2048 tokens): this 0.5 %, 1.0 of the tiles' estimate 1.0, 0.95
-// 1.1, 0.85 1.9, tiles alone 3.1.  Over 608 others of mixed k 0.85 0.2 %, 0.95 1.0, tiles alone 0.3; over 652 of one k 0.95 0.4, 1 0.6,
-// tiles alone 0.9.
+// 1024 180 / 158; all seven linears of Llama-2-7B on 256 tokens 115 / 110, on 512 189 / 193, on 768 264 / 272; 16 workgroups to a
+// panel: {q, k, v, down} of Llama-3-70B on 40 tokens 51 / 67.  What the slower form costs, of both stages' time, over 782 stages with a
+// long k (groups of 2 to 7 linears of three models, 0.55 to 1 bit, 33 to 2048 tokens, the device kept busy): this 0.4 %, 1.0 of the
+// tiles' estimate 0.9, 0.95 0.9, 0.85 1.8, tiles alone 3.0.  Over 608 others of mixed k 0.85 0.3 %, 0.95 1.0, tiles alone 0.4; over 652 of
+// one k 0.95 0.4, 1 0.6, tiles alone 1.0.
 bool panel_applies(int count, const void* const* x, int T, const int* K, const int* R, bool scaled, double* time) {
     constexpr int kLongK = 16 * kTileK;
     bool mixed = false;
@@ -604,8 +605,16 @@ bool panel_applies(int count, const void* const* x, int T, const int* K, const i
     }
     double shared = 0, panels = panel_time(count, T, K, R, scaled, &shared), margin = mixed ? 0.85 : 0.95;
     if (mixed && longest > kLongK && shared <= 12.0) {
-        margin = 1.05;
-        if (panels > 120.0) panels += 0.5 * (panels - 120.0);
+        double all = 0, own = 0;                 // products, those of the longest k
+        for (int p = 0; p < count; ++p) {
+            const double n = (double)K[p] * R[p];
+            all += n;
+            own += K[p] == longest ? n : 0.0;
+        }
+        if (shared >= 2.0 || own >= 0.5 * all) {
+            margin = 1.05;
+            if (panels > 120.0) panels += 0.5 * (panels - 120.0);
+        }
     }
     const double tiles = gemm_tiles_time(count, x, T, K, R, scaled);
     const bool take = panels < margin * tiles;

@@ -135,6 +135,7 @@ def test_sums_are_compared_with_the_launch_that_would_be_made(dev, tokens, weigh
     (640, [(4096, 1536, 4096), (11008, 2304, 4096)], 1),       # 90 / 85 / 94
     (1536, [(1024, 2048, 4096), (1024, 3072, 12288), (1024, 3072, 12288)], 0),      # k of 8 and 12 tiles: tiles ahead by 5 %
     (256, [(4096, 2048, 4096)] * 4 + [(4096, 3072, 11008)] * 2 + [(11008, 3072, 4096)], 1),      # 119 / 111
+    (768, [(4096, 2048, 4096)] * 4 + [(4096, 3072, 11008)] * 2 + [(11008, 3072, 4096)], 0),      # 264 / 272
     (1024, [(4096, 2048, 4096)] * 4 + [(4096, 3072, 11008)] * 2 + [(11008, 3072, 4096)], 0),     # 347 / 357
     (40, [(8192, 4096, 8192), (8192, 1024, 1024), (8192, 1024, 1024), (28672, 6400, 8192)], 0),     # 16 workgroups to a panel: 51 / 67
     (99, [(8192, 2560, 8192), (28672, 3840, 8192)], 0),        # 60 / 76
